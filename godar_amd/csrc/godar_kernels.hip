@@ -115,6 +115,37 @@ __device__ __forceinline__ int queue_slot_it(int qn, int it) {
     const int t = (int)(blockIdx.x % XCD_COUNT) * per + local;
     return t < qn ? t : -1;
 }
+// Entries of a queue of length qn taken by this wavefront when a wavefront
+// evaluates its floes' pairs together: `floes` consecutive entries of its
+// XCD's share at begin, begin + stride, ... below end.  Just enough floes for
+// one full pass of 64 pairs (by the mean superset length of the last build),
+// more only if the queue has more for every wavefront of the grid: with 64
+// floes of tens of candidates each, a wavefront works through all their pairs
+// one pass after the other while the rest of the GPU has nothing to do (one
+// MI355X, contact kernel: 320,000 floes in 24 members with about 43
+// candidates a floe, 2,100 of them queued, 0.45 -> 0.03 ms), while one floe
+// of two pairs per wavefront only spreads the same chain over more compute
+// units (2,501 floes, 130 queued: 0.029 ms with full passes, 0.037 without).
+// Queues with more than 16 floes for every wavefront keep 64: all wavefronts
+// are busy then, and full passes count for more (the 512-field ensemble's
+// 157,000 queued floes lost 0.03 ms per step with 39).
+struct QueueShare { int begin, end, stride, floes; };
+__device__ __forceinline__ QueueShare queue_share(const DS& S, int qn) {
+    const int per = (qn + XCD_COUNT - 1) / XCD_COUNT;
+    const int wpb = (int)(blockDim.x >> 6);
+    const int nw = (int)(gridDim.x / XCD_COUNT) * wpb;
+    const int w = (int)(blockIdx.x / XCD_COUNT) * wpb + (int)(threadIdx.x >> 6);
+    const int lo = (int)(blockIdx.x % XCD_COUNT) * per;
+    QueueShare q;
+    const int f = (per + nw - 1) / nw;
+    const int64_t entries = S.sblk[(S.N + SCAN_TILE - 1) / SCAN_TILE];   // supersets together
+    const int full = (int)min((int64_t)64, 64 * (int64_t)S.N / max(entries, (int64_t)1));
+    q.floes = f > 16 ? 64 : max(1, max(f, full));
+    q.begin = lo + w * q.floes;
+    q.end = min(qn, lo + per);
+    q.stride = nw * q.floes;
+    return q;
+}
 // the queue entry of this thread (split over the XCDs as queue_slot), or -1
 __device__ __forceinline__ int queue_entry(const DS& S, int c) {
     const QueueView v = queue_view(S, c);
@@ -1795,12 +1826,12 @@ __global__ __launch_bounds__(FLOE_BLOCK, MIXED ? 2 : 3) void k_contact(DS S) {
     if (*S.err) return;
     const int lane = (int)(threadIdx.x & 63);
     const QueueView qv = queue_view(S, 0);
-    // (the wavefront loops while any lane has an entry: its lanes share LDS
-    // and shuffles)
-    for (int it = 0;; ++it) {
-        const int qt = queue_slot_it(qv.total, it);
-        if (__ballot(qt >= 0) == 0) break;
-        const int k = qt >= 0 ? queue_at(S, 0, qv, qt) : -1;
+    // (the wavefront's lanes share LDS and shuffles: every lane runs each
+    // round, whether or not it has an entry)
+    const QueueShare qs = queue_share(S, qv.total);
+    for (int t0 = qs.begin; t0 < qs.end; t0 += qs.stride) {
+        const int qt = t0 + lane;
+        const int k = lane < qs.floes && qt < qs.end ? queue_at(S, 0, qv, qt) : -1;
         const bool act = k >= 0;
         const int64_t SS = S.S;
         int m = 0, f = 0, fs = 0, ni = 0, no = 0;
