@@ -25,13 +25,11 @@ __global__ void k_scan_total(DS, int);
 __global__ void k_scan_offsets(DS);
 template <bool M> __global__ void k_cand_dense(DS);
 template <bool M> __global__ void k_cand_dense_over(DS);
-__global__ void k_comp(DS);
 template <bool M> __global__ void k_contact(DS);
 template <bool M> __global__ void k_bond(DS);
 __global__ void k_stress(DS);
 template <bool M> __global__ void k_walls(DS);
 template <bool M> __global__ void k_repair(DS, int);
-__global__ void k_fixq(DS);
 template <bool M> __global__ void k_fixup(DS);
 template <bool M, bool R> __global__ void k_final(DS);
 __global__ void k_totals(DS, int64_t*);
@@ -107,7 +105,7 @@ struct godar_ctx {
     int64_t S = 0;
     int Mcap = 0;
     int CO = 32, CI = 32, HC = 16, BC = 16;
-    int SEEDK = 2, HEAPK = 16, TABK = 4;
+    int SEEDK = 2, HEAPK = 8;
     int block = 256;
     int sblock[GODAR_NSTAGES];          // threads per block of each stage's per-floe kernels
     int record = 0;
@@ -236,7 +234,6 @@ struct PairLists {
     double* od = nullptr;
     int64_t* ik = nullptr;
     uint32_t* evf = nullptr;
-    int32_t* ov = nullptr;
     BondTerms* bterm = nullptr;
     double *ssc = nullptr, *ssb = nullptr;
     int32_t* ibond = nullptr;
@@ -245,7 +242,7 @@ struct PairLists {
 };
 
 void free_lists(PairLists& L) {
-    dfree(L.oj); dfree(L.od); dfree(L.ik); dfree(L.evf); dfree(L.ov); dfree(L.bterm);
+    dfree(L.oj); dfree(L.od); dfree(L.ik); dfree(L.evf); dfree(L.bterm);
     dfree(L.ssc); dfree(L.ssb); dfree(L.ibond);
     for (int k = 0; k < 2; ++k) { dfree(L.hist[k]); dfree(L.bond[k]); }
 }
@@ -255,7 +252,7 @@ hipError_t alloc_lists(PairLists& L, int64_t S, int CO, int CI, int HC, int BC) 
     hipError_t e = hipSuccess;
     auto ok = [&](hipError_t x) { e = x; return x == hipSuccess; };
     bool good = ok(dalloc(&L.oj, S * CO)) && ok(dalloc(&L.od, S * CO)) && ok(dalloc(&L.ik, S * CI)) &&
-                ok(dalloc(&L.evf, S * CO)) && ok(dalloc(&L.ov, S * CO)) &&
+                ok(dalloc(&L.evf, S * CO)) &&
                 ok(dalloc(&L.bterm, S * BC)) && ok(dalloc(&L.ssc, S * CO)) &&
                 ok(dalloc(&L.ibond, S * CI)) && ok(dalloc(&L.ssb, S * CO));
     for (int k = 0; good && k < 2; ++k)
@@ -267,7 +264,7 @@ hipError_t alloc_lists(PairLists& L, int64_t S, int CO, int CI, int HC, int BC) 
 PairLists lists_of(const godar_ctx* c) {
     const DS& d = c->d;
     PairLists L;
-    L.oj = d.oj; L.od = d.od; L.ik = d.ik; L.evf = d.evf; L.ov = d.ov; L.bterm = d.bterm;
+    L.oj = d.oj; L.od = d.od; L.ik = d.ik; L.evf = d.evf; L.bterm = d.bterm;
     L.ssc = d.ssc; L.ssb = d.ssb; L.ibond = d.ibond;
     for (int k = 0; k < 2; ++k) { L.hist[k] = c->hist[k]; L.bond[k] = c->bond[k]; }
     return L;
@@ -275,7 +272,7 @@ PairLists lists_of(const godar_ctx* c) {
 
 void set_lists(godar_ctx* c, const PairLists& L) {
     DS& d = c->d;
-    d.oj = L.oj; d.od = L.od; d.ik = L.ik; d.evf = L.evf; d.ov = L.ov; d.bterm = L.bterm;
+    d.oj = L.oj; d.od = L.od; d.ik = L.ik; d.evf = L.evf; d.bterm = L.bterm;
     d.ssc = L.ssc; d.ssb = L.ssb; d.ibond = L.ibond;
     for (int k = 0; k < 2; ++k) { c->hist[k] = L.hist[k]; c->bond[k] = L.bond[k]; }
 }
@@ -311,7 +308,7 @@ void sync_ds(godar_ctx* c) {
     DS& d = c->d;
     d.S = c->S; d.N = c->N_used;
     d.CO = c->CO; d.CI = c->CI; d.HC = c->HC; d.BC = c->BC;
-    d.SEEDK = c->SEEDK; d.HEAPK = c->HEAPK; d.TABK = c->TABK;
+    d.SEEDK = c->SEEDK; d.HEAPK = c->HEAPK;
     d.record_forces = c->record;
     d.ncells = c->ncells_cap;
     d.qseg = qseg_of(c);   // XCD share of the candidate search (k_cand's grid, XCD-aware order)
@@ -575,16 +572,12 @@ int launch_step(godar_ctx* c, bool lean) {
     }
     {
         StageTimer t(c, 8);
-        // contact components (roots), then the ordered repair
-        hipLaunchKernelGGL(k_comp, grid_queue(N, FLOE_BLOCK), dim3(FLOE_BLOCK), 0, s, d);
-        hipLaunchKernelGGL(mixed ? k_repair<true> : k_repair<false>, dim3(nm), dim3(64), 0, s, d, nm);
+        hipLaunchKernelGGL(mixed ? k_repair<true> : k_repair<false>, dim3(nm), dim3(REPAIR_THREADS),
+                           0, s, d, nm);
     }
     {
         StageTimer t(c, 9);
-        // the touched floes into the fixup queue (laid out as the candidate
-        // search's grid, so that a wavefront's positions lie in one XCD
-        // share), then a few of them per wavefront
-        hipLaunchKernelGGL(k_fixq, grid_for(N, B[3], true), dim3(B[3]), 0, s, d);
+        // the floes the repair queued, a few of them per wavefront
         const int fb = std::max(XCD_COUNT, FIXUP_GRID_WAVES * 64 / B[9] / XCD_COUNT * XCD_COUNT);
         hipLaunchKernelGGL(mixed ? k_fixup<true> : k_fixup<false>, dim3(fb),
                            dim3(B[9]), (B[9] / 64) * FIX_LDS_PER_WAVE, s, d);
@@ -775,22 +768,17 @@ int godar_create(int64_t max_floes, int32_t max_members, int32_t precision, goda
     }
     ACHK(dalloc(&d.acc, (int64_t)NACC * S));
     ACHK(dalloc(&d.wout, S));
-    ACHK(dalloc(&d.wflag, (S + 3) / 4 * 4));   // whole 32-bit words (wflag_set)
+    ACHK(dalloc(&d.wflag, (S + 3) / 4 * 4));   // whole 32-bit words (set by word atomics)
     ACHK(dalloc(&d.cls, S));
     ACHK(dalloc(&d.qlist, (int64_t)NQUEUE * S));
     ACHK(dalloc(&d.bgat, S));
     ACHK(dalloc(&d.qn, (int64_t)NQUEUE * XCD_COUNT * QN_STRIDE));
-    ACHK(dalloc(&d.seeds, (int64_t)c->SEEDK * S));
+    ACHK(dalloc(&d.shape, (int64_t)c->SEEDK * S));
+    ACHK(dalloc(&d.rhead, S));
     ACHK(dalloc(&d.nseeds, max_members));
     ACHK(dalloc(&d.heap, (int64_t)c->HEAPK * S));
-    ACHK(dalloc(&d.etab, (int64_t)c->TABK * S));
-    ACHK(dalloc(&d.netab, max_members));
-    ACHK(dalloc(&d.wtab, S));
-    ACHK(dalloc(&d.nwtab, max_members));
-    ACHK(dalloc(&d.ovw, S));
-    ACHK(dalloc(&d.cur, 7 * S));
-    ACHK(dalloc(&d.dirty, (S + 3) / 4 * 4));   // whole 32-bit words (dirty_set)
-    ACHK(dalloc(&d.comp, S));
+    ACHK(dalloc(&d.cur, 6 * S));
+    ACHK(dalloc(&d.dirty, (S + 3) / 4 * 4));
     ACHK(dalloc(&d.wnz, S));
     ACHK(dalloc(&d.stats, 4 * (int64_t)max_members));
     ACHK(dalloc(&d.tcur, max_members));
@@ -851,8 +839,8 @@ int godar_destroy(godar_ctx* c) {
         free_lists(L);
         set_lists(c, L);
     }
-    dfree(d.wout); dfree(d.wflag); dfree(d.cls); dfree(d.qlist); dfree(d.qn); dfree(d.bgat); dfree(d.seeds); dfree(d.nseeds); dfree(d.heap); dfree(d.etab);
-    dfree(d.netab); dfree(d.wtab); dfree(d.nwtab); dfree(d.ovw); dfree(d.dirty); dfree(d.comp);
+    dfree(d.wout); dfree(d.wflag); dfree(d.cls); dfree(d.qlist); dfree(d.qn); dfree(d.bgat); dfree(d.shape); dfree(d.rhead); dfree(d.nseeds); dfree(d.heap);
+    dfree(d.dirty);
     dfree(d.wnz); dfree(d.stats); dfree(d.tcur); dfree(d.err); dfree(d.steps_done);
     dfree(d.sup); dfree(d.scnt); dfree(d.sout); dfree(d.soff); dfree(d.sblk); dfree(d.x0); dfree(d.rebuild);
     radix_free(c->rs);
@@ -876,12 +864,12 @@ static int64_t bytes_per_floe(const godar_ctx* c) {
     per += sizeof(FloeRec) + sizeof(GeoRec) + sizeof(ShelRec) + sizeof(KinRec);
     per += 4 + 4 /*pos_of, pos_id*/ + 4 * 8 /*wbc*/ + 4 /*member_of*/ + 4 + 4 /*ckey, cval*/;
     per += 4 + 4 /*ocnt, icnt*/ + 2 * (4 + 4) /*hcnt, bcnt*/;
-    per += (int64_t)c->CO * (8 + 8 + 4 + 4 + 8 + 8) + (int64_t)c->CI * (8 + 4);   // oj od evf ov ssc ssb; ik ibond
+    per += (int64_t)c->CO * (8 + 8 + 4 + 8 + 8) + (int64_t)c->CI * (8 + 4);   // oj od evf ssc ssb; ik ibond
     per += 2 * ((int64_t)c->HC * sizeof(HistRec) + (int64_t)c->BC * sizeof(BondRec));
     per += (int64_t)c->BC * sizeof(BondTerms) + 1 /*bgat*/;
     per += NACC * 8 + sizeof(WallOut) + 1 /*wflag*/ + 1 /*cls*/ + NQUEUE * 4 /*qlist*/;
-    per += (int64_t)c->SEEDK * 8 + (int64_t)c->HEAPK * 8 + (int64_t)c->TABK * sizeof(EventOut);
-    per += sizeof(WallOut) /*wtab*/ + 4 /*ovw*/ + 7 * 8 /*cur*/ + 1 + 1 /*dirty, wnz*/ + 4 /*comp*/;
+    per += (int64_t)c->SEEDK * sizeof(Reshape) + 4 /*rhead*/ + (int64_t)c->HEAPK * 8;
+    per += 6 * 8 /*cur*/ + 1 + 1 /*dirty, wnz*/;
     per += 33 * 8 /*fout*/ + 4 + 4 /*radix keys, values*/;
     per += (c->S > 0 ? c->sup_cap / c->S : 0) * 8 /*superset pool share*/ + 4 + 4 + 8 + 16 /*scnt sout soff x0*/;
     per += 1 /*sblk, per SCAN_TILE floes*/;
@@ -1509,7 +1497,6 @@ int godar_reserve(godar_ctx* c, int32_t outer, int32_t inner, int32_t histc, int
     bool good = ok(rows(nl.oj, ol.oj, sizeof(int64_t), c->CO, nCO)) &&
                 ok(rows(nl.od, ol.od, sizeof(double), c->CO, nCO)) &&
                 ok(rows(nl.evf, ol.evf, sizeof(uint32_t), c->CO, nCO)) &&
-                ok(rows(nl.ov, ol.ov, sizeof(int32_t), c->CO, nCO)) &&
                 ok(rows(nl.ssc, ol.ssc, sizeof(double), c->CO, nCO)) &&
                 ok(rows(nl.ssb, ol.ssb, sizeof(double), c->CO, nCO)) &&
                 ok(rows(nl.ik, ol.ik, sizeof(int64_t), c->CI, nCI)) &&
@@ -1862,18 +1849,17 @@ static bool grow_for(godar_ctx* c, uint32_t bits) {
         if (c->HEAPK >= 1024) return false;
         if (hipStreamSynchronize(c->stream) != hipSuccess) return false;
         // the larger pools first: on failure the current ones stay
-        uint64_t *seeds = nullptr, *heap = nullptr;
-        EventOut* etab = nullptr;
-        if (dalloc(&seeds, (int64_t)2 * c->SEEDK * c->S) != hipSuccess ||
-            dalloc(&heap, (int64_t)2 * c->HEAPK * c->S) != hipSuccess ||
-            dalloc(&etab, (int64_t)2 * c->TABK * c->S) != hipSuccess) {
-            dfree(seeds); dfree(heap); dfree(etab);
+        uint64_t* heap = nullptr;
+        Reshape* shape = nullptr;
+        if (dalloc(&shape, (int64_t)2 * c->SEEDK * c->S) != hipSuccess ||
+            dalloc(&heap, (int64_t)2 * c->HEAPK * c->S) != hipSuccess) {
+            dfree(shape); dfree(heap);
             (void)hipGetLastError();
             return false;
         }
-        dfree(c->d.seeds); dfree(c->d.heap); dfree(c->d.etab);
-        c->d.seeds = seeds; c->d.heap = heap; c->d.etab = etab;
-        c->SEEDK *= 2; c->HEAPK *= 2; c->TABK *= 2;
+        dfree(c->d.shape); dfree(c->d.heap);
+        c->d.shape = shape; c->d.heap = heap;
+        c->SEEDK *= 2; c->HEAPK *= 2;
         grew = true;
     }
     if (bits & ERR_SUP_CAP) {

@@ -50,13 +50,9 @@ struct ShelRec { double hfa, hfw, wx, wy; };
 struct KinRec { double u, v, omega, h, mass, inertia, theta; };
 
 // Per-position step flags (wflag): the floe touched a wall this step (wout
-// holds its terms); the repair recomputed its walls (wtab entry in ovw); the
-// repair touched the floe, so k_fixup re-gathers it.
-constexpr uint32_t WF_WALL = 1, WF_REPAIR_WALL = 2, WF_FIXUP = 4;
-// dirty bits (by storage slot, during the repair): the floe was reshaped (cur
-// rows 0-5 hold its properties); its iteration's query radius is kept (cur
-// row 6).  k_final clears them.
-constexpr uint32_t DIRTY_SHAPE = 1, DIRTY_RQ = 2;
+// holds its terms); its wall event is on the repair's list; the repair
+// touched the floe, so k_fixup re-gathers it.
+constexpr uint32_t WF_WALL = 1, WF_PENDING = 2, WF_FIXUP = 4;
 
 // Everything the kernels touch.  "id" arrays are indexed by a floe's storage
 // slot; "pos" arrays by the floe's position in this step's cell order.  Per-floe lists
@@ -65,12 +61,13 @@ struct DS {
     int64_t S;                 // floe capacity = stride of slot-major arrays
     int32_t N;                 // floe slots in use [0, N)
     int32_t CO, CI, HC, BC;    // outer / inner / history / bond list capacities
-    int32_t SEEDK, HEAPK, TABK;  // repair pool entries per floe slot
+    int32_t SEEDK, HEAPK;      // repair pool entries per floe slot
+    int32_t pad_s_;
     int32_t record_forces;
     int32_t ncells;            // cell slots (sentinel key = ncells)
     int32_t qseg;              // floe positions per XCD share of the candidate search
     int32_t repair_lanes;      // events the repair evaluates at once (1: one at a time)
-    int32_t repair_cap;        // pending repair keys held in LDS
+    int32_t repair_cap;        // entries of each repair list held in LDS
     int32_t pad_r_;
     // floe state by storage slot (current where rebuild[2] is clear, else
     // in the ordered copies)
@@ -100,11 +97,10 @@ struct DS {
     // candidate lists (pos rows; entries are partner positions)
     int32_t* ocnt;
     int64_t* oj;
-    double* od;
+    double* od;                // the search's distances; after it r(i) where evf has EV_SRI
     int32_t* icnt;
     int64_t* ik;
     uint32_t* evf;
-    int32_t* ov;               // repair table entry, valid where evf has EV_TABLE
     double *ssc, *ssb;         // [CO][S] pos: the pair's |(fcn,fct)| and |(fbn,fbt)|
                                // (written only when forces are recorded)
     // pair state, double-buffered (id rows; partner stored as id)
@@ -119,7 +115,6 @@ struct DS {
     double* acc;               // [NACC][S]
     WallOut* wout;             // [S], valid where WF_WALL is set
     uint8_t* wflag;            // [S rounded up to 4] WF_* bits
-    int32_t* ovw;              // [S] repair wall-table entry, valid where WF_REPAIR_WALL is set
     uint8_t* cls;              // [S] CLS_* bits
     // Candidate supersets: every floe within its query radius plus the
     // member's skin at the last build, (id << 32 | pos), floe k's at
@@ -148,17 +143,15 @@ struct DS {
     // QN_STRIDE ints), so that the counters' atomics spread over many lines.
     int32_t* qlist;            // [NQUEUE][S]
     int32_t* qn;               // [NQUEUE][XCD_COUNT] x QN_STRIDE
-    // ordered repair (id)
-    uint64_t* seeds;           // SEEDK per floe slot, member region starts at SEEDK*first
-    int32_t* nseeds;           // [members]
-    uint64_t* heap;            // HEAPK per floe slot
-    EventOut* etab;            // TABK per floe slot
-    int32_t* netab;
-    WallOut* wtab;             // one per floe slot
-    int32_t* nwtab;
-    double* cur;               // [7][S] r h mass inertia hfa hfw, query radius during repair
-    uint8_t* dirty;            // [S rounded up to 4] DIRTY_* bits
-    int32_t* comp;             // [S] by pos: contact component (union-find parent)
+    // ordered repair: reshape records, SEEDK per floe slot (a member's from
+    // SEEDK*first on), the seeds first; rhead is each floe's list of them
+    Reshape* shape;
+    int32_t* nseeds;           // [members] records the event kernels wrote
+    int32_t* rhead;            // [S] by pos: a record of the floe, -1: none this step
+    uint64_t* heap;            // HEAPK per floe slot: the repair's lists beyond LDS
+    double* cur;               // [6][S] r h mass inertia hfa hfw after the step's reshapes
+    uint8_t* dirty;            // [S rounded up to 4] 1: the floe was reshaped (cur holds its
+                               //     properties; by storage slot, k_final clears it)
     uint8_t* wnz;              // [S] by storage slot: 0 = the floe's wall history rows (wbc)
                                //     are all +0.0 (k_final then skips rewriting them)
     int64_t* stats;            // [members][4]

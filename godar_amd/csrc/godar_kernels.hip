@@ -2,8 +2,7 @@
 //
 //   k_begin -> [build steps: radix sort -> k_ranges -> k_sup ...] -> k_cand
 //    -> (k_contact -> k_walls on a side stream) beside k_bond
-//    -> k_comp -> k_repair -> k_fixq -> k_fixup
-//    -> k_final (which also gathers the bond terms)
+//    -> k_repair -> k_fixup -> k_final (which also gathers the bond terms)
 //
 // Sequential semantics of the reference (stepper.f90:71-280 visits floes i
 // in index order and, for each, its candidates j > i in ascending distance;
@@ -23,12 +22,12 @@
 //     and FP64 sums stay identical to the reference.
 //   * An event's speculative result is exact unless one of its floes was
 //     reshaped earlier in the sequence.  Events that ridge are seeds; the
-//     per-member k_repair walks, in sequence order, the seeds and every later
-//     event of each reshaped floe, recomputes them with the current floe
-//     properties and records the results.
-//   * k_fixq lists the floes touched by the repair, k_fixup re-gathers them,
-//     k_final applies the final floe properties, forcing, Coriolis, totals
-//     and integration.
+//     per-member k_repair settles which events reshape which floe, and to
+//     what, in the order of the sequence, and lists the floes whose terms
+//     that changes.
+//   * k_fixup evaluates those floes' events again, each with the properties
+//     its floes have at its place in the sequence, k_final applies the final
+//     floe properties, forcing, Coriolis, totals and integration.
 //
 // Layout: the per-step kernels run over floes in cell order ("pos"), reading
 // a sorted copy of the 96-byte floe records, so that a floe's neighbours sit
@@ -180,54 +179,38 @@ __device__ __forceinline__ double2 wind_at(const DS& S, int k) {
     return make_double2(h.wx, h.wy);
 }
 
-// Sets flag bits of position k's wflag byte from any lane or wavefront: the
-// byte shares a 32-bit word with three neighbours whose bits others may be
-// setting at the same time (the array is allocated in whole words).
-__device__ __forceinline__ void wflag_set(const DS& S, int k, uint32_t bits) {
-    atomicOr(reinterpret_cast<uint32_t*>(S.wflag + (k & ~3)), bits << (8 * (k & 3)));
+__device__ __forceinline__ void take_shape(const Reshape& w, Floe& F) {
+    F.r = w.r; F.h = w.h; F.mass = w.mass; F.inertia = w.inertia; F.hfa = w.hfa; F.hfw = w.hfw;
 }
 
-// Contact components of the step (union-find over the speculative contacts,
-// at positions): k_cand makes every floe its own root, k_contact unites the
-// floes of each contact, hooking the larger root under the smaller with a
-// compare-and-swap (a root's parent changes only there), and k_comp points
-// every contact floe at its root.  Parents are read and written at device
-// scope: other wavefronts change them during k_contact.
-__device__ __forceinline__ int comp_parent(const int32_t* p, int x) {
-    return __hip_atomic_load(p + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// Properties of a floe during the step's ordered sequence of events: F, the
+// properties it starts the step with, unless a reshape of it (list `head` of
+// the member's records) comes before event `key`; then those the last such
+// reshape left.
+__device__ __forceinline__ void floe_at_event(const Reshape* rec, int head, int64_t key, Floe& F) {
+    int best = -1;
+    int64_t bk = -1;
+    for (int p = head; p >= 0; p = rec[p].next)
+        if (rec[p].live && rec[p].key < key && rec[p].key > bk) { bk = rec[p].key; best = p; }
+    if (best >= 0) take_shape(rec[best], F);
 }
-__device__ __forceinline__ int comp_find(int32_t* p, int x) {
-    for (;;) {
-        const int px = comp_parent(p, x);
-        if (px == x) return x;
-        const int ppx = comp_parent(p, px);
-        // path halving: any ancestor may stand in for the parent
-        if (ppx != px) __hip_atomic_store(p + x, ppx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        x = px;
-    }
+// (the first reshape of the list, INT64_MAX if none)
+__device__ __forceinline__ int64_t first_reshape(const Reshape* rec, int head) {
+    int64_t k = INT64_MAX;
+    for (int p = head; p >= 0; p = rec[p].next)
+        if (rec[p].live && rec[p].key < k) k = rec[p].key;
+    return k;
 }
-__device__ __forceinline__ void comp_unite(int32_t* p, int a, int b) {
-    for (;;) {
-        a = comp_find(p, a);
-        b = comp_find(p, b);
-        if (a == b) return;
-        if (a < b) { const int t = a; a = b; b = t; }
-        if (atomicCAS(p + a, a, b) == a) return;
-    }
-}
-
-// floe at storage slot f and position k with the properties current during
-// the ordered repair
-__device__ __forceinline__ Floe load_floe_cur(const DS& S, int f, int k) {
-    // the current rows are read with the records (one round of loads) and
-    // taken where the floe was reshaped
-    Floe F = floe_at(S, k);
-    const bool d = (S.dirty[f] & DIRTY_SHAPE) != 0;
-    const double r = S.cur[0 * S.S + f], h = S.cur[1 * S.S + f], mass = S.cur[2 * S.S + f];
-    const double inertia = S.cur[3 * S.S + f], hfa = S.cur[4 * S.S + f], hfw = S.cur[5 * S.S + f];
-    F.r = d ? r : F.r; F.h = d ? h : F.h; F.mass = d ? mass : F.mass;
-    F.inertia = d ? inertia : F.inertia; F.hfa = d ? hfa : F.hfa; F.hfw = d ? hfw : F.hfw;
-    return F;
+// Records the reshape event `key` of the floes at kf (outer) and kj (-1: a
+// wall) gives the floe at kg, as record p of the member, and links it to the
+// floe's list.
+__device__ __forceinline__ void add_reshape(const DS& S, Reshape* rec, int p, int64_t key, int kg,
+                                            int kf, int kj, double r, double h, double mass,
+                                            double inertia, double hfa, double hfw) {
+    Reshape& w = rec[p];
+    w.key = key; w.r = r; w.h = h; w.mass = mass; w.inertia = inertia; w.hfa = hfa; w.hfw = hfw;
+    w.pos = kg; w.kf = kf; w.kj = kj; w.live = 1;
+    w.next = atomicExch(&S.rhead[kg], p);
 }
 
 __device__ __forceinline__ int cell_coord(double p, double cell, int g) {
@@ -277,41 +260,14 @@ __device__ __forceinline__ int find_entry(const int64_t* list, int64_t SS, int k
     int r = -1;
 #pragma unroll
     for (int s = LIST_PEEK - 1; s >= 0; --s) r = (s < n && id[s] == g) ? s : r;
-    for (int s = LIST_PEEK; r < 0 && s < n; ++s)
-        if (ent_id(list[(int64_t)s * SS + kp]) == g) r = s;
-    return r;
-}
-
-// (PEEK 1: one entry at a time, for kernels short of registers)
-template <int PEEK = LIST_PEEK>
-__device__ __forceinline__ void load_pair_state(const DS& S, int i, int j, PairState& ps) {
-    ps.deltat = 0.0; ps.thetarelc = 0.0; ps.fcn = 0.0; ps.fct = 0.0;
-    ps.bond = 0; ps.has_bond_rec = false;
-    ps.damage = ps.deltanb = ps.deltatb = ps.trb_ji = ps.trb_ij = 0.0;
-    ps.rb = ps.hb = ps.lb = ps.sb = ps.ib = 0.0;
-    // both lists are searched at once
-    const int hc = S.hcnt_old[i], bc = S.bcnt_old[i];
-    const int hq = find_partner<PEEK>(S.hist_old, S.S, i, hc, j);
-    const int bq = find_partner<PEEK>(S.bond_old, S.S, i, bc, j);
-    if (hq >= 0) {
-        const HistRec& hr = S.hist_old[(int64_t)hq * S.S + i];
-        ps.deltat = hr.deltat; ps.thetarelc = hr.thetarelc; ps.fcn = hr.fcn; ps.fct = hr.fct;
-    }
-    if (bq >= 0) {
-        const BondRec& b = S.bond_old[(int64_t)bq * S.S + i];
-        ps.has_bond_rec = true; ps.bond = b.bond; ps.damage = b.damage;
-        ps.deltanb = b.deltanb; ps.deltatb = b.deltatb; ps.trb_ji = b.trb_ji; ps.trb_ij = b.trb_ij;
-        ps.rb = b.rb; ps.hb = b.hb; ps.lb = b.lb; ps.sb = b.sb; ps.ib = b.ib;
-    }
-}
-
-// Record copy word by word (a struct copy is lowered through scratch memory).
-static_assert(sizeof(BondRec) % 8 == 0, "BondRec is copied in 8-byte words");
-__device__ __forceinline__ void copy_bond(BondRec* dst, const BondRec* src) {
-    const uint64_t* s = reinterpret_cast<const uint64_t*>(src);
-    uint64_t* d = reinterpret_cast<uint64_t*>(dst);
+    // (long lists: LIST_PEEK entries a round)
+    for (int s0 = LIST_PEEK; r < 0 && s0 < n; s0 += LIST_PEEK) {
 #pragma unroll
-    for (int w = 0; w < (int)(sizeof(BondRec) / 8); ++w) d[w] = s[w];
+        for (int s = 0; s < LIST_PEEK; ++s) id[s] = ent_id(list[(int64_t)min(s0 + s, n - 1) * SS + kp]);
+#pragma unroll
+        for (int s = LIST_PEEK - 1; s >= 0; --s) r = (s0 + s < n && id[s] == g) ? s0 + s : r;
+    }
+    return r;
 }
 
 __device__ __forceinline__ BondRec bond_from(const PairState& ps, int j) {
@@ -442,7 +398,7 @@ __global__ void k_begin(DS S, int lean, int nmembers) {
     if (build && i <= S.ncells) S.crange[i] = make_int2(0, 0);
     // per-member resets (thread m for member m)
     if (i < nmembers && member_live(S.members[i])) {
-        S.nseeds[i] = 0; S.netab[i] = 0; S.nwtab[i] = 0;
+        S.nseeds[i] = 0;
         S.stats[4 * i + 2] = 0; S.stats[4 * i + 3] = 0;
         S.tcur[i] = S.members[i].tstep;
     }
@@ -575,7 +531,7 @@ __device__ __forceinline__ void cand_finish(const DS& S, int k, int fs, const De
         if (!qb) S.bcnt_new[fs] = 0;
         S.wflag[k] = 0;
         S.bgat[k] = 0;
-        S.comp[k] = k;
+        S.rhead[k] = -1;
         S.cls[k] = qc ? CLS_CONTACT : 0;   // the fix-up sets CLS_BOND
     }
 }
@@ -1228,35 +1184,6 @@ constexpr int DENSE_WAVES_PER_SIMD = 3;   // the dense search's occupancy bound
 static_assert((DENSE_RING & (DENSE_RING - 1)) == 0 && DENSE_RING >= DENSE_BATCH + DENSE_WIN,
               "a ring of whole rows with room for a batch past the register part");
 
-__device__ __forceinline__ void bitonic_inner(int64_t* ke, int n, int lane) {
-    for (int size = 2; size <= n; size <<= 1) {
-        for (int stride = size >> 1; stride > 0; stride >>= 1) {
-            for (int i = lane; i < n; i += 64) {
-                const int pj = i ^ stride;
-                if (pj > i) {
-                    const bool up = (i & size) == 0;
-                    const int64_t e1 = ke[i], e2 = ke[pj];
-                    if ((e1 > e2) == up) { ke[i] = e2; ke[pj] = e1; }
-                }
-            }
-            __syncthreads();
-        }
-    }
-}
-
-template <typename T>
-__device__ __forceinline__ T wave_min(T v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = dmin(v, (T)__shfl_xor(v, off));
-    return v;
-}
-
-__device__ __forceinline__ int pow2_at_least(int n) {
-    int p = 1;
-    while (p < n) p <<= 1;
-    return p;
-}
-
 // Superset build of the dense members' floes (queue 3), one wavefront per
 // floe over its (2 span + 1)^2 cell block, 64 entries at a time: counts, or
 // the entries and the build positions.  The filled superset is then ordered
@@ -1820,7 +1747,7 @@ constexpr int CONTACT_LDS_PER_WAVE = 64 * (int)sizeof(ContactOut);
 // 3 wavefronts per SIMD: 0.0955 -> 0.0915 ms beside the bond kernel; FP64
 // would drop to 2 and keeps the bound of 3)
 template <bool MIXED>
-__global__ __launch_bounds__(FLOE_BLOCK, MIXED ? 2 : 3) void k_contact(DS S) {
+__global__ __launch_bounds__(FLOE_BLOCK, 3) void k_contact(DS S) {
     extern __shared__ unsigned char contact_lds[];
     ContactOut* co = reinterpret_cast<ContactOut*>(contact_lds + (threadIdx.x >> 6) * CONTACT_LDS_PER_WAVE);
     if (*S.err) return;
@@ -1928,7 +1855,6 @@ __global__ __launch_bounds__(FLOE_BLOCK, MIXED ? 2 : 3) void k_contact(DS S) {
                         kinematics(Fi, Fj, kn);
                         PairState ps;
                         load_contact_state(S, ofs, j, ps);
-                        comp_unite(S.comp, ko, qj);      // the contact joins the floes' components
                         bond_create(P, tstep, of - first, j - first, Fi, Fj, kn, ps);
                         EventOut o;
                         o.flags = 0;
@@ -1946,7 +1872,9 @@ __global__ __launch_bounds__(FLOE_BLOCK, MIXED ? 2 : 3) void k_contact(DS S) {
                         if (o.flags & EV_RIDGED) {
                             const int p = atomicAdd(&S.nseeds[om], 1);
                             if (p < S.SEEDK * S.members[om].n)
-                                S.seeds[(int64_t)S.SEEDK * first + p] = ((uint64_t)(of - first) << 16) | (uint64_t)s;
+                                add_reshape(S, S.shape + (int64_t)S.SEEDK * first, p,
+                                            ((int64_t)(of - first) << 16) | s, o.ridged == 0 ? ko : qj,
+                                            ko, qj, o.nr, o.nh, o.nmass, o.ninertia, o.nhfa, o.nhfw);
                             else
                                 over |= ERR_SEED_CAP;
                         }
@@ -2290,7 +2218,9 @@ __global__ __launch_bounds__(FLOE_BLOCK) void k_walls(DS S) {
         if (W.flags & 4u) {
             int p = atomicAdd(&S.nseeds[m], 1);
             if (p < S.SEEDK * S.members[m].n)
-                S.seeds[(int64_t)S.SEEDK * first + p] = ((uint64_t)(f - first) << 16) | WALL_SLOT;
+                add_reshape(S, S.shape + (int64_t)S.SEEDK * first, p,
+                            ((int64_t)(f - first) << 16) | WALL_SLOT, k, k, -1, W.nr, W.nh, W.nmass,
+                            W.ninertia, W.nhfa, W.nhfw);
             else
                 set_err(S, ERR_SEED_CAP);
         }
@@ -2298,622 +2228,395 @@ __global__ __launch_bounds__(FLOE_BLOCK) void k_walls(DS S) {
 }
 
 // ---------------------------------------------------------------------
-// 4. ordered repair, one member per block (one wavefront)
+// 4. ordered repair, one member per block
+//
+// An event reads the radius, thickness, mass and drafts of its two floes and
+// only a reshape changes those, so the result of the reference's sequence is
+// fixed by the reshapes alone: for every event that ridges, which floe it
+// reshapes and to what.  Events are named by their place in the sequence, key
+// (outer local index << 16 | slot), and each floe has a list of its reshape
+// records; an event takes the properties of the last record before its key.
+// Only a floe's contacts and walls can reshape it, and radii only shrink, so
+// the events that can ridge are the contacts and walls the event kernels
+// found at the start-of-step radii.
+//
+// The records start as the seeds (what ridges with the start-of-step
+// properties).  Round by round, every contact and wall event that comes after
+// a record that changed, on the same floe, is evaluated again, all of a
+// member's at once; one whose outcome differs from its record updates it,
+// which is a change for the next round.  When nothing changes, each event's
+// outcome follows from the records before it, and by induction over the keys
+// that is the sequence's own outcome, whatever order the rounds took.  The
+// rounds a member needs are the longest chain of reshapes that act on each
+// other, not the number of events behind them.
+//
+// What it costs is the chain of dependent loads of a round (event -> rows ->
+// records), about 8 us; most members have a handful of seeds, one round that
+// finds no later contact, and the closing pass that queues the floes whose
+// terms change.  (One MI355X, against committing the events in key order 64
+// at a time, which also took every candidate after a reshape through the
+// rounds and went on one event at a time past 1,024 pending: 262,144 floes of
+// one field with 43 candidates a floe and 80 seeds, FP64, 20 -> 0.043 ms per
+// step; 24 such fields, 320,000 floes, mixed, 0.23-0.9 -> 0.023; 2,501 floes
+// with 50 seeds 0.26 -> 0.027; the 512-field ensemble 0.064 -> 0.026.)
 // ---------------------------------------------------------------------
-struct Heap {
-    uint64_t* a;
-    int n, cap;
-    __device__ bool push(uint64_t k) {
-        if (n >= cap) return false;
-        int i = n++;
-        while (i > 0) {
-            int p = (i - 1) >> 1;
-            if (a[p] <= k) break;
-            a[i] = a[p];
-            i = p;
-        }
-        a[i] = k;
-        return true;
-    }
-    __device__ uint64_t pop() {
-        uint64_t top = a[0];
-        uint64_t last = a[--n];
-        int i = 0;
-        while (true) {
-            int l = 2 * i + 1;
-            if (l >= n) break;
-            int c = (l + 1 < n && a[l + 1] < a[l]) ? l + 1 : l;
-            if (a[c] >= last) break;
-            a[i] = a[c];
-            i = c;
-        }
-        if (n > 0) a[i] = last;
-        return top;
-    }
-};
-
-__device__ __forceinline__ void set_cur(const DS& S, int g, double r, double h, double mass,
-                                        double inertia, double hfa, double hfw) {
-    S.cur[0 * S.S + g] = r; S.cur[1 * S.S + g] = h; S.cur[2 * S.S + g] = mass;
-    S.cur[3 * S.S + g] = inertia; S.cur[4 * S.S + g] = hfa; S.cur[5 * S.S + g] = hfw;
-}
-
-// Sets bits of storage slot f's dirty byte (the word holds three other
-// floes' bytes, which other lanes may be setting; the array is allocated in
-// whole words).
-__device__ __forceinline__ void dirty_set(const DS& S, int f, uint32_t bits) {
-    atomicOr(reinterpret_cast<uint32_t*>(S.dirty + (f & ~3)), bits << (8 * (f & 3)));
-}
-
-// Query radius of the floe at slot fs (position kf) for the events of its
-// own iteration: its radius at the top of that iteration.  The first
-// committed event of the iteration keeps it (cur row 6); until then no event
-// of the iteration has reshaped the floe, so it is the current radius.
-__device__ __forceinline__ double block_rq(const DS& S, int fs, int kf) {
-    const uint8_t d = S.dirty[fs];
-    return (d & DIRTY_RQ) ? S.cur[6 * S.S + fs] : ((d & DIRTY_SHAPE) ? S.cur[fs] : S.geo[kf].r);
-}
-__device__ __forceinline__ void keep_block_rq(const DS& S, int fs, double rq) {
-    if (!(S.dirty[fs] & DIRTY_RQ)) {
-        S.cur[6 * S.S + fs] = rq;
-        dirty_set(S, fs, DIRTY_RQ);
-    }
-}
+constexpr int REPAIR_THREADS = 512;
+constexpr int REPAIR_LIST = 1024;        // entries of each list held in LDS
+constexpr int REPAIR_ROUNDS = 1 << 20;   // (never reached: every round settles one more key)
 
 // slot of partner id g in the outer list of the floe at position kp
 __device__ __forceinline__ int slot_of(const DS& S, int kp, int g) {
     return find_entry(S.oj, S.S, kp, S.ocnt[kp], g);
 }
 
-// write (or clear) owner i's new contact history entry for partner j; the
-// entry lives while any of its four values is non-zero
-__device__ __forceinline__ bool put_hist(const DS& S, int i, int j, const PairState& ps) {
-    const bool want = ps.deltat != 0.0 || ps.thetarelc != 0.0 || ps.fcn != 0.0 || ps.fct != 0.0;
-    const int n = S.hcnt_new[i];
-    int q = find_partner(S.hist_new, S.S, i, n, j);
-    if (want) {
-        if (q < 0) {
-            if (n >= S.HC) return false;
-            q = n;
-            S.hcnt_new[i] = n + 1;
-        }
-        HistRec hr; hr.j = j; hr.pad_ = 0; hr.deltat = ps.deltat; hr.thetarelc = ps.thetarelc;
-        hr.fcn = ps.fcn; hr.fct = ps.fct;
-        S.hist_new[(int64_t)q * S.S + i] = hr;
-    } else if (q >= 0) {
-        S.hist_new[(int64_t)q * S.S + i].j = -1;
-    }
-    return true;
+// Sets bits of position k's wflag byte; returns the byte as it was.
+__device__ __forceinline__ uint32_t wflag_fetch_set(const DS& S, int k, uint32_t bits) {
+    const int sh = 8 * (k & 3);
+    return (atomicOr(reinterpret_cast<uint32_t*>(S.wflag + (k & ~3)), bits << sh) >> sh) & 255u;
+}
+__device__ __forceinline__ void wflag_clear(const DS& S, int k, uint32_t bits) {
+    atomicAnd(reinterpret_cast<uint32_t*>(S.wflag + (k & ~3)), ~(bits << (8 * (k & 3))));
+}
+// a record list's head, changed by other wavefronts of the block
+__device__ __forceinline__ int rhead_at(const DS& S, int k) {
+    return __hip_atomic_load(S.rhead + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__device__ __forceinline__ bool put_bond(const DS& S, int i, int j, bool want, const BondRec& b) {
-    const int n = S.bcnt_new[i];
-    int q = find_partner(S.bond_new, S.S, i, n, j);
-    if (want) {
-        if (q < 0) {
-            if (n >= S.BC) return false;
-            q = n;
-            S.bcnt_new[i] = n + 1;
-        }
-        S.bond_new[(int64_t)q * S.S + i] = b;
-    } else if (q >= 0) {
-        S.bond_new[(int64_t)q * S.S + i].j = -1;
-    }
-    return true;
+// The floe at position k joins the fix-up queue (once).
+__device__ __forceinline__ void touch_floe(const DS& S, int k) {
+    if (!(wflag_fetch_set(S, k, WF_FIXUP) & WF_FIXUP)) enqueue_one(S, 4, k);
 }
 
-// Appends record r of every lane in `ma` to its owner i's list (count cnt[i],
-// capacity cap) in lane order.  The lanes of one owner are adjacent in the
-// batch (the keys are sorted by owner), so each takes the owner's count plus
-// its rank among them, and the last of them writes the new count: no lane
-// waits for another.  Every lane of the wavefront calls it.
-template <typename Rec>
-__device__ __forceinline__ void append_lanes(Rec* list, int32_t* cnt, int64_t SS, int cap,
-                                             uint64_t ma, int i, int n, const Rec& r,
-                                             uint32_t& over, uint32_t err) {
-    const int lane = (int)(threadIdx.x & 63);
-    const bool mine = (ma >> lane) & 1ull;
-    const uint64_t below = ma & ((1ull << lane) - 1ull);
-    const uint64_t above = ma & ~((2ull << lane) - 1ull);
-    const int prev = below ? 63 - __clzll((long long)below) : lane;
-    const int next = above ? __ffsll((long long)above) - 1 : lane;
-    const int iprev = __shfl(i, prev), inext = __shfl(i, next);
-    const bool head = mine && (!below || iprev != i);
-    const bool last = mine && (!above || inext != i);
-    const uint64_t hb = __ballot(head) & ((2ull << lane) - 1ull);
-    const int start = hb ? 63 - __clzll((long long)hb) : 0;
-    const int rank = __popcll(below & ~((1ull << start) - 1ull));
-    if (mine) {
-        const int at = n + rank;
-        if (at >= cap) over |= err;
-        else list[(int64_t)at * SS + i] = r;
-        if (last) cnt[i] = min(at + 1, cap);
-    }
-}
-
-// Lane versions of put_hist / put_bond for the batched repair: the lanes in
-// `on` hold committed events, in key order.  Records found are replaced (or
-// cleared) in place; new ones are appended in lane order.
-__device__ __forceinline__ void put_hist_lanes(const DS& S, bool on, int i, int j,
-                                               const PairState& ps, uint32_t& over) {
-    const bool want = on && (ps.deltat != 0.0 || ps.thetarelc != 0.0 || ps.fcn != 0.0 || ps.fct != 0.0);
-    HistRec hr;
-    hr.j = j; hr.pad_ = 0; hr.deltat = ps.deltat; hr.thetarelc = ps.thetarelc; hr.fcn = ps.fcn; hr.fct = ps.fct;
-    int q = -1, n = 0;
-    if (on) {
-        n = S.hcnt_new[i];
-        q = find_partner(S.hist_new, S.S, i, n, j);
-        if (q >= 0) {
-            if (want) S.hist_new[(int64_t)q * S.S + i] = hr;
-            else S.hist_new[(int64_t)q * S.S + i].j = -1;
-        }
-    }
-    append_lanes(S.hist_new, S.hcnt_new, S.S, S.HC, __ballot(want && q < 0), i, n, hr, over,
-                 ERR_HIST_CAP);
-}
-
-__device__ __forceinline__ void put_bond_lanes(const DS& S, bool on, int i, int j, bool want,
-                                               const BondRec& b, uint32_t& over) {
-    want = want && on;
-    int q = -1, n = 0;
-    if (on) {
-        n = S.bcnt_new[i];
-        q = find_partner(S.bond_new, S.S, i, n, j);
-        if (q >= 0) {
-            if (want) S.bond_new[(int64_t)q * S.S + i] = b;
-            else S.bond_new[(int64_t)q * S.S + i].j = -1;
-        }
-    }
-    append_lanes(S.bond_new, S.bcnt_new, S.S, S.BC, __ballot(want && q < 0), i, n, b, over,
-                 ERR_BOND_CAP);
-}
-
-// Progress of one member's repair (the same in every lane).
-struct RepairState {
-    int64_t last;        // key of the last event recomputed (-1: none)
-    int nt, nwt;         // repair table entries used
-    int64_t repaired;
+// The events after a record of the floe at kg: its inner pairs of later outer
+// floes, its own candidates from slot s0 on, its walls.  A wavefront takes
+// the records of its lanes together, 64 events at a time.
+struct LaterEvents {
+    int ni, s0, no;        // inner entries (0: none is later), own slots [s0, s0 + no)
+    int f;                 // local index of the record's outer floe
 };
-
-// Every later event of floe g, reshaped by event (f, s), goes onto the heap:
-// the pairs (i2, g) with f < i2 < g, then g's own events after s (all of
-// them if g != f) and g's walls.
-__device__ __forceinline__ void push_later_events(const DS& S, Heap& H, int first, int f, int s,
-                                                  int g, int kg, uint32_t& over) {
-    const int64_t SS = S.S;
-    const int gb = g - first;
-    if (g != f) {
-        const int gi = S.icnt[kg];
-        for (int q = 0; q < gi; ++q) {
-            const int64_t ei = S.ik[(int64_t)q * SS + kg];
-            const int i2 = ent_id(ei);
-            if (i2 <= f) continue;
-            const int sk = slot_of(S, ent_pos(ei), g);
-            if (sk >= 0 && !H.push(((uint64_t)(i2 - first) << 16) | (uint64_t)sk)) over |= ERR_REPAIR_CAP;
-        }
-    }
-    const int s0 = (g == f) ? s + 1 : 0;
-    const int gno = S.ocnt[kg];
-    for (int s2 = s0; s2 < gno; ++s2)
-        if (!H.push(((uint64_t)gb << 16) | (uint64_t)s2)) over |= ERR_REPAIR_CAP;
-    if (!H.push(((uint64_t)gb << 16) | WALL_SLOT)) over |= ERR_REPAIR_CAP;
+__device__ __forceinline__ LaterEvents later_events(const DS& S, int64_t key, int kg, int gid, int first) {
+    LaterEvents l;
+    const int s = (int)(key & 0xFFFF);
+    l.f = (int)(key >> 16);
+    const bool own = gid - first == l.f;          // the record's event is one of the floe's own
+    const int ni = S.icnt[kg], no = S.ocnt[kg];
+    l.ni = own ? 0 : ni;
+    l.s0 = own ? s + 1 : 0;
+    l.no = s == WALL_SLOT ? 0 : max(no - l.s0, 0);
+    if (s == WALL_SLOT) l.ni = 0;                 // (a floe's walls are its last event)
+    return l;
 }
-
-// Every contact floe (queue 0) points at the root of its contact component
-// (no unions run any more).  Every floe of a contact is in the queue.
-__global__ __launch_bounds__(FLOE_BLOCK) void k_comp(DS S) {
-    if (*S.err) return;
-    const QueueView qv = queue_view(S, 0);
-    for (int it = 0;; ++it) {
-        const int t = queue_slot_it(qv.total, it);
-        if (t < 0) break;
-        const int k = queue_at(S, 0, qv, t);
-        S.comp[k] = comp_find(S.comp, k);
-    }
-}
-
-// One event at a time off the binary heap in HBM (single lane).
-template <bool MIXED>
-__device__ void repair_serial(const DS& S, const DevParams& P, int first, int nmem, int tstep,
-                              Heap& H, EventOut* etab, int tcap, WallOut* wtab, RepairState& st,
-                              uint32_t& over) {
-    const int64_t SS = S.S;
-    while (H.n > 0 && !over) {
-        const uint64_t key = H.pop();
-        if ((int64_t)key == st.last) continue;
-        st.last = (int64_t)key;
-        const int b = (int)(key >> 16), s = (int)(key & 0xFFFF);
-        // keys name an event of this member (a broken key is an internal
-        // error, never an out-of-range access)
-        if (key >> 16 >= (uint64_t)nmem || (s != WALL_SLOT && s >= S.CO)) { over |= ERR_REPAIR_CAP; break; }
-        const int f = first + b;              // identity
-        const int fs = S.sid_of[f];           // storage slot
-        const int kf = S.pos_id[f];           // position (loaded beside the slot)
-        ++st.repaired;
-        if (s == WALL_SLOT) {
-            Floe F = load_floe_cur(S, fs, kf);
-            double hist[4] = {S.wbc[0 * SS + fs], S.wbc[1 * SS + fs], S.wbc[2 * SS + fs], S.wbc[3 * SS + fs]};
-            WallOut W;
-            walls<MIXED>(P, F, hist, W);
-            if (st.nwt >= nmem) { over |= ERR_REPAIR_CAP; break; }
-            wtab[st.nwt] = W;
-            S.ovw[kf] = st.nwt++;
-            wflag_set(S, kf, WF_REPAIR_WALL | WF_FIXUP);
-            if (W.flags & 4u) {
-                set_cur(S, fs, W.nr, W.nh, W.nmass, W.ninertia, W.nhfa, W.nhfw);
-                dirty_set(S, fs, DIRTY_SHAPE);
-            }
-            continue;
-        }
-        const double rq = block_rq(S, fs, kf);   // query radius at the top of iteration f
-        keep_block_rq(S, fs, rq);
-        const int64_t e = S.oj[(int64_t)s * SS + kf];
-        const int j = ent_id(e);
-        const int js = S.cval[ent_pos(e)];
-        Floe Fi = load_floe_cur(S, fs, kf);
-        Floe Fj = load_floe_cur(S, js, ent_pos(e));
-        wflag_set(S, kf, WF_FIXUP);
-        wflag_set(S, ent_pos(e), WF_FIXUP);
-        EventOut o;
-        const double dx = Fi.x - Fj.x, dy = Fi.y - Fj.y;
-        const double d = sqrt(dx * dx + dy * dy);
-        PairState ps;
-        load_pair_state(S, fs, j, ps);
-        if (!(d <= rq + P.rtree)) {
-            // no longer a candidate: the pair keeps its old state
-            o.flags = EV_REMOVED;
-            o.ridged = -1;
-        } else {
-            const double2 wf = wind_at(S, kf);
-            pair_event<MIXED>(P, tstep, b, j - first, Fi, Fj, wf.x, wf.y, P.uw, P.vw, ps, o, 0);
-        }
-        if (!put_hist(S, fs, j, ps)) over |= ERR_HIST_CAP;
-        if (!put_bond(S, fs, j, ps.has_bond_rec, bond_from(ps, j))) over |= ERR_BOND_CAP;
-        if (o.flags & EV_RIDGED) {
-            const int g = o.ridged == 0 ? f : j;
-            const int gs = o.ridged == 0 ? fs : js;
-            const int kg = o.ridged == 0 ? kf : ent_pos(e);
-            set_cur(S, gs, o.nr, o.nh, o.nmass, o.ninertia, o.nhfa, o.nhfw);
-            if (!(S.dirty[gs] & DIRTY_SHAPE)) {
-                dirty_set(S, gs, DIRTY_SHAPE);
-                push_later_events(S, H, first, f, s, g, kg, over);
-            }
-        }
-        if (st.nt >= tcap) { over |= ERR_REPAIR_CAP; break; }
-        etab[st.nt] = o;
-        S.ov[(int64_t)s * SS + kf] = st.nt++;
-        S.evf[(int64_t)s * SS + kf] = o.flags | EV_TABLE;
-    }
-}
-
-// number of a[0..n) below v (strictly, or at most v)
-__device__ __forceinline__ int count_below(const int64_t* a, int n, int64_t v, bool or_equal) {
-    int lo = 0, hi = n;
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        const bool left = or_equal ? a[mid] <= v : a[mid] < v;
-        if (left) lo = mid + 1; else hi = mid;
-    }
-    return lo;
-}
-
-// The recomputation follows the reference's loop order, key
-// (f - first) << 16 | slot.  Between two reshapes the recomputed events are
-// independent: an event reads the radius, thickness, mass, inertia and
-// drafts of its floes, which only a reshape changes, and writes the state of
-// its own pair.  So the wavefront evaluates the next `repair_lanes` pending
-// keys at once, one per lane, and commits them in key order up to and
-// including the first that reshapes a floe; the rest stay pending and are
-// evaluated again with the new state.  The pending keys are a sorted array in
-// LDS; those a reshape adds (every later event of the reshaped floe, produced
-// in order) are merged in.  A member whose pending keys outgrow `repair_cap`
-// continues one event at a time on its binary heap in HBM.
-constexpr int REPAIR_PCAP = 1024;    // pending keys held in LDS
-constexpr int REPAIR_NCAP = 512;     // keys one reshape adds, at most
 
 template <bool MIXED>
-__global__ __launch_bounds__(64) void k_repair(DS S, int nmembers) {
-    __shared__ int64_t pk[2][REPAIR_PCAP];
-    __shared__ int64_t nk[REPAIR_NCAP];
-    // each lane's result until the round decides whether it commits (one
-    // EventOut-sized slot per lane; a wall lane's WallOut uses its start)
-    __shared__ uint64_t stage_buf[64 * sizeof(EventOut) / 8];
-    __shared__ int tcomp[64];      // components of a round's reshaping lanes so far
-    // the member's parameters, copied to LDS: the physics reads them at LDS
-    // latency (this wavefront is the only one working on the member)
+__global__ __launch_bounds__(REPAIR_THREADS) void k_repair(DS S, int nmembers) {
+    __shared__ uint64_t wl[REPAIR_LIST];   // events to evaluate: outer position << 16 | slot
+    __shared__ int cl[REPAIR_LIST];        // records that changed
+    __shared__ int nw_, nc_, nn_, rep_, ns_;
+    __shared__ uint32_t over_;
+    // the member's parameters: the physics reads them at LDS latency
     __shared__ uint64_t pbuf[sizeof(DevParams) / 8];
     static_assert(sizeof(DevParams) % 8 == 0 && sizeof(DevParams) / 8 <= 64, "DevParams copied by lane");
     const int m = blockIdx.x;
-    if (m >= nmembers || *S.err) return;
-    if (!member_live(S.members[m])) return;
-    int ns = S.nseeds[m];
+    const int tid = (int)threadIdx.x, lane = tid & 63;
+    if (m >= nmembers) return;
+    // (the error word is read once for the block: all its wavefronts take the
+    // barriers below or none does)
+    if (tid == 0) {
+        const uint32_t err = *S.err;
+        const int n = S.nseeds[m];
+        const Member M = S.members[m];
+        ns_ = err || !member_live(M) ? 0 : min(n, S.SEEDK * M.n);
+        nn_ = ns_;
+        nw_ = nc_ = rep_ = 0;
+        over_ = 0;
+    }
+    __syncthreads();
+    const int ns = ns_;
     if (ns == 0) return;
-    if ((int)threadIdx.x < (int)(sizeof(DevParams) / 8))
-        pbuf[threadIdx.x] = reinterpret_cast<const uint64_t*>(S.params + m)[threadIdx.x];
+    // as many wavefronts as the events after the seeds fill (by the mean
+    // superset length of the last build); where the caller allows fewer than
+    // 64 lanes, the first wavefront with those
+    const int lanes = min(max(S.repair_lanes, 1), 64);
+    int waves = 1;
+    if (lanes == 64) {
+        const int64_t mean = 1 + S.sblk[(S.N + SCAN_TILE - 1) / SCAN_TILE] / S.N;
+        waves = (int)min((int64_t)(REPAIR_THREADS / 64), ((int64_t)ns * mean + 63) / 64);
+    }
+    const int width = lanes < 64 ? lanes : waves * 64;
+    if (tid >= waves * 64) return;
+    // records a wavefront takes at once from a list of n
+    auto share = [&](int n) { return min(lanes, (n + waves - 1) / waves); };
+    if (tid < (int)(sizeof(DevParams) / 8))
+        pbuf[tid] = reinterpret_cast<const uint64_t*>(S.params + m)[tid];
     __syncthreads();
     const DevParams& P = *reinterpret_cast<const DevParams*>(pbuf);
-    const int first = S.members[m].first;
-    const int nmem = S.members[m].n;
-    const int tstep = S.members[m].tstep;
+    const int first = S.members[m].first, nmem = S.members[m].n, tstep = S.members[m].tstep;
     const int64_t SS = S.S;
-    if (ns > S.SEEDK * nmem) ns = S.SEEDK * nmem;
-    const int lane = (int)threadIdx.x;
-    const uint64_t lt = lane ? ((~0ull) >> (64 - lane)) : 0ull;
-    const uint64_t* seeds = S.seeds + (int64_t)S.SEEDK * first;
-    EventOut* etab = S.etab + (int64_t)S.TABK * first;
-    const int tcap = S.TABK * nmem;
-    WallOut* wtab = S.wtab + first;
-    RepairState st;
-    st.last = -1; st.nt = 0; st.nwt = 0; st.repaired = 0;
+    Reshape* rec = S.shape + (int64_t)S.SEEDK * first;
+    const int reccap = S.SEEDK * nmem;
+    // lists beyond LDS: the member's share of `heap`, half for each
+    const int cap = min(max(S.repair_cap, 1), REPAIR_LIST);
+    uint64_t* whbm = S.heap + (int64_t)S.HEAPK * first;
+    const int hcap = S.HEAPK / 2 * nmem;
+    uint64_t* chbm = whbm + hcap;
     uint32_t over = 0;
-    Heap H;
-    H.a = S.heap + (int64_t)S.HEAPK * first;
-    H.n = 0;
-    H.cap = S.HEAPK * nmem;
-    EventOut* stage_e = reinterpret_cast<EventOut*>(stage_buf);
-    WallOut& stage_w_mine = *reinterpret_cast<WallOut*>(stage_e + threadIdx.x);
-    const int lanes = min(max(S.repair_lanes, 1), 64);
-    const int cap = min(max(S.repair_cap, 1), REPAIR_PCAP);
-    bool serial = lanes == 1 || ns > cap;
-    int cb = 0, head = 0, np = 0;
-    if (serial) {
-        if (lane == 0)
-            for (int p = 0; p < ns; ++p)
-                if (!H.push(seeds[p])) over |= ERR_REPAIR_CAP;
-    } else {
-        const int p2 = pow2_at_least(ns);
-        for (int i = lane; i < p2; i += 64) pk[0][i] = i < ns ? (int64_t)seeds[i] : INT64_MAX;
+    auto put_event = [&](int k, int s) {
+        const uint64_t w = ((uint64_t)(uint32_t)k << 16) | (uint32_t)s;
+        const int at = atomicAdd(&nw_, 1);
+        if (at < cap) wl[at] = w;
+        else if (at - cap < hcap) whbm[at - cap] = w;
+        else over |= ERR_REPAIR_CAP;
+    };
+    auto put_change = [&](int p) {
+        const int at = atomicAdd(&nc_, 1);
+        if (at < cap) cl[at] = p;
+        else if (at - cap < hcap) chbm[at - cap] = (uint64_t)p;
+        else over |= ERR_REPAIR_CAP;
+    };
+    // the records c0 .. of a list of n (at(i): record index), a lane each, and
+    // every event after them, fn(record lane's values, event)
+    auto each_later = [&](int cnt, auto&& fn) {
+        int incl = cnt;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int v = __shfl_up(incl, off);
+            if (lane >= off) incl += v;
+        }
+        const int start = incl - cnt, total = __shfl(incl, 63);
+        for (int c0 = 0; c0 < total; c0 += 64) {
+            const int idx = c0 + lane;
+            int own = 0;
+#pragma unroll
+            for (int step = 32; step > 0; step >>= 1)
+                if (__shfl(start, own + step) <= idx) own += step;
+            const int at = idx - __shfl(start, own);
+            fn(own, idx < total ? at : -1);
+        }
+    };
+    int nchg = ns;
+    bool seeds = true;       // (the first round's changes: the seeds, records 0 .. ns - 1)
+    for (int round = 0;; ++round) {
+        // ---- the contact and wall events after the changed records
+        const int rpw = share(nchg);
+        for (int c0 = 0; c0 < nchg; c0 += waves * rpw) {
+            const int ci = c0 + (tid >> 6) * rpw + lane;
+            const bool act = lane < rpw && ci < nchg;
+            int kg = 0, gid = 0, wl1 = 0;
+            LaterEvents l{0, 0, 0, 0};
+            GeoRec gg;
+            gg.x = gg.y = gg.r = 0.0;
+            if (act) {
+                const int p = seeds ? ci : ci < cap ? cl[ci] : (int)chbm[ci - cap];
+                const int64_t key = rec[p].key;
+                kg = rec[p].pos;
+                gg = S.geo[kg];
+                gid = gg.id;
+                l = later_events(S, key, kg, gid, first);
+                wl1 = (key & 0xFFFF) != WALL_SLOT && (S.wflag[kg] & WF_WALL) ? 1 : 0;
+            }
+            each_later(l.ni + l.no + wl1, [&](int own, int local) {
+                const int ko = __shfl(kg, own), go = __shfl(gid, own), fo = __shfl(l.f, own);
+                const int nio = __shfl(l.ni, own), s0 = __shfl(l.s0, own), noo = __shfl(l.no, own);
+                const double ox = __shfl(gg.x, own), oy = __shfl(gg.y, own), orr = __shfl(gg.r, own);
+                if (local < 0) return;
+                int ke = ko, s = WALL_SLOT;
+                bool want = true;
+                if (local < nio + noo) {
+                    const bool inner = local < nio;
+                    const int64_t e = inner ? S.ik[(int64_t)local * SS + ko]
+                                            : S.oj[(int64_t)(s0 + local - nio) * SS + ko];
+                    const int q = ent_pos(e);
+                    const GeoRec o = S.geo[q];
+                    // the pair's overlap as k_contact evaluates it
+                    const double dx = inner ? o.x - ox : ox - o.x, dy = inner ? o.y - oy : oy - o.y;
+                    const double dn = (inner ? o.r + orr : orr + o.r) - sqrt(dx * dx + dy * dy);
+                    want = dn > 0 && (!inner || ent_id(e) - first > fo);
+                    ke = inner ? q : ko;
+                    s = inner ? (want ? slot_of(S, q, go) : -1) : s0 + local - nio;
+                    want = want && s >= 0;
+                }
+                if (!want) return;
+                const bool listed = s == WALL_SLOT ? (wflag_fetch_set(S, ke, WF_PENDING) & WF_PENDING) != 0
+                                                   : (atomicOr(&S.evf[(int64_t)s * SS + ke], EV_PENDING) & EV_PENDING) != 0;
+                if (!listed) put_event(ke, s);
+            });
+        }
+        if (over) atomicOr(&over_, over);
         __syncthreads();
-        bitonic_inner(pk[0], p2, lane);
-        np = ns;
-    }
-    while (!serial && np > 0) {
-        const int nb = min(np, lanes);
-        const int64_t key = lane < nb ? pk[cb][head + lane] : INT64_MAX;
-        const int64_t prev = lane == 0 ? st.last : (lane < nb ? pk[cb][head + lane - 1] : INT64_MAX);
-        bool act = lane < nb && key != prev;            // repeated keys are done once
-        // keys name an event of this member (a broken key is an internal
-        // error, never an out-of-range access)
-        if (act && (key < 0 || (key >> 16) >= nmem || ((key & 0xFFFF) != WALL_SLOT && (key & 0xFFFF) >= S.CO))) {
-            over |= ERR_REPAIR_CAP;
-            act = false;
-        }
-        if (__ballot(over != 0)) break;
-        const int64_t kk = act ? key : 0;
-        const int b = (int)(kk >> 16), s = (int)(kk & 0xFFFF);
-        const int f = first + b;
-        const bool wall = act && s == WALL_SLOT;
-        const bool pair = act && s != WALL_SLOT;
-        int fs = 0, kf = 0, j = 0, js = 0, kj = 0, ridged = -1, ca = -1, cbm = -1;
-        bool reshape = false;
-        uint32_t oflags = 0;
-        double rql = 0.0, nr = 0.0, nh = 0.0, nmass = 0.0, ninertia = 0.0, nhfa = 0.0, nhfw = 0.0;
-        PairState ps;
-        if (act) {
-            fs = S.sid_of[f];
-            kf = S.pos_id[f];
-        }
-        if (wall) {
-            ca = cbm = S.comp[kf];
-            Floe F = load_floe_cur(S, fs, kf);
-            double hist[4] = {S.wbc[0 * SS + fs], S.wbc[1 * SS + fs], S.wbc[2 * SS + fs], S.wbc[3 * SS + fs]};
-            WallOut W;
-            walls<MIXED>(P, F, hist, W);
-            stage_w_mine = W;
-            reshape = (W.flags & 4u) != 0;
-            nr = W.nr; nh = W.nh; nmass = W.nmass; ninertia = W.ninertia; nhfa = W.nhfa; nhfw = W.nhfw;
-        }
-        if (pair) {
-            rql = block_rq(S, fs, kf);
-            const int64_t e = S.oj[(int64_t)s * SS + kf];
-            j = ent_id(e);
-            kj = ent_pos(e);
-            js = S.cval[kj];
-            ca = S.comp[kf];
-            cbm = S.comp[kj];
-            Floe Fi = load_floe_cur(S, fs, kf);
-            Floe Fj = load_floe_cur(S, js, kj);
-            const double dx = Fi.x - Fj.x, dy = Fi.y - Fj.y;
-            const double d = sqrt(dx * dx + dy * dy);
-            load_pair_state(S, fs, j, ps);
-            EventOut o;
-            if (!(d <= rql + P.rtree)) {
-                o.flags = EV_REMOVED;
-                o.ridged = -1;
-            } else {
-                const double2 wf = wind_at(S, kf);
-                pair_event<MIXED>(P, tstep, b, j - first, Fi, Fj, wf.x, wf.y, P.uw, P.vw, ps, o, 0);
-            }
-            stage_e[lane] = o;
-            oflags = o.flags;
-            reshape = (o.flags & EV_RIDGED) != 0;
-            ridged = o.ridged;
-            nr = o.nr; nh = o.nh; nmass = o.nmass; ninertia = o.ninertia; nhfa = o.nhfa; nhfw = o.nhfw;
-        }
-        // Commit every event of the batch whose floes no uncommitted event
-        // before it (in key order) can still change, and whose reshape no
-        // such event can still read.  A floe changes only when an event of it
-        // ridges, so only through contacts: within its contact component
-        // (comp, from the step's contacts at its start radii; radii only
-        // shrink).  An event before a lane that is not committed yet (a
-        // deferred lane, one a reshape adds, one those add in turn) belongs
-        // to a component of T, the components of the reshaping lanes before
-        // it (a lane waits when a floe of it lies in T, so its own component
-        // is in T if it ridges at all), or it reads floes in T and their
-        // candidate neighbours.  So, going through the reshaping lanes in
-        // order: the component of each joins T, and the later lanes in T
-        // wait; a reshaping lane itself waits if a waiting lane before it
-        // reads the floe it reshapes or a candidate neighbour of that floe
-        // lies in T.  (A lane that waits ridges nothing new: if its floes
-        // touch, they share a component in T; if not, it cannot ridge.)
-        uint64_t defer = 0, done = 0;
-        int nT = 0;
-        const uint64_t rsh = __ballot(reshape);
-        const int kgl = (wall || ridged == 0) ? kf : kj;     // the floe a reshaping lane reshapes
-        for (;;) {
-            const uint64_t t = rsh & ~defer & ~done;
-            if (!t) break;
-            const int cl = __ffsll((long long)t) - 1;
-            done |= 1ull << cl;
-            const int cc = __shfl(ca, cl);
-            const int kgc = __shfl(kgl, cl);
-            bool exposed = __ballot(lane < cl && ((defer >> lane) & 1ull) && (kf == kgc || (pair && kj == kgc))) != 0;
-            if (!exposed && nT > 0) {
-                const int no_g = S.ocnt[kgc], ncand = no_g + S.icnt[kgc];
-                bool hit = false;
-                for (int q0 = 0; q0 < ncand; q0 += 64) {
-                    const int q = q0 + lane;
-                    if (q < ncand) {
-                        const int64_t e = q < no_g ? S.oj[(int64_t)q * SS + kgc] : S.ik[(int64_t)(q - no_g) * SS + kgc];
-                        const int cn = S.comp[ent_pos(e)];
-                        for (int u = 0; u < nT; ++u) hit = hit || cn == tcomp[u];
-                    }
-                    if (__ballot(hit)) break;
-                }
-                exposed = __ballot(hit) != 0;
-            }
-            if (exposed) defer |= 1ull << cl;
-            if (lane == 0) tcomp[nT] = cc;
-            ++nT;
-            wave_lds_sync();
-            defer |= __ballot(act && lane > cl && (ca == cc || cbm == cc));
-        }
-        const bool com = act && !((defer >> lane) & 1ull);
-        const uint64_t mce = __ballot(com && pair), mcw = __ballot(com && wall);
-        const int rank_e = __popcll(mce & lt), rank_w = __popcll(mcw & lt);
-        if (st.nt + __popcll(mce) > tcap || st.nwt + __popcll(mcw) > nmem) { over |= ERR_REPAIR_CAP; break; }
-        if (com && pair) {
-            const int at = st.nt + rank_e;
-            etab[at] = stage_e[lane];
-            wflag_set(S, kf, WF_FIXUP);
-            wflag_set(S, kj, WF_FIXUP);
-            S.ov[(int64_t)s * SS + kf] = at;
-            S.evf[(int64_t)s * SS + kf] = oflags | EV_TABLE;
-            keep_block_rq(S, fs, rql);
-        }
-        if (com && wall) {
-            const int at = st.nwt + rank_w;
-            wtab[at] = stage_w_mine;
-            S.ovw[kf] = at;
-            wflag_set(S, kf, WF_REPAIR_WALL | WF_FIXUP);
-        }
-        put_hist_lanes(S, com && pair, fs, j, ps, over);
-        put_bond_lanes(S, com && pair, fs, j, ps.has_bond_rec, bond_from(ps, j), over);
-        int g = 0, gs = 0, kg = 0;
-        bool adds = false;
-        if (com && reshape) {
-            g = (wall || ridged == 0) ? f : j;
-            gs = (wall || ridged == 0) ? fs : js;
-            kg = (wall || ridged == 0) ? kf : kj;
-            set_cur(S, gs, nr, nh, nmass, ninertia, nhfa, nhfw);
-            // a wall is a floe's last event: nothing of it follows
-            adds = !wall && !(S.dirty[gs] & DIRTY_SHAPE);
-            dirty_set(S, gs, DIRTY_SHAPE);
-        }
-        st.nt += __popcll(mce);
-        st.nwt += __popcll(mcw);
-        st.repaired += __popcll(mce | mcw);
-        // the next round starts with the deferred keys, in order, then the
-        // keys after the batch; one equal to the batch's last key is dropped
-        // if that key is done (its first lane committed, or it repeats the
-        // key done before the batch)
-        const int64_t lastkey = __shfl(key, nb - 1);
-        const uint64_t same = __ballot(lane < nb && key == lastkey);
-        const int fl = __ffsll((long long)same) - 1;
-        // (a first lane that is not active repeats the key done before)
-        const bool last_done = __shfl((int)act, fl) ? !((defer >> fl) & 1ull) : true;
-        const int nd = __popcll(defer);
-        int skip = 0;
-        if (last_done)
-            while (nb + skip < np && pk[cb][head + nb + skip] == lastkey) ++skip;
-        st.last = last_done ? lastkey : -1;
-        wave_lds_sync();
-        // deferred keys go just before the keys after the batch
-        const int nhead = head + nb + skip - nd;
-        if ((defer >> lane) & 1ull) pk[cb][nhead + __popcll(defer & lt)] = key;
-        wave_lds_sync();
-        if (__ballot(over != 0)) break;
-        head = nhead;
-        np = np - nb - skip + nd;
-        if (!__ballot(adds)) continue;
-        // each committed reshape (of a floe not reshaped before) adds every
-        // later event of its floe g: one sorted run per reshape, the runs
-        // sorted together when there are several
-        const uint64_t madd = __ballot(adds);
-        const int rest = np;
-        int K = 0;
-        bool spill_heap = false;
-        for (uint64_t ma = madd; ma; ma &= ma - 1) {
-            const int cl = __ffsll((long long)ma) - 1;
-            const int gc = __shfl(g, cl), fc = __shfl(f, cl), kgc = __shfl(kg, cl);
-            const int sc = __shfl(s, cl);
-            const int gi = gc != fc ? S.icnt[kgc] : 0;
-            const int s0 = gc == fc ? sc + 1 : 0;
-            const int gno = S.ocnt[kgc];
-            const int kmax = gi + max(gno - s0, 0) + 1;
-            if (K + kmax > REPAIR_NCAP || rest + K + kmax > cap) { spill_heap = true; break; }
-            for (int q0 = 0; q0 < gi; q0 += 64) {
-                const int q = q0 + lane;
-                bool ok = false;
-                int64_t nkey = 0;
-                if (q < gi) {
-                    const int64_t ei = S.ik[(int64_t)q * SS + kgc];
-                    const int i2 = ent_id(ei);
-                    if (i2 > fc) {
-                        const int sk = slot_of(S, ent_pos(ei), gc);
-                        if (sk >= 0) { ok = true; nkey = ((int64_t)(i2 - first) << 16) | sk; }
-                    }
-                }
-                const uint64_t mk = __ballot(ok);
-                if (ok) nk[K + __popcll(mk & lt)] = nkey;
-                K += __popcll(mk);
-            }
-            for (int s2 = s0 + lane; s2 < gno; s2 += 64) nk[K + s2 - s0] = ((int64_t)(gc - first) << 16) | s2;
-            K += max(gno - s0, 0);
-            if (lane == 0) nk[K] = ((int64_t)(gc - first) << 16) | WALL_SLOT;
-            K += 1;
-        }
-        if (spill_heap) {
-            // too many pending keys for LDS: on to the heap in HBM
-            if (lane == 0) {
-                for (int i = 0; i < rest; ++i)
-                    if (!H.push((uint64_t)pk[cb][head + i])) over |= ERR_REPAIR_CAP;
-            }
-            for (uint64_t ma = madd; ma; ma &= ma - 1) {
-                const int cl = __ffsll((long long)ma) - 1;
-                const int gc = __shfl(g, cl), fc = __shfl(f, cl), kgc = __shfl(kg, cl);
-                const int sc = __shfl(s, cl);
-                if (lane == 0) push_later_events(S, H, first, fc, sc, gc, kgc, over);
-            }
-            serial = true;
+        const int nw = min(nw_, cap + hcap);
+        const bool stop = nw == 0 || over_ != 0 || round >= REPAIR_ROUNDS;
+        __syncthreads();
+        if (stop) {
+            if (round >= REPAIR_ROUNDS) over |= ERR_REPAIR_CAP;
             break;
         }
-        wave_lds_sync();
-        if (__popcll(madd) > 1) {
-            const int p2 = pow2_at_least(K);
-            for (int i = K + lane; i < p2; i += 64) nk[i] = INT64_MAX;
-            wave_lds_sync();
-            bitonic_inner(nk, p2, lane);
+        if (tid == 0) { nw_ = 0; nc_ = 0; }
+        // ---- their outcome, from the records before them
+        for (int w0 = 0; w0 < nw; w0 += width) {
+            const bool act = tid < width && w0 + tid < nw;
+            int kf = 0, kj = -1, s = WALL_SLOT, who = -1, hf = -1, hj = -1;
+            int64_t key = 0;
+            double nr = 0.0, nh = 0.0, nmass = 0.0, ninertia = 0.0, nhfa = 0.0, nhfw = 0.0;
+            if (act) {
+                const int wi = w0 + tid;
+                const uint64_t w = wi < cap ? wl[wi] : whbm[wi - cap];
+                kf = (int)(w >> 16);
+                s = (int)(w & 0xFFFF);
+                const int f = S.geo[kf].id;
+                key = ((int64_t)(f - first) << 16) | s;
+                hf = rhead_at(S, kf);
+                Floe Fi = floe_at(S, kf);
+                if (s == WALL_SLOT) {
+                    floe_at_event(rec, hf, key, Fi);
+                    double hist[4] = {0.0, 0.0, 0.0, 0.0};   // (no part in a reshape)
+                    WallOut W;
+                    walls<MIXED>(P, Fi, hist, W);
+                    who = (W.flags & 4u) ? 0 : -1;
+                    nr = W.nr; nh = W.nh; nmass = W.nmass; ninertia = W.ninertia; nhfa = W.nhfa; nhfw = W.nhfw;
+                } else {
+                    kj = ent_pos(S.oj[(int64_t)s * SS + kf]);
+                    hj = rhead_at(S, kj);
+                    Floe Fj = floe_at(S, kj);
+                    // the query radius: the outer floe's at the top of its iteration
+                    Floe Fq = Fi;
+                    floe_at_event(rec, hf, key & ~0xFFFFll, Fq);
+                    floe_at_event(rec, hf, key, Fi);
+                    floe_at_event(rec, hj, key, Fj);
+                    Kin kn;
+                    kinematics(Fi, Fj, kn);
+                    if (kn.dist <= Fq.r + P.rtree && kn.deltan > 0) {
+                        PairState ps{};                      // (no part in a reshape)
+                        EventOut o;
+                        o.flags = 0;
+                        o.ridged = -1;
+                        contact_part<MIXED>(P, Fi, Fj, kn, ps, o);
+                        if (o.flags & EV_RIDGED) {
+                            who = o.ridged;
+                            nr = o.nr; nh = o.nh; nmass = o.nmass; ninertia = o.ninertia; nhfa = o.nhfa; nhfw = o.nhfw;
+                        }
+                    }
+                }
+            }
+            __syncthreads();        // every outcome is known before a record changes
+            if (act) {
+                int xf = -1, xj = -1;      // the event's records, of either floe
+                for (int p = hf; p >= 0; p = rec[p].next)
+                    if (rec[p].key == key) xf = p;
+                for (int p = hj; p >= 0; p = rec[p].next)
+                    if (rec[p].key == key) xj = p;
+                if (xf >= 0 && who != 0 && rec[xf].live) { rec[xf].live = 0; put_change(xf); }
+                if (xj >= 0 && who != 1 && rec[xj].live) { rec[xj].live = 0; put_change(xj); }
+                if (who >= 0) {
+                    const int x = who == 0 ? xf : xj;
+                    if (x < 0) {
+                        const int p = atomicAdd(&nn_, 1);
+                        if (p < reccap) {
+                            add_reshape(S, rec, p, key, who == 0 ? kf : kj, kf, kj, nr, nh, nmass, ninertia, nhfa, nhfw);
+                            put_change(p);
+                        } else {
+                            over |= ERR_SEED_CAP;
+                        }
+                    } else if (!rec[x].live || rec[x].r != nr || rec[x].h != nh) {
+                        Reshape& w = rec[x];
+                        w.r = nr; w.h = nh; w.mass = nmass; w.inertia = ninertia; w.hfa = nhfa; w.hfw = nhfw;
+                        w.live = 1;
+                        put_change(x);
+                    }
+                }
+                if (s == WALL_SLOT) wflag_clear(S, kf, WF_PENDING);
+                else atomicAnd(&S.evf[(int64_t)s * SS + kf], ~EV_PENDING);
+            }
+            __syncthreads();
         }
-        // merge the two sorted runs (pending keys first among equals)
-        const int64_t* A = &pk[cb][head];
-        int64_t* O = pk[cb ^ 1];
-        for (int i = lane; i < rest; i += 64) O[i + count_below(nk, K, A[i], false)] = A[i];
-        for (int i = lane; i < K; i += 64) O[i + count_below(A, rest, nk[i], true)] = nk[i];
-        wave_lds_sync();
-        cb ^= 1;
-        head = 0;
-        np = rest + K;
+        nchg = min(nc_, cap + hcap);
+        seeds = false;
+        if (nchg == 0) break;
     }
-    if (serial && lane == 0)
-        repair_serial<MIXED>(S, P, first, nmem, tstep, H, etab, tcap, wtab, st, over);
-    if (lane == 0) {
-        S.netab[m] = st.nt;
-        S.nwtab[m] = st.nwt;
+    if (over) atomicOr(&over_, over);
+    __syncthreads();
+    if (over_) {
+        if (tid == 0) set_err(S, over_);
+        return;
+    }
+    // ---- the floes whose terms change: those of every event with a record,
+    // every reshaped floe, and the partners of its later events that can
+    // notice (in contact, bonded, or near enough for their own sheltering).
+    // Counted on the way: the seeds and the events after a reshape of one of
+    // their floes (each once).
+    const int nn = nn_;
+    const bool bond_step = tstep == 1 && P.restart != 1 && P.cohesion;
+    int counted = 0;
+    const int rpw = share(nn);
+    for (int c0 = 0; c0 < nn; c0 += waves * rpw) {
+        const int p = c0 + (tid >> 6) * rpw + lane;
+        const bool act = lane < rpw && p < nn;
+        int kg = 0, gid = 0, bown = 0, wall = 0;
+        int64_t key = 0;
+        LaterEvents l{0, 0, 0, 0};
+        GeoRec gg;
+        gg.x = gg.y = gg.r = 0.0;
+        if (act) {
+            key = rec[p].key;
+            kg = rec[p].pos;
+            const int kf = rec[p].kf, kj = rec[p].kj;
+            touch_floe(S, kf);
+            if (kj >= 0) touch_floe(S, kj);
+            gg = S.geo[kg];
+            gid = gg.id;
+            const int hk = rhead_at(S, kg);
+            const int64_t k0 = first_reshape(rec, hk);
+            if (p < ns) {
+                // a seed that is not after a reshape of either floe
+                const int ko = kg == kf ? kj : kf;
+                const int64_t ko0 = ko >= 0 ? first_reshape(rec, rhead_at(S, ko)) : INT64_MAX;
+                if (!(k0 < key) && !(ko0 < key)) ++counted;
+            }
+            if (rec[p].live && k0 == key) {
+                l = later_events(S, key, kg, gid, first);
+                wall = (key & 0xFFFF) != WALL_SLOT ? 1 : 0;
+                bown = S.bcnt_old[S.cval[kg]];
+            }
+        }
+        counted += wall;
+        each_later(l.ni + l.no, [&](int own, int local) {
+            const int ko = __shfl(kg, own), go = __shfl(gid, own), fo = __shfl(l.f, own);
+            const int nio = __shfl(l.ni, own), s0 = __shfl(l.s0, own), bo = __shfl(bown, own);
+            const double ox = __shfl(gg.x, own), oy = __shfl(gg.y, own), orr = __shfl(gg.r, own);
+            if (local < 0) return;
+            const bool inner = local < nio;
+            const int64_t e = inner ? S.ik[(int64_t)local * SS + ko]
+                                    : S.oj[(int64_t)(s0 + local - nio) * SS + ko];
+            const int q = ent_pos(e);
+            if (inner && ent_id(e) - first <= fo) return;     // before the reshape
+            const GeoRec o = S.geo[q];
+            const ShelRec sh = S.shel[q];
+            const int hq = rhead_at(S, q);
+            const int bc = inner ? S.bcnt_old[S.cval[q]] : bo;
+            // the partner's own reshape may come before the event too: counted
+            // from the outer floe's side
+            bool both = false;
+            if (hq >= 0) {
+                const int64_t ek = inner ? ((int64_t)(ent_id(e) - first) << 16) | slot_of(S, q, go)
+                                         : ((int64_t)(go - first) << 16) | (s0 + local - nio);
+                both = first_reshape(rec, hq) < ek;
+            }
+            if (!(both && inner)) ++counted;
+            const double dx = inner ? o.x - ox : ox - o.x, dy = inner ? o.y - oy : oy - o.y;
+            const double dn = (inner ? o.r + orr : orr + o.r) - sqrt(dx * dx + dy * dy);
+            // (radii only shrink: a term that is exactly 1 stays so)
+            using T = typename Prec<MIXED>::T;
+            const T lim = sizeof(T) == 4 ? T(20) : T(40), dnt = T(dn);
+            const bool far = dnt < T(0) && T((double)0.18f) * -dnt >= lim * T(sh.hfa) &&
+                             T((double)0.18f) * -dnt >= lim * T(sh.hfw);
+            if (dn > 0 || bc > 0 || (bond_step && dn >= -P.bond_lim) || (P.shelter && !far)) touch_floe(S, q);
+        });
+    }
+    atomicAdd(&rep_, counted);
+    __syncthreads();
+    if (tid == 0) {
         S.stats[4 * m + 2] = ns;
-        S.stats[4 * m + 3] = st.repaired;
+        S.stats[4 * m + 3] = rep_;
     }
-    if (over) set_err(S, over);
 }
 
 // ---------------------------------------------------------------------
@@ -2923,6 +2626,9 @@ __global__ __launch_bounds__(64) void k_repair(DS S, int nmembers) {
 // wavefront: one pass of 64 results).
 constexpr int FIX_LDS_PER_WAVE = 64 * (int)sizeof(EventOut);
 static_assert(sizeof(EventOut) % 8 == 0, "EventOut is copied in 8-byte words");
+// (LDS copies only) the event's new contact history, in nr, nh, nmass,
+// ninertia, is to be appended to the owner's list for partner `ridged`
+constexpr uint32_t EV_PUT_HIST = 1u << 15;
 
 __device__ __forceinline__ void copy_event(EventOut* dst, const EventOut* src) {
     const uint64_t* s = reinterpret_cast<const uint64_t*>(src);
@@ -2931,20 +2637,68 @@ __device__ __forceinline__ void copy_event(EventOut* dst, const EventOut* src) {
     for (int w = 0; w < (int)(sizeof(EventOut) / 8); ++w) d[w] = s[w];
 }
 
+// Where the records of pair (i, j), owner i by storage slot and partner j by
+// identity, are in the owner's lists, old and new (-1: none).  The counts and
+// the first two partners of all four lists are requested together.
+struct PairRefs { int hist, bond, hist_new, bond_new; };
+__device__ __forceinline__ PairRefs find_pair(const DS& S, int i, int j) {
+    const int64_t SS = S.S;
+    const int64_t h1 = (int64_t)min(1, S.HC - 1) * SS + i, b1 = (int64_t)min(1, S.BC - 1) * SS + i;
+    const int n[4] = {S.hcnt_old[i], S.bcnt_old[i], S.hcnt_new[i], S.bcnt_new[i]};
+    const int j0[4] = {S.hist_old[i].j, S.bond_old[i].j, S.hist_new[i].j, S.bond_new[i].j};
+    const int j1[4] = {S.hist_old[h1].j, S.bond_old[b1].j, S.hist_new[h1].j, S.bond_new[b1].j};
+    int q[4];
+#pragma unroll
+    for (int l = 0; l < 4; ++l) q[l] = (n[l] > 0 && j0[l] == j) ? 0 : (n[l] > 1 && j1[l] == j) ? 1 : -1;
+    for (int p = 2; q[0] < 0 && p < n[0]; ++p) if (S.hist_old[(int64_t)p * SS + i].j == j) q[0] = p;
+    for (int p = 2; q[1] < 0 && p < n[1]; ++p) if (S.bond_old[(int64_t)p * SS + i].j == j) q[1] = p;
+    for (int p = 2; q[2] < 0 && p < n[2]; ++p) if (S.hist_new[(int64_t)p * SS + i].j == j) q[2] = p;
+    for (int p = 2; q[3] < 0 && p < n[3]; ++p) if (S.bond_new[(int64_t)p * SS + i].j == j) q[3] = p;
+    PairRefs r;
+    r.hist = q[0]; r.bond = q[1]; r.hist_new = q[2]; r.bond_new = q[3];
+    return r;
+}
+// The pair's old state (contact history, bond record) at those places.
+__device__ __forceinline__ void pair_state_at(const DS& S, int i, const PairRefs& r, PairState& ps) {
+    ps.deltat = 0.0; ps.thetarelc = 0.0; ps.fcn = 0.0; ps.fct = 0.0;
+    ps.bond = 0; ps.has_bond_rec = false;
+    ps.damage = ps.deltanb = ps.deltatb = ps.trb_ji = ps.trb_ij = 0.0;
+    ps.rb = ps.hb = ps.lb = ps.sb = ps.ib = 0.0;
+    if (r.hist >= 0) {
+        const HistRec& hr = S.hist_old[(int64_t)r.hist * S.S + i];
+        ps.deltat = hr.deltat; ps.thetarelc = hr.thetarelc; ps.fcn = hr.fcn; ps.fct = hr.fct;
+    }
+    if (r.bond >= 0) {
+        const BondRec& b = S.bond_old[(int64_t)r.bond * S.S + i];
+        ps.has_bond_rec = true; ps.bond = b.bond; ps.damage = b.damage;
+        ps.deltanb = b.deltanb; ps.deltatb = b.deltatb; ps.trb_ji = b.trb_ji; ps.trb_ij = b.trb_ij;
+        ps.rb = b.rb; ps.hb = b.hb; ps.lb = b.lb; ps.sb = b.sb; ps.ib = b.ib;
+    }
+}
+
 // The floes the repair touched re-gather every event of theirs, in the
 // reference's order (inner pairs by ascending outer index, then their own
-// candidates in distance order): the repair's result where the table holds
-// one, else the event evaluated again (its inputs are final).  All the
+// candidates in distance order), each event with the properties its floes
+// have at its place in the sequence (their reshape records).  The owner's new
+// pair state and flags are written again from these results; a pair that is
+// no longer a candidate when its outer floe's turn comes (the query radius
+// shrank) keeps its old state.  Pairs that add nothing (apart, not bonded,
+// too far to shelter) are passed over after their distance.  All the
 // wavefront's events are evaluated together, 64 a pass (each lane finds its
 // event's floe among the lanes), and after each pass every floe adds its own
 // in order, so that a floe with many candidates does not hold one lane
-// through all of them.
+// through all of them.  It is bound by the chain of loads of one event (queue
+// -> list entry -> rows -> the owner's lists -> records), so each round of
+// that chain requests all it can at once.  (One MI355X: 0.025-0.028 ms with a
+// few to a few thousand touched floes of sparse fields, 0.033 for 24 dense
+// fields, 0.10 when every partner of a reshaped floe was gathered again.)
 template <bool MIXED>
 __global__ __launch_bounds__(FLOE_BLOCK, 2) void k_fixup(DS S) {
+    using T = typename Prec<MIXED>::T;
     extern __shared__ unsigned char fix_lds[];
     EventOut* ev = reinterpret_cast<EventOut*>(fix_lds + (threadIdx.x >> 6) * FIX_LDS_PER_WAVE);
-    // The floes the repair touched (the fixup queue, filled by k_fixq), a few
-    // per wavefront: every wavefront of the grid (about one resident round)
+    // The touched floes (the fixup queue, filled by k_repair), a few per
+    // wavefront: every wavefront of the grid (about one resident round)
     // takes F consecutive entries, F as small as the queue allows, so that
     // the floes' re-gathers run side by side rather than in a few long
     // wavefronts.
@@ -2967,6 +2721,7 @@ __global__ __launch_bounds__(FLOE_BLOCK, 2) void k_fixup(DS S) {
         const int f = act ? S.geo[k].id : 0;
         const int fs = act ? (int)S.cval[k] : 0;
         const int ni = act ? S.icnt[k] : 0, no = act ? S.ocnt[k] : 0;
+        const int hk = act ? S.rhead[k] : -1;
         const int cnt = ni + no;
         int incl = cnt;
 #pragma unroll
@@ -2978,6 +2733,7 @@ __global__ __launch_bounds__(FLOE_BLOCK, 2) void k_fixup(DS S) {
         const int64_t SS = S.S;
         double acc[NACC];
         acc_init(acc);
+        uint32_t over = 0;
         for (int c0 = 0; c0 < total; c0 += 64) {
             const int idx = c0 + lane;
             int own = 0;
@@ -2986,49 +2742,149 @@ __global__ __launch_bounds__(FLOE_BLOCK, 2) void k_fixup(DS S) {
                 if (__shfl(start, own + step) <= idx) own += step;
             const int ko = __shfl(k, own), om = __shfl(m, own), of = __shfl(f, own);
             const int ofs = __shfl(fs, own), oni = __shfl(ni, own), ostart = __shfl(start, own);
+            const int oh = __shfl(hk, own);
+            bool adds = false;
             if (idx < total) {
                 const DevParams& P = S.params[om];
-                const int tstep = S.members[om].tstep;
-                const int first = S.members[om].first;
-                const EventOut* etab = S.etab + (int64_t)S.TABK * first;
+                const Member Mb = S.members[om];
+                const int rst = P.restart, coh = P.cohesion, shl = P.shelter;
+                const double rtree = P.rtree, blim = P.bond_lim;
+                const int tstep = Mb.tstep, first = Mb.first;
+                const Reshape* rec = S.shape + (int64_t)S.SEEDK * first;
                 const int local = idx - ostart;
                 const bool inner = local < oni;
-                int tab = -1, qp = 0, pid = 0;
-                if (inner) {
-                    const int64_t e = S.ik[(int64_t)local * SS + ko];
-                    pid = ent_id(e);
-                    qp = ent_pos(e);
-                    const int sk = slot_of(S, qp, of);
-                    tab = sk >= 0 && (S.evf[(int64_t)sk * SS + qp] & EV_TABLE) ? S.ov[(int64_t)sk * SS + qp] : -1;
-                } else {
-                    const int s2 = local - oni;
-                    tab = (S.evf[(int64_t)s2 * SS + ko] & EV_TABLE) ? S.ov[(int64_t)s2 * SS + ko] : -1;
-                    const int64_t e = S.oj[(int64_t)s2 * SS + ko];
-                    pid = ent_id(e);
-                    qp = ent_pos(e);
+                const int64_t e = inner ? S.ik[(int64_t)local * SS + ko] : S.oj[(int64_t)(local - oni) * SS + ko];
+                const int pid = ent_id(e), qp = ent_pos(e);
+                // outer floe a, inner floe b; their rows, requested at once
+                const int ka = inner ? qp : ko, kb = inner ? ko : qp;
+                const int ia = inner ? pid : of, ib = inner ? of : pid;
+                const int hq = S.rhead[qp];
+                const int sq = S.cval[qp];
+                Floe Fa = floe_at(S, ka), Fb = floe_at(S, kb);
+                const double2 wa = wind_at(S, ka);
+                const int sa = inner ? sq : ofs;
+                // the owner's lists, old and new
+                const PairRefs pr = find_pair(S, sa, ib);
+                const double dx = Fa.x - Fb.x, dy = Fa.y - Fb.y;
+                const double d = sqrt(dx * dx + dy * dy);
+                const double dn = Fa.r + Fb.r - d;
+                // the properties at the event, the outer floe's radius at the
+                // top of its iteration
+                bool removed = false;
+                EventOut o;
+                o.ridged = -1;
+                // the event's own record: the floe it reshapes, and to what
+                auto own_record = [&](const Reshape& w, int side) {
+                    if (w.kf != ka || w.kj != kb) return;
+                    o.ridged = side;
+                    o.nr = w.r; o.nh = w.h; o.nmass = w.mass;
+                    o.ninertia = w.inertia; o.nhfa = w.hfa; o.nhfw = w.hfw;
+                };
+                if ((oh >= 0) | (hq >= 0)) {
+                    const int al = ia - first;
+                    int sl = inner ? -1 : local - oni;      // (the slot of an inner pair only where it decides)
+                    // last record before the event: of a, of b; of a before its
+                    // iteration
+                    int wa_ = -1, wb_ = -1, wq_ = -1;
+                    int64_t ka_ = -1, kb_ = -1, kq_ = -1;
+                    auto before = [&](const Reshape& w) {
+                        const int rf = (int)(w.key >> 16);
+                        if (rf != al) return rf < al;
+                        if (w.kf == ka && w.kj == kb) return false;   // the event's own
+                        if (sl < 0) sl = slot_of(S, qp, of);
+                        return (int)(w.key & 0xFFFF) < sl;
+                    };
+                    for (int p = inner ? hq : oh; p >= 0; p = rec[p].next) {
+                        const Reshape& w = rec[p];
+                        if (!w.live) continue;
+                        own_record(w, 0);
+                        if ((int)(w.key >> 16) < al && w.key > kq_) { kq_ = w.key; wq_ = p; }
+                        if (w.key > ka_ && before(w)) { ka_ = w.key; wa_ = p; }
+                    }
+                    for (int p = inner ? oh : hq; p >= 0; p = rec[p].next) {
+                        const Reshape& w = rec[p];
+                        if (!w.live) continue;
+                        own_record(w, 1);
+                        if (w.key > kb_ && before(w)) { kb_ = w.key; wb_ = p; }
+                    }
+                    const double rq = wq_ >= 0 ? rec[wq_].r : Fa.r;
+                    removed = !(d <= rq + rtree);
+                    if (wa_ >= 0) take_shape(rec[wa_], Fa);
+                    if (wb_ >= 0) take_shape(rec[wb_], Fb);
                 }
-                if (tab >= 0) {
-                    copy_event(&ev[lane], &etab[tab]);
-                    if (ev[lane].flags & EV_REMOVED) ev[lane].flags = 0;   // adds nothing
-                } else {
-                    // inner: pair (i, f) with i's wind; outer: pair (f, j) with f's wind
+                // (the start-of-step overlap is the largest the pair can have)
+                const T lim = sizeof(T) == 4 ? T(20) : T(40), dnt = T(dn);
+                const bool far = dnt < T(0) && T((double)0.18f) * -dnt >= lim * T(inner ? Fb.hfa : Fa.hfa) &&
+                                 T((double)0.18f) * -dnt >= lim * T(inner ? Fb.hfw : Fa.hfw);
+                const bool bond_step = (tstep == 1) & (rst != 1) & (coh != 0);
+                adds = dn > 0 || pr.bond >= 0 || (bond_step && dn >= -blim) || (shl && !far) || removed ||
+                       (S.record_forces && !inner && oh >= 0);
+                if (adds) {
                     PairState ps;
-                    load_pair_state<1>(S, inner ? (int)S.cval[qp] : ofs, inner ? of : pid, ps);
-                    const double2 w = wind_at(S, inner ? qp : ko);
-                    Floe Fa = floe_at(S, inner ? qp : ko), Fb = floe_at(S, inner ? ko : qp);
-                    EventOut o;
-                    pair_event<MIXED>(P, tstep, (inner ? pid : of) - first, (inner ? of : pid) - first,
-                                      Fa, Fb, w.x, w.y, P.uw, P.vw, ps, o, inner ? 2 : 1);
+                    pair_state_at(S, sa, pr, ps);
+                    if (removed) {
+                        // no longer a candidate: the pair keeps its old state
+                        o.flags = EV_REMOVED;
+                        o.sc = o.sbd = o.sri = 0.0;
+                    } else {
+                        pair_event<MIXED>(P, tstep, ia - first, ib - first, Fa, Fb, wa.x, wa.y, P.uw, P.vw,
+                                          ps, o, inner ? 2 : 1);
+                    }
+                    if (!inner) {
+                        const int64_t at = (int64_t)(local - oni) * SS + ko;
+                        S.evf[at] = (S.evf[at] & 0xffff0000u) | o.flags | (S.record_forces ? EV_SRI : 0u);
+                        if (S.record_forces) { S.ssc[at] = o.sc; S.ssb[at] = o.sbd; S.od[at] = o.sri; }
+                        // the pair's new records, each in its place; a history
+                        // with no place yet is the owner's lane's to append
+                        if (pr.bond_new >= 0) {
+                            if (ps.has_bond_rec) S.bond_new[(int64_t)pr.bond_new * SS + ofs] = bond_from(ps, pid);
+                            else S.bond_new[(int64_t)pr.bond_new * SS + ofs].j = -1;
+                        } else if (ps.has_bond_rec) {
+                            const int p = atomicAdd(&S.bcnt_new[ofs], 1);
+                            if (p < S.BC) S.bond_new[(int64_t)p * SS + ofs] = bond_from(ps, pid);
+                            else over |= ERR_BOND_CAP;
+                        }
+                        const bool hist = ps.deltat != 0.0 || ps.thetarelc != 0.0 || ps.fcn != 0.0 || ps.fct != 0.0;
+                        HistRec hr;
+                        hr.j = hist ? pid : -1; hr.pad_ = 0;
+                        hr.deltat = ps.deltat; hr.thetarelc = ps.thetarelc; hr.fcn = ps.fcn; hr.fct = ps.fct;
+                        if (pr.hist_new >= 0) {
+                            S.hist_new[(int64_t)pr.hist_new * SS + ofs] = hr;
+                        } else if (hist) {
+                            o.nr = hr.deltat; o.nh = hr.thetarelc; o.nmass = hr.fcn; o.ninertia = hr.fct;
+                            o.ridged = pid;
+                            o.flags |= EV_PUT_HIST;
+                        }
+                    }
                     copy_event(&ev[lane], &o);
                 }
             }
+            const uint64_t am = __ballot(adds);
             wave_lds_sync();
             // every floe adds this pass's events of its own, in order
             if (act) {
-                const int lo = max(start, c0), hi = min(start + cnt, c0 + 64);
-                for (int i2 = lo; i2 < hi; ++i2) {
-                    if (i2 - start < ni) apply_j(acc, ev[i2 - c0]);
-                    else apply_i(acc, ev[i2 - c0]);
+                const int lo = max(start, c0) - c0, hi = min(start + cnt, c0 + 64) - c0;
+                uint64_t mine = hi > lo ? am & (~0ull >> (64 - hi)) & (~0ull << lo) : 0ull;
+                for (; mine; mine &= mine - 1) {
+                    const int i2 = __ffsll((long long)mine) - 1;
+                    const EventOut& o = ev[i2];
+                    if (c0 + i2 - start < ni) {
+                        apply_j(acc, o);
+                    } else {
+                        apply_i(acc, o);
+                        if (o.flags & EV_PUT_HIST) {
+                            const int n = S.hcnt_new[fs];
+                            if (n < S.HC) {
+                                HistRec hr;
+                                hr.j = o.ridged; hr.pad_ = 0;
+                                hr.deltat = o.nr; hr.thetarelc = o.nh; hr.fcn = o.nmass; hr.fct = o.ninertia;
+                                S.hist_new[(int64_t)n * SS + fs] = hr;
+                                S.hcnt_new[fs] = n + 1;
+                            } else {
+                                over |= ERR_HIST_CAP;
+                            }
+                        }
+                    }
                 }
             }
             wave_lds_sync();
@@ -3037,16 +2893,32 @@ __global__ __launch_bounds__(FLOE_BLOCK, 2) void k_fixup(DS S) {
 #pragma unroll
             for (int a = 0; a < NACC; ++a) S.acc[a * SS + k] = acc[a];
             S.cls[k] = CLS_CONTACT | CLS_BOND;
+            if (hk >= 0) {
+                const Member Mb = S.members[m];
+                const Reshape* rec = S.shape + (int64_t)S.SEEDK * Mb.first;
+                const DevParams& P = S.params[m];
+                if (S.wflag[k] & WF_WALL) {
+                    // its walls, with the properties it has when their turn comes
+                    Floe Fw = floe_at(S, k);
+                    floe_at_event(rec, hk, ((int64_t)(f - Mb.first) << 16) | WALL_SLOT, Fw);
+                    double hist[4] = {S.wbc[0 * SS + fs], S.wbc[1 * SS + fs], S.wbc[2 * SS + fs], S.wbc[3 * SS + fs]};
+                    WallOut W;
+                    walls<MIXED>(P, Fw, hist, W);
+                    if (W.flags & 1u) S.wout[k] = W;
+                    else wflag_clear(S, k, WF_WALL);
+                }
+                // the properties the step leaves it with
+                if (first_reshape(rec, hk) != INT64_MAX) {
+                    Floe Fn;
+                    floe_at_event(rec, hk, INT64_MAX, Fn);
+                    S.cur[0 * SS + fs] = Fn.r; S.cur[1 * SS + fs] = Fn.h; S.cur[2 * SS + fs] = Fn.mass;
+                    S.cur[3 * SS + fs] = Fn.inertia; S.cur[4 * SS + fs] = Fn.hfa; S.cur[5 * SS + fs] = Fn.hfw;
+                    S.dirty[fs] = 1;
+                }
+            }
         }
+        if (over) set_err(S, over);
     }
-}
-
-// The positions the repair touched (WF_FIXUP) into the fixup queue, one
-// atomic per wavefront; the grid is laid out as the candidate search's.
-__global__ __launch_bounds__(FLOE_BLOCK) void k_fixq(DS S) {
-    const int k = xcd_block() * blockDim.x + threadIdx.x;
-    const bool want = k < S.N && !*S.err && (S.wflag[k] & WF_FIXUP);
-    enqueue(S, want, 4, k);
 }
 
 // ---------------------------------------------------------------------
@@ -3071,7 +2943,6 @@ __global__ __launch_bounds__(FLOE_BLOCK) void k_stress(DS S) {
     if (m < 0) return;
     const int f = me.id;
     const int64_t SS = S.S;
-    const EventOut* etab = S.etab + (int64_t)S.TABK * S.members[m].first;
     double a[NACC];
     a[A_SXX] = a[A_SYY] = a[A_SXY] = a[A_SYX] = 0.0;
     // pairs (i, f), f inner, ascending i
@@ -3081,16 +2952,12 @@ __global__ __launch_bounds__(FLOE_BLOCK) void k_stress(DS S) {
         const int qi = ent_pos(e);
         const int s = slot_of(S, qi, f);
         if (s < 0) continue;
-        const int idx = (S.evf[(int64_t)s * SS + qi] & EV_TABLE) ? S.ov[(int64_t)s * SS + qi] : -1;
+        const int64_t at = (int64_t)s * SS + qi;
+        const uint32_t fl = S.evf[at];
+        if (fl & EV_REMOVED) continue;
         const GeoRec gi = S.geo[qi];
-        double sc, sb, ri;
-        if (idx >= 0) {
-            const EventOut& o = etab[idx];
-            if (o.flags & EV_REMOVED) continue;
-            sc = o.sc; sb = o.sbd; ri = o.sri;
-        } else {
-            sc = S.ssc[(int64_t)s * SS + qi]; sb = S.ssb[(int64_t)s * SS + qi]; ri = gi.r;
-        }
+        const double sc = S.ssc[at], sb = S.ssb[at];
+        const double ri = (fl & EV_SRI) ? S.od[at] : gi.r;
         const double dx = gi.x - me.x, dy = gi.y - me.y;
         const double dist = sqrt(dx * dx + dy * dy);
         const double c = (me.x - gi.x) / dist, sn = (me.y - gi.y) / dist;
@@ -3101,15 +2968,11 @@ __global__ __launch_bounds__(FLOE_BLOCK) void k_stress(DS S) {
     for (int s = 0; s < no; ++s) {
         const int64_t e = S.oj[s * SS + k];
         const int qj = ent_pos(e);
-        const int idx = (S.evf[s * SS + k] & EV_TABLE) ? S.ov[s * SS + k] : -1;
-        double sc, sb, ri;
-        if (idx >= 0) {
-            const EventOut& o = etab[idx];
-            if (o.flags & EV_REMOVED) continue;
-            sc = o.sc; sb = o.sbd; ri = o.sri;
-        } else {
-            sc = S.ssc[s * SS + k]; sb = S.ssb[s * SS + k]; ri = me.r;
-        }
+        const int64_t at = (int64_t)s * SS + k;
+        const uint32_t fl = S.evf[at];
+        if (fl & EV_REMOVED) continue;
+        const double sc = S.ssc[at], sb = S.ssb[at];
+        const double ri = (fl & EV_SRI) ? S.od[at] : me.r;
         const GeoRec gj = S.geo[qj];
         const double dx = me.x - gj.x, dy = me.y - gj.y;
         const double dist = sqrt(dx * dx + dy * dy);
@@ -3149,15 +3012,13 @@ __global__ __launch_bounds__(FLOE_BLOCK, (MIXED && !REC) ? 5 : 4) void k_final(D
     const DevParams& P = S.params[m];
     const int64_t SS = S.S;
     const uint8_t dflags = S.dirty[f];
-    const bool dirty = (dflags & DIRTY_SHAPE) != 0;
+    const bool dirty = dflags != 0;
     if (dirty) {
         F.r = S.cur[0 * SS + f]; F.h = S.cur[1 * SS + f]; F.mass = S.cur[2 * SS + f];
         F.inertia = S.cur[3 * SS + f]; F.hfa = S.cur[4 * SS + f]; F.hfw = S.cur[5 * SS + f];
     }
     WallOut W;
-    if (wf & WF_REPAIR_WALL) {
-        W = S.wtab[S.members[m].first + S.ovw[k]];   // recomputed by the repair
-    } else if (wf & WF_WALL) {
+    if (wf & WF_WALL) {
         W = S.wout[k];
     } else {
         // no wall touched: reset_boundary(i, 0) cleared every wall history

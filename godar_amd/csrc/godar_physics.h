@@ -165,7 +165,11 @@ __device__ __forceinline__ void bond_create(const DevParams& P, int tstep, int g
 // Contact of a pair with deltan > 0: contact_forces (contact_forces.f90:1-87)
 // with plastic_contact/update_shape (ridging.f90:1-99) and coulomb
 // (physics.f90:1-33).  fi/fj are reshaped in place when ridging occurs.
-template <bool MIXED>
+// KNOWN: o already holds what update_shape leaves (ridged and the six new
+// properties, from an evaluation with the same floes), so the lens area's
+// two arc cosines, the longest chain of the event in FP64, are not taken
+// again.
+template <bool MIXED, bool KNOWN = false>
 __device__ __forceinline__ void contact_part(const DevParams& P, Floe& fi, Floe& fj, const Kin& k,
                                              PairState& ps, EventOut& o) {
     using T = typename Prec<MIXED>::T;
@@ -206,27 +210,38 @@ __device__ __forceinline__ void contact_part(const DevParams& P, Floe& fi, Floe&
             fcn = dmin(fcn, snc * h2 * dr);
             fct = ktc * T(ps.deltat) - gamt * T(k.velt);
             // update_shape, ridging.f90:36-99 (FP64 volume bookkeeping)
-            double hmin64 = fmin(fi.h, fj.h);
-            double ri = fi.r, rj = fj.r;
-            double dij = (dist * dist - rj * rj + ri * ri) / (2.0 * dist);
-            double dji = (dist * dist - ri * ri + rj * rj) / (2.0 * dist);
-            double area = ri * ri * ridge_acos<MIXED>(dij / ri) - dij * delt_ridge / 2.0
-                        + rj * rj * ridge_acos<MIXED>(dji / rj) - dji * delt_ridge / 2.0;
-            double vol = fmax(area * hmin64 / 2.0, 0.0);
-            // the thinner floe is reshaped; its six properties are selected
-            // field by field (a pointer to either floe, or a select of whole
-            // records, would force both floes out of registers)
             int who = -1;
-            if (hmin64 == fi.h) who = 0;
-            else if (hmin64 == fj.h) who = 1;
+            Floe w;
+            if constexpr (KNOWN) {
+                who = o.ridged;
+                w.r = o.nr; w.h = o.nh; w.mass = o.nmass;
+                w.inertia = o.ninertia; w.hfa = o.nhfa; w.hfw = o.nhfw;
+            } else {
+                double hmin64 = fmin(fi.h, fj.h);
+                double ri = fi.r, rj = fj.r;
+                double dij = (dist * dist - rj * rj + ri * ri) / (2.0 * dist);
+                double dji = (dist * dist - ri * ri + rj * rj) / (2.0 * dist);
+                double area = ri * ri * ridge_acos<MIXED>(dij / ri) - dij * delt_ridge / 2.0
+                            + rj * rj * ridge_acos<MIXED>(dji / rj) - dji * delt_ridge / 2.0;
+                double vol = fmax(area * hmin64 / 2.0, 0.0);
+                // the thinner floe is reshaped; its six properties are selected
+                // field by field (a pointer to either floe, or a select of whole
+                // records, would force both floes out of registers)
+                if (hmin64 == fi.h) who = 0;
+                else if (hmin64 == fj.h) who = 1;
+                if (who >= 0) {
+                    const double rw = who == 0 ? fi.r : fj.r;
+                    const double hw = who == 0 ? fi.h : fj.h;
+                    double dh = vol / (P.pi * (rw * rw));
+                    w.r = rw * sqrt(hw / (hw + dh));
+                    w.h = hw + dh;
+                    floe_properties(P, w);
+                    o.ridged = who;
+                    o.nr = w.r; o.nh = w.h; o.nmass = w.mass;
+                    o.ninertia = w.inertia; o.nhfa = w.hfa; o.nhfw = w.hfw;
+                }
+            }
             if (who >= 0) {
-                Floe w;
-                const double rw = who == 0 ? fi.r : fj.r;
-                const double hw = who == 0 ? fi.h : fj.h;
-                double dh = vol / (P.pi * (rw * rw));
-                w.r = rw * sqrt(hw / (hw + dh));
-                w.h = hw + dh;
-                floe_properties(P, w);
                 const bool wi = who == 0;
                 fi.r = wi ? w.r : fi.r;             fj.r = wi ? fj.r : w.r;
                 fi.h = wi ? w.h : fi.h;             fj.h = wi ? fj.h : w.h;
@@ -236,9 +251,6 @@ __device__ __forceinline__ void contact_part(const DevParams& P, Floe& fi, Floe&
                 fi.hfa = wi ? w.hfa : fi.hfa;       fj.hfa = wi ? fj.hfa : w.hfa;
                 fi.hfw = wi ? w.hfw : fi.hfw;       fj.hfw = wi ? fj.hfw : w.hfw;
                 o.flags |= EV_RIDGED;
-                o.ridged = who;
-                o.nr = w.r; o.nh = w.h; o.nmass = w.mass;
-                o.ninertia = w.inertia; o.nhfa = w.hfa; o.nhfw = w.hfw;
             }
             delt_ridge = delt_ridge_of(fi.r, fj.r, dist);
             dr = T(delt_ridge);
@@ -385,21 +397,21 @@ __device__ __forceinline__ double stale_contact_magnitude(const PairState& ps) {
 }
 
 // One pair event (i < j), the body of stepper.f90:89-271 for one (j,i).
-// fi/fj are updated in place if ridging reshapes one of them.  ps is updated
-// to the pair's new state.  Returns the gather terms in `o`.
+// fi/fj are updated in place if ridging reshapes one of them, to the
+// properties o holds (contact_part's KNOWN).  ps is updated to the pair's new
+// state.  Returns the gather terms in `o`.
 template <bool MIXED>
 __device__ __forceinline__ void pair_event(const DevParams& P, int tstep, int gi, int gj,
                                            Floe& fi, Floe& fj, double uai, double vai,
                                            double uwi, double vwi, PairState& ps,
                                            EventOut& o, int side = 0) {
     o.flags = 0;
-    o.ridged = -1;
     o.sbd = 0.0;
     Kin k;
     kinematics(fi, fj, k);
     bond_create(P, tstep, gi, gj, fi, fj, k, ps);
     if (k.deltan > 0) {
-        contact_part<MIXED>(P, fi, fj, k, ps, o);
+        contact_part<MIXED, true>(P, fi, fj, k, ps, o);
     } else {
         // reset_contact, reset.f90:1-15; the last contact forces stay
         ps.thetarelc = 0.0;

@@ -109,8 +109,20 @@ struct HistRec {
     double deltat, thetarelc, fcn, fct;
 };
 
-// Per-event result the gather needs, kept in the repair table for events
-// the ordered repair recomputed.  Field names follow the stepper.f90
+// A reshape of a floe by one event of the step (ridging): the event's key
+// (outer local index << 16 | slot; slot WALL_SLOT: the floe's walls), the
+// properties it leaves the floe with, the next record of the same floe.
+struct Reshape {
+    int64_t key;
+    double r, h, mass, inertia, hfa, hfw;
+    int32_t pos;           // position of the reshaped floe
+    int32_t next;          // next record of the floe (member's record index), -1: none
+    int32_t kf, kj;        // positions of the event's outer and inner floe (-1: walls)
+    int32_t live;          // 0: the event no longer reshapes this floe
+    int32_t pad_;
+};
+
+// Per-event result the gather needs.  Field names follow the stepper.f90
 // accumulation lines (113-146 contact, 165-198 bond, 215-223 shelter).
 struct EventOut {
     uint32_t flags;        // EV_* bits
@@ -135,7 +147,8 @@ enum : uint32_t {
     EV_RIDGED  = 1u << 2,
     EV_REMOVED = 1u << 3,   // no longer a candidate (query radius shrank)
     EV_SHELTER = 1u << 4,
-    EV_TABLE   = 1u << 5,   // (evf only) the repair table holds the event: ov is its entry
+    EV_PENDING = 1u << 5,   // (evf only, during the repair) on the list of events to evaluate
+    EV_SRI     = 1u << 6,   // (evf only) od holds r(i) after the event (stress diagnostics)
 };
 
 // Wall result of one floe (verify_bc, boundaries.f90:1-97).

@@ -198,7 +198,7 @@ class Context:
 
     def set_repair(self, lanes: int = 64, pending: int = 1024):
         """Ridging repair: events evaluated at once (1: one at a time) and
-        pending events kept on chip.  Results do not depend on either."""
+        entries of its lists kept on chip.  Results do not depend on either."""
         self._chk(self.L.godar_set_repair(self.h, int(lanes), int(pending)))
 
     def set_stage_block(self, stage: int, threads: int):

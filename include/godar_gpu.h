@@ -226,10 +226,10 @@ int godar_set_stage_block(godar_ctx *ctx, int32_t stage, int32_t threads);
  * floes fit on the GPU at once) instead of the thread search (0: every
  * member, a huge value: none).  Results do not depend on it. */
 int godar_set_dense_search(godar_ctx *ctx, int32_t floes);
-/* Ridging repair: the number of pending events one member evaluates at once
- * (1-64, default 64; 1: one at a time) and the pending events kept in on-chip
- * memory (1-1024, default 1024) before the member continues one event at a
- * time.  Results do not depend on either. */
+/* Ridging repair: the number of events one wavefront of a member evaluates
+ * at once (1-64, default 64; fewer than 64: one wavefront per member) and the
+ * entries of each of its lists kept in on-chip memory (1-1024, default 1024)
+ * before they go on in device memory.  Results do not depend on either. */
 int godar_set_repair(godar_ctx *ctx, int32_t lanes, int32_t pending);
 /* Candidate supersets of members added afterwards reach `frac` x (max r +
  * rtree) beyond each floe's query radius (0-1, default 0.1).  The cell sort

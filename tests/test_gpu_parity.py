@@ -244,6 +244,24 @@ def test_repair_components_bitwise():
     assert worst < FP64_REL_TOL and seeds > 50, (worst, seeds)
 
 
+@pytest.mark.parametrize("n,rtree", [(2, 1500.0), (130, 9000.0), (1500, 1500.0), (1500, 9000.0)])
+def test_repair_sizes_and_list_lengths(n, rtree):
+    """The ordered repair from a single pair to hundreds of seeds in one
+    member (more than one wavefront's lanes, one full pass, several), with
+    short candidate lists and lists of a few hundred: bitwise the oracle's
+    sequential step."""
+    f = kick(squeeze(g.make_field(n, 11, radius="uniform", r_lo=500.0, r_hi=1500.0, h_median=1.0,
+                                  h_sigma=0.3, packing=0.6, box=9000.0 if n == 2 else None,
+                                  wind_speed=15.0, current_speed=0.2, gap=0.5, placement="rsa"),
+                     0.96), 2, speed=0.6)
+    if n == 2:
+        f.x, f.y = np.array([3000.0, 3000.0 + f.r.sum() - 20.0]), np.array([4000.0, 4000.0])
+    p = config0_params(f, sigmanc_crit=1e5, rtree=rtree)
+    worst, seeds, repaired = _lockstep(f, p, 6)
+    print(f"[repair] {n} floes, rtree {rtree:.0f}: {seeds} seeds, {repaired} events", flush=True)
+    assert worst == 0.0 and seeds > 0 and repaired >= seeds, (worst, seeds, repaired)
+
+
 def test_superset_skin_bitwise():
     """Candidate lists taken from skinned supersets (rebuilt only after a floe
     has moved far enough) give the same trajectory, bitwise, as a full cell
