@@ -16,9 +16,15 @@ ARCH = os.environ.get("GODAR_ARCH", "gfx950")
 
 # -ffp-contract=off keeps FP64 rounding identical to the reference (no fused
 # multiply-adds); packed FP32 instructions are disabled on this target.
+# -disable-machine-licm keeps the compiler from hoisting the physics' FP64
+# constants out of the kernels' work loops: it held hundreds of them in scalar
+# registers, spilled to vector registers and those to scratch (k_contact FP64
+# 476 scalar spills and 160 B of scratch -> 26 and 40 B, k_repair 711 -> 7 and
+# 140 -> 98 VGPRs, k_walls 155 -> 120), though each costs one move where used
+# (262,144 floes FP64: contacts 0.038 -> 0.031 ms, fix-up 0.047 -> 0.032).
 FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-shared",
-    "-ffp-contract=off",
+    "-ffp-contract=off", "-mllvm", "-disable-machine-licm",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-command-line-argument",
 ]
