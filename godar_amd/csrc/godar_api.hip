@@ -23,8 +23,6 @@ template <bool F> __global__ void k_sup_dense(DS);
 __global__ void k_scan_tiles(DS);
 __global__ void k_scan_total(DS, int);
 __global__ void k_scan_offsets(DS);
-template <bool M> __global__ void k_cand_dense(DS);
-template <bool M> __global__ void k_cand_dense_over(DS);
 template <bool M> __global__ void k_contact(DS);
 template <bool M> __global__ void k_bond(DS);
 __global__ void k_stress(DS);
@@ -33,6 +31,7 @@ template <bool M> __global__ void k_repair(DS, int);
 template <bool M> __global__ void k_fixup(DS);
 template <bool M, bool R> __global__ void k_final(DS);
 __global__ void k_totals(DS, int64_t*);
+__global__ void k_pairs(DS, int, int*, int2*, int);
 
 __global__ void k_fill_u8(uint8_t* p, int64_t n, uint8_t v) {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -122,7 +121,8 @@ struct godar_ctx {
     int64_t wpool_dev_cap = 0;
     int wgrids_dev_cap = 0;
     DS d{};
-    // double-buffered pair state
+    // double-buffered positions and pair state
+    GeoRec* geo[2] = {nullptr, nullptr};
     HistRec* hist[2] = {nullptr, nullptr};
     int32_t* hcnt[2] = {nullptr, nullptr};
     BondRec* bond[2] = {nullptr, nullptr};
@@ -279,6 +279,7 @@ void set_lists(godar_ctx* c, const PairLists& L) {
 
 void bind_parity(godar_ctx* c) {
     int o = c->parity, n = 1 - c->parity;
+    c->d.geo = c->geo[o]; c->d.geo_new = c->geo[n];
     c->d.hist_old = c->hist[o]; c->d.hist_new = c->hist[n];
     c->d.hcnt_old = c->hcnt[o]; c->d.hcnt_new = c->hcnt[n];
     c->d.bond_old = c->bond[o]; c->d.bond_new = c->bond[n];
@@ -314,6 +315,7 @@ void sync_ds(godar_ctx* c) {
     d.qseg = qseg_of(c);   // XCD share of the candidate search (k_cand's grid, XCD-aware order)
     d.repair_lanes = c->repair_lanes;
     d.repair_cap = c->repair_cap;
+    d.near_lim = c->precision == GODAR_MIXED ? 20.0f : 40.0f;
     d.sup_cap = c->sup_cap;
     d.bkey = c->rs.keys_alt;
     d.bval = c->rs.vals_alt;
@@ -497,16 +499,10 @@ int launch_step(godar_ctx* c, bool lean) {
     int nm = c->Mcap;
     const bool mixed = c->precision == GODAR_MIXED;
     bool any_dense = false;
-    int64_t dense_n = 0;
-    for (int k = 0; k < c->Mcap; ++k)
-        if (c->members[k].active && c->dparams[k].dense) { any_dense = true; dense_n += c->members[k].n; }
-    // The dense search runs a thread per dense floe (blocks of one
-    // wavefront, or of two that split the supersets when the dense floes
-    // fit on the GPU at once; each block with its list of near pairs in
-    // LDS); the superset
-    // builds keep 1,024 wavefronts per XCD: they return at once on most
-    // steps, and dispatching many more would cost more than they save.
-    const dim3 dense_grid(XCD_COUNT * (int)std::max<int64_t>(1, (dense_n + XCD_COUNT * 64 - 1) / (XCD_COUNT * 64)));
+    for (int k = 0; k < c->Mcap; ++k) any_dense |= c->members[k].active && c->dparams[k].dense;
+    // (the superset builds of dense members keep 1,024 wavefronts per XCD:
+    // they return at once on most steps, and dispatching many more would cost
+    // more than they save)
     if (!lean) {
         StageTimer t(c, 2);
         hipLaunchKernelGGL(k_ranges, grid_for(N, B[2], false), dim3(B[2]), 0, s, d);
@@ -526,18 +522,6 @@ int launch_step(godar_ctx* c, bool lean) {
         // LDS: one list of (floe, candidate) pairs per wavefront
         hipLaunchKernelGGL(mixed ? k_cand<true> : k_cand<false>, grid_for(N, B[3], true),
                            dim3(B[3]), (B[3] / 64) * CAND_LDS_PER_WAVE, s, d);
-        if (any_dense) {
-            // a thread per dense floe, a contiguous share of the list per XCD
-            // two wavefronts per 64 floes (one per half of the supersets)
-            // when they all fit on the GPU at once: a shorter chain per
-            // wavefront; with more floes, one wavefront takes both halves
-            const bool two = dense_n <= (int64_t)c->ncu * 4 * DENSE_WAVES_PER_SIMD * 32;
-            auto kd = mixed ? (two ? k_cand_dense<true, true> : k_cand_dense<true, false>)
-                            : (two ? k_cand_dense<false, true> : k_cand_dense<false, false>);
-            hipLaunchKernelGGL(kd, dense_grid, dim3(two ? 128 : 64), 0, s, d);
-            hipLaunchKernelGGL(mixed ? k_cand_dense_over<true> : k_cand_dense_over<false>,
-                               grid_for(N, FLOE_BLOCK, true), dim3(FLOE_BLOCK), 0, s, d);
-        }
     }
     // contacts, bonds and walls touch disjoint state (the flag words both
     // the contact and the bond kernel set are set with atomicOr), so they may
@@ -740,7 +724,8 @@ int godar_create(int64_t max_floes, int32_t max_members, int32_t precision, goda
         return GODAR_ERR_HIP;
     }
     ACHK(dalloc(&d.rec, S));
-    ACHK(dalloc(&d.geo, S));
+    ACHK(dalloc(&c->geo[0], S));
+    ACHK(dalloc(&c->geo[1], S));
     ACHK(dalloc(&d.shel, S));
     ACHK(dalloc(&d.kin, S));
     ACHK(dalloc(&d.pos_of, S));
@@ -788,7 +773,10 @@ int godar_create(int64_t max_floes, int32_t max_members, int32_t precision, goda
     c->sup_cap = 8 * S;
     ACHK(dalloc(&d.sup, c->sup_cap));
     ACHK(dalloc(&d.scnt, S));
-    ACHK(dalloc(&d.sout, S));
+    ACHK(dalloc(&d.snear, S));
+    ACHK(dalloc(&d.nb, S));
+    ACHK(dalloc(&d.nbmin, S));
+    ACHK(dalloc(&d.nearsum, 1));
     ACHK(dalloc(&d.soff, S));
     ACHK(dalloc(&d.sblk, S / SCAN_TILE + 2));
     ACHK(dalloc(&d.x0, S));
@@ -798,6 +786,9 @@ int godar_create(int64_t max_floes, int32_t max_members, int32_t precision, goda
     (void)hipMemsetAsync(d.err, 0, sizeof(uint32_t), c->stream);
     (void)hipMemsetAsync(d.steps_done, 0, sizeof(int64_t), c->stream);
     (void)hipMemsetAsync(d.scnt, 0, sizeof(int32_t) * S, c->stream);
+    (void)hipMemsetAsync(d.nbmin, 0, sizeof(float) * S, c->stream);
+    for (int k = 0; k < 2; ++k)       // (member -1: no floe yet)
+        (void)hipMemsetAsync(c->geo[k], 0xFF, sizeof(GeoRec) * S, c->stream);
     (void)hipMemsetAsync(d.qn, 0, sizeof(int32_t) * NQUEUE * XCD_COUNT * QN_STRIDE, c->stream);
     hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, c->stream, d.rebuild, 2, 1);
     hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, c->stream, d.rebuild + 2, 1, 0);
@@ -826,7 +817,7 @@ int godar_destroy(godar_ctx* c) {
     DS& d = c->d;
     double* dbl[] = {d.wbc, d.acc, d.cur, d.fout};
     for (double* p : dbl) dfree(p);
-    dfree(d.rec); dfree(d.geo); dfree(d.shel); dfree(d.kin); dfree(d.pos_of); dfree(d.pos_id);
+    dfree(d.rec); dfree(c->geo[0]); dfree(c->geo[1]); dfree(d.shel); dfree(d.kin); dfree(d.pos_of); dfree(d.pos_id);
     dfree(d.member_of); dfree(d.gid_of); dfree(d.sid_of); dfree(d.members);
     DevParams* pp = const_cast<DevParams*>(d.params); dfree(pp);
     WindGridDesc* wg = const_cast<WindGridDesc*>(d.wgrids); dfree(wg);
@@ -842,7 +833,7 @@ int godar_destroy(godar_ctx* c) {
     dfree(d.wout); dfree(d.wflag); dfree(d.cls); dfree(d.qlist); dfree(d.qn); dfree(d.bgat); dfree(d.shape); dfree(d.rhead); dfree(d.nseeds); dfree(d.heap);
     dfree(d.dirty);
     dfree(d.wnz); dfree(d.stats); dfree(d.tcur); dfree(d.err); dfree(d.steps_done);
-    dfree(d.sup); dfree(d.scnt); dfree(d.sout); dfree(d.soff); dfree(d.sblk); dfree(d.x0); dfree(d.rebuild);
+    dfree(d.sup); dfree(d.scnt); dfree(d.snear); dfree(d.nb); dfree(d.nbmin); dfree(d.nearsum); dfree(d.soff); dfree(d.sblk); dfree(d.x0); dfree(d.rebuild);
     radix_free(c->rs);
     collect_events(c);
     for (hipEvent_t e : c->ev_pool) (void)hipEventDestroy(e);
@@ -861,7 +852,7 @@ const char* godar_last_error(const godar_ctx* c) { return c ? c->err.c_str() : "
 // list capacities.
 static int64_t bytes_per_floe(const godar_ctx* c) {
     int64_t per = 0;
-    per += sizeof(FloeRec) + sizeof(GeoRec) + sizeof(ShelRec) + sizeof(KinRec);
+    per += sizeof(FloeRec) + 2 * sizeof(GeoRec) + sizeof(ShelRec) + sizeof(KinRec);
     per += 4 + 4 /*pos_of, pos_id*/ + 4 * 8 /*wbc*/ + 4 /*member_of*/ + 4 + 4 /*ckey, cval*/;
     per += 4 + 4 /*ocnt, icnt*/ + 2 * (4 + 4) /*hcnt, bcnt*/;
     per += (int64_t)c->CO * (8 + 8 + 4 + 8 + 8) + (int64_t)c->CI * (8 + 4);   // oj od evf ssc ssb; ik ibond
@@ -871,7 +862,7 @@ static int64_t bytes_per_floe(const godar_ctx* c) {
     per += (int64_t)c->SEEDK * sizeof(Reshape) + 4 /*rhead*/ + (int64_t)c->HEAPK * 8;
     per += 6 * 8 /*cur*/ + 1 + 1 /*dirty, wnz*/;
     per += 33 * 8 /*fout*/ + 4 + 4 /*radix keys, values*/;
-    per += (c->S > 0 ? c->sup_cap / c->S : 0) * 8 /*superset pool share*/ + 4 + 4 + 8 + 16 /*scnt sout soff x0*/;
+    per += (c->S > 0 ? c->sup_cap / c->S : 0) * 8 /*superset pool share*/ + 4 + 4 + 8 + 16 + 4 + 4 /*scnt snear soff x0 nb nbmin*/;
     per += 1 /*sblk, per SCAN_TILE floes*/;
     return per;
 }
@@ -1038,6 +1029,7 @@ int godar_member_add(godar_ctx* c, const godar_params* p, int32_t n, const doubl
         HIPCHK(c, hipMemset(c->bcnt[k] + first, 0, sizeof(int32_t) * n));
     }
     HIPCHK(c, hipMemset(d.dirty + first, 0, n));
+    HIPCHK(c, hipMemset(d.nbmin + first, 0, sizeof(float) * n));
     HIPCHK(c, hipMemset(d.wnz + first, 0, n));        // wall history rows zeroed above
     std::vector<int32_t> mo(n, m);
     HIPCHK(c, hipMemcpy(d.member_of + first, mo.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice));
@@ -1445,6 +1437,7 @@ int godar_set_bonds(godar_ctx* c, int32_t m, int32_t nb, const int32_t* bi, cons
         HIPCHK(c, hipMemcpy(c->bond[o] + q * S + mm.first, recs.data() + (int64_t)q * mm.n,
                             sizeof(BondRec) * mm.n, hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->bcnt[o] + mm.first, cnt.data(), sizeof(int32_t) * mm.n, hipMemcpyHostToDevice));
+    force_rebuild(c);   // the supersets keep bonded pairs
     return GODAR_OK;
 }
 
@@ -1591,6 +1584,7 @@ int build_period(godar_ctx* c, double frac, double* period) {
     std::vector<KinRec> kin(std::max(N, 1));
     std::vector<GeoRec> geo(std::max(N, 1));
     HIPCHK(c, hipStreamSynchronize(c->stream));
+    sync_ds(c);
     HIPCHK(c, hipMemcpy(kin.data(), c->d.kin, sizeof(KinRec) * N, hipMemcpyDeviceToHost));
     HIPCHK(c, hipMemcpy(geo.data(), c->d.geo, sizeof(GeoRec) * N, hipMemcpyDeviceToHost));
     std::vector<double> vmax(c->Mcap, 0.0);
@@ -1798,15 +1792,16 @@ int godar_sync(godar_ctx* c) {
     bool was_pending = c->pending;
     c->pending = false;
     if (e == ERR_NEED_BUILD && was_pending) {
-        // a lean step found a build due: it and the steps after it did
-        // nothing; back to the last complete step, and the rest again with
-        // the build kernels
+        // a lean step found a build due, or a floe's drafts outgrew its lists:
+        // that step and the ones after it did nothing; back to the last
+        // complete step, and the rest again with the build kernels
         int64_t now = 0;
         rc = steps_done(c, &now);
         if (rc != GODAR_OK) return rc;
         c->parity = c->pend_parity ^ (int)((now - c->pend_done0) & 1);
         bind_parity(c);
-        HIPCHK(c, hipMemset(c->d.err, 0, sizeof(uint32_t)));
+        HIPCHK(c, hipMemsetAsync(c->d.dirty, 0, c->S, c->stream));
+        HIPCHK(c, hipMemsetAsync(c->d.err, 0, sizeof(uint32_t), c->stream));
         const int64_t left = c->pend_launched - (now - c->pend_done0);
         c->need_full = true;
         c->full_hold = FULL_HOLD;
@@ -1827,8 +1822,9 @@ int godar_sync(godar_ctx* c) {
             c->parity = c->pend_parity ^ (int)((now - c->pend_done0) & 1);
             bind_parity(c);
         }
-        HIPCHK(c, hipMemset(c->d.dirty, 0, c->S));
-        HIPCHK(c, hipMemset(c->d.err, 0, sizeof(uint32_t)));
+        HIPCHK(c, hipMemsetAsync(c->d.dirty, 0, c->S, c->stream));
+        HIPCHK(c, hipMemsetAsync(c->d.err, 0, sizeof(uint32_t), c->stream));
+        HIPCHK(c, hipStreamSynchronize(c->stream));
         c->last_err_bits = e;
         return fail(c, GODAR_ERR_CAPACITY, "step aborted:" + err_text(e));
     }
@@ -1987,7 +1983,35 @@ int godar_get_pairs(godar_ctx* c, int32_t m, int32_t kind, int32_t cap, int32_t*
     const Member& mm = c->members[m];
     int64_t S = c->S;
     std::vector<std::pair<int32_t, int32_t>> out;
-    if (kind == GODAR_PAIRS_CANDIDATE || kind == GODAR_PAIRS_CONTACT) {
+    if (kind == GODAR_PAIRS_CANDIDATE) {
+        // the step's lists hold the pairs that can matter; all of the
+        // candidates come from the supersets, counted first
+        sync_ds(c);
+        int n = 0, *dn = nullptr;
+        int2* dp = nullptr;
+        HIPCHK(c, hipMalloc(&dn, sizeof(int)));
+        hipError_t e = hipSuccess;
+        auto pass = [&](int want) {
+            hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, c->stream, dn, (int64_t)1, 0);
+            if (c->N_used > 0)
+                hipLaunchKernelGGL(k_pairs, dim3((c->N_used + 255) / 256), dim3(256), 0, c->stream, c->d, m, dn, dp, want);
+            e = hipMemcpyAsync(&n, dn, sizeof(int), hipMemcpyDeviceToHost, c->stream);
+            if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+        };
+        pass(0);
+        if (e == hipSuccess && n > 0 && cap > 0) {
+            const int want = n;
+            std::vector<int2> h(want);
+            e = hipMalloc(&dp, sizeof(int2) * want);
+            if (e == hipSuccess) pass(want);
+            if (e == hipSuccess) e = hipMemcpy(h.data(), dp, sizeof(int2) * want, hipMemcpyDeviceToHost);
+            for (const int2& p : h) out.push_back({p.x, p.y});
+        }
+        (void)hipFree(dp);
+        (void)hipFree(dn);
+        HIPCHK(c, e);
+        if (cap == 0) { *count = n; return GODAR_OK; }
+    } else if (kind == GODAR_PAIRS_CONTACT) {
         // the member's floes occupy a contiguous range of this step's cell order
         std::vector<int32_t> pos(mm.n);
         HIPCHK(c, hipMemcpy(pos.data(), c->d.pos_of + mm.first, sizeof(int32_t) * mm.n, hipMemcpyDeviceToHost));
@@ -2011,7 +2035,7 @@ int godar_get_pairs(godar_ctx* c, int32_t m, int32_t kind, int32_t cap, int32_t*
             for (int s = 0; s < cnt[r0] && s < cmax; ++s) {
                 uint32_t fl = ef[(int64_t)s * len + r0];
                 if (fl & EV_REMOVED) continue;
-                if (kind == GODAR_PAIRS_CONTACT && !(fl & EV_CONTACT)) continue;
+                if (!(fl & EV_CONTACT)) continue;
                 out.push_back({c->perm[m][i], (int32_t)(oj[(int64_t)s * len + r0] >> 32) - mm.first});
             }
         }
@@ -2069,8 +2093,9 @@ int godar_get_totals(godar_ctx* c, int64_t* out) {
     HIPCHK(c, hipStreamSynchronize(c->stream));
     int64_t* dout = nullptr;
     HIPCHK(c, hipMalloc(&dout, 5 * sizeof(int64_t)));
-    HIPCHK(c, hipMemset(dout, 0, 5 * sizeof(int64_t)));
     sync_ds(c);
+    // (on the context's stream, which the null stream's memset would not wait for)
+    hipLaunchKernelGGL(k_zero_i64, dim3(1), dim3(64), 0, c->stream, dout, 5);
     if (c->N_used > 0)
         hipLaunchKernelGGL(k_totals, dim3((c->N_used + 255) / 256), dim3(256), 0, c->stream, c->d, dout);
     hipLaunchKernelGGL(k_member_totals, dim3(1), dim3(256), 0, c->stream, c->d, c->Mcap, dout + 3);

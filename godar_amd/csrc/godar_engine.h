@@ -68,6 +68,7 @@ struct DS {
     int32_t qseg;              // floe positions per XCD share of the candidate search
     int32_t repair_lanes;      // events the repair evaluates at once (1: one at a time)
     int32_t repair_cap;        // entries of each repair list held in LDS
+    float near_lim;            // shelter_min's limit: 20 (FP32 force laws) or 40
     int32_t pad_r_;
     // floe state by storage slot (current where rebuild[2] is clear, else
     // in the ordered copies)
@@ -89,7 +90,8 @@ struct DS {
     uint32_t *ckey, *cval;     // sort keys / floe ids, sorted (cval[pos] = storage slot)
     uint32_t *bkey, *bval;     // the sort's input, written by k_begin (the sort's scratch)
     int2* crange;              // [ncells+1] (start, end) in cell order
-    GeoRec* geo;               // [S] pos
+    GeoRec* geo;               // [S] pos: at the start of the step
+    GeoRec* geo_new;           // [S] pos: at its end (the two change places every step)
     ShelRec* shel;             // [S] pos (wind at the floe this step)
     KinRec* kin;               // [S] pos
     int32_t* pos_of;           // [S] storage slot -> pos
@@ -117,7 +119,7 @@ struct DS {
     uint8_t* wflag;            // [S rounded up to 4] WF_* bits
     uint8_t* cls;              // [S] CLS_* bits
     // Candidate supersets: every floe within its query radius plus the
-    // member's skin at the last build, (id << 32 | pos), floe k's at
+    // member's skin at the last build, (bound << 32 | pos), floe k's at
     // sup[soff[k] .. soff[k] + scnt[k]).  They are rebuilt (cell binning,
     // sort, search) only on steps that start with *rebuild set: after a
     // change of members, or once some floe has moved more than 0.45 skin from
@@ -127,10 +129,12 @@ struct DS {
     int64_t* sup;              // [sup_cap]
     int64_t sup_cap;
     int32_t* scnt;             // [S] by pos
-    int32_t* sout;             // [S] by pos, dense members: the superset holds its outer
-                               // entries (partner id above the floe's) first, by (distance
-                               // at the build, id), then the inner ones by id; sout is the
-                               // outer count (-1: left in scan order, too long to order)
+    int32_t* snear;            // [S] by pos: the first entries, which the search reads (all
+                               // of them but in dense members, see k_sup_dense)
+    float* nb;                 // [S] by pos: how far apart a pair of the floe may be and
+                               // still matter to it (dense members; at the build)
+    float* nbmin;              // [S] by storage slot: nb is at least this (0: no demand)
+    int64_t* nearsum;          // sum of snear
     int64_t* soff;             // [S] by pos
     int64_t* sblk;             // [S / SCAN_TILE + 2] scan of per-tile totals
     double2* x0;               // [S] by pos (positions stand between builds)

@@ -32,7 +32,8 @@
 // Layout: the per-step kernels run over floes in cell order ("pos"), reading
 // a sorted copy of the 96-byte floe records, so that a floe's neighbours sit
 // close in memory.  Pair state persists per floe id.  List entries pack the
-// partner as (id << 32 | pos).
+// partner as (id << 32 | pos).  The lists hold the candidates that can matter
+// (all of them but in dense members, see k_sup_dense).
 #include "godar_engine.h"
 #include "godar_physics.h"
 #include <type_traits>
@@ -117,8 +118,8 @@ __device__ __forceinline__ int queue_slot_it(int qn, int it) {
 // Entries of a queue of length qn taken by this wavefront when a wavefront
 // evaluates its floes' pairs together: `floes` consecutive entries of its
 // XCD's share at begin, begin + stride, ... below end.  Just enough floes for
-// one full pass of 64 pairs (by the mean superset length of the last build),
-// more only if the queue has more for every wavefront of the grid: with 64
+// one full pass of 64 pairs (by the mean number of superset entries the search
+// reads), more only if the queue has more for every wavefront of the grid: with 64
 // floes of tens of candidates each, a wavefront works through all their pairs
 // one pass after the other while the rest of the GPU has nothing to do (one
 // MI355X, contact kernel: 320,000 floes in 24 members with about 43
@@ -137,7 +138,7 @@ __device__ __forceinline__ QueueShare queue_share(const DS& S, int qn) {
     const int lo = (int)(blockIdx.x % XCD_COUNT) * per;
     QueueShare q;
     const int f = (per + nw - 1) / nw;
-    const int64_t entries = S.sblk[(S.N + SCAN_TILE - 1) / SCAN_TILE];   // supersets together
+    const int64_t entries = *S.nearsum;     // entries the search reads
     const int full = (int)min((int64_t)64, 64 * (int64_t)S.N / max(entries, (int64_t)1));
     q.floes = f > 16 ? 64 : max(1, max(f, full));
     q.begin = lo + w * q.floes;
@@ -161,6 +162,33 @@ __device__ __forceinline__ int ent_id(int64_t e) { return (int)(e >> 32); }
 __device__ __forceinline__ int ent_pos(int64_t e) { return (int)(uint32_t)(e & 0xffffffffll); }
 __device__ __forceinline__ int64_t ent(int id, int pos) {
     return ((int64_t)id << 32) | (int64_t)(uint32_t)pos;
+}
+
+// Superset entries: the partner's position and, in the high half, the bound
+// (a float): the pair is listed only while its floes are no further apart
+// than that (see k_sup_dense).
+constexpr float SUP_KEEP = __builtin_inff();
+__device__ __forceinline__ int64_t sup_ent(float bound, int pos) {
+    return ((int64_t)__float_as_int(bound) << 32) | (int64_t)(uint32_t)pos;
+}
+__device__ __forceinline__ double sup_bound(int64_t e) { return (double)__int_as_float((int)(e >> 32)); }
+// The pair at positions a and b is listed from now on whatever its distance
+// (it has a contact history or a bond): its entries of both supersets.
+__device__ __forceinline__ void sup_keep(const DS& S, int a, int b) {
+#pragma unroll
+    for (int side = 0; side < 2; ++side) {
+        const int k = side ? b : a, q = side ? a : b;
+        int64_t* se = S.sup + S.soff[k];
+        const int n = S.snear[k];
+        for (int i0 = 0; i0 < n; i0 += 4) {
+            int64_t e[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) e[u] = se[min(i0 + u, n - 1)];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (ent_pos(e[u]) == q) se[min(i0 + u, n - 1)] = sup_ent(SUP_KEEP, q);
+        }
+    }
 }
 
 // floe at position k of this step's cell order
@@ -194,12 +222,17 @@ __device__ __forceinline__ void floe_at_event(const Reshape* rec, int head, int6
         if (rec[p].live && rec[p].key < key && rec[p].key > bk) { bk = rec[p].key; best = p; }
     if (best >= 0) take_shape(rec[best], F);
 }
-// (the first reshape of the list, INT64_MAX if none)
-__device__ __forceinline__ int64_t first_reshape(const Reshape* rec, int head) {
+// (the record of the list's first reshape, -1 if none; its key, INT64_MAX)
+__device__ __forceinline__ int first_record(const Reshape* rec, int head) {
+    int best = -1;
     int64_t k = INT64_MAX;
     for (int p = head; p >= 0; p = rec[p].next)
-        if (rec[p].live && rec[p].key < k) k = rec[p].key;
-    return k;
+        if (rec[p].live && rec[p].key < k) { k = rec[p].key; best = p; }
+    return best;
+}
+__device__ __forceinline__ int64_t first_reshape(const Reshape* rec, int head) {
+    const int p = first_record(rec, head);
+    return p >= 0 ? rec[p].key : INT64_MAX;
 }
 // Records the reshape event `key` of the floes at kf (outer) and kj (-1: a
 // wall) gives the floe at kg, as record p of the member, and links it to the
@@ -396,6 +429,7 @@ __global__ void k_begin(DS S, int lean, int nmembers) {
     // (the dense-search queue stands between builds)
     if (i < NQUEUE * XCD_COUNT && (build || i / XCD_COUNT != 3)) S.qn[i * QN_STRIDE] = 0;
     if (build && i <= S.ncells) S.crange[i] = make_int2(0, 0);
+    if (build && i == 0) *S.nearsum = 0;
     // per-member resets (thread m for member m)
     if (i < nmembers && member_live(S.members[i])) {
         S.nseeds[i] = 0;
@@ -433,6 +467,14 @@ __global__ void k_begin(DS S, int lean, int nmembers) {
     S.bkey[f] = (uint32_t)(P.cell_base + cy * P.gx + cx);
 }
 
+// Distance beyond which a floe's sheltering terms are exactly 1 (shelter_min;
+// lim: 20 in FP32, 40 in FP64), from its own drafts; the room kept for the
+// drafts to grow before the next build.
+constexpr double NEAR_ROOM = 1.25;
+__device__ __forceinline__ double near_reach(double lim, double hfa, double hfw) {
+    return lim * fmax(hfa, hfw) / (double)0.18f;
+}
+
 // The floe records in the current order and the wind at each floe
 // (winds_currents, forcing.f90:1-29); on build steps the cell ranges over the
 // sorted keys.  Between builds the order stands and k_final writes these
@@ -459,6 +501,12 @@ __global__ void k_ranges(DS S) {
     if (m >= 0) {
         S.pos_id[g.id] = k;
         if (*S.rebuild) {
+            // how far apart a pair of this floe may be and still matter to it
+            const DevParams& P = S.params[m];
+            double nb = P.shelter ? NEAR_ROOM * near_reach(S.near_lim, fr.hfa, fr.hfw) : 0.0;
+            if (P.cohesion) nb = fmax(nb, P.bond_lim);
+            nb = fmax(nb, (double)S.nbmin[f]) * (1.0 + 1e-6);
+            S.nb[k] = P.dense && nb < 1e30 ? (float)nb : SUP_KEEP;
             const uint32_t key = S.ckey[k];
             if (k == 0 || S.ckey[k - 1] != key) S.crange[key].x = k;
             if (k == S.N - 1 || S.ckey[k + 1] != key) S.crange[key].y = k + 1;
@@ -508,32 +556,28 @@ __device__ __forceinline__ void enqueue(const DS& S, bool want, int c, int k) {
 // Finishing writes of one floe's search (any search shape): list counts,
 // per-slot resets, sheltering minima and the per-step resets of its rows
 // (fs: the floe's storage slot).
-template <bool MIXED>
 __device__ __forceinline__ void cand_finish(const DS& S, int k, int fs, const DevParams& P, int no,
-                                            int ni, double sha, double shw, bool qc, bool qb,
-                                            int lane0, int lanes) {
+                                            int ni, double sha, double shw, bool qc, bool qb) {
     const int64_t SS = S.S;
     const uint32_t fl = P.shelter ? EV_SHELTER : 0u;
-    for (int s2 = lane0; s2 < no; s2 += lanes) {
+    for (int s2 = 0; s2 < no; ++s2) {
         S.evf[s2 * SS + k] = fl;
         if (S.record_forces) {
             S.ssc[s2 * SS + k] = 0.0;
             S.ssb[s2 * SS + k] = 0.0;
         }
     }
-    for (int s2 = lane0; s2 < ni; s2 += lanes) S.ibond[s2 * SS + k] = 0;
-    if (lane0 == 0) {
-        S.ocnt[k] = no;
-        S.icnt[k] = ni;
-        S.acc[A_SHA * SS + k] = sha;
-        S.acc[A_SHW * SS + k] = shw;
-        if (!qc) S.hcnt_new[fs] = 0;
-        if (!qb) S.bcnt_new[fs] = 0;
-        S.wflag[k] = 0;
-        S.bgat[k] = 0;
-        S.rhead[k] = -1;
-        S.cls[k] = qc ? CLS_CONTACT : 0;   // the fix-up sets CLS_BOND
-    }
+    for (int s2 = 0; s2 < ni; ++s2) S.ibond[s2 * SS + k] = 0;
+    S.ocnt[k] = no;
+    S.icnt[k] = ni;
+    S.acc[A_SHA * SS + k] = sha;
+    S.acc[A_SHW * SS + k] = shw;
+    if (!qc) S.hcnt_new[fs] = 0;
+    if (!qb) S.bcnt_new[fs] = 0;
+    S.wflag[k] = 0;
+    S.bgat[k] = 0;
+    S.rhead[k] = -1;
+    S.cls[k] = qc ? CLS_CONTACT : 0;   // the fix-up sets CLS_BOND
 }
 
 constexpr int SCAN_BATCH = 4;
@@ -605,7 +649,7 @@ __device__ __forceinline__ int sup_thread(const DS& S, int k, const GeoRec& me, 
             const double thr = g[u].id > f ? rad : g[u].r + reach;
             // a superset: the margin only adds entries
             if (dx * dx + dy * dy <= thr * thr * (1.0 + 1e-12)) {
-                if (FILL) out[n] = ent(g[u].id, q);
+                if (FILL) out[n] = sup_ent(SUP_KEEP, q);
                 ++n;
             }
         }
@@ -624,7 +668,7 @@ constexpr int CAND_LDS_PER_WAVE = CAND_TCAP * (8 + 8 + 1) + 64 * 4 + CAND_TCAP *
 // resets of the floe's rows.  The head of each candidate list is sorted in
 // registers while it is built, the rest in its slots in HBM.
 //
-// WAVE: every lane of the wavefront calls it (act: the lane has a floe).  The
+// Every lane of the wavefront calls it (act: the lane has a floe).  The
 // wavefront's supersets lie one after the other in the pool; they are tested
 // together, 64 consecutive entries a round (each lane finds the entry's
 // owner among the lanes), and the entries within the query radius are listed
@@ -634,8 +678,8 @@ constexpr int CAND_LDS_PER_WAVE = CAND_TCAP * (8 + 8 + 1) + 64 * 4 + CAND_TCAP *
 // classification terms of all the listed pairs are evaluated together, 64 at
 // a time; each floe then takes the minimum of its own terms (a minimum of
 // fmin terms does not depend on the order or on which lane computed them).
-// Otherwise, or when the pairs outnumber CAND_TCAP, each lane scans its own
-// superset SCAN_BATCH records at a time and evaluates its own terms.
+// When the pairs outnumber CAND_TCAP, each lane scans its own superset and
+// evaluates its own terms.
 // The rows of position k (and its storage slot's counts) that the search
 // reads first, loaded at once as soon as k is known.
 struct CandPre {
@@ -647,14 +691,14 @@ __device__ __forceinline__ CandPre cand_pre(const DS& S, int k) {
     CandPre c;
     c.msh = S.shel[k];
     c.fs = S.cval[k];
-    c.L = S.scnt[k];
+    c.L = S.snear[k];
     c.soff = S.soff[k];
     c.hc = S.hcnt_old[c.fs];
     c.bc = S.bcnt_old[c.fs];
     return c;
 }
 
-template <bool MIXED, bool WAVE>
+template <bool MIXED>
 __device__ __forceinline__ void cand_thread(const DS& S, int k, const GeoRec& me, const CandPre& pre,
                                             int m, bool act, bool& qc, bool& qb, bool& qw,
                                             unsigned char* lds) {
@@ -769,7 +813,7 @@ __device__ __forceinline__ void cand_thread(const DS& S, int k, const GeoRec& me
     // the pairs whose terms the second pass evaluates (indices into the above)
     uint16_t* tx = reinterpret_cast<uint16_t*>(lds + 17 * CAND_TCAP + 64 * 4);
     int nneed = 0;
-    if (WAVE) {
+    {
         const int lane = (int)(threadIdx.x & 63);
         const uint64_t lt = lane ? ((~0ull) >> (64 - lane)) : 0ull;
         int incl = L;
@@ -832,7 +876,9 @@ __device__ __forceinline__ void cand_thread(const DS& S, int k, const GeoRec& me
                 // correctly rounded, so it cannot cross a margin of 1e-12)
                 if (dist2 <= thr * thr * (1.0 + 1e-12)) {
                     d = sqrt(dist2);
-                    hit = d <= thr;
+                    // (the same overlap on either side of the pair, so both
+                    // floes list it or neither does)
+                    hit = d <= thr && orr + o.r - d >= -sup_bound(e);
                 }
                 if (hit) {
                     // The second pass changes nothing for a pair out of
@@ -880,16 +926,20 @@ __device__ __forceinline__ void cand_thread(const DS& S, int k, const GeoRec& me
         }
     }
     if (!flat && act) {
-        // (the wavefront search is the common path: this one keeps fewer
+        // (the wavefront's common search is the common path: this one keeps few
         // records in flight, which keeps the kernel's registers down)
-        constexpr int B = WAVE ? 2 : SCAN_BATCH;
+        constexpr int B = 2;
         const int64_t* se = S.sup + soff;
         for (int v0 = 0; v0 < L; v0 += B) {
             GeoRec g[B];
             int qq[B];
+            double bd[B];
 #pragma unroll
-            for (int u = 0; u < B; ++u)
-                qq[u] = ent_pos(se[min(v0 + u, L - 1)]);   // the last entry stands in past the end
+            for (int u = 0; u < B; ++u) {
+                const int64_t e = se[min(v0 + u, L - 1)];   // the last entry stands in past the end
+                qq[u] = ent_pos(e);
+                bd[u] = sup_bound(e);
+            }
 #pragma unroll
             for (int u = 0; u < B; ++u) g[u] = S.geo[qq[u]];
 #pragma unroll
@@ -901,7 +951,7 @@ __device__ __forceinline__ void cand_thread(const DS& S, int k, const GeoRec& me
                 const double thr = o->id > f ? rad : o->r + rtree;
                 if (dist2 > thr * thr * (1.0 + 1e-12)) continue;
                 const double d = sqrt(dist2);
-                if (!(d <= thr)) continue;
+                if (!(d <= thr) || !(me.r + o->r - d >= -bd[u])) continue;
                 insert(o->id, qq[u], d);
             }
         }
@@ -1031,22 +1081,23 @@ __device__ __forceinline__ void cand_thread(const DS& S, int k, const GeoRec& me
         if (s2 < ni) ik[s2 * SS + k] = ri[s2];
     }
     if (over) set_err(S, over);
-    cand_finish<MIXED>(S, k, fs, P, no, ni, double(sha), double(shw), qc, qb, 0, 1);
+    cand_finish(S, k, fs, P, no, ni, double(sha), double(shw), qc, qb);
 }
 
 // Superset build, thread per floe (members that are not dense; span 1 or
 // 2 cells on each side): counts (FILL false) or entries and the build
 // positions x0 (FILL true).  The count pass lists the dense members' floes in
-// queue 3 for k_sup_dense and k_cand_dense.  Only on build steps.
+// queue 3 for k_sup_dense.  Only on build steps.
 template <bool FILL>
 __global__ __launch_bounds__(FLOE_BLOCK) void k_sup(DS S) {
     if (!*S.rebuild || *S.err) return;
     const int k = xcd_block() * blockDim.x + threadIdx.x;
     bool qd = false;
+    int n = 0;
     if (k < S.N) {
         const GeoRec me = S.geo[k];
         if (me.member < 0) {
-            if (!FILL) S.scnt[k] = 0;
+            if (!FILL) S.scnt[k] = S.snear[k] = 0;
         } else {
             const DevParams& P = S.params[me.member];
             if (P.dense) {
@@ -1056,12 +1107,18 @@ __global__ __launch_bounds__(FLOE_BLOCK) void k_sup(DS S) {
                 else sup_thread<1, true>(S, k, me, P, S.sup + S.soff[k]);
                 S.x0[k] = make_double2(me.x, me.y);
             } else {
-                S.scnt[k] = P.span == 2 ? sup_thread<2, false>(S, k, me, P, nullptr)
-                                        : sup_thread<1, false>(S, k, me, P, nullptr);
+                n = P.span == 2 ? sup_thread<2, false>(S, k, me, P, nullptr)
+                                : sup_thread<1, false>(S, k, me, P, nullptr);
+                S.scnt[k] = S.snear[k] = n;
             }
         }
     }
-    enqueue(S, qd, 3, k);
+    if (!FILL) {
+        enqueue(S, qd, 3, k);
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off);
+        if ((threadIdx.x & 63) == 0 && n) atomicAdd((unsigned long long*)S.nearsum, (unsigned long long)n);
+    }
 }
 
 // Superset offsets: per-tile totals, their exclusive scan (one workgroup;
@@ -1133,13 +1190,11 @@ __global__ __launch_bounds__(FLOE_BLOCK) void k_cand(DS S) {
     }
     const bool slot_used = inr && me.member >= 0;
     const int m = slot_used ? me.member : 0;
-    const bool dense = S.params[m].dense != 0;
     const bool ok = !*S.err;
-    // floes of dense members: k_cand_dense
     extern __shared__ unsigned char cand_lds[];
-    const bool act = slot_used & ok & !dense;
-    cand_thread<MIXED, true>(S, k, me, pre, m, act, qc, qb, qw,
-                             cand_lds + (threadIdx.x >> 6) * CAND_LDS_PER_WAVE);
+    const bool act = slot_used & ok;
+    cand_thread<MIXED>(S, k, me, pre, m, act, qc, qb, qw,
+                       cand_lds + (threadIdx.x >> 6) * CAND_LDS_PER_WAVE);
     if (inr && ok && !slot_used) {
         S.ocnt[k] = 0;
         S.icnt[k] = 0;
@@ -1149,54 +1204,36 @@ __global__ __launch_bounds__(FLOE_BLOCK) void k_cand(DS S) {
     enqueue(S, qw, 2, k);
 }
 
-// Dense members (many floes per cell): a thread per floe, over its superset
-// as the build ordered it (outer entries by distance at the build, then inner
-// ones by id).  Inner candidates therefore come in list order and are
-// appended; outer ones come in nearly the order of their current distance
-// (floes move little between builds), so each is inserted among the last
-// DENSE_WIN entries, which stay in registers (most simply take their top),
-// and only the rare entry that belongs below them is inserted into the part
-// of the list in HBM.
-// The lists are slot-major (slot s of floe k at s * S + k), so a thread that
-// stored each entry as it found it would touch a line per entry, 64 lines per
-// store of a wavefront.  Instead the scan takes the outer part of the
-// supersets in one pass and the inner part in another (one after the other,
-// or in two wavefronts over the same floes), so that the lanes' lists grow
-// nearly in step, and each thread stages its rows in a ring of its own in
-// LDS; the wavefront writes a row out for all its floes at once when every
-// thread still scanning has passed it, or when a thread needs the room.
-// A row a thread reaches after its wavefront wrote it out goes straight to
-// HBM; a thread that inserts below its register part first writes its staged
-// outer rows out and keeps its outer list in HBM from then on.
-// Sheltering terms are needed only for pairs close enough that
-// exp(-0.18 |dn/cos| / hf) still counts (shelter_min); the threads list those
-// pairs in LDS (slots taken by ballot, no atomic) and the wavefront evaluates
-// them 64 at a time, each floe taking the minimum of its own (an LDS atomic:
-// a minimum does not depend on the order of its terms).  A superset left in
-// scan order (longer than SUP_ORDER_CAP) goes to the thread search
-// (k_cand_dense_over).
-constexpr int DENSE_OVER = -1;   // ocnt of a dense floe left to the thread search
-constexpr int DENSE_WIN = 4;     // outer candidates in registers
-constexpr int DENSE_NEAR = 512;  // near pairs listed per wavefront
-constexpr int DENSE_BATCH = 5;   // superset entries a thread loads at once (mixed precision)
-constexpr int DENSE_RING = 16;   // list rows a thread stages in LDS
-constexpr int DENSE_WAVES_PER_SIMD = 3;   // the dense search's occupancy bound
-static_assert((DENSE_RING & (DENSE_RING - 1)) == 0 && DENSE_RING >= DENSE_BATCH + DENSE_WIN,
-              "a ring of whole rows with room for a batch past the register part");
-
 // Superset build of the dense members' floes (queue 3), one wavefront per
 // floe over its (2 span + 1)^2 cell block, 64 entries at a time: counts, or
-// the entries and the build positions.  The filled superset is then ordered
-// as the dense search reads it: outer entries (partner id above the floe's)
-// first, by (distance at the build, id), then inner entries by id; each
-// entry goes to its rank, counted over the floe's entries in LDS.  A
-// superset longer than SUP_ORDER_CAP stays in scan order (sout = -1).  Only
-// on build steps.
-constexpr int SUP_ORDER_CAP = 256;   // (16 bytes of LDS per entry: 4 KB per wavefront)
+// the entries and the build positions.  Only on build steps.
+//
+// In these members (power-law radii, say) the query radius r + rtree holds
+// tens of floes, nearly all of them kilometres away: no contact, no bond, and
+// a sheltering term that is exactly 1.  A pair can only matter while its
+// floes are no further apart than the larger of their two bounds nb (the
+// reach of their own sheltering, with room for the drafts to grow, and the
+// distance bonds form at), or if it has a contact history or a bond.  So the
+// entries that can come within their bound before the next build go first
+// (snear of them, each with its bound; SUP_KEEP for pairs with a history or a
+// bond, which k_contact and k_bond set on the entries of new ones), and the
+// step's search reads those alone and lists the pairs within their bound: of
+// 59 entries and 43 candidates a floe (power-law radii on [200, 5000] m at
+// packing 0.7), 9-11 and 2.4-4.2.  (One MI355X, against a search and lists of
+// all candidates: 320,000 floes mixed, search 0.39 -> 0.11 ms, integration
+// 0.088 -> 0.034, bonds 0.034 -> 0.016; 262,144 floes FP64, search 0.38 ->
+// 0.16; 1,000 floes 0.114 -> 0.041.)  The others only answer which pairs were
+// candidates (k_pairs) and how many events a reshape came before (k_repair).
+// A reshape whose drafts outgrow their room ends the step, which is run again
+// with a build and more room (k_fixup).
+__device__ __forceinline__ bool has_records(const DS& S, int i, int j) {
+    const int hc = S.hcnt_old[i], bc = S.bcnt_old[i];
+    if (hc == 0 && bc == 0) return false;
+    return find_partner(S.hist_old, S.S, i, hc, j) >= 0 || find_partner(S.bond_old, S.S, i, bc, j) >= 0;
+}
+
 template <bool FILL>
 __global__ __launch_bounds__(64) void k_sup_dense(DS S) {
-    __shared__ double od_[FILL ? SUP_ORDER_CAP : 1];
-    __shared__ int64_t oe_[FILL ? SUP_ORDER_CAP : 1];
     if (!*S.rebuild || *S.err) return;
     const int lane = threadIdx.x;
     const QueueView qv = queue_view(S, 3);
@@ -1206,16 +1243,19 @@ __global__ __launch_bounds__(64) void k_sup_dense(DS S) {
     const int per = (nq + XCD_COUNT - 1) / XCD_COUNT;
     const int t1 = min(nq, xcd * per + per);
     const uint64_t lt = lane ? ((~0ull) >> (64 - lane)) : 0ull;
+    int64_t sum = 0;
     for (int t = xcd * per + bi; t < t1; t += nb) {
         const int k = queue_at(S, 3, qv, t);
         const GeoRec me = S.geo[k];
         const DevParams& P = S.params[me.member];
         const double rad = me.r + P.rtree + P.skin, reach = P.rtree + P.skin;
-        const int f = me.id;
+        const int f = me.id, fs = S.cval[k];
+        const float nbme = S.nb[k];
         const int sp = P.span;
         const int cx = cell_coord(me.x, P.cell, P.gx), cy = cell_coord(me.y, P.cell, P.gy);
         int64_t* out = FILL ? S.sup + S.soff[k] : nullptr;
-        int n = 0;
+        const int snear = FILL ? S.snear[k] : 0;
+        int n = 0, nn = 0;
         const int a0 = max(cx - sp, 0), a1 = min(cx + sp, P.gx - 1);
         for (int b = cy - sp; b <= cy + sp; ++b) {
             if (b < 0 || b >= P.gy) continue;
@@ -1227,485 +1267,48 @@ __global__ __launch_bounds__(64) void k_sup_dense(DS S) {
             }
             for (int base = lo; base < hi; base += 64) {
                 const int q = base + lane;
-                bool in = false;
-                int oid = 0;
+                bool in = false, near = false;
+                float bound = 0.0f;
                 if (q < hi && q != k) {
                     const GeoRec o = S.geo[q];
-                    const double dx = me.x - o.x, dy = me.y - o.y;
-                    oid = o.id;
+                    const double dx = me.x - o.x, dy = me.y - o.y, d2 = dx * dx + dy * dy;
                     const double thr = o.id > f ? rad : o.r + reach;
-                    in = dx * dx + dy * dy <= thr * thr * (1.0 + 1e-12);
-                }
-                const uint64_t mi = __ballot(in);
-                if (FILL && in) out[n + (int)__popcll(mi & lt)] = ent(oid, q);
-                n += (int)__popcll(mi);
-            }
-        }
-        if (FILL) {
-            if (n <= SUP_ORDER_CAP) {
-                // outer entries carry their build distance, inner ones -1
-                int nout = 0;
-                for (int v = lane; v < n; v += 64) {
-                    const int64_t e = out[v];
-                    const GeoRec o = S.geo[ent_pos(e)];
-                    const double dx = me.x - o.x, dy = me.y - o.y;
-                    const bool outer = ent_id(e) > f;
-                    od_[v] = outer ? sqrt(dx * dx + dy * dy) : -1.0;
-                    oe_[v] = e;
-                    nout += (int)__popcll(__ballot(outer));
-                }
-                nout = __shfl(nout, 0);
-                wave_lds_sync();
-                for (int v = lane; v < n; v += 64) {
-                    const double dv = od_[v];
-                    const int64_t ev = oe_[v];
-                    int rank = 0;
-                    if (dv >= 0.0) {
-                        for (int u = 0; u < n; ++u) {
-                            const double du = od_[u];
-                            rank += (du >= 0.0 && (du < dv || (du == dv && oe_[u] < ev))) ? 1 : 0;
-                        }
-                    } else {
-                        rank = nout;
-                        for (int u = 0; u < n; ++u) rank += (od_[u] < 0.0 && oe_[u] < ev) ? 1 : 0;
+                    in = d2 <= thr * thr * (1.0 + 1e-12);
+                    if (in) {
+                        bound = fmaxf(nbme, S.nb[q]);
+                        if (o.id > f ? has_records(S, fs, o.id) : has_records(S, S.cval[q], f)) bound = SUP_KEEP;
+                        const double w = me.r + o.r + (double)bound + P.skin;
+                        near = d2 <= w * w * (1.0 + 1e-12);
                     }
-                    out[rank] = ev;
                 }
-                if (lane == 0) S.sout[k] = nout;
-                wave_lds_sync();
-            } else if (lane == 0) {
-                S.sout[k] = -1;
+                const uint64_t mi = __ballot(in), mn = __ballot(near);
+                if (FILL && in)
+                    out[near ? nn + (int)__popcll(mn & lt) : snear + (n - nn) + (int)__popcll(mi & ~mn & lt)] =
+                        sup_ent(bound, q);
+                n += (int)__popcll(mi);
+                nn += (int)__popcll(mn);
             }
         }
         if (lane == 0) {
-            if (FILL) S.x0[k] = make_double2(me.x, me.y);
-            else S.scnt[k] = n;
-        }
-    }
-}
-
-// A pair whose sheltering terms are needed (its distance is recomputed from
-// the two positions, the same expression as the scan's).
-struct DenseNear {
-    int32_t q;                   // partner position
-    uint8_t lane, outer;
-    uint16_t pad_;
-};
-
-// Order-preserving map of doubles to unsigned keys (a < b iff key(a) < key(b)
-// for non-NaN values), for minima taken with integer atomics.
-__device__ __forceinline__ uint64_t ord_key(double v) {
-    const uint64_t u = (uint64_t)__double_as_longlong(v);
-    return (u >> 63) ? ~u : (u | (1ull << 63));
-}
-__device__ __forceinline__ double ord_val(uint64_t k) {
-    return __longlong_as_double((long long)((k >> 63) ? (k & ~(1ull << 63)) : ~k));
-}
-
-// W2: two wavefronts over the same 64 floes, one per half of the
-// supersets (for dense queues that fit on the GPU at once); else one
-// wavefront takes both halves, one after the other.  (DENSE_WAVES_PER_SIMD
-// wavefronts per SIMD: the registers of a batch of partner rows and of two
-// sets of superset entries, 5 in mixed precision and 4 in FP64, and the LDS
-// of the rings and the near-pair list fit them without spilling.)
-template <bool MIXED, bool W2>
-__global__ __launch_bounds__(W2 ? 128 : 64, DENSE_WAVES_PER_SIMD) void k_cand_dense(DS S) {
-    using T = typename Prec<MIXED>::T;
-    __shared__ DenseNear nr[DENSE_NEAR];
-    __shared__ uint64_t mina[64], minw[64];
-    // staged rows of each wavefront: row r of lane l at (r % DENSE_RING) * 64 + l
-    __shared__ int64_t ring2_[W2 ? 2 : 1][DENSE_RING * 64];
-    __shared__ int xni[W2 ? 64 : 1];    // the inner wavefront's counts, flags and errors
-    __shared__ uint32_t xfl[W2 ? 64 : 1], xover[W2 ? 64 : 1];
-    __shared__ int ncnt_[2], err0;      // near pairs listed by each wavefront
-    // (the error word is read once for the block: a block that sets it may
-    // finish between the two wavefronts' starts, and both must take the
-    // barriers below or neither)
-    if (threadIdx.x == 0) err0 = *S.err;
-    __syncthreads();
-    if (err0) return;
-    // (W2: wavefront 0 the outer lists, 1 the inner ones)
-    const int lane = threadIdx.x & 63, wv = W2 ? (int)(threadIdx.x >> 6) : 0;
-    int64_t* const ring_ = ring2_[wv];
-    int k = -1;
-    {
-        const QueueView qv = queue_view(S, 3);
-        const int per = (qv.total + XCD_COUNT - 1) / XCD_COUNT;
-        const int local = (int)(blockIdx.x / XCD_COUNT) * 64 + lane;
-        const int t = (int)(blockIdx.x % XCD_COUNT) * per + local;
-        if (local < per && t < qv.total) k = queue_at(S, 3, qv, t);
-    }
-    GeoRec me;
-    me.x = me.y = me.r = 0.0;
-    me.id = 0;
-    me.member = -1;
-    int L = 0, nout = 0;
-    int64_t soff = 0;
-    if (k >= 0) {
-        me = S.geo[k];
-        if (me.member >= 0) {   // (-1: member past its stop step, nothing to do)
-            L = S.scnt[k];
-            nout = S.sout[k];
-            soff = S.soff[k];
-        }
-    }
-    bool act = k >= 0 && me.member >= 0;
-    if (act && nout < 0) {
-        if (wv == 0) S.ocnt[k] = DENSE_OVER;   // superset in scan order: the thread search
-        act = false;
-    }
-    const uint64_t one_key = ord_key(1.0);
-    if (wv == 0) {
-        mina[lane] = minw[lane] = one_key;
-    }
-    const int m = act ? me.member : 0;
-    const DevParams& P = S.params[m];
-    // the parameters every entry of the scan reads, held in registers (the
-    // list stores below could otherwise alias them); the bond parameters, the
-    // wind and the floe's sheltering record are read again where needed, so
-    // that the registers go to the batch of partners
-    const double rtree = P.rtree;
-    const bool shelter = P.shelter != 0;
-    const double rad = me.r + rtree;
-    const int f = me.id;
-    const int first = S.members[m].first;
-    const bool bond_step = act && S.members[m].tstep == 1 && P.restart != 1 && P.cohesion;
-    const T lim = sizeof(T) == 4 ? T(20) : T(40);
-    T lha = T(0), lhw = T(0);   // lim times the floe's two drafts
-    int fs = 0;
-    bool qc = false, qb = false;
-    if (act) {
-        const ShelRec sh = S.shel[k];
-        lha = lim * T(sh.hfa);
-        lhw = lim * T(sh.hfw);
-        fs = S.cval[k];
-        qc = S.hcnt_old[fs] > 0;
-        qb = S.bcnt_old[fs] > 0;
-    }
-    if (!act) L = nout = 0;
-    T sha = T(1), shw = T(1);
-    __syncthreads();
-    const int64_t SS = S.S;
-    int64_t* oj = S.oj;
-    const int64_t* se = S.sup + soff;
-    // the last min(no, DENSE_WIN) outer entries, ascending: slots [no - nw, no)
-    double wd[DENSE_WIN];
-    int64_t we[DENSE_WIN];
-#pragma unroll
-    for (int w = 0; w < DENSE_WIN; ++w) {
-        wd[w] = __longlong_as_double(0x7ff0000000000000ll);
-        we[w] = INT64_MAX;
-    }
-    int no = 0, ni = 0, nw = 0;
-    // rows below bo (outer) and bi (inner) are in HBM, a lane's rows from
-    // there on in its ring; od: this lane's outer list is all in HBM
-    int bo = 0, bi = 0;
-    bool od = false;
-    uint32_t over = 0;
-    // near pairs: this wavefront's part of the list (W2: half each) and the
-    // count of pairs listed so far
-    const int ncap = W2 ? DENSE_NEAR / 2 : DENSE_NEAR, nofs = wv * (DENSE_NEAR / 2);
-    int nbase = 0;
-    const uint64_t lt = lane ? ((~0ull) >> (64 - lane)) : 0ull;
-    auto rslot = [&](int r) { return (r & (DENSE_RING - 1)) * 64 + lane; };
-    auto less = [](double ad, int64_t ae, double bd, int64_t be) {
-        return ad < bd || (ad == bd && ent_id(ae) < ent_id(be));
-    };
-    // (the part of the list in HBM keeps no distances: the rare entry that
-    // belongs below the register part compares with a slot's entry by its
-    // distance recomputed from the positions, the same expression)
-    auto dist_of = [&](int64_t e) {
-        const GeoRec o = S.geo[ent_pos(e)];
-        const double dx = me.x - o.x, dy = me.y - o.y;
-        return sqrt(dx * dx + dy * dy);
-    };
-    auto put_outer = [&](int s, int64_t e) {
-        if (od || s < bo) oj[(int64_t)s * SS + k] = e;
-        else ring_[rslot(s)] = e;
-    };
-    auto insert_outer = [&](double xd, int64_t xe) {
-        if (no >= S.CO) { over |= ERR_OUTER_CAP; return; }
-        if (nw == DENSE_WIN && less(xd, xe, wd[0], we[0])) {
-            if (!od) {
-                // the staged rows [bo, no - DENSE_WIN) out first
-                for (int s = bo; s < no - DENSE_WIN; ++s) oj[(int64_t)s * SS + k] = ring_[rslot(s)];
-                od = true;
+            if (FILL) {
+                S.x0[k] = make_double2(me.x, me.y);
+            } else {
+                S.scnt[k] = n;
+                S.snear[k] = nn;
             }
-            // below the register part: into the part in HBM, whose slots
-            // [0, no - DENSE_WIN) move up by one from x's place on
-            int p = no - DENSE_WIN;
-            while (p > 0) {
-                const int64_t ep = oj[(int64_t)(p - 1) * SS + k];
-                if (!less(xd, xe, dist_of(ep), ep)) break;
-                oj[(int64_t)p * SS + k] = ep;
-                --p;
-            }
-            oj[(int64_t)p * SS + k] = xe;
-            ++no;
-            return;
         }
-        if (nw == DENSE_WIN) {
-            // the smallest register entry is final: to its slot
-            put_outer(no - DENSE_WIN, we[0]);
-            // (most entries come above the whole register part: they take
-            // its top without the insertion below)
-            const bool top = !less(xd, xe, wd[DENSE_WIN - 1], we[DENSE_WIN - 1]);
-#pragma unroll
-            for (int w = 0; w < DENSE_WIN - 1; ++w) { wd[w] = wd[w + 1]; we[w] = we[w + 1]; }
-            if (top) {
-                wd[DENSE_WIN - 1] = xd;
-                we[DENSE_WIN - 1] = xe;
-                ++no;
-                return;
-            }
-            wd[DENSE_WIN - 1] = __longlong_as_double(0x7ff0000000000000ll);
-            we[DENSE_WIN - 1] = INT64_MAX;
-            --nw;
-        }
-        // insertion into the sorted register part (empty slots hold keys
-        // above every entry)
-#pragma unroll
-        for (int w = 0; w < DENSE_WIN; ++w) {
-            const bool lt = less(xd, xe, wd[w], we[w]);
-            const double td = wd[w];
-            const int64_t te = we[w];
-            wd[w] = lt ? xd : td;
-            we[w] = lt ? xe : te;
-            xd = lt ? td : xd;
-            xe = lt ? te : xe;
-        }
-        ++nw;
-        ++no;
-    };
-    // row bo (bi) out to HBM for every lane that has it staged (the whole
-    // wavefront takes part)
-    auto out_outer = [&]() {
-        if (!od && no - nw > bo) oj[(int64_t)bo * SS + k] = ring_[rslot(bo)];
-        ++bo;
-    };
-    auto out_inner = [&]() {
-        if (ni > bi) S.ik[(int64_t)bi * SS + k] = ring_[rslot(bi)];
-        ++bi;
-    };
-    constexpr int B = MIXED ? DENSE_BATCH : DENSE_BATCH - 1;
-    // one pass over a part of every lane's superset: outer entries [0, nout),
-    // then inner ones [nout, L), entry t of the part at the same step
-    auto scan = [&](auto outer_part) {
-        constexpr bool outer = decltype(outer_part)::value;
-        const int vb = outer ? 0 : nout;
-        const int n = outer ? nout : L - nout;
-        int nmax = n;
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) nmax = max(nmax, __shfl_xor(nmax, off));
-        // a batch's superset entries are requested with the batch before, in
-        // the other of two register sets (a copy from one set to the other
-        // would wait for the loads); the last entry stands in past the end
-        int64_t ea[B], eb[B];
-#pragma unroll
-        for (int u = 0; u < B; ++u) ea[u] = eb[u] = 0;
-        if (n > 0) {
-#pragma unroll
-            for (int u = 0; u < B; ++u) ea[u] = se[vb + min(u, n - 1)];
-        }
-        auto batch = [&](const int t0, const int64_t (&ev)[B], int64_t (&en)[B]) {
-            const bool run = t0 < n;
-            // rows out: each row that every lane still scanning has passed,
-            // and those that make room for this batch (at most B rows, the
-            // register part's included)
-            for (;;) {
-                const int c = outer ? no - nw : ni;
-                const int b = outer ? bo : bi;
-                const bool mine = outer ? !od : true;
-                if (!__ballot(mine && c > b)) break;
-                if (!__ballot(run && mine && (outer ? no : ni) + B > b + DENSE_RING) &&
-                    __ballot(run && mine && c <= b))
-                    break;
-                if (outer) out_outer(); else out_inner();
-            }
-            // (every lane takes part in the batch, so that the near-pair
-            // count below stays the same in all of them)
-            GeoRec g[B];
-            if (run) {
-#pragma unroll
-                for (int u = 0; u < B; ++u) g[u] = S.geo[ent_pos(ev[u])];
-                if (t0 + B < n) {
-#pragma unroll
-                    for (int u = 0; u < B; ++u) en[u] = se[vb + min(t0 + B + u, n - 1)];
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < B; ++u) {
-                const GeoRec& o = g[u];
-                const double dx = me.x - o.x, dy = me.y - o.y;
-                const double dist2 = dx * dx + dy * dy;
-                const double thr = outer ? rad : o.r + rtree;
-                // far beyond the radius: no square root needed
-                bool inr = run && t0 + u < n && !(dist2 > thr * thr * (1.0 + 1e-12));
-                double d = 0.0;
-                if (inr) d = sqrt(dist2);
-                inr = inr && d <= thr;
-                // outer: pair (f, j) with f the outer floe i of the event;
-                // inner: pair (j, f) with f the inner floe j
-                const double deltan = outer ? me.r + o.r - d : o.r + me.r - d;
-                const T dn = T(deltan);
-                bool near = false;
-                if (inr) {
-                    if (deltan > 0) qc = true;
-                    if (outer && bond_step && deltan >= -P.bond_lim &&
-                        bond_keep(f - first, ent_id(ev[u]) - first, P.bond_seed, P.bond_thr24))
-                        qb = true;
-                    near = shelter && (!(dn < T(0) && T((double)0.18f) * -dn >= lha) ||
-                                       !(dn < T(0) && T((double)0.18f) * -dn >= lhw));
-                }
-                // near pairs take consecutive slots of the wavefront's part of
-                // the list, counted by ballot (the same count in every lane)
-                const uint64_t mn = __ballot(near);
-                const int slot = nbase + (int)__popcll(mn & lt);
-                nbase += (int)__popcll(mn);
-                if (near) {
-                    {
-                        if (slot < ncap) {
-                            DenseNear r;
-                            r.q = ent_pos(ev[u]); r.lane = (uint8_t)lane; r.outer = outer ? 1 : 0;
-                            r.pad_ = 0;
-                            nr[nofs + slot] = r;
-                        } else {
-                            // list full: this thread takes the terms itself
-                            const double nx = outer ? o.x - me.x : me.x - o.x;
-                            const double ny = outer ? o.y - me.y : me.y - o.y;
-                            const double cosa = nx / d, sina = ny / d;
-                            const ShelRec ms = S.shel[k];
-                            const ShelRec oh = S.shel[ent_pos(ev[u])];
-                            const T c0t = T(cosa), s0t = T(sina);
-                            const T c = outer ? -c0t : c0t, sn = outer ? -s0t : s0t;
-                            const T ux = outer ? T(ms.wx) : T(oh.wx), uy = outer ? T(ms.wy) : T(oh.wy);
-                            sha = shelter_min(sha, T(oh.hfa), T(ms.hfa), dn, c, sn, ux, uy);
-                            shw = shelter_min(shw, T(oh.hfw), T(ms.hfw), dn, c, sn, T(P.uw), T(P.vw));
-                        }
-                    }
-                }
-                if (!inr) continue;
-                if (outer) {
-                    insert_outer(d, ev[u]);
-                } else if (ni < S.CI) {
-                    if (ni < bi) S.ik[(int64_t)ni * SS + k] = ev[u];
-                    else ring_[rslot(ni)] = ev[u];
-                    ++ni;
-                } else {
-                    over |= ERR_INNER_CAP;
-                }
-            }
-            if (outer && run && t0 + B >= n) {
-                // the lane's last outer entries: its register part is final
-#pragma unroll
-                for (int w = 0; w < DENSE_WIN; ++w)
-                    if (w < nw) put_outer(no - nw + w, we[w]);
-                nw = 0;
-            }
-        };
-        for (int t0 = 0; t0 < nmax; t0 += 2 * B) {
-            batch(t0, ea, eb);
-            if (t0 + B < nmax) batch(t0 + B, eb, ea);
-        }
-    };
-    if (wv == 0) {
-        scan(std::true_type{});
-        // every staged outer row out (each lane's register part went to its
-        // rows with its last batch): the ring is free for the inner half
-        while (__ballot(!od && no > bo)) out_outer();
+        sum += nn;
     }
-    if (!W2 || wv == 1) {
-        scan(std::false_type{});
-        while (__ballot(ni > bi)) out_inner();
-        if (W2) {
-            xni[lane] = ni;
-            xfl[lane] = qc ? 1u : 0u;
-            xover[lane] = over;
-        }
-    }
-    if (lane == 0) ncnt_[wv] = min(nbase, ncap);
-    // minima a thread took itself (near-pair list full) join the LDS ones
-    if (sha < T(1)) atomicMin((unsigned long long*)&mina[lane], (unsigned long long)ord_key((double)sha));
-    if (shw < T(1)) atomicMin((unsigned long long*)&minw[lane], (unsigned long long)ord_key((double)shw));
-    // sheltering terms of the listed near pairs, across the lanes (every lane
-    // takes part in each round; the listing thread's floe comes by shuffle)
-    ShelRec msh;
-    msh.hfa = msh.hfw = msh.wx = msh.wy = 0.0;
-    if (act) msh = S.shel[k];
-    __syncthreads();
-    // (W2: the two wavefronts take alternate rounds of 64 pairs)
-    const int nn0 = ncnt_[0], nn = nn0 + (W2 ? ncnt_[1] : 0);
-    for (int i0 = wv * 64; i0 < nn; i0 += W2 ? 128 : 64) {
-        const int i = i0 + lane;
-        DenseNear r;
-        r.q = 0; r.lane = 0; r.outer = 0; r.pad_ = 0;
-        if (i < nn) r = nr[i < nn0 ? i : DENSE_NEAR / 2 + (i - nn0)];
-        const int ow = r.lane;
-        const double ox = __shfl(me.x, ow), oy = __shfl(me.y, ow), orr = __shfl(me.r, ow);
-        const double ohfa = __shfl(msh.hfa, ow), ohfw = __shfl(msh.hfw, ow);
-        const double owx = __shfl(msh.wx, ow), owy = __shfl(msh.wy, ow);
-        const double ouw = __shfl(P.uw, ow), ovw = __shfl(P.vw, ow);
-        if (i < nn) {
-            const GeoRec o = S.geo[r.q];
-            const ShelRec oh = S.shel[r.q];
-            const bool outer = r.outer != 0;
-            const double ddx = ox - o.x, ddy = oy - o.y;
-            const double d = sqrt(ddx * ddx + ddy * ddy);
-            // outer: f takes hsf*(j,f) with -cosa, -sina of f -> j and its own
-            // wind; inner: cosa/sina from j to f and j's wind
-            const double deltan = outer ? orr + o.r - d : o.r + orr - d;
-            const double nx = outer ? o.x - ox : ox - o.x;
-            const double ny = outer ? o.y - oy : oy - o.y;
-            const double cosa = nx / d, sina = ny / d;
-            const T dn = T(deltan), c0t = T(cosa), s0t = T(sina);
-            const T c = outer ? -c0t : c0t, sn = outer ? -s0t : s0t;
-            const T ux = outer ? T(owx) : T(oh.wx), uy = outer ? T(owy) : T(oh.wy);
-            const T ta = shelter_min(T(1), T(oh.hfa), T(ohfa), dn, c, sn, ux, uy);
-            const T tw = shelter_min(T(1), T(oh.hfw), T(ohfw), dn, c, sn, T(ouw), T(ovw));
-            if (ta < T(1)) atomicMin((unsigned long long*)&mina[ow], (unsigned long long)ord_key((double)ta));
-            if (tw < T(1)) atomicMin((unsigned long long*)&minw[ow], (unsigned long long)ord_key((double)tw));
-        }
-    }
-    __syncthreads();
-    if (wv != 0 || !act) return;
-    sha = T(ord_val(mina[lane]));
-    shw = T(ord_val(minw[lane]));
-    if (W2) {
-        ni = xni[lane];
-        qc = qc || (xfl[lane] & 1u);
-        over |= xover[lane];
-    }
-    if (over) set_err(S, over);
-    const bool qw = me.y - me.r < 0 || me.y + me.r > P.ny || me.x - me.r < 0 || me.x + me.r > P.nx;
-    cand_finish<MIXED>(S, k, fs, P, no, ni, double(sha), double(shw), qc, qb, 0, 1);
-    if (qc) enqueue_one(S, 0, k);
-    if (qb) enqueue_one(S, 1, k);
-    if (qw) enqueue_one(S, 2, k);
-}
-
-// The thread search for the dense floes whose candidates overflow the dense
-// search's LDS lists (marked DENSE_OVER in ocnt, which every dense floe's
-// search writes each step).  One thread per entry of the dense queue.
-template <bool MIXED>
-__global__ __launch_bounds__(FLOE_BLOCK) void k_cand_dense_over(DS S) {
-    if (*S.err) return;
-    const int k = queue_entry(S, 3);
-    if (k < 0 || S.ocnt[k] != DENSE_OVER) return;
-    const GeoRec me = S.geo[k];
-    const CandPre pre = cand_pre(S, k);
-    bool qc = false, qb = false, qw = false;
-    cand_thread<MIXED, false>(S, k, me, pre, me.member, true, qc, qb, qw, nullptr);
-    if (qc) enqueue_one(S, 0, k);
-    if (qb) enqueue_one(S, 1, k);
-    if (qw) enqueue_one(S, 2, k);
+    if (!FILL && lane == 0 && sum) atomicAdd((unsigned long long*)S.nearsum, (unsigned long long)sum);
 }
 
 // ---------------------------------------------------------------------
 // 3. speculative events + per-floe gather + owner state writes
 // ---------------------------------------------------------------------
 // Contact state of pair (i, j), owner i by storage slot, partner j by
-// identity: history, last contact forces and whether it is bonded.
-__device__ __forceinline__ void load_contact_state(const DS& S, int i, int j, PairState& ps) {
+// identity: history, last contact forces and whether it is bonded.  Returns
+// whether it has a history.
+__device__ __forceinline__ bool load_contact_state(const DS& S, int i, int j, PairState& ps) {
     ps.deltat = 0.0; ps.thetarelc = 0.0; ps.fcn = 0.0; ps.fct = 0.0;
     ps.bond = 0; ps.has_bond_rec = false;
     ps.damage = ps.deltanb = ps.deltatb = ps.trb_ji = ps.trb_ij = 0.0;
@@ -1723,6 +1326,7 @@ __device__ __forceinline__ void load_contact_state(const DS& S, int i, int j, Pa
         ps.has_bond_rec = true;
         ps.bond = S.bond_old[(int64_t)bq * S.S + i].bond;
     }
+    return hq >= 0;
 }
 
 // Contact terms of the queued floes (contact_forces, plastic_contact,
@@ -1854,7 +1458,7 @@ __global__ __launch_bounds__(FLOE_BLOCK, 3) void k_contact(DS S) {
                         Kin kn;
                         kinematics(Fi, Fj, kn);
                         PairState ps;
-                        load_contact_state(S, ofs, j, ps);
+                        const bool had = load_contact_state(S, ofs, j, ps);
                         bond_create(P, tstep, of - first, j - first, Fi, Fj, kn, ps);
                         EventOut o;
                         o.flags = 0;
@@ -1868,6 +1472,7 @@ __global__ __launch_bounds__(FLOE_BLOCK, 3) void k_contact(DS S) {
                         if (ps.deltat != 0.0 || ps.thetarelc != 0.0 || ps.fcn != 0.0 || ps.fct != 0.0) {
                             r.kind |= 2;
                             r.deltat = ps.deltat; r.thetarelc = ps.thetarelc; r.fcn = ps.fcn; r.fct = ps.fct;
+                            if (!had && P.dense) sup_keep(S, ko, qj);
                         }
                         if (o.flags & EV_RIDGED) {
                             const int p = atomicAdd(&S.nseeds[om], 1);
@@ -1965,6 +1570,7 @@ __device__ __forceinline__ bool bond_event(const DS& S, const DevParams& P, int 
     if (rq < 0) {
         if (nb < S.BC) rq = nb++;
         else { over |= ERR_BOND_CAP; return false; }
+        if (P.dense) sup_keep(S, k, qj);
     }
     S.bond_new[(int64_t)rq * SS + fs] = bond_from(ps, j);
     if (!(o.flags & EV_BONDED)) return false;
@@ -2542,53 +2148,67 @@ __global__ __launch_bounds__(REPAIR_THREADS) void k_repair(DS S, int nmembers) {
     // every reshaped floe, and the partners of its later events that can
     // notice (in contact, bonded, or near enough for their own sheltering).
     // Counted on the way: the seeds and the events after a reshape of one of
-    // their floes (each once).
+    // their floes (each once), over all candidates, listed or not, so from
+    // the supersets.
     const int nn = nn_;
     const bool bond_step = tstep == 1 && P.restart != 1 && P.cohesion;
+    const double rtree = P.rtree;
     int counted = 0;
     const int rpw = share(nn);
     for (int c0 = 0; c0 < nn; c0 += waves * rpw) {
         const int p = c0 + (tid >> 6) * rpw + lane;
         const bool act = lane < rpw && p < nn;
-        int kg = 0, gid = 0, bown = 0, wall = 0;
-        int64_t key = 0;
-        LaterEvents l{0, 0, 0, 0};
+        int kg = 0, gid = 0, bown = 0, cnt = 0, fr = 0, idr = 0;
+        int64_t soff = 0;
+        double dr = -1.0;           // the record's pair, if it is one of the floe's own
         GeoRec gg;
         gg.x = gg.y = gg.r = 0.0;
         if (act) {
-            key = rec[p].key;
+            const int64_t key = rec[p].key;
             kg = rec[p].pos;
             const int kf = rec[p].kf, kj = rec[p].kj;
             touch_floe(S, kf);
             if (kj >= 0) touch_floe(S, kj);
             gg = S.geo[kg];
             gid = gg.id;
-            const int hk = rhead_at(S, kg);
-            const int64_t k0 = first_reshape(rec, hk);
+            const int64_t k0 = first_reshape(rec, rhead_at(S, kg));
             if (p < ns) {
                 // a seed that is not after a reshape of either floe
                 const int ko = kg == kf ? kj : kf;
                 const int64_t ko0 = ko >= 0 ? first_reshape(rec, rhead_at(S, ko)) : INT64_MAX;
                 if (!(k0 < key) && !(ko0 < key)) ++counted;
             }
-            if (rec[p].live && k0 == key) {
-                l = later_events(S, key, kg, gid, first);
-                wall = (key & 0xFFFF) != WALL_SLOT ? 1 : 0;
+            // (a floe's walls are its last event)
+            if (rec[p].live && k0 == key && (key & 0xFFFF) != WALL_SLOT) {
+                ++counted;           // its walls come after
+                cnt = S.scnt[kg];
+                soff = S.soff[kg];
+                fr = (int)(key >> 16);
                 bown = S.bcnt_old[S.cval[kg]];
+                if (kg == kf) {
+                    const GeoRec gj = S.geo[kj];
+                    const double dx = gg.x - gj.x, dy = gg.y - gj.y;
+                    dr = sqrt(dx * dx + dy * dy);
+                    idr = gj.id;
+                }
             }
         }
-        counted += wall;
-        each_later(l.ni + l.no, [&](int own, int local) {
-            const int ko = __shfl(kg, own), go = __shfl(gid, own), fo = __shfl(l.f, own);
-            const int nio = __shfl(l.ni, own), s0 = __shfl(l.s0, own), bo = __shfl(bown, own);
+        each_later(cnt, [&](int own, int local) {
+            const int go = __shfl(gid, own), fo = __shfl(fr, own), bo = __shfl(bown, own), ido = __shfl(idr, own);
+            const int64_t so = __shfl(soff, own);
+            const double dro = __shfl(dr, own);
             const double ox = __shfl(gg.x, own), oy = __shfl(gg.y, own), orr = __shfl(gg.r, own);
             if (local < 0) return;
-            const bool inner = local < nio;
-            const int64_t e = inner ? S.ik[(int64_t)local * SS + ko]
-                                    : S.oj[(int64_t)(s0 + local - nio) * SS + ko];
-            const int q = ent_pos(e);
-            if (inner && ent_id(e) - first <= fo) return;     // before the reshape
+            const int q = ent_pos(S.sup[so + local]);
             const GeoRec o = S.geo[q];
+            const bool inner = o.id < go;                 // the floe is the pair's inner one
+            const double dx = ox - o.x, dy = oy - o.y;
+            const double d = sqrt(dx * dx + dy * dy);
+            if (!(d <= (inner ? o.r : orr) + rtree)) return;        // not a candidate
+            // after the record: in a later iteration, or later in the same one
+            const bool later = dro >= 0.0 ? !inner && (d > dro || (d == dro && o.id > ido))
+                                          : !inner || o.id - first > fo;
+            if (!later) return;
             const ShelRec sh = S.shel[q];
             const int hq = rhead_at(S, q);
             const int bc = inner ? S.bcnt_old[S.cval[q]] : bo;
@@ -2596,13 +2216,22 @@ __global__ __launch_bounds__(REPAIR_THREADS) void k_repair(DS S, int nmembers) {
             // from the outer floe's side
             bool both = false;
             if (hq >= 0) {
-                const int64_t ek = inner ? ((int64_t)(ent_id(e) - first) << 16) | slot_of(S, q, go)
-                                         : ((int64_t)(go - first) << 16) | (s0 + local - nio);
-                both = first_reshape(rec, hq) < ek;
+                const int pq = first_record(rec, hq);
+                if (pq >= 0) {
+                    const Reshape& w = rec[pq];
+                    const int al = (inner ? o.id : go) - first, wf = (int)(w.key >> 16);
+                    if (wf != al) {
+                        both = wf < al;
+                    } else if ((w.key & 0xFFFF) != WALL_SLOT) {
+                        const GeoRec a = S.geo[w.kf], b = S.geo[w.kj];
+                        const double ex = a.x - b.x, ey = a.y - b.y;
+                        const double de = sqrt(ex * ex + ey * ey);
+                        both = de < d || (de == d && b.id < (inner ? go : o.id));
+                    }
+                }
             }
             if (!(both && inner)) ++counted;
-            const double dx = inner ? o.x - ox : ox - o.x, dy = inner ? o.y - oy : oy - o.y;
-            const double dn = (inner ? o.r + orr : orr + o.r) - sqrt(dx * dx + dy * dy);
+            const double dn = orr + o.r - d;
             // (radii only shrink: a term that is exactly 1 stays so)
             using T = typename Prec<MIXED>::T;
             const T lim = sizeof(T) == 4 ? T(20) : T(40), dnt = T(dn);
@@ -2782,7 +2411,6 @@ __global__ __launch_bounds__(FLOE_BLOCK, 2) void k_fixup(DS S) {
                 };
                 if ((oh >= 0) | (hq >= 0)) {
                     const int al = ia - first;
-                    int sl = inner ? -1 : local - oni;      // (the slot of an inner pair only where it decides)
                     // last record before the event: of a, of b; of a before its
                     // iteration
                     int wa_ = -1, wb_ = -1, wq_ = -1;
@@ -2790,9 +2418,15 @@ __global__ __launch_bounds__(FLOE_BLOCK, 2) void k_fixup(DS S) {
                     auto before = [&](const Reshape& w) {
                         const int rf = (int)(w.key >> 16);
                         if (rf != al) return rf < al;
-                        if (w.kf == ka && w.kj == kb) return false;   // the event's own
-                        if (sl < 0) sl = slot_of(S, qp, of);
-                        return (int)(w.key & 0xFFFF) < sl;
+                        const int ws = (int)(w.key & 0xFFFF);
+                        if (!inner) return ws < local - oni;
+                        // the same outer floe's event with another partner, or its
+                        // walls: by distance, as its list is
+                        if (ws == WALL_SLOT || w.kj == kb) return false;
+                        const GeoRec wf = S.geo[w.kf], wj = S.geo[w.kj];
+                        const double ex = wf.x - wj.x, ey = wf.y - wj.y;
+                        const double de = sqrt(ex * ex + ey * ey);
+                        return de < d || (de == d && wj.id < ib);
                     };
                     for (int p = inner ? hq : oh; p >= 0; p = rec[p].next) {
                         const Reshape& w = rec[p];
@@ -2843,6 +2477,7 @@ __global__ __launch_bounds__(FLOE_BLOCK, 2) void k_fixup(DS S) {
                             const int p = atomicAdd(&S.bcnt_new[ofs], 1);
                             if (p < S.BC) S.bond_new[(int64_t)p * SS + ofs] = bond_from(ps, pid);
                             else over |= ERR_BOND_CAP;
+                            if (P.dense) sup_keep(S, ko, qp);
                         }
                         const bool hist = ps.deltat != 0.0 || ps.thetarelc != 0.0 || ps.fcn != 0.0 || ps.fct != 0.0;
                         HistRec hr;
@@ -2853,6 +2488,7 @@ __global__ __launch_bounds__(FLOE_BLOCK, 2) void k_fixup(DS S) {
                         } else if (hist) {
                             o.nr = hr.deltat; o.nh = hr.thetarelc; o.nmass = hr.fcn; o.ninertia = hr.fct;
                             o.ridged = pid;
+                            if (P.dense) sup_keep(S, ko, qp);
                             o.flags |= EV_PUT_HIST;
                         }
                     }
@@ -2914,6 +2550,14 @@ __global__ __launch_bounds__(FLOE_BLOCK, 2) void k_fixup(DS S) {
                     S.cur[0 * SS + fs] = Fn.r; S.cur[1 * SS + fs] = Fn.h; S.cur[2 * SS + fs] = Fn.mass;
                     S.cur[3 * SS + fs] = Fn.inertia; S.cur[4 * SS + fs] = Fn.hfa; S.cur[5 * SS + fs] = Fn.hfw;
                     S.dirty[fs] = 1;
+                    // drafts that outgrew the floe's bound: its lists may lack a
+                    // pair, so the step runs again with a build and more room
+                    const double reach = P.shelter ? near_reach(S.near_lim, Fn.hfa, Fn.hfw) : 0.0;
+                    if (1.01 * reach > (double)S.nb[k]) {
+                        S.nbmin[fs] = (float)fmin(NEAR_ROOM * reach, 1e30);
+                        atomicOr(S.rebuild, BUILD_DUE);
+                        set_err(S, ERR_NEED_BUILD);
+                    }
                 }
             }
         }
@@ -3008,7 +2652,10 @@ __global__ __launch_bounds__(FLOE_BLOCK, (MIXED && !REC) ? 5 : 4) void k_final(D
     // every earlier kernel of the step has finished: the step is complete
     if (k == 0) *S.steps_done += 1;
     const int m = me.member;
-    if (m < 0) return;
+    if (m < 0) {
+        S.geo_new[k] = me;
+        return;
+    }
     const DevParams& P = S.params[m];
     const int64_t SS = S.S;
     const uint8_t dflags = S.dirty[f];
@@ -3108,7 +2755,7 @@ __global__ __launch_bounds__(FLOE_BLOCK, (MIXED && !REC) ? 5 : 4) void k_final(D
     {
         GeoRec g;
         g.x = out.x; g.y = out.y; g.r = out.r; g.id = me.id; g.member = m;
-        S.geo[k] = g;
+        S.geo_new[k] = g;
         KinRec q;
         q.u = out.u; q.v = out.v; q.omega = out.omega; q.h = out.h; q.mass = out.mass;
         q.inertia = out.inertia; q.theta = out.theta;
@@ -3134,17 +2781,47 @@ __global__ __launch_bounds__(FLOE_BLOCK, (MIXED && !REC) ? 5 : 4) void k_final(D
     }
 }
 
-// per-member totals of the last step: candidates, contacts (evf flags) and
-// current bonds; diagnostics only
+// The candidate pairs of the floe at position k in the last step (the
+// reference's kNearest within r(i) + rtree): those of its superset within the
+// query radius, by the positions the step started from (the other of the two
+// position buffers) and its radius at the top of its iteration; fn(partner's
+// identity) for each.
+template <typename F>
+__device__ __forceinline__ void each_candidate(const DS& S, int k, const GeoRec& me, F&& fn) {
+    const int m = me.member;
+    const double rtree = S.params[m].rtree;
+    const int first = S.members[m].first;
+    const Reshape* rec = S.shape + (int64_t)S.SEEDK * first;
+    Floe Fq;
+    Fq.r = me.r;
+    floe_at_event(rec, S.rhead[k], (int64_t)(me.id - first) << 16, Fq);
+    const int64_t* se = S.sup + S.soff[k];
+    const int n = S.scnt[k];
+    for (int i0 = 0; i0 < n; i0 += 4) {
+        GeoRec o[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) o[u] = S.geo_new[ent_pos(se[min(i0 + u, n - 1)])];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const double dx = me.x - o[u].x, dy = me.y - o[u].y;
+            if (i0 + u < n && o[u].id > me.id && sqrt(dx * dx + dy * dy) <= Fq.r + rtree) fn(o[u].id);
+        }
+    }
+}
+
+// totals of the last step: candidates, contacts (evf flags) and current
+// bonds; diagnostics only
 __global__ void k_totals(DS S, int64_t* out) {
     int k = blockIdx.x * blockDim.x + threadIdx.x;
     int64_t c = 0, ct = 0, bd = 0;
     if (k < S.N && S.geo[k].member >= 0) {
+        const GeoRec me = S.geo_new[k];
         int no = S.ocnt[k];
+        if (me.member >= 0) each_candidate(S, k, me, [&](int) { ++c; });
+        else no = 0;
         for (int s = 0; s < no; ++s) {
             uint32_t fl = S.evf[(int64_t)s * S.S + k];
             if (fl & EV_REMOVED) continue;
-            ++c;
             if (fl & EV_CONTACT) ++ct;
         }
         int f = S.cval[k];
@@ -3167,17 +2844,25 @@ __global__ void k_totals(DS S, int64_t* out) {
     }
 }
 
+// Member m's candidate pairs of the last step, as (i, j) in the caller's
+// indices, in no order: counted in *n, the first `cap` written to `out`.
+__global__ void k_pairs(DS S, int m, int* n, int2* out, int cap) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= S.N) return;
+    const GeoRec me = S.geo_new[k];
+    if (me.member != m) return;
+    const int first = S.members[m].first;
+    each_candidate(S, k, me, [&](int j) {
+        const int at = atomicAdd(n, 1);
+        if (at < cap) out[at] = make_int2(me.id - first, j - first);
+    });
+}
+
 // explicit instantiations used by the host launcher
 template __global__ void k_sup<false>(DS);
 template __global__ void k_sup<true>(DS);
 template __global__ void k_sup_dense<false>(DS);
 template __global__ void k_sup_dense<true>(DS);
-template __global__ void k_cand_dense<false, false>(DS);
-template __global__ void k_cand_dense<false, true>(DS);
-template __global__ void k_cand_dense<true, false>(DS);
-template __global__ void k_cand_dense<true, true>(DS);
-template __global__ void k_cand_dense_over<false>(DS);
-template __global__ void k_cand_dense_over<true>(DS);
 template __global__ void k_cand<false>(DS);
 template __global__ void k_cand<true>(DS);
 template __global__ void k_contact<false>(DS);

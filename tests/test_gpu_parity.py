@@ -517,6 +517,44 @@ def test_dense_search_matches_thread_search():
             assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("what", ["separating", "thickening"])
+def test_dense_lists_keep_every_pair_that_matters(what):
+    """The dense members' step lists hold only pairs near enough to matter;
+    state and stresses stay those of the oracle's step over all candidates,
+    and the candidate pairs reported are all of them: pairs that part by up to
+    900 m with bonds and contact histories of theirs (further than their floes
+    shelter each other), and floes that ridging thickens past the room their
+    lists were built with (up to 1.5 times)."""
+    from oracle_py import OracleSim
+    if what == "separating":
+        f = kick(squeeze(packed_box(40, 5, box=1.6e4), 0.99), 1, speed=30.0)
+        p = config0_params(f, rtree=9000.0, eb=1e2, bond_lim=60.0, sigmatb_crit=1e12,
+                           sigmacb_crit=1e12, tau_crit=1e12)
+        steps = 40
+    else:
+        f = kick(squeeze(packed_box(64, 3), 0.9), 1, speed=1.0)
+        p = config0_params(f, sigmanc_crit=3e4, rtree=6000.0)
+        steps = 30
+    ctx = _ctx(f.n)
+    ctx.set_dense_search(0)
+    ctx.record_forces(True)
+    m = ctx.add_field(p, f)
+    O = OracleSim(p, f)
+    for t in range(1, steps + 1):
+        ctx.step(1)
+        O.step()
+        cand, cont = _oracle_pairs(O)
+        assert _pairs(ctx, m, "candidate") == cand and _pairs(ctx, m, "contact") == cont, t
+        assert ctx.totals()["candidates"] == len(cand), t
+        a, b = ctx.floes(m), O.state()
+        for k in STATE:
+            assert np.array_equal(a[k], b[k]), (t, k)
+        fa, fb = ctx.forces(m), O.forces()
+        for k in ("tsigxx", "tsigyy", "tsigxy", "tsigyx"):
+            assert np.max(np.abs(fa[k] - fb[k])) <= 1e-13 * np.max(np.abs(fb[k])), (t, k)
+    ctx.close()
+
+
 def test_dense_search_long_lists_and_unordered_supersets():
     """Dense floes with long candidate lists give the same lists, sheltering
     and trajectories through the dense search as through the thread search,
