@@ -129,10 +129,10 @@ struct DS {
     int64_t* sup;              // [sup_cap]
     int64_t sup_cap;
     int32_t* scnt;             // [S] by pos
-    int32_t* snear;            // [S] by pos: the first entries, which the search reads (all
-                               // of them but in dense members, see k_sup_dense)
+    int32_t* snear;            // [S] by pos: the first entries, those that can come within
+                               // their bound and that the search reads
     float* nb;                 // [S] by pos: how far apart a pair of the floe may be and
-                               // still matter to it (dense members; at the build)
+                               // still matter to it (at the build)
     float* nbmin;              // [S] by storage slot: nb is at least this (0: no demand)
     int64_t* nearsum;          // sum of snear
     int64_t* soff;             // [S] by pos

@@ -33,7 +33,7 @@
 // a sorted copy of the 96-byte floe records, so that a floe's neighbours sit
 // close in memory.  Pair state persists per floe id.  List entries pack the
 // partner as (id << 32 | pos).  The lists hold the candidates that can matter
-// (all of them but in dense members, see k_sup_dense).
+// (sup_bound_of).
 #include "godar_engine.h"
 #include "godar_physics.h"
 #include <type_traits>
@@ -139,7 +139,8 @@ __device__ __forceinline__ QueueShare queue_share(const DS& S, int qn) {
     QueueShare q;
     const int f = (per + nw - 1) / nw;
     const int64_t entries = *S.nearsum;     // entries the search reads
-    const int full = (int)min((int64_t)64, 64 * (int64_t)S.N / max(entries, (int64_t)1));
+    // (a floe in contact has about 1.6 listed pairs for each entry of the mean)
+    const int full = (int)min((int64_t)64, 40 * (int64_t)S.N / max(entries, (int64_t)1));
     q.floes = f > 16 ? 64 : max(1, max(f, full));
     q.begin = lo + w * q.floes;
     q.end = min(qn, lo + per);
@@ -166,7 +167,7 @@ __device__ __forceinline__ int64_t ent(int id, int pos) {
 
 // Superset entries: the partner's position and, in the high half, the bound
 // (a float): the pair is listed only while its floes are no further apart
-// than that (see k_sup_dense).
+// than that (sup_bound_of).
 constexpr float SUP_KEEP = __builtin_inff();
 __device__ __forceinline__ int64_t sup_ent(float bound, int pos) {
     return ((int64_t)__float_as_int(bound) << 32) | (int64_t)(uint32_t)pos;
@@ -175,18 +176,19 @@ __device__ __forceinline__ double sup_bound(int64_t e) { return (double)__int_as
 // The pair at positions a and b is listed from now on whatever its distance
 // (it has a contact history or a bond): its entries of both supersets.
 __device__ __forceinline__ void sup_keep(const DS& S, int a, int b) {
+    int64_t *sa = S.sup + S.soff[a], *sb = S.sup + S.soff[b];
+    const int na = S.snear[a], nb = S.snear[b];
+    for (int i0 = 0; i0 < max(na, nb); i0 += 4) {
+        int64_t ea[4], eb[4];
 #pragma unroll
-    for (int side = 0; side < 2; ++side) {
-        const int k = side ? b : a, q = side ? a : b;
-        int64_t* se = S.sup + S.soff[k];
-        const int n = S.snear[k];
-        for (int i0 = 0; i0 < n; i0 += 4) {
-            int64_t e[4];
+        for (int u = 0; u < 4; ++u) {
+            ea[u] = sa[min(i0 + u, max(na - 1, 0))];
+            eb[u] = sb[min(i0 + u, max(nb - 1, 0))];
+        }
 #pragma unroll
-            for (int u = 0; u < 4; ++u) e[u] = se[min(i0 + u, n - 1)];
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                if (ent_pos(e[u]) == q) se[min(i0 + u, n - 1)] = sup_ent(SUP_KEEP, q);
+        for (int u = 0; u < 4; ++u) {
+            if (i0 + u < na && ent_pos(ea[u]) == b) sa[i0 + u] = sup_ent(SUP_KEEP, b);
+            if (i0 + u < nb && ent_pos(eb[u]) == a) sb[i0 + u] = sup_ent(SUP_KEEP, a);
         }
     }
 }
@@ -506,7 +508,7 @@ __global__ void k_ranges(DS S) {
             double nb = P.shelter ? NEAR_ROOM * near_reach(S.near_lim, fr.hfa, fr.hfw) : 0.0;
             if (P.cohesion) nb = fmax(nb, P.bond_lim);
             nb = fmax(nb, (double)S.nbmin[f]) * (1.0 + 1e-6);
-            S.nb[k] = P.dense && nb < 1e30 ? (float)nb : SUP_KEEP;
+            S.nb[k] = nb < 1e30 ? (float)nb : SUP_KEEP;
             const uint32_t key = S.ckey[k];
             if (k == 0 || S.ckey[k - 1] != key) S.crange[key].x = k;
             if (k == S.N - 1 || S.ckey[k + 1] != key) S.crange[key].y = k + 1;
@@ -583,16 +585,50 @@ __device__ __forceinline__ void cand_finish(const DS& S, int k, int fs, const De
 constexpr int SCAN_BATCH = 4;
 constexpr int LIST_REGS = 4;
 
+// The query radius r + rtree holds many floes that are far away: no contact,
+// no bond, and a sheltering term that is exactly 1 (with power-law radii on
+// [200, 5000] m, nearly all of a floe's 43 candidates).  A pair can only matter
+// while its floes are no further apart than the larger of their two bounds nb
+// (the reach of their own sheltering, with room for the drafts to grow, and
+// the distance bonds form at), or if it has a contact history or a bond.  So
+// a superset puts the entries that can come within their bound before the
+// next build first (snear of them), each entry with its bound (SUP_KEEP for
+// pairs with a history or a bond; k_contact and k_bond set it on the entries
+// of new ones), and the step's search reads those alone and lists the pairs
+// within their bound: 9-11 of 59 entries and 2.4-4.2 of 43 candidates a floe
+// at packing 0.7 of the power-law radii, 2.2-2.5 of 3.6 and 1.5-1.7 of 2.6
+// with radii on [500, 2000] m at 0.55.  (One MI355X, against a search and
+// lists of all candidates: 320,000 power-law floes mixed, search 0.39 -> 0.11
+// ms, integration 0.088 -> 0.034, bonds 0.034 -> 0.016; 262,144 FP64, search
+// 0.38 -> 0.16; 1,000 floes 0.114 -> 0.041; the 512-field ensemble of radii on
+// [500, 2000] m, search 0.136 -> 0.115.)
+// The other entries only answer which pairs were candidates (k_pairs) and how
+// many events a reshape came before (k_repair).  A reshape whose drafts
+// outgrow their room ends the step, which is run again with a build and more
+// room (k_fixup).
+__device__ __forceinline__ bool has_records(const DS& S, int i, int j) {
+    const int hc = S.hcnt_old[i], bc = S.bcnt_old[i];
+    if (hc == 0 && bc == 0) return false;
+    return find_partner(S.hist_old, S.S, i, hc, j) >= 0 || find_partner(S.bond_old, S.S, i, bc, j) >= 0;
+}
+// bound of the pair of floe f (storage slot fs, bound nbf) and floe j at q
+__device__ __forceinline__ float sup_bound_of(const DS& S, int f, int fs, float nbf, int j, int q) {
+    const bool keep = j > f ? has_records(S, fs, j) : has_records(S, S.cval[q], f);
+    return keep ? SUP_KEEP : fmaxf(nbf, S.nb[q]);
+}
+
 // Candidate superset of one floe by one thread over its (2 SPAN + 1)^2 cell
 // block: every floe j within (j > f ? r(f) : r(j)) + rtree + skin.  The cells
 // of one row of the block are consecutive in the cell order, so each row is
 // one contiguous range of positions; every cell range is read at once
 // (indices clamped into the grid, cells outside it masked out afterwards) and
-// the rows, taken as one sequence, SCAN_BATCH records at a time.  FILL
-// writes the entries at `out`; either way the count is returned.
+// the rows, taken as one sequence, SCAN_BATCH records at a time.  Returns the
+// counts of all entries and of those that can come within their bound
+// (sup_bound_of); FILL writes the entries at `out`, the latter (`snear`)
+// first.
 template <int SPAN, bool FILL>
-__device__ __forceinline__ int sup_thread(const DS& S, int k, const GeoRec& me, const DevParams& P,
-                                          int64_t* out) {
+__device__ __forceinline__ int2 sup_thread(const DS& S, int k, const GeoRec& me, const DevParams& P,
+                                           int64_t* out, int snear) {
     constexpr int R = 2 * SPAN + 1;
     const int cx = cell_coord(me.x, P.cell, P.gx), cy = cell_coord(me.y, P.cell, P.gy);
     int2 rg[R][R];
@@ -624,7 +660,9 @@ __device__ __forceinline__ int sup_thread(const DS& S, int k, const GeoRec& me, 
     }
     const int f = me.id;
     const double rad = me.r + P.rtree + P.skin, reach = P.rtree + P.skin;
-    int n = 0;
+    const int fs = S.cval[k];
+    const float nbme = S.nb[k];
+    int n = 0, nn = 0;
     for (int v0 = 0; v0 < L; v0 += SCAN_BATCH) {
         GeoRec g[SCAN_BATCH];
         int qq[SCAN_BATCH];
@@ -648,13 +686,18 @@ __device__ __forceinline__ int sup_thread(const DS& S, int k, const GeoRec& me, 
             const double dx = me.x - g[u].x, dy = me.y - g[u].y;
             const double thr = g[u].id > f ? rad : g[u].r + reach;
             // a superset: the margin only adds entries
-            if (dx * dx + dy * dy <= thr * thr * (1.0 + 1e-12)) {
-                if (FILL) out[n] = sup_ent(SUP_KEEP, q);
+            const double d2 = dx * dx + dy * dy;
+            if (d2 <= thr * thr * (1.0 + 1e-12)) {
+                const float bound = sup_bound_of(S, f, fs, nbme, g[u].id, q);
+                const double w = me.r + g[u].r + (double)bound + P.skin;
+                const bool near = d2 <= w * w * (1.0 + 1e-12);
+                if (FILL) out[near ? nn : snear + n - nn] = sup_ent(bound, q);
                 ++n;
+                nn += near ? 1 : 0;
             }
         }
     }
-    return n;
+    return make_int2(n, nn);
 }
 
 // (floe, candidate) pairs of one wavefront in LDS: entry, distance (inner:
@@ -1103,13 +1146,15 @@ __global__ __launch_bounds__(FLOE_BLOCK) void k_sup(DS S) {
             if (P.dense) {
                 qd = !FILL;
             } else if (FILL) {
-                if (P.span == 2) sup_thread<2, true>(S, k, me, P, S.sup + S.soff[k]);
-                else sup_thread<1, true>(S, k, me, P, S.sup + S.soff[k]);
+                int64_t* out = S.sup + S.soff[k];
+                if (P.span == 2) sup_thread<2, true>(S, k, me, P, out, S.snear[k]);
+                else sup_thread<1, true>(S, k, me, P, out, S.snear[k]);
                 S.x0[k] = make_double2(me.x, me.y);
             } else {
-                n = P.span == 2 ? sup_thread<2, false>(S, k, me, P, nullptr)
-                                : sup_thread<1, false>(S, k, me, P, nullptr);
-                S.scnt[k] = S.snear[k] = n;
+                const int2 c = P.span == 2 ? sup_thread<2, false>(S, k, me, P, nullptr, 0)
+                                           : sup_thread<1, false>(S, k, me, P, nullptr, 0);
+                S.scnt[k] = c.x;
+                S.snear[k] = n = c.y;
             }
         }
     }
@@ -1207,31 +1252,6 @@ __global__ __launch_bounds__(FLOE_BLOCK) void k_cand(DS S) {
 // Superset build of the dense members' floes (queue 3), one wavefront per
 // floe over its (2 span + 1)^2 cell block, 64 entries at a time: counts, or
 // the entries and the build positions.  Only on build steps.
-//
-// In these members (power-law radii, say) the query radius r + rtree holds
-// tens of floes, nearly all of them kilometres away: no contact, no bond, and
-// a sheltering term that is exactly 1.  A pair can only matter while its
-// floes are no further apart than the larger of their two bounds nb (the
-// reach of their own sheltering, with room for the drafts to grow, and the
-// distance bonds form at), or if it has a contact history or a bond.  So the
-// entries that can come within their bound before the next build go first
-// (snear of them, each with its bound; SUP_KEEP for pairs with a history or a
-// bond, which k_contact and k_bond set on the entries of new ones), and the
-// step's search reads those alone and lists the pairs within their bound: of
-// 59 entries and 43 candidates a floe (power-law radii on [200, 5000] m at
-// packing 0.7), 9-11 and 2.4-4.2.  (One MI355X, against a search and lists of
-// all candidates: 320,000 floes mixed, search 0.39 -> 0.11 ms, integration
-// 0.088 -> 0.034, bonds 0.034 -> 0.016; 262,144 floes FP64, search 0.38 ->
-// 0.16; 1,000 floes 0.114 -> 0.041.)  The others only answer which pairs were
-// candidates (k_pairs) and how many events a reshape came before (k_repair).
-// A reshape whose drafts outgrow their room ends the step, which is run again
-// with a build and more room (k_fixup).
-__device__ __forceinline__ bool has_records(const DS& S, int i, int j) {
-    const int hc = S.hcnt_old[i], bc = S.bcnt_old[i];
-    if (hc == 0 && bc == 0) return false;
-    return find_partner(S.hist_old, S.S, i, hc, j) >= 0 || find_partner(S.bond_old, S.S, i, bc, j) >= 0;
-}
-
 template <bool FILL>
 __global__ __launch_bounds__(64) void k_sup_dense(DS S) {
     if (!*S.rebuild || *S.err) return;
@@ -1275,8 +1295,7 @@ __global__ __launch_bounds__(64) void k_sup_dense(DS S) {
                     const double thr = o.id > f ? rad : o.r + reach;
                     in = d2 <= thr * thr * (1.0 + 1e-12);
                     if (in) {
-                        bound = fmaxf(nbme, S.nb[q]);
-                        if (o.id > f ? has_records(S, fs, o.id) : has_records(S, S.cval[q], f)) bound = SUP_KEEP;
+                        bound = sup_bound_of(S, f, fs, nbme, o.id, q);
                         const double w = me.r + o.r + (double)bound + P.skin;
                         near = d2 <= w * w * (1.0 + 1e-12);
                     }
@@ -1472,7 +1491,7 @@ __global__ __launch_bounds__(FLOE_BLOCK, 3) void k_contact(DS S) {
                         if (ps.deltat != 0.0 || ps.thetarelc != 0.0 || ps.fcn != 0.0 || ps.fct != 0.0) {
                             r.kind |= 2;
                             r.deltat = ps.deltat; r.thetarelc = ps.thetarelc; r.fcn = ps.fcn; r.fct = ps.fct;
-                            if (!had && P.dense) sup_keep(S, ko, qj);
+                            if (!had) sup_keep(S, ko, qj);
                         }
                         if (o.flags & EV_RIDGED) {
                             const int p = atomicAdd(&S.nseeds[om], 1);
@@ -1570,7 +1589,7 @@ __device__ __forceinline__ bool bond_event(const DS& S, const DevParams& P, int 
     if (rq < 0) {
         if (nb < S.BC) rq = nb++;
         else { over |= ERR_BOND_CAP; return false; }
-        if (P.dense) sup_keep(S, k, qj);
+        sup_keep(S, k, qj);
     }
     S.bond_new[(int64_t)rq * SS + fs] = bond_from(ps, j);
     if (!(o.flags & EV_BONDED)) return false;
@@ -2477,7 +2496,7 @@ __global__ __launch_bounds__(FLOE_BLOCK, 2) void k_fixup(DS S) {
                             const int p = atomicAdd(&S.bcnt_new[ofs], 1);
                             if (p < S.BC) S.bond_new[(int64_t)p * SS + ofs] = bond_from(ps, pid);
                             else over |= ERR_BOND_CAP;
-                            if (P.dense) sup_keep(S, ko, qp);
+                            sup_keep(S, ko, qp);
                         }
                         const bool hist = ps.deltat != 0.0 || ps.thetarelc != 0.0 || ps.fcn != 0.0 || ps.fct != 0.0;
                         HistRec hr;
@@ -2488,7 +2507,7 @@ __global__ __launch_bounds__(FLOE_BLOCK, 2) void k_fixup(DS S) {
                         } else if (hist) {
                             o.nr = hr.deltat; o.nh = hr.thetarelc; o.nmass = hr.fcn; o.ninertia = hr.fct;
                             o.ridged = pid;
-                            if (P.dense) sup_keep(S, ko, qp);
+                            sup_keep(S, ko, qp);
                             o.flags |= EV_PUT_HIST;
                         }
                     }
@@ -2653,7 +2672,8 @@ __global__ __launch_bounds__(FLOE_BLOCK, (MIXED && !REC) ? 5 : 4) void k_final(D
     if (k == 0) *S.steps_done += 1;
     const int m = me.member;
     if (m < 0) {
-        S.geo_new[k] = me;
+        // (only the member is read of such a row)
+        S.geo_new[k].member = m;
         return;
     }
     const DevParams& P = S.params[m];

@@ -30,8 +30,7 @@ struct DevParams {
     uint32_t bond_thr24;
     uint64_t bond_seed;
     int32_t wind_grid;     // -1: uniform ua/va, else index into the wind-grid table
-    int32_t dense;         // 1: many floes per cell; the supersets put the pairs that can
-                           // matter first (k_sup_dense)
+    int32_t dense;         // 1: many floes per cell; a wavefront builds each superset
     int32_t span;          // cells searched on each side (cell >= (max r + rtree + skin) / span)
     int32_t pad2_;
     double skin;           // candidate supersets reach this far beyond the query radius
