@@ -15,9 +15,10 @@
 #include <vector>
 
 namespace godar {
-__global__ void k_begin(DS, int, int);
+__global__ void k_begin(DS, int);
 __global__ void k_ranges(DS);
-template <bool M> __global__ void k_cand(DS);
+template <bool M> __global__ void k_cand(DS, int, int);
+template <bool M> __global__ void k_events(DS, int, int, int);
 template <bool F> __global__ void k_sup(DS);
 template <bool F> __global__ void k_sup_dense(DS);
 __global__ void k_scan_tiles(DS);
@@ -94,12 +95,6 @@ struct Range { int64_t first, n; };
 
 struct godar_ctx {
     hipStream_t stream = nullptr;
-    // The contact and wall kernels run beside the bond kernel, on a side
-    // stream forked from and joined back to `stream` by events (a captured
-    // step graph takes the same branches); steps timed stage by stage run
-    // them one after another.
-    hipStream_t side = nullptr;
-    hipEvent_t efork = nullptr, ejoin = nullptr;
     int precision = GODAR_FP64;
     int64_t S = 0;
     int Mcap = 0;
@@ -121,8 +116,9 @@ struct godar_ctx {
     int64_t wpool_dev_cap = 0;
     int wgrids_dev_cap = 0;
     DS d{};
-    // double-buffered positions and pair state
+    // double-buffered positions, queue counters and pair state
     GeoRec* geo[2] = {nullptr, nullptr};
+    int32_t* qn[2] = {nullptr, nullptr};
     HistRec* hist[2] = {nullptr, nullptr};
     int32_t* hcnt[2] = {nullptr, nullptr};
     BondRec* bond[2] = {nullptr, nullptr};
@@ -280,6 +276,7 @@ void set_lists(godar_ctx* c, const PairLists& L) {
 void bind_parity(godar_ctx* c) {
     int o = c->parity, n = 1 - c->parity;
     c->d.geo = c->geo[o]; c->d.geo_new = c->geo[n];
+    c->d.qn = c->qn[o]; c->d.qn_next = c->qn[n];
     c->d.hist_old = c->hist[o]; c->d.hist_new = c->hist[n];
     c->d.hcnt_old = c->hcnt[o]; c->d.hcnt_new = c->hcnt[n];
     c->d.bond_old = c->bond[o]; c->d.bond_new = c->bond[n];
@@ -482,13 +479,10 @@ int launch_step(godar_ctx* c, bool lean) {
     // Steps that start with d.rebuild set bin, sort and search the cells and
     // build the candidate supersets; the other steps' build kernels return at
     // once (the launch sequence, and a captured graph, is the same).
-    {
+    if (!lean) {
         StageTimer t(c, 0);
-        // (a lean step only resets the queue counters and the members' words)
-        const int nt = lean ? std::max(c->Mcap, NQUEUE * XCD_COUNT)
-                            : std::max({N, c->ncells_cap + 1, NQUEUE * XCD_COUNT, c->Mcap});
-        hipLaunchKernelGGL(k_begin, grid_for(nt, B[0], false), dim3(B[0]), 0, s, d, lean ? 1 : 0,
-                           (int)c->Mcap);
+        const int nt = std::max({N, c->ncells_cap + 1, NQUEUE * XCD_COUNT});
+        hipLaunchKernelGGL(k_begin, grid_for(nt, B[0], false), dim3(B[0]), 0, s, d, (int)c->Mcap);
     }
     int bits = 1;
     while ((1u << bits) <= (uint32_t)c->ncells_cap && bits < 32) ++bits;
@@ -521,38 +515,34 @@ int launch_step(godar_ctx* c, bool lean) {
         StageTimer t(c, 3);
         // LDS: one list of (floe, candidate) pairs per wavefront
         hipLaunchKernelGGL(mixed ? k_cand<true> : k_cand<false>, grid_for(N, B[3], true),
-                           dim3(B[3]), (B[3] / 64) * CAND_LDS_PER_WAVE, s, d);
+                           dim3(B[3]), (B[3] / 64) * CAND_LDS_PER_WAVE, s, d, lean ? 1 : 0, nm);
     }
-    // contacts, bonds and walls touch disjoint state (the flag words both
-    // the contact and the bond kernel set are set with atomicOr), so they may
-    // run together: contacts and walls on the side stream, bonds (the
-    // longest) on the step's stream, whose next kernel waits for the side
-    // stream once
-    const bool fork = !c->prof;
-    hipStream_t sc = fork ? c->side : s;
-    if (fork) {
-        (void)hipEventRecord(c->efork, s);
-        (void)hipStreamWaitEvent(sc, c->efork, 0);
-    }
-    {
-        StageTimer t(c, 4);
-        // LDS: one pass of 64 pair results per wavefront
-        hipLaunchKernelGGL(mixed ? k_contact<true> : k_contact<false>, grid_queue(N, B[4]),
-                           dim3(B[4]), (B[4] / 64) * CONTACT_LDS_PER_WAVE, sc, d);
-    }
-    {
-        StageTimer t(c, 7);
-        hipLaunchKernelGGL(mixed ? k_walls<true> : k_walls<false>, grid_queue(N, B[7]),
-                           dim3(B[7]), 0, sc, d);
-    }
-    {
-        StageTimer t(c, 5);
-        hipLaunchKernelGGL(mixed ? k_bond<true> : k_bond<false>, grid_queue(N, B[5]),
-                           dim3(B[5]), 0, s, d);
-    }
-    if (fork) {
-        (void)hipEventRecord(c->ejoin, sc);
-        (void)hipStreamWaitEvent(s, c->ejoin, 0);
+    if (!c->prof) {
+        // contacts, bonds and walls in one launch, as many single-wavefront
+        // blocks of each per XCD as the floes could fill, capped
+        const int per = (N + XCD_COUNT * 64 - 1) / (XCD_COUNT * 64);
+        const int nb = std::min(per, QUEUE_GRID_WAVES / XCD_COUNT);
+        const int nc = std::min(4 * per, QUEUE_GRID_WAVES / XCD_COUNT);   // (queue_share: fewer floes each)
+        const int nw = std::min(per, WALL_GRID_WAVES / XCD_COUNT);
+        hipLaunchKernelGGL(mixed ? k_events<true> : k_events<false>, dim3(XCD_COUNT * (nw + nc + nb)),
+                           dim3(64), CONTACT_LDS_PER_WAVE, s, d, nw, nc, nb);
+    } else {
+        {
+            StageTimer t(c, 4);
+            // LDS: one pass of 64 pair results per wavefront
+            hipLaunchKernelGGL(mixed ? k_contact<true> : k_contact<false>, grid_queue(N, B[4]),
+                               dim3(B[4]), (B[4] / 64) * CONTACT_LDS_PER_WAVE, s, d);
+        }
+        {
+            StageTimer t(c, 7);
+            hipLaunchKernelGGL(mixed ? k_walls<true> : k_walls<false>, grid_queue(N, B[7]),
+                               dim3(B[7]), 0, s, d);
+        }
+        {
+            StageTimer t(c, 5);
+            hipLaunchKernelGGL(mixed ? k_bond<true> : k_bond<false>, grid_queue(N, B[5]),
+                               dim3(B[5]), 0, s, d);
+        }
     }
     {
         StageTimer t(c, 8);
@@ -688,8 +678,8 @@ int godar_create(int64_t max_floes, int32_t max_members, int32_t precision, goda
     *out = nullptr;
     godar_ctx* c = new godar_ctx();
     c->precision = precision;
-    // default block sizes: 256 threads, except the bond and wall stages,
-    // which run beside the contact stage (64), and the integration (128);
+    // default block sizes: 256 threads, except the bond and wall stages (64)
+    // and the integration (128);
     // measured on the 512-field ensemble and the served mix
     for (int k = 0; k < GODAR_NSTAGES; ++k) c->sblock[k] = FLOE_BLOCK;
     c->sblock[5] = c->sblock[7] = 64;
@@ -705,9 +695,6 @@ int godar_create(int64_t max_floes, int32_t max_members, int32_t precision, goda
     DS& d = c->d;
     int64_t S = c->S;
     hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
-    if (e == hipSuccess) e = hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking);
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&c->ejoin, hipEventDisableTiming);
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&c->efork, hipEventDisableTiming);
 #define ACHK(x)                                        \
     do {                                               \
         e = (x);                                       \
@@ -757,7 +744,7 @@ int godar_create(int64_t max_floes, int32_t max_members, int32_t precision, goda
     ACHK(dalloc(&d.cls, S));
     ACHK(dalloc(&d.qlist, (int64_t)NQUEUE * S));
     ACHK(dalloc(&d.bgat, S));
-    ACHK(dalloc(&d.qn, (int64_t)NQUEUE * XCD_COUNT * QN_STRIDE));
+    for (int k = 0; k < 2; ++k) ACHK(dalloc(&c->qn[k], (int64_t)NQUEUE * XCD_COUNT * QN_STRIDE));
     ACHK(dalloc(&d.shape, (int64_t)c->SEEDK * S));
     ACHK(dalloc(&d.rhead, S));
     ACHK(dalloc(&d.nseeds, max_members));
@@ -789,7 +776,8 @@ int godar_create(int64_t max_floes, int32_t max_members, int32_t precision, goda
     (void)hipMemsetAsync(d.nbmin, 0, sizeof(float) * S, c->stream);
     for (int k = 0; k < 2; ++k)       // (member -1: no floe yet)
         (void)hipMemsetAsync(c->geo[k], 0xFF, sizeof(GeoRec) * S, c->stream);
-    (void)hipMemsetAsync(d.qn, 0, sizeof(int32_t) * NQUEUE * XCD_COUNT * QN_STRIDE, c->stream);
+    for (int k = 0; k < 2; ++k)
+        (void)hipMemsetAsync(c->qn[k], 0, sizeof(int32_t) * NQUEUE * XCD_COUNT * QN_STRIDE, c->stream);
     hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, c->stream, d.rebuild, 2, 1);
     hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, c->stream, d.rebuild + 2, 1, 0);
     (void)hipMemsetAsync(d.dirty, 0, (S + 3) / 4 * 4, c->stream);
@@ -830,16 +818,13 @@ int godar_destroy(godar_ctx* c) {
         free_lists(L);
         set_lists(c, L);
     }
-    dfree(d.wout); dfree(d.wflag); dfree(d.cls); dfree(d.qlist); dfree(d.qn); dfree(d.bgat); dfree(d.shape); dfree(d.rhead); dfree(d.nseeds); dfree(d.heap);
+    dfree(d.wout); dfree(d.wflag); dfree(d.cls); dfree(d.qlist); dfree(c->qn[0]); dfree(c->qn[1]); dfree(d.bgat); dfree(d.shape); dfree(d.rhead); dfree(d.nseeds); dfree(d.heap);
     dfree(d.dirty);
     dfree(d.wnz); dfree(d.stats); dfree(d.tcur); dfree(d.err); dfree(d.steps_done);
     dfree(d.sup); dfree(d.scnt); dfree(d.snear); dfree(d.nb); dfree(d.nbmin); dfree(d.nearsum); dfree(d.soff); dfree(d.sblk); dfree(d.x0); dfree(d.rebuild);
     radix_free(c->rs);
     collect_events(c);
     for (hipEvent_t e : c->ev_pool) (void)hipEventDestroy(e);
-    if (c->ejoin) (void)hipEventDestroy(c->ejoin);
-    if (c->side) (void)hipStreamDestroy(c->side);
-    if (c->efork) (void)hipEventDestroy(c->efork);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
     return GODAR_OK;
@@ -1682,12 +1667,8 @@ int godar_autotune(godar_ctx* c, int32_t trial) {
     if (rc != GODAR_OK) return rc;
     for (int st = 0; st < GODAR_NSTAGES; ++st) {
         if (!tunable_stage(st)) continue;
-        // The bond and wall kernels run beside the contact kernel (the
-        // contacts and walls on a side stream), where single-wavefront blocks
-        // fit in the room the others leave;
-        // timed one kernel after another, as here, larger blocks look as
-        // fast, but overlapped 256-thread bond blocks cost about 3 % of a
-        // step at the mid-run of the 512-field ensemble.
+        // (outside steps timed stage by stage, contacts, bonds and walls are
+        // one launch of single-wavefront blocks, whatever their sizes here)
         if (st == 5 || st == 7) {
             c->sblock[st] = 64;
             continue;
@@ -1826,6 +1807,7 @@ int godar_sync(godar_ctx* c) {
         HIPCHK(c, hipMemsetAsync(c->d.err, 0, sizeof(uint32_t), c->stream));
         HIPCHK(c, hipStreamSynchronize(c->stream));
         c->last_err_bits = e;
+        c->need_full = true;   // (the queue counters of the failed step are k_begin's to clear)
         return fail(c, GODAR_ERR_CAPACITY, "step aborted:" + err_text(e));
     }
     return GODAR_OK;
@@ -2104,7 +2086,7 @@ int godar_get_totals(godar_ctx* c, int64_t* out) {
     if (e == hipSuccess) e = hipMemcpy(out + 6, dout + 3, 2 * sizeof(int64_t), hipMemcpyDeviceToHost);
     std::vector<int32_t> q((size_t)NQUEUE * XCD_COUNT * QN_STRIDE, 0);
     if (e == hipSuccess)
-        e = hipMemcpy(q.data(), c->d.qn, q.size() * sizeof(int32_t), hipMemcpyDeviceToHost);
+        e = hipMemcpy(q.data(), c->d.qn_next, q.size() * sizeof(int32_t), hipMemcpyDeviceToHost);
     for (int k = 0; k < 3; ++k) {
         out[3 + k] = 0;
         for (int x = 0; x < XCD_COUNT; ++x) out[3 + k] += q[(size_t)(k * XCD_COUNT + x) * QN_STRIDE];
@@ -2132,7 +2114,7 @@ int godar_get_totals_noalloc(godar_ctx* c, int64_t* out) {
     hipLaunchKernelGGL(k_zero_i64, dim3(1), dim3(64), 0, c->stream, w, GODAR_NTOTALS);
     if (c->N_used > 0)
         hipLaunchKernelGGL(k_totals, dim3((c->N_used + 255) / 256), dim3(256), 0, c->stream, c->d, w);
-    hipLaunchKernelGGL(k_queue_totals, dim3(1), dim3(64), 0, c->stream, c->d.qn, w + 3);
+    hipLaunchKernelGGL(k_queue_totals, dim3(1), dim3(64), 0, c->stream, c->d.qn_next, w + 3);
     hipLaunchKernelGGL(k_member_totals, dim3(1), dim3(256), 0, c->stream, c->d, c->Mcap, w + 6);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipMemcpyAsync(out, w, GODAR_NTOTALS * sizeof(int64_t), hipMemcpyDeviceToHost, c->stream));

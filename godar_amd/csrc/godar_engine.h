@@ -24,6 +24,7 @@ constexpr int NQUEUE = 5;         // work queues: contact, bond, wall, dense sea
 constexpr int QN_STRIDE = 64;     // ints between queue counters (256 B)
 constexpr int SCAN_TILE = 1024;   // positions per tile of the superset offset scan
 constexpr int QUEUE_GRID_WAVES = 4096;   // wavefronts launched for a queue kernel at most
+constexpr int WALL_GRID_WAVES = 256;     // wavefronts of the walls beside contacts and bonds at most
 constexpr int FIXUP_GRID_WAVES = 2048;   // wavefronts of the fix-up (about one resident round)
 
 // Per-floe record (96 bytes) by storage slot.  Between builds of the cell
@@ -147,6 +148,7 @@ struct DS {
     // QN_STRIDE ints), so that the counters' atomics spread over many lines.
     int32_t* qlist;            // [NQUEUE][S]
     int32_t* qn;               // [NQUEUE][XCD_COUNT] x QN_STRIDE
+    int32_t* qn_next;          // the next step's (the two change places every step)
     // ordered repair: reshape records, SEEDK per floe slot (a member's from
     // SEEDK*first on), the seeds first; rhead is each floe's list of them
     Reshape* shape;

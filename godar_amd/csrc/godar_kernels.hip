@@ -1,8 +1,8 @@
 // Kernels of the GODAR step pipeline (one launch sequence per step):
 //
-//   k_begin -> [build steps: radix sort -> k_ranges -> k_sup ...] -> k_cand
-//    -> (k_contact -> k_walls on a side stream) beside k_bond
-//    -> k_repair -> k_fixup -> k_final (which also gathers the bond terms)
+//   [steps with the build kernels: k_begin -> radix sort -> k_ranges -> k_sup ...]
+//    -> k_cand -> k_events (contacts, bonds, walls) -> k_repair -> k_fixup
+//    -> k_final (which also gathers the bond terms)
 //
 // Sequential semantics of the reference (stepper.f90:71-280 visits floes i
 // in index order and, for each, its candidates j > i in ascending distance;
@@ -10,10 +10,9 @@
 // thickness) are reproduced as follows:
 //   * The event kernels evaluate every pair event with the start-of-step
 //     floe properties.  Contact, bond and sheltering terms feed disjoint
-//     accumulators, so each kind has a kernel of its own: the candidate
+//     accumulators, so each kind has code of its own: the candidate
 //     search k_cand also computes every floe's sheltering minima and queues
-//     the floes that have contact, bond or wall work for k_contact, k_bond
-//     and k_walls.  One thread per
+//     the floes that have contact, bond or wall work.  One thread per
 //     floe gathers its own contributions in the reference's per-floe order:
 //     first the pairs where it is the inner index (ascending outer index),
 //     then its own candidates in distance order.  Contact and sheltering
@@ -61,16 +60,17 @@ __device__ __forceinline__ int xcd_block() {
     return (int)(blockIdx.x % XCD_COUNT) * per + (int)(blockIdx.x / XCD_COUNT);
 }
 
-// Entry of a work queue of length qn for this thread, or -1.  Each XCD takes
-// one contiguous share of the queue (the grid, sized for all floes, always
-// has enough threads per XCD), so that short queues still spread over all
+// The blocks a queue's kernel runs: this block's XCD, its index among the
+// XCD's blocks of the same work and their number.  Each XCD takes one
+// contiguous share of the queue, so that short queues still spread over all
 // XCDs and each XCD's share sits together in its L2.
-__device__ __forceinline__ int queue_slot(int qn) {
-    const int per = (qn + XCD_COUNT - 1) / XCD_COUNT;
-    const int local = (int)(blockIdx.x / XCD_COUNT) * (int)blockDim.x + (int)threadIdx.x;
-    if (local >= per) return -1;
-    const int t = (int)(blockIdx.x % XCD_COUNT) * per + local;
-    return t < qn ? t : -1;
+struct QueueBlocks { int xcd, block, blocks; };
+__device__ __forceinline__ QueueBlocks queue_blocks() {
+    QueueBlocks b;
+    b.xcd = (int)(blockIdx.x % XCD_COUNT);
+    b.block = (int)(blockIdx.x / XCD_COUNT);
+    b.blocks = (int)(gridDim.x / XCD_COUNT);
+    return b;
 }
 
 __device__ __forceinline__ int32_t* qcount(const DS& S, int c, int x) {
@@ -103,16 +103,15 @@ __device__ __forceinline__ int queue_at(const DS& S, int c, const QueueView& v, 
     }
     return S.qlist[(int64_t)c * S.S + idx];
 }
-// Slot of this thread's it-th entry of a queue of length qn, or -1: the
-// grid may be smaller than the queue (the host caps the queue kernels' grids
-// at QUEUE_GRID_WAVES wavefronts), so each thread takes every
-// (threads per XCD)-th entry of its XCD's share.
-__device__ __forceinline__ int queue_slot_it(int qn, int it) {
+// Slot of this thread's it-th entry of a queue of length qn, or -1: there may
+// be fewer blocks than the queue fills (the host caps them at
+// QUEUE_GRID_WAVES wavefronts), so each thread takes every (threads per
+// XCD)-th entry of its XCD's share.
+__device__ __forceinline__ int queue_slot_it(const QueueBlocks& b, int qn, int it) {
     const int per = (qn + XCD_COUNT - 1) / XCD_COUNT;
-    const int local = ((int)(blockIdx.x / XCD_COUNT) + it * (int)(gridDim.x / XCD_COUNT)) * (int)blockDim.x +
-                      (int)threadIdx.x;
+    const int local = (b.block + it * b.blocks) * (int)blockDim.x + (int)threadIdx.x;
     if (local >= per) return -1;
-    const int t = (int)(blockIdx.x % XCD_COUNT) * per + local;
+    const int t = b.xcd * per + local;
     return t < qn ? t : -1;
 }
 // Entries of a queue of length qn taken by this wavefront when a wavefront
@@ -130,12 +129,12 @@ __device__ __forceinline__ int queue_slot_it(int qn, int it) {
 // are busy then, and full passes count for more (the 512-field ensemble's
 // 157,000 queued floes lost 0.03 ms per step with 39).
 struct QueueShare { int begin, end, stride, floes; };
-__device__ __forceinline__ QueueShare queue_share(const DS& S, int qn) {
+__device__ __forceinline__ QueueShare queue_share(const DS& S, const QueueBlocks& b, int qn) {
     const int per = (qn + XCD_COUNT - 1) / XCD_COUNT;
     const int wpb = (int)(blockDim.x >> 6);
-    const int nw = (int)(gridDim.x / XCD_COUNT) * wpb;
-    const int w = (int)(blockIdx.x / XCD_COUNT) * wpb + (int)(threadIdx.x >> 6);
-    const int lo = (int)(blockIdx.x % XCD_COUNT) * per;
+    const int nw = b.blocks * wpb;
+    const int w = b.block * wpb + (int)(threadIdx.x >> 6);
+    const int lo = b.xcd * per;
     QueueShare q;
     const int f = (per + nw - 1) / nw;
     const int64_t entries = *S.nearsum;     // entries the search reads
@@ -146,12 +145,6 @@ __device__ __forceinline__ QueueShare queue_share(const DS& S, int qn) {
     q.end = min(qn, lo + per);
     q.stride = nw * q.floes;
     return q;
-}
-// the queue entry of this thread (split over the XCDs as queue_slot), or -1
-__device__ __forceinline__ int queue_entry(const DS& S, int c) {
-    const QueueView v = queue_view(S, c);
-    const int t = queue_slot(v.total);
-    return t < 0 ? -1 : queue_at(S, c, v, t);
 }
 // appends position k to queue c from a single lane
 __device__ __forceinline__ void enqueue_one(const DS& S, int c, int k) {
@@ -404,14 +397,22 @@ __global__ void k_spill(DS S, int host) {
     S.rec[f] = r;
 }
 
-// First kernel of every step, over max(N, cells) threads.  A step launched
-// without the build kernels (lean) that finds a build or a refresh due sets
-// ERR_NEED_BUILD and does nothing else (every later kernel of the step then
-// returns at once and the host runs the step again with them); with the
-// build kernels, BUILD_SOON alone is enough to build.  Then:
-//  * the queue counters (the dense-search list, queue 3, only on build steps:
-//    it lists positions, which change only then) and, on build steps, the
-//    cell ranges;
+// The per-member resets of a step (thread i of `threads` takes members i,
+// i + threads, ...).
+__device__ __forceinline__ void member_resets(const DS& S, int i, int threads, int nmembers) {
+    for (; i < nmembers; i += threads) {
+        if (!member_live(S.members[i])) continue;
+        S.nseeds[i] = 0;
+        S.stats[4 * i + 2] = 0; S.stats[4 * i + 3] = 0;
+        S.tcur[i] = S.members[i].tstep;
+    }
+}
+
+// First kernel of a step with the build kernels, over max(N, cells) threads
+// (a step without them, lean, starts with k_cand).  BUILD_SOON alone is
+// enough to build.
+//  * the queue counters (k_final clears the next step's, which a failed step
+//    leaves as they are) and, on build steps, the cell ranges;
 //  * thread i as position: rec from the ordered copies where they are newer,
 //    on build and refresh steps (k_spill's work; k_ranges clears the flag);
 //  * thread i as storage slot: the per-member resets of the step and, on
@@ -419,26 +420,16 @@ __global__ void k_spill(DS S, int host) {
 //    input buffers (bkey, bval).  The position is read from the ordered copy
 //    where that is newer than rec (it is the same value the spill writes),
 //    so the spill and the keys need no order between them.
-__global__ void k_begin(DS S, int lean, int nmembers) {
+__global__ void k_begin(DS S, int nmembers) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (*S.err) return;
-    if (lean && ((S.rebuild[0] & BUILD_DUE) || S.rebuild[1])) {
-        if (i == 0) atomicOr(S.err, ERR_NEED_BUILD);
-        return;
-    }
-    const bool build = !lean && S.rebuild[0] != 0, refresh = !lean && S.rebuild[1] != 0;
+    const bool build = S.rebuild[0] != 0, refresh = S.rebuild[1] != 0;
     const bool newer = S.rebuild[2] != 0;
-    // (the dense-search queue stands between builds)
-    if (i < NQUEUE * XCD_COUNT && (build || i / XCD_COUNT != 3)) S.qn[i * QN_STRIDE] = 0;
+    if (i < NQUEUE * XCD_COUNT) S.qn[i * QN_STRIDE] = 0;
     if (build && i <= S.ncells) S.crange[i] = make_int2(0, 0);
     if (build && i == 0) *S.nearsum = 0;
-    // per-member resets (thread m for member m)
-    if (i < nmembers && member_live(S.members[i])) {
-        S.nseeds[i] = 0;
-        S.stats[4 * i + 2] = 0; S.stats[4 * i + 3] = 0;
-        S.tcur[i] = S.members[i].tstep;
-    }
-    if (lean || i >= S.N) return;   // (a lean step's grid covers the counters and members only)
+    member_resets(S, i, (int)(gridDim.x * blockDim.x), nmembers);
+    if (i >= S.N) return;
     if (newer && (build || refresh)) {
         const GeoRec g = S.geo[i];
         const uint32_t fs = S.cval[i];
@@ -1220,8 +1211,12 @@ __global__ __launch_bounds__(SCAN_TILE) void k_scan_offsets(DS S) {
     if (k < S.N) S.soff[k] = S.sblk[blockIdx.x] + ex;
 }
 
+// (lean: the step has no build kernels.  It then starts here, with the
+// per-member resets; if a build or a refresh is due it sets ERR_NEED_BUILD and
+// does nothing else: every later kernel of the step returns at once and the
+// host runs the step again with them.)
 template <bool MIXED>
-__global__ __launch_bounds__(FLOE_BLOCK) void k_cand(DS S) {
+__global__ __launch_bounds__(FLOE_BLOCK) void k_cand(DS S, int lean, int nmembers) {
     const int k = xcd_block() * blockDim.x + threadIdx.x;
     bool qc = false, qb = false, qw = false;
     // every row the search starts from is requested before anything is
@@ -1235,7 +1230,13 @@ __global__ __launch_bounds__(FLOE_BLOCK) void k_cand(DS S) {
     }
     const bool slot_used = inr && me.member >= 0;
     const int m = slot_used ? me.member : 0;
-    const bool ok = !*S.err;
+    // (the build flags stand while this kernel runs)
+    const bool due = lean && ((S.rebuild[0] & BUILD_DUE) | S.rebuild[1]) != 0;
+    const bool ok = !*S.err && !due;
+    if (lean && blockIdx.x == 0) {
+        if (due && threadIdx.x == 0) atomicOr(S.err, ERR_NEED_BUILD);
+        if (ok) member_resets(S, (int)threadIdx.x, (int)blockDim.x, nmembers);
+    }
     extern __shared__ unsigned char cand_lds[];
     const bool act = slot_used & ok;
     cand_thread<MIXED>(S, k, me, pre, m, act, qc, qb, qw,
@@ -1366,19 +1367,13 @@ struct ContactOut {
 };
 constexpr int CONTACT_LDS_PER_WAVE = 64 * (int)sizeof(ContactOut);
 
-// (the mixed-precision instance gets 163 VGPRs from the looser bound, still
-// 3 wavefronts per SIMD: 0.0955 -> 0.0915 ms beside the bond kernel; FP64
-// would drop to 2 and keeps the bound of 3)
 template <bool MIXED>
-__global__ __launch_bounds__(FLOE_BLOCK, 3) void k_contact(DS S) {
-    extern __shared__ unsigned char contact_lds[];
-    ContactOut* co = reinterpret_cast<ContactOut*>(contact_lds + (threadIdx.x >> 6) * CONTACT_LDS_PER_WAVE);
-    if (*S.err) return;
+__device__ __forceinline__ void contacts(const DS& S, const QueueBlocks& qb, ContactOut* co) {
     const int lane = (int)(threadIdx.x & 63);
     const QueueView qv = queue_view(S, 0);
     // (the wavefront's lanes share LDS and shuffles: every lane runs each
     // round, whether or not it has an entry)
-    const QueueShare qs = queue_share(S, qv.total);
+    const QueueShare qs = queue_share(S, qb, qv.total);
     for (int t0 = qs.begin; t0 < qs.end; t0 += qs.stride) {
         const int qt = t0 + lane;
         const int k = lane < qs.floes && qt < qs.end ? queue_at(S, 0, qv, qt) : -1;
@@ -1639,23 +1634,18 @@ constexpr int BOND_TCAP = 256;
 // records are listed in LDS and evaluated one per lane, so that an owner with
 // several bonds does not hold its lane through all of them; owners whose
 // bonds form this step (step 1) append new records in candidate order and
-// walk their own lists.  (3 wavefronts per SIMD, without spills: at 4 the
-// kernel spilled 40 bytes, and the step, where it shares the GPU with the
-// contact and wall kernels, ran 1.3 % slower.)
+// walk their own lists.
 template <bool MIXED>
-__global__ __launch_bounds__(FLOE_BLOCK, 3) void k_bond(DS S) {
-    __shared__ uint32_t recs[FLOE_BLOCK / 64][BOND_TCAP];
-    if (*S.err) return;
+__device__ __forceinline__ void bonds(const DS& S, const QueueBlocks& qb, uint32_t* rl) {
     const QueueView qv = queue_view(S, 1);
     // (the wavefront loops while any lane has an entry: its lanes share LDS
     // and shuffles)
     for (int it = 0;; ++it) {
-        const int qt = queue_slot_it(qv.total, it);
+        const int qt = queue_slot_it(qb, qv.total, it);
         if (__ballot(qt >= 0) == 0) break;
         const int k = qt >= 0 ? queue_at(S, 1, qv, qt) : -1;
         const bool act = k >= 0;
         const int lane = (int)(threadIdx.x & 63);
-        uint32_t* rl = recs[threadIdx.x >> 6];
         const int64_t SS = S.S;
         int m = 0, fs = 0, no = 0, bco = 0, fid = 0, tstep = 0, first = 0;
         bool bond_step = false;
@@ -1817,14 +1807,13 @@ __device__ __forceinline__ void gather_bonds(const DS& S, int k, int ni, int no,
 
 // Walls of the queued floes (verify_bc, boundaries.f90:1-97).
 template <bool MIXED>
-__global__ __launch_bounds__(FLOE_BLOCK) void k_walls(DS S) {
-    if (*S.err) return;
+__device__ __forceinline__ void wall_contacts(const DS& S, const QueueBlocks& qb) {
     // no later kernel of the step reads the build flag; k_final raises it
     // again when a floe has moved too far for the supersets
-    if (blockIdx.x == 0 && threadIdx.x == 0) { S.rebuild[0] = 0; S.rebuild[1] = 0; }
+    if (qb.xcd == 0 && qb.block == 0 && threadIdx.x == 0) { S.rebuild[0] = 0; S.rebuild[1] = 0; }
     const QueueView qv = queue_view(S, 2);
     for (int it = 0;; ++it) {
-        const int t = queue_slot_it(qv.total, it);
+        const int t = queue_slot_it(qb, qv.total, it);
         if (t < 0) break;
         const int k = queue_at(S, 2, qv, t);
         const GeoRec me = S.geo[k];
@@ -1850,6 +1839,61 @@ __global__ __launch_bounds__(FLOE_BLOCK) void k_walls(DS S) {
                 set_err(S, ERR_SEED_CAP);
         }
     }
+}
+
+// The three kinds of events of a step: they touch disjoint state (the flag
+// words that both contacts and bonds set are set with atomicOr), so they run
+// in one launch, single-wavefront blocks of contacts and bonds alternating so
+// that both are under way from the start, the few of the walls first.  (One
+// launch instead of three on two streams takes the fork, the join and two
+// kernel starts out of the step: with the steps' k_begin gone as well, 94 ->
+// 76 us a step at 1,000 floes in mixed precision and 145 -> 126 us at 24
+// members of 2,700; at 512 members, where each kind fills the chip by itself,
+// it is the same to 1%.)  Steps timed stage by stage run
+// them one after another, in the kernels below.
+template <bool MIXED>
+__global__ __launch_bounds__(64, 3) void k_events(DS S, int nwall, int ncontact, int nbond) {
+    extern __shared__ __align__(16) unsigned char ev_lds[];
+    if (*S.err) return;
+    QueueBlocks qb;
+    qb.xcd = (int)(blockIdx.x % XCD_COUNT);
+    int b = (int)(blockIdx.x / XCD_COUNT);
+    if (b < nwall) {
+        qb.block = b;
+        qb.blocks = nwall;
+        wall_contacts<MIXED>(S, qb);
+        return;
+    }
+    b -= nwall;
+    const int both = 2 * min(ncontact, nbond);
+    const bool contact = b < both ? (b & 1) == 0 : ncontact > nbond;
+    qb.block = b < both ? b >> 1 : b - both / 2;
+    if (contact) {
+        qb.blocks = ncontact;
+        contacts<MIXED>(S, qb, reinterpret_cast<ContactOut*>(ev_lds));
+    } else {
+        qb.blocks = nbond;
+        bonds<MIXED>(S, qb, reinterpret_cast<uint32_t*>(ev_lds));
+    }
+}
+static_assert(BOND_TCAP * 4 <= CONTACT_LDS_PER_WAVE, "k_events' LDS holds either list");
+
+template <bool MIXED>
+__global__ __launch_bounds__(FLOE_BLOCK, 3) void k_contact(DS S) {
+    extern __shared__ unsigned char contact_lds[];
+    if (*S.err) return;
+    contacts<MIXED>(S, queue_blocks(), reinterpret_cast<ContactOut*>(contact_lds + (threadIdx.x >> 6) * CONTACT_LDS_PER_WAVE));
+}
+template <bool MIXED>
+__global__ __launch_bounds__(FLOE_BLOCK, 3) void k_bond(DS S) {
+    __shared__ uint32_t recs[FLOE_BLOCK / 64][BOND_TCAP];
+    if (*S.err) return;
+    bonds<MIXED>(S, queue_blocks(), recs[threadIdx.x >> 6]);
+}
+template <bool MIXED>
+__global__ __launch_bounds__(FLOE_BLOCK) void k_walls(DS S) {
+    if (*S.err) return;
+    wall_contacts<MIXED>(S, queue_blocks());
 }
 
 // ---------------------------------------------------------------------
@@ -2660,6 +2704,8 @@ __global__ __launch_bounds__(FLOE_BLOCK) void k_stress(DS S) {
 template <bool MIXED, bool REC>
 __global__ __launch_bounds__(FLOE_BLOCK, (MIXED && !REC) ? 5 : 4) void k_final(DS S) {
     int k = blockIdx.x * blockDim.x + threadIdx.x;
+    // the next step's queue counters
+    if (k < NQUEUE * XCD_COUNT && !*S.err) S.qn_next[k * QN_STRIDE] = 0;
     if (k >= S.N) return;
     // the position's rows are requested at once, before anything is tested
     const GeoRec me = S.geo[k];
@@ -2883,8 +2929,10 @@ template __global__ void k_sup<false>(DS);
 template __global__ void k_sup<true>(DS);
 template __global__ void k_sup_dense<false>(DS);
 template __global__ void k_sup_dense<true>(DS);
-template __global__ void k_cand<false>(DS);
-template __global__ void k_cand<true>(DS);
+template __global__ void k_cand<false>(DS, int, int);
+template __global__ void k_cand<true>(DS, int, int);
+template __global__ void k_events<false>(DS, int, int, int);
+template __global__ void k_events<true>(DS, int, int, int);
 template __global__ void k_contact<false>(DS);
 template __global__ void k_contact<true>(DS);
 template __global__ void k_bond<false>(DS);
