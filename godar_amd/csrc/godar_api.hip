@@ -32,7 +32,10 @@ template <bool M> __global__ void k_repair(DS, int);
 template <bool M> __global__ void k_fixup(DS);
 template <bool M, bool R> __global__ void k_final(DS);
 __global__ void k_totals(DS, int64_t*);
-__global__ void k_pairs(DS, int, int*, int2*, int);
+__global__ void k_status(DS, int, HostStatus*);
+template <int W> __global__ void k_read(DS, int, int, int, double*);
+template <int K> __global__ void k_pairs(DS, int, PairOut*, int);
+__global__ void k_take_count(int32_t*, int32_t*);
 
 __global__ void k_fill_u8(uint8_t* p, int64_t n, uint8_t v) {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -165,6 +168,12 @@ struct godar_ctx {
     int device = 0;                     // the GPU the context lives on
     int ncu = 256;                      // its compute units
     int64_t* totals_scratch = nullptr;  // device address of that GPU's `scratch`
+    // pinned host memory the GPU writes: the step status and, from the first
+    // read-back on, the staging area (stage_bytes), with an event per half
+    HostStatus* status = nullptr;
+    unsigned char* stage = nullptr;
+    hipEvent_t estage[2] = {nullptr, nullptr};
+    int64_t done = 0;                   // steps completed, as of the last godar_sync
 };
 
 namespace {
@@ -358,17 +367,126 @@ int upload_members_only(godar_ctx* c) {
     return GODAR_OK;
 }
 
-// steps completed without error since the context was created
-int steps_done(godar_ctx* c, int64_t* out) {
-    HIPCHK(c, hipMemcpyAsync(out, c->d.steps_done, sizeof(int64_t), hipMemcpyDeviceToHost, c->stream));
+// Waits for the context's stream and brings the step status back: the error
+// word, the steps completed and the members (their step numbers).
+int read_status(godar_ctx* c) {
+    sync_ds(c);
+    hipLaunchKernelGGL(k_status, dim3(1), dim3(256), 0, c->stream, c->d, c->Mcap, c->status);
+    HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipStreamSynchronize(c->stream));
+    std::memcpy(c->members.data(), c->status->members(), sizeof(Member) * c->Mcap);
     return GODAR_OK;
 }
 
-int download_members(godar_ctx* c) {
-    HIPCHK(c, hipMemcpyAsync(c->members.data(), c->d.members, sizeof(Member) * c->Mcap,
-                             hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+// steps completed without error since the context was created
+int steps_done(godar_ctx* c, int64_t* out) {
+    if (c->pending) {
+        int rc = read_status(c);
+        if (rc != GODAR_OK) return rc;
+        *out = c->status->steps_done;
+    } else {
+        *out = c->done;
+    }
+    return GODAR_OK;
+}
+
+int download_members(godar_ctx* c) { return read_status(c); }
+
+// The staging area of the read-backs: two halves, so that the host copies one
+// out while the GPU fills the other.  4 MiB keep a half (2 MiB) above the
+// size where the launch and the wait still count and within a core's caches.
+constexpr size_t STAGE_BYTES = 4u << 20;
+
+int ensure_stage(godar_ctx* c) {
+    for (hipEvent_t& e : c->estage)
+        if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+            e = nullptr;
+            (void)hipGetLastError();
+            return fail(c, GODAR_ERR_NOMEM, "read-back: no event");
+        }
+    if (!c->stage && hipHostMalloc((void**)&c->stage, STAGE_BYTES) != hipSuccess) {
+        c->stage = nullptr;
+        (void)hipGetLastError();
+        return fail(c, GODAR_ERR_NOMEM, "read-back: out of pinned host memory");
+    }
+    return GODAR_OK;
+}
+
+// Rows of member m in the caller's floe order (W: READ_FLOES, ..., `rows`
+// rows) into dst[row] (null: not wanted), by way of the staging area.
+template <int W>
+int read_rows(godar_ctx* c, int32_t m, int rows, double* const* dst) {
+    int rc = ensure_stage(c);
+    if (rc != GODAR_OK) return rc;
+    sync_ds(c);
+    const int n = c->members[m].n;
+    const int part = (int)(STAGE_BYTES / 2 / sizeof(double) / rows) & ~63;
+    const int parts = (n + part - 1) / part;
+    auto half = [&](int p) { return reinterpret_cast<double*>(c->stage + (p & 1) * (STAGE_BYTES / 2)); };
+    auto launch = [&](int p) {
+        const int cnt = std::min(part, n - p * part);
+        hipLaunchKernelGGL(k_read<W>, dim3((cnt + 63) / 64), dim3(64), 0, c->stream, c->d, m, p * part, cnt, half(p));
+        hipError_t e = hipGetLastError();
+        return e == hipSuccess ? hipEventRecord(c->estage[p & 1], c->stream) : e;
+    };
+    HIPCHK(c, launch(0));
+    for (int p = 0; p < parts; ++p) {
+        if (p + 1 < parts) HIPCHK(c, launch(p + 1));
+        HIPCHK(c, hipEventSynchronize(c->estage[p & 1]));
+        const int cnt = std::min(part, n - p * part);
+        for (int k = 0; k < rows; ++k)
+            if (dst[k]) std::memcpy(dst[k] + (int64_t)p * part, half(p) + (int64_t)k * cnt, sizeof(double) * cnt);
+    }
+    return GODAR_OK;
+}
+
+// Member m's pairs of kind K (PAIRS_*): counted into *n, and where `want`
+// listed, in no order, in the staging area or, past its room, in `more`.
+template <int K>
+int read_pairs(godar_ctx* c, int32_t m, bool want, const PairOut** list, std::vector<PairOut>& more, int* n) {
+    int rc = ensure_stage(c);
+    if (rc != GODAR_OK) return rc;
+    sync_ds(c);
+    auto pass = [&](PairOut* out, int cap) -> hipError_t {
+        if (c->N_used > 0)
+            hipLaunchKernelGGL(k_pairs<K>, dim3((c->N_used + 255) / 256), dim3(256), 0, c->stream, c->d, m, out, cap);
+        hipLaunchKernelGGL(k_take_count, dim3(1), dim3(1), 0, c->stream, c->d.npairs, &c->status->npairs);
+        hipError_t e = hipGetLastError();
+        if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+        *n = c->status->npairs;
+        return e;
+    };
+    const int room = want ? (int)(STAGE_BYTES / sizeof(PairOut)) : 0;
+    *list = reinterpret_cast<const PairOut*>(c->stage);
+    HIPCHK(c, pass(reinterpret_cast<PairOut*>(c->stage), room));
+    if (!want || *n <= room) return GODAR_OK;
+    more.resize(*n);
+    const int cap = *n;
+    PairOut* dev = nullptr;
+    hipError_t e = hipMalloc(&dev, sizeof(PairOut) * cap);
+    if (e == hipSuccess) e = pass(dev, cap);
+    if (e == hipSuccess) e = hipMemcpy(more.data(), dev, sizeof(PairOut) * cap, hipMemcpyDeviceToHost);
+    (void)hipFree(dev);
+    HIPCHK(c, e);
+    *list = more.data();
+    return GODAR_OK;
+}
+
+// Member m's pairs of kind K in order, those wanted by a caller with room for
+// `cap` of them; without room only counted.
+template <int K>
+int ordered_pairs(godar_ctx* c, int32_t m, int32_t cap, std::vector<PairOut>& out, int32_t* count) {
+    const PairOut* list = nullptr;
+    std::vector<PairOut> more;
+    int n = 0;
+    int rc = read_pairs<K>(c, m, cap > 0, &list, more, &n);
+    if (rc != GODAR_OK) return rc;
+    *count = n;
+    if (cap > 0) out.assign(list, list + n);
+    std::sort(out.begin(), out.end(), [](const PairOut& a, const PairOut& b) {
+        return a.i != b.i ? a.i < b.i : a.j < b.j;
+    });
+    if ((int64_t)out.size() > cap) out.resize(cap);
     return GODAR_OK;
 }
 
@@ -756,6 +874,8 @@ int godar_create(int64_t max_floes, int32_t max_members, int32_t precision, goda
     ACHK(dalloc(&d.tcur, max_members));
     ACHK(dalloc(&d.fout, 33 * S));
     ACHK(dalloc(&d.err, 1));
+    ACHK(dalloc(&d.npairs, 1));
+    ACHK(hipHostMalloc((void**)&c->status, HostStatus::bytes(max_members)));
     ACHK(dalloc(&d.steps_done, 1));
     c->sup_cap = 8 * S;
     ACHK(dalloc(&d.sup, c->sup_cap));
@@ -771,6 +891,7 @@ int godar_create(int64_t max_floes, int32_t max_members, int32_t precision, goda
     ACHK(radix_alloc(c->rs, S));
 #undef ACHK
     (void)hipMemsetAsync(d.err, 0, sizeof(uint32_t), c->stream);
+    (void)hipMemsetAsync(d.npairs, 0, sizeof(int32_t), c->stream);
     (void)hipMemsetAsync(d.steps_done, 0, sizeof(int64_t), c->stream);
     (void)hipMemsetAsync(d.scnt, 0, sizeof(int32_t) * S, c->stream);
     (void)hipMemsetAsync(d.nbmin, 0, sizeof(float) * S, c->stream);
@@ -820,11 +941,15 @@ int godar_destroy(godar_ctx* c) {
     }
     dfree(d.wout); dfree(d.wflag); dfree(d.cls); dfree(d.qlist); dfree(c->qn[0]); dfree(c->qn[1]); dfree(d.bgat); dfree(d.shape); dfree(d.rhead); dfree(d.nseeds); dfree(d.heap);
     dfree(d.dirty);
-    dfree(d.wnz); dfree(d.stats); dfree(d.tcur); dfree(d.err); dfree(d.steps_done);
+    dfree(d.wnz); dfree(d.stats); dfree(d.tcur); dfree(d.err); dfree(d.npairs); dfree(d.steps_done);
     dfree(d.sup); dfree(d.scnt); dfree(d.snear); dfree(d.nb); dfree(d.nbmin); dfree(d.nearsum); dfree(d.soff); dfree(d.sblk); dfree(d.x0); dfree(d.rebuild);
     radix_free(c->rs);
     collect_events(c);
     for (hipEvent_t e : c->ev_pool) (void)hipEventDestroy(e);
+    for (hipEvent_t e : c->estage)
+        if (e) (void)hipEventDestroy(e);
+    if (c->stage) (void)hipHostFree(c->stage);
+    if (c->status) (void)hipHostFree(c->status);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
     return GODAR_OK;
@@ -1764,21 +1889,18 @@ int godar_use_graphs(godar_ctx* c, int32_t on) {
 
 int godar_sync(godar_ctx* c) {
     if (!c) return GODAR_ERR_ARG;
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    collect_events(c);
-    uint32_t e = 0;
-    HIPCHK(c, hipMemcpy(&e, c->d.err, sizeof(uint32_t), hipMemcpyDeviceToHost));
-    int rc = download_members(c);
+    int rc = read_status(c);
     if (rc != GODAR_OK) return rc;
+    collect_events(c);
+    const uint32_t e = c->status->err;
+    const int64_t now = c->status->steps_done;
+    c->done = now;
     bool was_pending = c->pending;
     c->pending = false;
     if (e == ERR_NEED_BUILD && was_pending) {
         // a lean step found a build due, or a floe's drafts outgrew its lists:
         // that step and the ones after it did nothing; back to the last
         // complete step, and the rest again with the build kernels
-        int64_t now = 0;
-        rc = steps_done(c, &now);
-        if (rc != GODAR_OK) return rc;
         c->parity = c->pend_parity ^ (int)((now - c->pend_done0) & 1);
         bind_parity(c);
         HIPCHK(c, hipMemsetAsync(c->d.dirty, 0, c->S, c->stream));
@@ -1797,9 +1919,6 @@ int godar_sync(godar_ctx* c) {
         // fixes the pair-state parity.  Repair flags and the error word are
         // cleared so the caller can reserve more room and step again.
         if (was_pending) {
-            int64_t now = 0;
-            rc = steps_done(c, &now);
-            if (rc != GODAR_OK) return rc;
             c->parity = c->pend_parity ^ (int)((now - c->pend_done0) & 1);
             bind_parity(c);
         }
@@ -1913,160 +2032,46 @@ int godar_get_floes(godar_ctx* c, int32_t m, double* x, double* y, double* u, do
                     double* theta, double* omega, double* r, double* h, double* mass,
                     double* inertia, double* hfa, double* hfw) {
     if (!valid_member(c, m)) return fail(c, GODAR_ERR_ARG, "get_floes: bad member");
-    spill(c);
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    const Member& mm = c->members[m];
-    std::vector<FloeRec> recs(mm.n);
-    HIPCHK(c, hipMemcpy(recs.data(), c->d.rec + mm.first, sizeof(FloeRec) * mm.n, hipMemcpyDeviceToHost));
-    double* dst[] = {x, y, u, v, theta, omega, r, h, mass, inertia, hfa, hfw};
-    const std::vector<int32_t>& pm = c->perm[m];   // storage offset -> caller's index
-    for (int t = 0; t < mm.n; ++t) {
-        const FloeRec& q = recs[t];
-        double val[12] = {q.x, q.y, q.u, q.v, q.theta, q.omega, q.r, q.h, q.mass, q.inertia, q.hfa, q.hfw};
-        for (int k = 0; k < 12; ++k)
-            if (dst[k]) dst[k][pm[t]] = val[k];
-    }
-    return GODAR_OK;
+    double* const dst[] = {x, y, u, v, theta, omega, r, h, mass, inertia, hfa, hfw};
+    return read_rows<READ_FLOES>(c, m, 12, dst);
 }
 
 int godar_get_forces(godar_ctx* c, int32_t m, double* f) {
     if (!valid_member(c, m) || !f) return fail(c, GODAR_ERR_ARG, "get_forces: bad argument");
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    const Member& mm = c->members[m];
-    const std::vector<int32_t>& pm = c->perm[m];
-    std::vector<double> row(mm.n);
-    for (int k = 0; k < 33; ++k) {
-        HIPCHK(c, hipMemcpy(row.data(), c->d.fout + k * c->S + mm.first, sizeof(double) * mm.n,
-                            hipMemcpyDeviceToHost));
-        for (int t = 0; t < mm.n; ++t) f[(int64_t)k * mm.n + pm[t]] = row[t];
-    }
-    return GODAR_OK;
+    double* dst[NFORCE];
+    for (int k = 0; k < NFORCE; ++k) dst[k] = f + (int64_t)k * c->members[m].n;
+    return read_rows<READ_FORCES>(c, m, NFORCE, dst);
 }
 
 int godar_get_walls(godar_ctx* c, int32_t m, double* w) {
     if (!valid_member(c, m) || !w) return fail(c, GODAR_ERR_ARG, "get_walls: bad argument");
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    const Member& mm = c->members[m];
-    const std::vector<int32_t>& pm = c->perm[m];
-    std::vector<double> row(mm.n);
-    for (int k = 0; k < 4; ++k) {
-        HIPCHK(c, hipMemcpy(row.data(), c->d.wbc + k * c->S + mm.first, sizeof(double) * mm.n,
-                            hipMemcpyDeviceToHost));
-        for (int t = 0; t < mm.n; ++t) w[(int64_t)k * mm.n + pm[t]] = row[t];
-    }
-    return GODAR_OK;
+    double* dst[4];
+    for (int k = 0; k < 4; ++k) dst[k] = w + (int64_t)k * c->members[m].n;
+    return read_rows<READ_WALLS>(c, m, 4, dst);
 }
 
 int godar_get_pairs(godar_ctx* c, int32_t m, int32_t kind, int32_t cap, int32_t* pi, int32_t* pj,
                     int32_t* count) {
     if (!valid_member(c, m) || !count || cap < 0 || (cap > 0 && (!pi || !pj)))
         return fail(c, GODAR_ERR_ARG, "get_pairs: bad argument");
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    const Member& mm = c->members[m];
-    int64_t S = c->S;
-    std::vector<std::pair<int32_t, int32_t>> out;
-    if (kind == GODAR_PAIRS_CANDIDATE) {
-        // the step's lists hold the pairs that can matter; all of the
-        // candidates come from the supersets, counted first
-        sync_ds(c);
-        int n = 0, *dn = nullptr;
-        int2* dp = nullptr;
-        HIPCHK(c, hipMalloc(&dn, sizeof(int)));
-        hipError_t e = hipSuccess;
-        auto pass = [&](int want) {
-            hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, c->stream, dn, (int64_t)1, 0);
-            if (c->N_used > 0)
-                hipLaunchKernelGGL(k_pairs, dim3((c->N_used + 255) / 256), dim3(256), 0, c->stream, c->d, m, dn, dp, want);
-            e = hipMemcpyAsync(&n, dn, sizeof(int), hipMemcpyDeviceToHost, c->stream);
-            if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-        };
-        pass(0);
-        if (e == hipSuccess && n > 0 && cap > 0) {
-            const int want = n;
-            std::vector<int2> h(want);
-            e = hipMalloc(&dp, sizeof(int2) * want);
-            if (e == hipSuccess) pass(want);
-            if (e == hipSuccess) e = hipMemcpy(h.data(), dp, sizeof(int2) * want, hipMemcpyDeviceToHost);
-            for (const int2& p : h) out.push_back({p.x, p.y});
-        }
-        (void)hipFree(dp);
-        (void)hipFree(dn);
-        HIPCHK(c, e);
-        if (cap == 0) { *count = n; return GODAR_OK; }
-    } else if (kind == GODAR_PAIRS_CONTACT) {
-        // the member's floes occupy a contiguous range of this step's cell order
-        std::vector<int32_t> pos(mm.n);
-        HIPCHK(c, hipMemcpy(pos.data(), c->d.pos_of + mm.first, sizeof(int32_t) * mm.n, hipMemcpyDeviceToHost));
-        int32_t p0 = *std::min_element(pos.begin(), pos.end());
-        int32_t len = *std::max_element(pos.begin(), pos.end()) - p0 + 1;
-        std::vector<int32_t> cnt(len);
-        HIPCHK(c, hipMemcpy(cnt.data(), c->d.ocnt + p0, sizeof(int32_t) * len, hipMemcpyDeviceToHost));
-        int32_t cmax = 0;
-        for (int32_t v : cnt) cmax = std::max(cmax, v);
-        cmax = std::min(cmax, c->CO);
-        std::vector<int64_t> oj((int64_t)cmax * len);
-        std::vector<uint32_t> ef((int64_t)cmax * len);
-        for (int s = 0; s < cmax; ++s) {
-            HIPCHK(c, hipMemcpy(oj.data() + (int64_t)s * len, c->d.oj + s * S + p0,
-                                sizeof(int64_t) * len, hipMemcpyDeviceToHost));
-            HIPCHK(c, hipMemcpy(ef.data() + (int64_t)s * len, c->d.evf + s * S + p0,
-                                sizeof(uint32_t) * len, hipMemcpyDeviceToHost));
-        }
-        for (int i = 0; i < mm.n; ++i) {
-            int32_t r0 = pos[i] - p0;
-            for (int s = 0; s < cnt[r0] && s < cmax; ++s) {
-                uint32_t fl = ef[(int64_t)s * len + r0];
-                if (fl & EV_REMOVED) continue;
-                if (!(fl & EV_CONTACT)) continue;
-                out.push_back({c->perm[m][i], (int32_t)(oj[(int64_t)s * len + r0] >> 32) - mm.first});
-            }
-        }
-    } else if (kind == GODAR_PAIRS_BOND) {
-        int o = c->parity;
-        std::vector<int32_t> cnt(mm.n);
-        HIPCHK(c, hipMemcpy(cnt.data(), c->bcnt[o] + mm.first, sizeof(int32_t) * mm.n, hipMemcpyDeviceToHost));
-        std::vector<BondRec> rec(mm.n);
-        for (int q = 0; q < c->BC; ++q) {
-            HIPCHK(c, hipMemcpy(rec.data(), c->bond[o] + q * S + mm.first, sizeof(BondRec) * mm.n,
-                                hipMemcpyDeviceToHost));
-            for (int i = 0; i < mm.n; ++i)
-                if (q < cnt[i] && rec[i].j >= 0 && rec[i].bond == 1)
-                    out.push_back({c->perm[m][i], rec[i].j - mm.first});
-        }
-    } else {
-        return fail(c, GODAR_ERR_ARG, "get_pairs: bad kind");
-    }
-    std::sort(out.begin(), out.end());
-    *count = (int32_t)out.size();
-    for (int32_t k = 0; k < cap && k < (int32_t)out.size(); ++k) { pi[k] = out[k].first; pj[k] = out[k].second; }
+    std::vector<PairOut> out;
+    int rc;
+    if (kind == GODAR_PAIRS_CANDIDATE) rc = ordered_pairs<PAIRS_CANDIDATE>(c, m, cap, out, count);
+    else if (kind == GODAR_PAIRS_CONTACT) rc = ordered_pairs<PAIRS_CONTACT>(c, m, cap, out, count);
+    else if (kind == GODAR_PAIRS_BOND) rc = ordered_pairs<PAIRS_BOND>(c, m, cap, out, count);
+    else return fail(c, GODAR_ERR_ARG, "get_pairs: bad kind");
+    if (rc != GODAR_OK) return rc;
+    for (size_t k = 0; k < out.size(); ++k) { pi[k] = out[k].i; pj[k] = out[k].j; }
     return GODAR_OK;
 }
 
 int godar_get_bond_state(godar_ctx* c, int32_t m, int32_t cap, double* st, int32_t* count) {
     if (!valid_member(c, m) || !count || cap < 0 || (cap > 0 && !st))
         return fail(c, GODAR_ERR_ARG, "get_bond_state: bad argument");
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    const Member& mm = c->members[m];
-    int64_t S = c->S;
-    int o = c->parity;
-    std::vector<int32_t> cnt(mm.n);
-    HIPCHK(c, hipMemcpy(cnt.data(), c->bcnt[o] + mm.first, sizeof(int32_t) * mm.n, hipMemcpyDeviceToHost));
-    std::vector<std::pair<std::pair<int32_t, int32_t>, BondRec>> out;
-    std::vector<BondRec> rec(mm.n);
-    for (int q = 0; q < c->BC; ++q) {
-        HIPCHK(c, hipMemcpy(rec.data(), c->bond[o] + q * S + mm.first, sizeof(BondRec) * mm.n,
-                            hipMemcpyDeviceToHost));
-        for (int i = 0; i < mm.n; ++i)
-            if (q < cnt[i] && rec[i].j >= 0 && rec[i].bond == 1)
-                out.push_back({{c->perm[m][i], rec[i].j - mm.first}, rec[i]});
-    }
-    std::sort(out.begin(), out.end(), [](const auto& a, const auto& b) { return a.first < b.first; });
-    *count = (int32_t)out.size();
-    for (int32_t k = 0; k < cap && k < (int32_t)out.size(); ++k) {
-        const BondRec& b = out[k].second;
-        double v[11] = {(double)b.bond, b.damage, b.deltanb, b.deltatb, b.trb_ji, b.trb_ij, b.rb, b.hb, b.lb, b.sb, b.ib};
-        std::memcpy(st + 11 * (int64_t)k, v, sizeof(v));
-    }
+    std::vector<PairOut> out;
+    int rc = ordered_pairs<PAIRS_BOND>(c, m, cap, out, count);
+    if (rc != GODAR_OK) return rc;
+    for (size_t k = 0; k < out.size(); ++k) std::memcpy(st + 11 * k, out[k].v, sizeof(out[k].v));
     return GODAR_OK;
 }
 

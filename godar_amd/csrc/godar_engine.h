@@ -164,7 +164,28 @@ struct DS {
     int32_t* tcur;             // [members] number of the step in progress (set at its start)
     double* fout;              // [33][S] (id)
     uint32_t* err;
+    int32_t* npairs;           // pairs k_pairs has counted (0 between calls)
     int64_t* steps_done;       // steps completed without error (whole context)
+};
+
+// What the host reads after steps, in pinned host memory that k_status
+// writes: one launch and one wait bring all of it back (copies of their own
+// for each word cost 15-20 us each, most of a small member's step).
+struct HostStatus {
+    int64_t steps_done;
+    uint32_t err;
+    int32_t npairs;            // the last pair list's length (k_take_count)
+    __host__ __device__ Member* members() { return reinterpret_cast<Member*>(this + 1); }
+    static size_t bytes(int nmembers) { return sizeof(HostStatus) + sizeof(Member) * nmembers; }
+};
+
+// Rows k_read gives (12, NFORCE and 4 of them) and pairs k_pairs lists.
+enum { READ_FLOES, READ_FORCES, READ_WALLS };
+enum { PAIRS_CANDIDATE, PAIRS_CONTACT, PAIRS_BOND };
+constexpr int NFORCE = 33;
+struct PairOut {
+    int32_t i, j;              // in the caller's indices
+    double v[11];              // PAIRS_BOND: the bond's state, as godar_set_bonds takes it
 };
 
 }  // namespace godar

@@ -269,19 +269,19 @@ class Context:
     # ------------------------------------------------------------ read-back
     def floes(self, m: int) -> dict:
         n = self.sizes[m]
-        outs = [np.zeros(n) for _ in STATE_KEYS]
+        outs = [np.empty(n) for _ in STATE_KEYS]   # (every entry is written)
         self._chk(self.L.godar_get_floes(self.h, int(m), *[_ptr(a) for a in outs]))
         return dict(zip(STATE_KEYS, outs))
 
     def forces(self, m: int) -> dict:
         n = self.sizes[m]
-        f = np.zeros((33, n))
+        f = np.empty((33, n))
         self._chk(self.L.godar_get_forces(self.h, int(m), _ptr(f)))
         return dict(zip(FORCE_KEYS, f))
 
     def walls(self, m: int) -> dict:
         n = self.sizes[m]
-        w = np.zeros((4, n))
+        w = np.empty((4, n))
         self._chk(self.L.godar_get_walls(self.h, int(m), _ptr(w)))
         return dict(zip(["deltat_bc1", "deltat_bc2", "theta_bc1", "theta_bc2"], w))
 

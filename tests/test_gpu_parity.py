@@ -12,6 +12,8 @@ Bars:
   * batch invariance: a member's trajectory does not depend on its batch
     mates (bitwise), in FP64 and in mixed precision.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -618,6 +620,67 @@ def test_checkpoint_restore_continues_exactly():
             assert np.array_equal(got[k], want[k]), (prec, k)
         for k in ("tfx", "tfy", "m", *STRESS):
             assert np.array_equal(gotf[k], wantf[k]), (prec, k)
+
+
+@pytest.mark.parametrize("n", [1, 64, 65, 7937, 21825, 24000])
+def test_read_back_in_parts(n):
+    """Floes, forces and pair lists read back through the staging area are
+    those of a checkpoint and of the field: below, at and past the sizes where
+    a read takes a second part (7,936 floes of force columns, 21,824 of floe
+    state) and where a list outgrows the area (43,690 pairs), for a member
+    behind another one, while it steps, and after it has stopped."""
+    side = int(np.ceil(np.sqrt(n)))
+    rng = np.random.default_rng(n)
+    a, b = np.arange(n) % side, np.arange(n) // side
+    f = g.config0_member(51, 100)
+    mate = g.config0_member(52, 100)
+    f.x, f.y = 2000.0 * a + 1000.0, 2000.0 * b + 1000.0
+    f.r, f.h = 995.0 + rng.uniform(-2, 2, n), rng.uniform(0.8, 1.2, n)
+    order = rng.permutation(n)
+    f.x, f.y = f.x[order], f.y[order]
+    f.theta, f.omega = np.zeros(n), np.zeros(n)
+    f.u, f.v = rng.normal(0, 0.01, n), rng.normal(0, 0.01, n)
+    f.box = 2000.0 * side
+    p = config0_params(f, bond_lim=20.0, rtree=1500.0, ridging=0)
+    ctx = _ctx(n + mate.n, 2)
+    ctx.add_field(config0_params(mate), mate)
+    m = ctx.add_field(p, f)
+    ctx.run_until(m, 2)
+    ctx.step(1)
+    # a lattice of gaps below bond_lim: every pair of neighbours is a
+    # candidate and no other pair is, and the seeded share of them bonds
+    at = np.full(side * side + side, -1)
+    at[order] = np.arange(n)
+    pos = order
+    pairs = set()
+    for d, ok in ((1, pos % side < side - 1), (side, np.ones(n, bool))):
+        q = at[pos + d]
+        ok = ok & (q >= 0)
+        pairs |= {(min(i, j), max(i, j)) for i, j in zip(np.arange(n)[ok].tolist(), q[ok].tolist())}
+    assert _pairs(ctx, m, "candidate") == sorted(pairs)
+    pairs = {(i, j) for i, j in pairs if g.bond_keep(i, j, p.bond_seed, p.bond_frac)}
+    assert _pairs(ctx, m, "bond") == sorted(pairs)
+    assert _pairs(ctx, m, "contact") == []
+    s0 = ctx.floes(m)
+    ctx.step(1)                      # the member's last step
+    for _ in range(2):
+        s1, fo = ctx.floes(m), ctx.forces(m)
+        # the integration's own update (integration.f90:1-38), rounded the same
+        assert np.array_equal(s1["u"], s0["u"] + fo["tfx"] / s0["mass"] * p.dt)
+        assert np.array_equal(s1["v"], s0["v"] + fo["tfy"] / s0["mass"] * p.dt)
+        assert np.array_equal(s1["omega"], s0["omega"] + fo["m"] / s0["inertia"] * p.dt)
+        block = ctx.checkpoint(m, p)
+        head = 40 + ctypes.sizeof(p)
+        ck = np.frombuffer(block, np.float64, 12 * n, head).reshape(n, 12)
+        for c, k in enumerate(["x", "y", "u", "v", "omega", "r", "h", "mass", "inertia", "hfa", "hfw", "theta"]):
+            assert np.array_equal(s1[k], ck[:, c]), k
+        tail = np.frombuffer(block, np.uint8)[-88 * len(pairs):] if pairs else np.zeros(0, np.uint8)
+        damage = np.frombuffer(tail.tobytes(), np.float64).reshape(-1, 11)[:, 1]
+        # (the block lists a floe's bonds in record order, the state by partner)
+        assert np.array_equal(np.sort(ctx.bond_state(m)["damage"]), np.sort(damage))
+        ctx.step(3)                  # the member has stopped, its mate goes on
+    assert ctx.tstep(m) == 3
+    ctx.close()
 
 
 def test_forcing_change_takes_effect_next_step():
