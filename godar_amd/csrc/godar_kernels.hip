@@ -546,35 +546,7 @@ __device__ __forceinline__ void enqueue(const DS& S, bool want, int c, int k) {
 //    bond records (or a bond of its own forms this step), the wall queue if
 //    it crosses the box.
 // ---------------------------------------------------------------------
-// Finishing writes of one floe's search (any search shape): list counts,
-// per-slot resets, sheltering minima and the per-step resets of its rows
-// (fs: the floe's storage slot).
-__device__ __forceinline__ void cand_finish(const DS& S, int k, int fs, const DevParams& P, int no,
-                                            int ni, double sha, double shw, bool qc, bool qb) {
-    const int64_t SS = S.S;
-    const uint32_t fl = P.shelter ? EV_SHELTER : 0u;
-    for (int s2 = 0; s2 < no; ++s2) {
-        S.evf[s2 * SS + k] = fl;
-        if (S.record_forces) {
-            S.ssc[s2 * SS + k] = 0.0;
-            S.ssb[s2 * SS + k] = 0.0;
-        }
-    }
-    for (int s2 = 0; s2 < ni; ++s2) S.ibond[s2 * SS + k] = 0;
-    S.ocnt[k] = no;
-    S.icnt[k] = ni;
-    S.acc[A_SHA * SS + k] = sha;
-    S.acc[A_SHW * SS + k] = shw;
-    if (!qc) S.hcnt_new[fs] = 0;
-    if (!qb) S.bcnt_new[fs] = 0;
-    S.wflag[k] = 0;
-    S.bgat[k] = 0;
-    S.rhead[k] = -1;
-    S.cls[k] = qc ? CLS_CONTACT : 0;   // the fix-up sets CLS_BOND
-}
-
 constexpr int SCAN_BATCH = 4;
-constexpr int LIST_REGS = 4;
 
 // The query radius r + rtree holds many floes that are far away: no contact,
 // no bond, and a sheltering term that is exactly 1 (with power-law radii on
@@ -692,28 +664,35 @@ __device__ __forceinline__ int2 sup_thread(const DS& S, int k, const GeoRec& me,
 }
 
 // (floe, candidate) pairs of one wavefront in LDS: entry, distance (inner:
-// -1) and owner lane, then the per-lane pair counts
+// -1) and owner lane, the per-lane pair counts and the pairs whose terms are
+// evaluated
 constexpr int CAND_TCAP = 512;
 constexpr int CAND_LDS_PER_WAVE = CAND_TCAP * (8 + 8 + 1) + 64 * 4 + CAND_TCAP * 2;
+static_assert(CAND_TCAP < 1 << 10, "the per-lane counts are packed 10 bits each");
 
 // Neighbour search of one floe by one thread: its candidate lists are the
-// entries of its superset within the query radius, inserted into the
-// slot-major rows, then sheltering minima, classification and the per-step
-// resets of the floe's rows.  The head of each candidate list is sorted in
-// registers while it is built, the rest in its slots in HBM.
+// entries of its superset within the query radius, in the slot-major rows
+// (the outer ones by distance and identity, the inner ones by identity), then
+// sheltering minima, classification and the per-step resets of the floe's
+// rows.
 //
 // Every lane of the wavefront calls it (act: the lane has a floe).  The
 // wavefront's supersets lie one after the other in the pool; they are tested
 // together, 64 consecutive entries a round (each lane finds the entry's
 // owner among the lanes), and the entries within the query radius are listed
 // in LDS (`lds`, CAND_LDS_PER_WAVE bytes for this wavefront) in superset
-// order, so each owner's are contiguous.  Each floe inserts its own into its
-// lists in that order (as its own scan would), and the sheltering and
-// classification terms of all the listed pairs are evaluated together, 64 at
-// a time; each floe then takes the minimum of its own terms (a minimum of
-// fmin terms does not depend on the order or on which lane computed them).
-// When the pairs outnumber CAND_TCAP, each lane scans its own superset and
-// evaluates its own terms.
+// order, so each owner's are contiguous.  Then one lane per listed pair
+// counts how many of its owner's come before it and writes the entry to that
+// place (inserting them one after the other, a lane per floe, held the
+// wavefront for its longest list, whose part past a few entries in registers
+// went through memory: 320,000 power-law floes mixed 109 -> 60 us, 40,015 57
+// -> 33, 262,144 FP64 164 -> 76; radii on [500, 2000] m, 1.7 pairs a floe, the
+// same), and the
+// sheltering and classification terms of the pairs that need them are
+// evaluated together, 64 at a time; each floe then takes the minimum of its
+// own terms (a minimum of fmin terms does not depend on which lane computed
+// them).  Floes whose pairs outnumber CAND_TCAP together are taken in smaller
+// groups; one that does by itself inserts its entries in memory.
 // The rows of position k (and its storage slot's counts) that the search
 // reads first, loaded at once as soon as k is known.
 struct CandPre {
@@ -732,6 +711,81 @@ __device__ __forceinline__ CandPre cand_pre(const DS& S, int k) {
     return c;
 }
 
+// The lists, minima and flags of one floe with more pairs than the
+// wavefront's LDS holds, by its lane alone: insertion in memory (the outer
+// list's distances in S.od), the terms as they come.
+template <bool MIXED>
+__device__ __forceinline__ void cand_single(const DS& S, int k, int m, bool bond_step, int& no, int& ni,
+                                            typename Prec<MIXED>::T& sha, typename Prec<MIXED>::T& shw,
+                                            bool& qc, bool& qb) {
+    using T = typename Prec<MIXED>::T;
+    const GeoRec me = S.geo[k];
+    const CandPre pre = cand_pre(S, k);
+    const DevParams& P = S.params[m];
+    const int first = S.members[m].first;
+    const int64_t SS = S.S;
+    const int f = me.id;
+    const double rad = me.r + P.rtree;
+    const int64_t* se = S.sup + pre.soff;
+    for (int v = 0; v < pre.L; ++v) {
+        const int64_t e0 = se[v];
+        const int q = ent_pos(e0);
+        const GeoRec o = S.geo[q];
+        const int j = o.id;
+        const bool outer = j > f;
+        const double dx = me.x - o.x, dy = me.y - o.y;
+        const double dist2 = dx * dx + dy * dy;
+        const double thr = outer ? rad : o.r + P.rtree;
+        if (dist2 > thr * thr * (1.0 + 1e-12)) continue;
+        const double d = sqrt(dist2);
+        if (!(d <= thr) || !(me.r + o.r - d >= -sup_bound(e0))) continue;
+        const int64_t e = ent(j, q);
+        if (outer && no < S.CO) {
+            int p = no;
+            for (; p > 0; --p) {
+                const double dp = S.od[(p - 1) * SS + k];
+                const int64_t ep = S.oj[(p - 1) * SS + k];
+                if (dp < d || (dp == d && ent_id(ep) < j)) break;
+                S.od[p * SS + k] = dp;
+                S.oj[p * SS + k] = ep;
+            }
+            S.od[p * SS + k] = d;
+            S.oj[p * SS + k] = e;
+            S.evf[no * SS + k] = P.shelter ? EV_SHELTER : 0u;
+            if (S.record_forces) { S.ssc[no * SS + k] = 0.0; S.ssb[no * SS + k] = 0.0; }
+        } else if (!outer && ni < S.CI) {
+            int p = ni;
+            for (; p > 0; --p) {
+                const int64_t ep = S.ik[(p - 1) * SS + k];
+                if (ep < e) break;
+                S.ik[p * SS + k] = ep;
+            }
+            S.ik[p * SS + k] = e;
+            S.ibond[ni * SS + k] = 0;
+        }
+        ++(outer ? no : ni);
+        // outer: pair (f, j), f the outer floe i of the event, which takes
+        // hsf*(j,f) evaluated with -cosa, -sina; inner: pair (j, f), cosa/sina
+        // point from j to f, which takes hsf*(j,f) with j's wind
+        const double deltan = outer ? me.r + o.r - d : o.r + me.r - d;
+        if (deltan > 0) qc = true;
+        if (outer && bond_step && deltan >= -P.bond_lim &&
+            bond_keep(f - first, j - first, P.bond_seed, P.bond_thr24))
+            qb = true;
+        if (P.shelter) {
+            const double nx = outer ? o.x - me.x : me.x - o.x;
+            const double ny = outer ? o.y - me.y : me.y - o.y;
+            const double cosa = nx / d, sina = ny / d;
+            const ShelRec oh = S.shel[q];
+            const T dn = T(deltan), c0t = T(cosa), s0t = T(sina);
+            const T c = outer ? -c0t : c0t, sn = outer ? -s0t : s0t;
+            const T ux = outer ? T(pre.msh.wx) : T(oh.wx), uy = outer ? T(pre.msh.wy) : T(oh.wy);
+            sha = shelter_min(sha, T(oh.hfa), T(pre.msh.hfa), dn, c, sn, ux, uy);
+            shw = shelter_min(shw, T(oh.hfw), T(pre.msh.hfw), dn, c, sn, T(P.uw), T(P.vw));
+        }
+    }
+}
+
 template <bool MIXED>
 __device__ __forceinline__ void cand_thread(const DS& S, int k, const GeoRec& me, const CandPre& pre,
                                             int m, bool act, bool& qc, bool& qb, bool& qw,
@@ -742,40 +796,20 @@ __device__ __forceinline__ void cand_thread(const DS& S, int k, const GeoRec& me
     // between them, which would turn into a chain of single loads
     const DevParams& P = S.params[m];
     const Member Mb = S.members[m];
-    const double rtree = P.rtree, pnx = P.nx, pny = P.ny, uw = P.uw, vw = P.vw, blim = P.bond_lim;
+    const double rtree = P.rtree, pnx = P.nx, pny = P.ny;
     const int coh = P.cohesion, rst = P.restart, shl = P.shelter;
-    const uint32_t bthr = P.bond_thr24;
-    const uint64_t bseed = P.bond_seed;
     const double mx = act ? me.x : 0.0, my = act ? me.y : 0.0, mr = act ? me.r : 0.0;
-    const double rad = mr + rtree;
     const int f = act ? me.id : 0;
-    const int first = Mb.first;
     const bool bond_step = act & (Mb.tstep == 1) & (rst != 1) & (coh != 0);
-    ShelRec msh;
-    msh.hfa = msh.hfw = msh.wx = msh.wy = 0.0;
-    const T uwi = T(uw), vwi = T(vw);
     T sha = T(1), shw = T(1);
+    double hfa = 0.0, hfw = 0.0;
     int fs = 0;
     int no = 0, ni = 0;
-    uint32_t over = 0;
     const int64_t SS = S.S;
-    int64_t* oj = S.oj;
-    int64_t* ik = S.ik;
-    // the first LIST_REGS entries of each list stay in registers while the
-    // lists are built (sorted; empty slots hold keys above every entry), the
-    // rest are sorted in their slots in HBM
-    double rd[LIST_REGS];
-    int64_t re[LIST_REGS], ri[LIST_REGS];
-#pragma unroll
-    for (int t = 0; t < LIST_REGS; ++t) {
-        rd[t] = __longlong_as_double(0x7ff0000000000000ll);
-        re[t] = INT64_MAX;
-        ri[t] = INT64_MAX;
-    }
     int L = 0;
     int64_t soff = 0;
     if (act) {
-        msh = pre.msh;
+        hfa = pre.msh.hfa; hfw = pre.msh.hfw;
         fs = pre.fs;
         qc = pre.hc > 0;
         qb = pre.bc > 0;
@@ -783,129 +817,80 @@ __device__ __forceinline__ void cand_thread(const DS& S, int k, const GeoRec& me
         L = pre.L;
         soff = pre.soff;
     }
-    // one candidate j at position q and distance d into the floe's lists
-    auto insert = [&](int j, int q, double d) {
-        if (j > f) {
-            if (no >= S.CO) { over |= ERR_OUTER_CAP; return; }
-            // insertion by (distance, id) into the register part; the entry
-            // that leaves it is the largest so far
-            double xd = d;
-            int64_t xe = ent(j, q);
-#pragma unroll
-            for (int t = 0; t < LIST_REGS; ++t) {
-                const bool lt = xd < rd[t] || (xd == rd[t] && ent_id(xe) < ent_id(re[t]));
-                const double td = rd[t];
-                const int64_t te = re[t];
-                rd[t] = lt ? xd : td;
-                re[t] = lt ? xe : te;
-                xd = lt ? td : xd;
-                xe = lt ? te : xe;
-            }
-            if (no >= LIST_REGS) {
-                int p = no;
-                while (p > LIST_REGS) {
-                    double dp = S.od[(p - 1) * SS + k];
-                    int64_t ep = oj[(p - 1) * SS + k];
-                    if (dp < xd || (dp == xd && ent_id(ep) < ent_id(xe))) break;
-                    S.od[p * SS + k] = dp;
-                    oj[p * SS + k] = ep;
-                    --p;
-                }
-                S.od[p * SS + k] = xd;
-                oj[p * SS + k] = xe;
-            }
-            ++no;
-        } else {
-            if (ni >= S.CI) { over |= ERR_INNER_CAP; return; }
-            int64_t xe = ent(j, q);
-#pragma unroll
-            for (int t = 0; t < LIST_REGS; ++t) {
-                const bool lt = xe < ri[t];
-                const int64_t te = ri[t];
-                ri[t] = lt ? xe : te;
-                xe = lt ? te : xe;
-            }
-            if (ni >= LIST_REGS) {
-                int p = ni;
-                while (p > LIST_REGS) {
-                    int64_t ep = ik[(p - 1) * SS + k];
-                    if (ep < xe) break;
-                    ik[p * SS + k] = ep;
-                    --p;
-                }
-                ik[p * SS + k] = xe;
-            }
-            ++ni;
-        }
-    };
-    bool flat = false;          // the wavefront's pairs are listed in LDS
-    int abase = 0, acount = 0, atotal = 0;
     int64_t* te = reinterpret_cast<int64_t*>(lds);                      // entry, then the water term
     double* td = reinterpret_cast<double*>(lds + 8 * CAND_TCAP);         // distance (inner: -1), then the air term
-    uint8_t* to = lds + 16 * CAND_TCAP;                                   // owner lane, then flags | 0x80
-    int32_t* tn = reinterpret_cast<int32_t*>(lds + 17 * CAND_TCAP);      // pairs per lane
-    // the pairs whose terms the second pass evaluates (indices into the above)
+    uint8_t* to = lds + 16 * CAND_TCAP;                                   // owner lane, then flags
+    // per lane: pairs, outer ones << 10, pairs whose terms are needed << 20
+    int32_t* tn = reinterpret_cast<int32_t*>(lds + 17 * CAND_TCAP);
+    // the pairs whose terms the last pass evaluates (indices into the above)
     uint16_t* tx = reinterpret_cast<uint16_t*>(lds + 17 * CAND_TCAP + 64 * 4);
-    int nneed = 0;
-    {
-        const int lane = (int)(threadIdx.x & 63);
-        const uint64_t lt = lane ? ((~0ull) >> (64 - lane)) : 0ull;
-        int incl = L;
+    const int lane = (int)(threadIdx.x & 63);
+    const uint64_t lt = lane ? ((~0ull) >> (64 - lane)) : 0ull;
+    int incl = L;
 #pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const int v = __shfl_up(incl, off);
-            if (lane >= off) incl += v;
-        }
-        const int start = incl - L, totalL = __shfl(incl, 63);
+    for (int off = 1; off < 64; off <<= 1) {
+        const int v = __shfl_up(incl, off);
+        if (lane >= off) incl += v;
+    }
+    const int start = incl - L, totalL = __shfl(incl, 63);
+    // the floe's switches for the other passes: sheltering on (bit 0), bonds
+    // may form this step (bit 1)
+    const int pflags = (shl != 0 ? 1 : 0) | (bond_step ? 2 : 0);
+    // an entry's owner: the last lane whose superset starts at or before
+    // it (lanes without entries share the next one's start); idx < totalL
+    auto owner_of = [&](int idx) {
+        int own = 0;
+#pragma unroll
+        for (int step = 32; step > 0; step >>= 1)
+            if (__shfl(start, own + step) <= idx) own += step;
+        return own;
+    };
+    auto entry_at = [&](int idx, int own) -> int64_t {
+        return S.sup[__shfl(soff, own) + (idx - __shfl(start, own))];
+    };
+    // the floes [g0, g1) of the wavefront at a time: all of them, as a rule
+    uint64_t alone = 0;         // lanes of floes that list their pairs by themselves
+    for (int g0 = 0, gs = 64; g0 < 64;) {
+        const int g1 = min(g0 + gs, 64);
+        const int lo = __shfl(start, g0), hi = g1 < 64 ? __shfl(start, g1 & 63) : totalL;
+        int atotal = 0, nneed = 0;
         tn[lane] = 0;
         wave_lds_sync();
         bool ovf = false;
-        // the floe's switches for the second pass: sheltering on (bit 0), bonds
-        // may form this step (bit 1)
-        const int pflags = (shl != 0 ? 1 : 0) | (bond_step ? 2 : 0);
-        // an entry's owner: the last lane whose superset starts at or before
-        // it (lanes without entries share the next one's start); idx < totalL
-        auto owner_of = [&](int idx) {
-            int own = 0;
-#pragma unroll
-            for (int step = 32; step > 0; step >>= 1)
-                if (__shfl(start, own + step) <= idx) own += step;
-            return own;
-        };
-        auto entry_at = [&](int idx, int own) -> int64_t {
-            return S.sup[__shfl(soff, own) + (idx - __shfl(start, own))];
-        };
-        // each round's superset entries are requested during the round
-        // before (a lane past the end reads the last entry again)
-        int own_nxt = 0;
-        int64_t e_nxt = 0;
-        if (totalL > 0) {
-            own_nxt = owner_of(min(lane, totalL - 1));
-            e_nxt = entry_at(min(lane, totalL - 1), own_nxt);
+        // each round's superset entries are requested two rounds before and
+        // their floes one round before (a lane past the end reads the last
+        // entry again)
+        int own = 0, own_nxt = 0;
+        int64_t e = 0, e_nxt = 0;
+        GeoRec o = {};
+        if (lo < hi) {
+            own = owner_of(min(lo + lane, hi - 1));
+            e = entry_at(min(lo + lane, hi - 1), own);
+            own_nxt = owner_of(min(lo + 64 + lane, hi - 1));
+            e_nxt = entry_at(min(lo + 64 + lane, hi - 1), own_nxt);
+            o = S.geo[ent_pos(e)];
         }
-        for (int c0 = 0; c0 < totalL; c0 += 64) {
+        for (int c0 = lo; c0 < hi; c0 += 64) {
             const int idx = c0 + lane;
-            const int own = own_nxt;
-            const int64_t e = e_nxt;
-            if (c0 + 64 < totalL) {
-                const int idn = min(idx + 64, totalL - 1);
-                own_nxt = owner_of(idn);
-                e_nxt = entry_at(idn, own_nxt);
+            int own_2 = 0;
+            int64_t e_2 = 0;
+            GeoRec o_nxt = o;
+            if (c0 + 64 < hi) {
+                o_nxt = S.geo[ent_pos(e_nxt)];
+                own_2 = owner_of(min(idx + 128, hi - 1));
+                e_2 = entry_at(min(idx + 128, hi - 1), own_2);
             }
-            const double ox = __shfl(mx, own), oy = __shfl(my, own), orad = __shfl(rad, own);
+            const double ox = __shfl(mx, own), oy = __shfl(my, own);
             const double ort = __shfl(rtree, own), orr = __shfl(mr, own);
-            const double ohfa = __shfl(msh.hfa, own), ohfw = __shfl(msh.hfw, own);
+            const double ohfa = __shfl(hfa, own), ohfw = __shfl(hfw, own);
             const int of = __shfl(f, own), ofl = __shfl(pflags, own);
             bool hit = false, need = false;
             double d = 0.0;
-            int j = 0, q = 0;
-            if (idx < totalL) {
-                q = ent_pos(e);
-                const GeoRec o = S.geo[q];
+            const int j = o.id, q = ent_pos(e);
+            if (idx < hi) {
                 const double dx = ox - o.x, dy = oy - o.y;
                 const double dist2 = dx * dx + dy * dy;
-                j = o.id;
-                const double thr = j > of ? orad : o.r + ort;
+                const double thr = j > of ? orr + ort : o.r + ort;
                 // far beyond the radius: no square root needed (sqrt is
                 // correctly rounded, so it cannot cross a margin of 1e-12)
                 if (dist2 <= thr * thr * (1.0 + 1e-12)) {
@@ -915,7 +900,7 @@ __device__ __forceinline__ void cand_thread(const DS& S, int k, const GeoRec& me
                     hit = d <= thr && orr + o.r - d >= -sup_bound(e);
                 }
                 if (hit) {
-                    // The second pass changes nothing for a pair out of
+                    // The last pass changes nothing for a pair out of
                     // contact, with no bond forming this step, whose two
                     // sheltering terms are exactly 1: the test shelter_min
                     // makes (the same overlap, the floe's own drafts, type T).
@@ -935,187 +920,153 @@ __device__ __forceinline__ void cand_thread(const DS& S, int k, const GeoRec& me
                 te[at] = ent(j, q);
                 td[at] = j > of ? d : -1.0;
                 to[at] = (uint8_t)own;
-                atomicAdd(&tn[own], 1);
+                atomicAdd(&tn[own], 1 + (j > of ? 1 << 10 : 0) + (need ? 1 << 20 : 0));
                 if (need) tx[nneed + __popcll(mn & lt)] = (uint16_t)at;
             }
             atotal += __popcll(mh);
             nneed += __popcll(mn);
+            own = own_nxt; e = e_nxt; o = o_nxt;
+            own_nxt = own_2; e_nxt = e_2;
         }
         wave_lds_sync();
-        if (!ovf) {
-            flat = true;
-            acount = tn[lane];
-            int ai = acount;
+        if (ovf) {
+            if (g1 - g0 > 1) { gs = (g1 - g0) / 2; continue; }
+            alone |= 1ull << g0;
+            g0 = g1;
+            continue;
+        }
+        const int mine = tn[lane];
+        const int acount = mine & 1023;
+        int ai = mine;                        // (no field carries: at most CAND_TCAP in all)
 #pragma unroll
-            for (int off = 1; off < 64; off <<= 1) {
-                const int v = __shfl_up(ai, off);
-                if (lane >= off) ai += v;
-            }
-            abase = ai - acount;
-            if (act)
-                for (int i = abase; i < abase + acount; ++i) {
-                    const double dv = td[i];
-                    insert(ent_id(te[i]), ent_pos(te[i]), dv);
+        for (int off = 1; off < 64; off <<= 1) {
+            const int v = __shfl_up(ai, off);
+            if (lane >= off) ai += v;
+        }
+        const int bases = ai - mine;
+        const int abase = bases & 1023, nbase = bases >> 20, ncount = mine >> 20;
+        if (lane >= g0 && lane < g1) {
+            no = (mine >> 10) & 1023;
+            ni = acount - no;
+        }
+        // every listed pair to its place in its owner's list, with the
+        // per-step resets of its rows
+        for (int c0 = 0; c0 < atotal; c0 += 64) {
+            const int idx = min(c0 + lane, atotal - 1);
+            const int ow = to[idx];
+            const int b = __shfl(abase, ow), n = __shfl(acount, ow), fl_o = __shfl(pflags, ow);
+            const int64_t en = te[idx];
+            const double d = td[idx];
+            const int id = ent_id(en);
+            int before = 0;
+            if (d >= 0.0) {
+                for (int t = b; t < b + n; ++t) {
+                    const double dt = td[t];
+                    before += dt >= 0.0 && (dt < d || (dt == d && ent_id(te[t]) < id));
                 }
-        }
-    }
-    if (!flat && act) {
-        // (the wavefront's common search is the common path: this one keeps few
-        // records in flight, which keeps the kernel's registers down)
-        constexpr int B = 2;
-        const int64_t* se = S.sup + soff;
-        for (int v0 = 0; v0 < L; v0 += B) {
-            GeoRec g[B];
-            int qq[B];
-            double bd[B];
-#pragma unroll
-            for (int u = 0; u < B; ++u) {
-                const int64_t e = se[min(v0 + u, L - 1)];   // the last entry stands in past the end
-                qq[u] = ent_pos(e);
-                bd[u] = sup_bound(e);
+            } else {
+                for (int t = b; t < b + n; ++t) before += td[t] < 0.0 && ent_id(te[t]) < id;
             }
-#pragma unroll
-            for (int u = 0; u < B; ++u) g[u] = S.geo[qq[u]];
-#pragma unroll
-            for (int u = 0; u < B; ++u) {
-                if (v0 + u >= L) continue;
-                const GeoRec* o = &g[u];
-                const double dx = me.x - o->x, dy = me.y - o->y;
-                const double dist2 = dx * dx + dy * dy;
-                const double thr = o->id > f ? rad : o->r + rtree;
-                if (dist2 > thr * thr * (1.0 + 1e-12)) continue;
-                const double d = sqrt(dist2);
-                if (!(d <= thr) || !(me.r + o->r - d >= -bd[u])) continue;
-                insert(o->id, qq[u], d);
+            if (c0 + lane < atotal) {
+                const int64_t at = before * SS + (k - lane + ow);
+                if (d >= 0.0) {
+                    if (before < S.CO) {
+                        S.oj[at] = en;
+                        S.evf[at] = (fl_o & 1) ? EV_SHELTER : 0u;
+                        if (S.record_forces) { S.ssc[at] = 0.0; S.ssb[at] = 0.0; }
+                    }
+                } else if (before < S.CI) {
+                    S.ik[at] = en;
+                    S.ibond[at] = 0;
+                }
             }
         }
-    }
-    // sheltering and classification over the pairs found.  A minimum and an
-    // "any" do not depend on the order of their terms.
-    if (flat) {
-        const int lane = (int)(threadIdx.x & 63);
-        wave_lds_sync();
+        // sheltering and classification over the pairs that need it.  A
+        // minimum and an "any" do not depend on the order of their terms.
+        // (A pair's terms replace the entry of the pair whose number among
+        // all listed equals its own among those that need them: no later one
+        // still to be read.)
         for (int c0 = 0; c0 < nneed; c0 += 64) {
             const bool valid = c0 + lane < nneed;
             const int idx = valid ? (int)tx[c0 + lane] : 0;
-            int64_t e = 0;
+            int64_t en = 0;
             double d = -1.0;
-            int own = lane;
-            if (valid) { e = te[idx]; d = td[idx]; own = to[idx]; }
-            // the pair's floe's member parameters, from its lane
-            const int ko = __shfl(k, own);
-            const int first_o = __shfl(first, own);
-            const int bst_o = __shfl((int)bond_step, own), shl_o = __shfl(shl, own);
-            const double blim_o = __shfl(blim, own), uw_o = __shfl(uw, own), vw_o = __shfl(vw, own);
-            const uint32_t thr_o = (uint32_t)__shfl((int)bthr, own);
-            const uint64_t seed_o = __shfl(bseed, own);
+            int ow = lane;
+            if (valid) { en = te[idx]; d = td[idx]; ow = to[idx]; }
+            // (the member parameters are read again: kept for this pass they
+            // cost the search its fourth wavefront per SIMD)
+            const int ko = k - lane + ow;
+            const int om = __shfl(m, ow), fl_o = __shfl(pflags, ow);
             T ta = T(1), tw = T(1);
             uint32_t fl = 0;
             if (valid) {
-                const int q = ent_pos(e);
+                const int q = ent_pos(en);
                 const GeoRec mo = S.geo[ko];
-                const GeoRec o = S.geo[q];
+                const GeoRec go = S.geo[q];
                 const ShelRec oh = S.shel[q];
                 const ShelRec mh = S.shel[ko];
                 const bool outer = d >= 0.0;
                 double dd = d;
                 if (!outer) {
-                    const double dx = mo.x - o.x, dy = mo.y - o.y;
+                    const double dx = mo.x - go.x, dy = mo.y - go.y;
                     dd = sqrt(dx * dx + dy * dy);
                 }
                 // outer: pair (f, j), f the outer floe i of the event; inner:
                 // pair (j, f), f the inner floe j
-                const double deltan = outer ? mo.r + o.r - dd : o.r + mo.r - dd;
+                const double deltan = outer ? mo.r + go.r - dd : go.r + mo.r - dd;
                 if (deltan > 0) fl |= 1u;
-                if (outer && bst_o && deltan >= -blim_o &&
-                    bond_keep(mo.id - first_o, ent_id(e) - first_o, seed_o, thr_o))
-                    fl |= 2u;
-                if (shl_o) {
+                const DevParams& Po = S.params[om];
+                if (outer && (fl_o & 2) && deltan >= -Po.bond_lim) {
+                    const int first = S.members[om].first;
+                    if (bond_keep(mo.id - first, ent_id(en) - first, Po.bond_seed, Po.bond_thr24)) fl |= 2u;
+                }
+                if (fl_o & 1) {
                     // outer: floe f takes hsf*(j,f), evaluated with -cosa,
                     // -sina of the direction f -> j; inner: cosa/sina point
                     // from j to f and f takes hsf*(j,f) with j's wind
-                    const double nx = outer ? o.x - mo.x : mo.x - o.x;
-                    const double ny = outer ? o.y - mo.y : mo.y - o.y;
+                    const double nx = outer ? go.x - mo.x : mo.x - go.x;
+                    const double ny = outer ? go.y - mo.y : mo.y - go.y;
                     const double cosa = nx / dd, sina = ny / dd;
                     const T dn = T(deltan), c0t = T(cosa), s0t = T(sina);
                     const T c = outer ? -c0t : c0t, sn = outer ? -s0t : s0t;
                     const T ux = outer ? T(mh.wx) : T(oh.wx), uy = outer ? T(mh.wy) : T(oh.wy);
                     ta = shelter_min(T(1), T(oh.hfa), T(mh.hfa), dn, c, sn, ux, uy);
-                    tw = shelter_min(T(1), T(oh.hfw), T(mh.hfw), dn, c, sn, T(uw_o), T(vw_o));
+                    tw = shelter_min(T(1), T(oh.hfw), T(mh.hfw), dn, c, sn, T(Po.uw), T(Po.vw));
                 }
             }
+            wave_lds_sync();
             if (valid) {
-                td[idx] = (double)ta;
-                te[idx] = __double_as_longlong((double)tw);
-                to[idx] = (uint8_t)(fl | 0x80u);
+                td[c0 + lane] = (double)ta;
+                te[c0 + lane] = __double_as_longlong((double)tw);
+                to[c0 + lane] = (uint8_t)fl;
             }
         }
         wave_lds_sync();
-        if (act) {
-            for (int i = abase; i < abase + acount; ++i) {
-                if (!(to[i] & 0x80u)) continue;      // not evaluated: terms 1, no flags
+        if (lane >= g0 && lane < g1) {
+            for (int i = nbase; i < nbase + ncount; ++i) {
                 sha = dmin(sha, T(td[i]));
                 shw = dmin(shw, T(__longlong_as_double(te[i])));
                 qc = qc || (to[i] & 1u);
                 qb = qb || (to[i] & 2u);
             }
         }
-    } else if (act) {
-        auto outer_terms = [&](int64_t e, double d) {
-            const int j = ent_id(e), q = ent_pos(e);
-            const GeoRec o = S.geo[q];
-            // pair (f, j): f is the outer floe i of the event
-            const double deltan = me.r + o.r - d;
-            if (deltan > 0) qc = true;
-            if (!qb && bond_step && deltan >= -blim &&
-                bond_keep(f - first, j - first, bseed, bthr))
-                qb = true;
-            if (shl) {
-                // floe f takes hsf*(j,f), evaluated with -cosa, -sina
-                const double cosa = (o.x - me.x) / d, sina = (o.y - me.y) / d;
-                const ShelRec oh = S.shel[q];
-                const T dn = T(deltan), c = T(cosa), sn = T(sina);
-                sha = shelter_min(sha, T(oh.hfa), T(msh.hfa), dn, -c, -sn, T(msh.wx), T(msh.wy));
-                shw = shelter_min(shw, T(oh.hfw), T(msh.hfw), dn, -c, -sn, uwi, vwi);
-            }
-        };
-        auto inner_terms = [&](int64_t e) {
-            const int q = ent_pos(e);
-            const GeoRec o = S.geo[q];
-            const double dx = me.x - o.x, dy = me.y - o.y;
-            const double d = sqrt(dx * dx + dy * dy);
-            // pair (j, f): f is the inner floe j of the event
-            const double deltan = o.r + me.r - d;
-            if (deltan > 0) qc = true;
-            if (shl) {
-                // cosa/sina point from j to f; floe f takes hsf*(j,f) with j's wind
-                const double cosa = (me.x - o.x) / d, sina = (me.y - o.y) / d;
-                const ShelRec oh = S.shel[q];
-                const T dn = T(deltan), c = T(cosa), sn = T(sina);
-                sha = shelter_min(sha, T(oh.hfa), T(msh.hfa), dn, c, sn, T(oh.wx), T(oh.wy));
-                shw = shelter_min(shw, T(oh.hfw), T(msh.hfw), dn, c, sn, uwi, vwi);
-            }
-        };
-#pragma unroll
-        for (int s2 = 0; s2 < LIST_REGS; ++s2)
-            if (s2 < no) outer_terms(re[s2], rd[s2]);
-        for (int s2 = LIST_REGS; s2 < no; ++s2) outer_terms(oj[s2 * SS + k], S.od[s2 * SS + k]);
-#pragma unroll
-        for (int s2 = 0; s2 < LIST_REGS; ++s2)
-            if (s2 < ni) inner_terms(ri[s2]);
-        for (int s2 = LIST_REGS; s2 < ni; ++s2) inner_terms(ik[s2 * SS + k]);
+        wave_lds_sync();
+        g0 = g1;
     }
     if (!act) return;
-    // the register part of the lists goes to its slots
-#pragma unroll
-    for (int s2 = 0; s2 < LIST_REGS; ++s2) {
-        if (s2 < no) {
-            oj[s2 * SS + k] = re[s2];   // (distances are only read back beyond the register part)
-        }
-        if (s2 < ni) ik[s2 * SS + k] = ri[s2];
-    }
+    if (alone >> lane & 1) cand_single<MIXED>(S, k, m, bond_step, no, ni, sha, shw, qc, qb);
+    const uint32_t over = (no > S.CO ? ERR_OUTER_CAP : 0u) | (ni > S.CI ? ERR_INNER_CAP : 0u);
     if (over) set_err(S, over);
-    cand_finish(S, k, fs, P, no, ni, double(sha), double(shw), qc, qb);
+    S.ocnt[k] = min(no, S.CO);
+    S.icnt[k] = min(ni, S.CI);
+    S.acc[A_SHA * SS + k] = double(sha);
+    S.acc[A_SHW * SS + k] = double(shw);
+    if (!qc) S.hcnt_new[fs] = 0;
+    if (!qb) S.bcnt_new[fs] = 0;
+    S.wflag[k] = 0;
+    S.bgat[k] = 0;
+    S.rhead[k] = -1;
+    S.cls[k] = qc ? CLS_CONTACT : 0;   // the fix-up sets CLS_BOND
 }
 
 // Superset build, thread per floe (members that are not dense; span 1 or

@@ -592,6 +592,37 @@ def test_dense_search_long_lists_and_unordered_supersets():
             assert np.array_equal(ha, hb)
 
 
+@pytest.mark.parametrize("n", [9, 200, 700])
+def test_search_takes_floes_in_groups(n):
+    """Small floes of such draft that all of them matter to each other: 64
+    floes' pairs that just outnumber the search's room per wavefront (512: 64
+    floes of 8 pairs just fit, 200 floes go two at a time), and 700 floes that
+    each outnumber it alone.  Lists, state and forces are the oracle's."""
+    from oracle_py import OracleSim
+    f = kick(g.make_field(n, 11, radius="uniform", r_lo=15.0, r_hi=25.0, h_median=30.0, h_sigma=0.1,
+                          packing=0.1, wind_speed=15.0, current_speed=0.2, gap=1.0), 3)
+    p = config0_params(f, rtree=9000.0)
+    # (9 floes: copies of the member fill the wavefronts)
+    copies = 16 if n == 9 else 1
+    ctx = _ctx(copies * n, copies)
+    ctx.reserve(outer=1024, inner=1024)
+    m = [ctx.add_field(p, f) for _ in range(copies)][-1]
+    O = OracleSim(p, f)
+    for t in range(1, 4):
+        ctx.step(1)
+        O.step()
+        cand, cont = _oracle_pairs(O)
+        assert len(cand) == n * (n - 1) // 2
+        assert _pairs(ctx, m, "candidate") == cand and _pairs(ctx, m, "contact") == cont, t
+        a, b = ctx.floes(m), O.state()
+        for k in STATE:
+            assert np.array_equal(a[k], b[k]), (t, k)
+        fa, fb = ctx.forces(m), O.forces()
+        for k in ("hsfa_min", "hsfw_min", "tfx", "tfy"):
+            assert _rel(fa[k], fb[k]) <= FP64_REL_TOL, (t, k)
+    ctx.close()
+
+
 def test_checkpoint_restore_continues_exactly():
     """A member restored from a checkpoint (floes, walls, contact histories
     with last contact forces, bond strain state, step number) continues
