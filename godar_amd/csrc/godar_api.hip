@@ -17,7 +17,7 @@
 namespace godar {
 __global__ void k_begin(DS, int);
 __global__ void k_ranges(DS);
-template <bool M> __global__ void k_cand(DS, int, int);
+template <bool M> __global__ void k_cand(DS, int, int, int);
 template <bool M> __global__ void k_events(DS, int, int, int);
 template <bool F> __global__ void k_sup(DS);
 template <bool F> __global__ void k_sup_dense(DS);
@@ -578,6 +578,17 @@ static dim3 grid_for(int N, int B, bool xcd) {
 // Queue kernels loop over their entries: at most QUEUE_GRID_WAVES
 // wavefronts (about one round of resident wavefronts), so that short queues
 // do not launch a wavefront per 64 floes that finds nothing to do.
+// Floes per wavefront of the candidate search: its passes over the floes'
+// pairs take 64 pairs a round, one round behind the other, so with room on the
+// chip fewer floes per wavefront end sooner (a power of two, as the queues'
+// shares are made of 64s): 1,000 floes 17 -> 10 us, 40,015 power-law floes 33 ->
+// 19, 100,000 38 -> 28; with 2,048 wavefronts on the way, twice as many cost
+// 65,000 floes on [500, 2000] m 17 -> 26 us and 320,000 power-law ones 61 -> 62.
+static int cand_floes(int N) {
+    int f = 64;
+    while (f > CAND_MIN_FLOES && N / f < CAND_WAVES) f /= 2;
+    return f;
+}
 static dim3 grid_queue(int N, int B) {
     const int cap = QUEUE_GRID_WAVES * 64 / B / XCD_COUNT * XCD_COUNT;
     const dim3 g = grid_for(N, B, true);
@@ -632,8 +643,9 @@ int launch_step(godar_ctx* c, bool lean) {
     {
         StageTimer t(c, 3);
         // LDS: one list of (floe, candidate) pairs per wavefront
-        hipLaunchKernelGGL(mixed ? k_cand<true> : k_cand<false>, grid_for(N, B[3], true),
-                           dim3(B[3]), (B[3] / 64) * CAND_LDS_PER_WAVE, s, d, lean ? 1 : 0, nm);
+        const int floes = cand_floes(N);
+        hipLaunchKernelGGL(mixed ? k_cand<true> : k_cand<false>, grid_for(N, B[3] / 64 * floes, true),
+                           dim3(B[3]), (B[3] / 64) * CAND_LDS_PER_WAVE, s, d, lean ? 1 : 0, nm, floes);
     }
     if (!c->prof) {
         // contacts, bonds and walls in one launch, as many single-wavefront
@@ -860,6 +872,7 @@ int godar_create(int64_t max_floes, int32_t max_members, int32_t precision, goda
     ACHK(dalloc(&d.wout, S));
     ACHK(dalloc(&d.wflag, (S + 3) / 4 * 4));   // whole 32-bit words (set by word atomics)
     ACHK(dalloc(&d.cls, S));
+    ACHK(dalloc(&d.rcnt, S));
     ACHK(dalloc(&d.qlist, (int64_t)NQUEUE * S));
     ACHK(dalloc(&d.bgat, S));
     for (int k = 0; k < 2; ++k) ACHK(dalloc(&c->qn[k], (int64_t)NQUEUE * XCD_COUNT * QN_STRIDE));
@@ -939,7 +952,7 @@ int godar_destroy(godar_ctx* c) {
         free_lists(L);
         set_lists(c, L);
     }
-    dfree(d.wout); dfree(d.wflag); dfree(d.cls); dfree(d.qlist); dfree(c->qn[0]); dfree(c->qn[1]); dfree(d.bgat); dfree(d.shape); dfree(d.rhead); dfree(d.nseeds); dfree(d.heap);
+    dfree(d.wout); dfree(d.wflag); dfree(d.cls); dfree(d.rcnt); dfree(d.qlist); dfree(c->qn[0]); dfree(c->qn[1]); dfree(d.bgat); dfree(d.shape); dfree(d.rhead); dfree(d.nseeds); dfree(d.heap);
     dfree(d.dirty);
     dfree(d.wnz); dfree(d.stats); dfree(d.tcur); dfree(d.err); dfree(d.npairs); dfree(d.steps_done);
     dfree(d.sup); dfree(d.scnt); dfree(d.snear); dfree(d.nb); dfree(d.nbmin); dfree(d.nearsum); dfree(d.soff); dfree(d.sblk); dfree(d.x0); dfree(d.rebuild);
@@ -968,7 +981,7 @@ static int64_t bytes_per_floe(const godar_ctx* c) {
     per += (int64_t)c->CO * (8 + 8 + 4 + 8 + 8) + (int64_t)c->CI * (8 + 4);   // oj od evf ssc ssb; ik ibond
     per += 2 * ((int64_t)c->HC * sizeof(HistRec) + (int64_t)c->BC * sizeof(BondRec));
     per += (int64_t)c->BC * sizeof(BondTerms) + 1 /*bgat*/;
-    per += NACC * 8 + sizeof(WallOut) + 1 /*wflag*/ + 1 /*cls*/ + NQUEUE * 4 /*qlist*/;
+    per += NACC * 8 + sizeof(WallOut) + 1 /*wflag*/ + 1 /*cls*/ + 4 /*rcnt*/ + NQUEUE * 4 /*qlist*/;
     per += (int64_t)c->SEEDK * sizeof(Reshape) + 4 /*rhead*/ + (int64_t)c->HEAPK * 8;
     per += 6 * 8 /*cur*/ + 1 + 1 /*dirty, wnz*/;
     per += 33 * 8 /*fout*/ + 4 + 4 /*radix keys, values*/;

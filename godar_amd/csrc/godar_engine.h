@@ -24,6 +24,8 @@ constexpr int NQUEUE = 5;         // work queues: contact, bond, wall, dense sea
 constexpr int QN_STRIDE = 64;     // ints between queue counters (256 B)
 constexpr int SCAN_TILE = 1024;   // positions per tile of the superset offset scan
 constexpr int QUEUE_GRID_WAVES = 4096;   // wavefronts launched for a queue kernel at most
+constexpr int CAND_WAVES = 2048;           // wavefronts below which the search takes fewer floes each
+constexpr int CAND_MIN_FLOES = 8;
 constexpr int WALL_GRID_WAVES = 256;     // wavefronts of the walls beside contacts and bonds at most
 constexpr int FIXUP_GRID_WAVES = 2048;   // wavefronts of the fix-up (about one resident round)
 
@@ -119,6 +121,7 @@ struct DS {
     WallOut* wout;             // [S], valid where WF_WALL is set
     uint8_t* wflag;            // [S rounded up to 4] WF_* bits
     uint8_t* cls;              // [S] CLS_* bits
+    uint32_t* rcnt;            // [S] old contact histories | old bond records << 16
     // Candidate supersets: every floe within its query radius plus the
     // member's skin at the last build, (bound << 32 | pos), floe k's at
     // sup[soff[k] .. soff[k] + scnt[k]).  They are rebuilt (cell binning,

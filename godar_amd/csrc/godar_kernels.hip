@@ -146,6 +146,21 @@ __device__ __forceinline__ QueueShare queue_share(const DS& S, const QueueBlocks
     q.stride = nw * q.floes;
     return q;
 }
+// The bond queue's: a wavefront evaluates its owners' records (1.2 each) 64 a
+// round, so half as many owners while the wavefronts are not all taken keeps
+// most of them to one round.
+__device__ __forceinline__ QueueShare bond_share(const QueueBlocks& b, int qn) {
+    const int per = (qn + XCD_COUNT - 1) / XCD_COUNT;
+    const int wpb = (int)(blockDim.x >> 6);
+    const int nw = b.blocks * wpb;
+    const int lo = b.xcd * per;
+    QueueShare q;
+    q.floes = per > 32 * nw ? 64 : 32;
+    q.begin = lo + (b.block * wpb + (int)(threadIdx.x >> 6)) * q.floes;
+    q.end = min(qn, lo + per);
+    q.stride = nw * q.floes;
+    return q;
+}
 // appends position k to queue c from a single lane
 __device__ __forceinline__ void enqueue_one(const DS& S, int c, int k) {
     const int x = k / S.qseg;
@@ -274,29 +289,52 @@ __device__ __forceinline__ int find_partner(const Rec* list, int64_t SS, int i, 
     return q;
 }
 
-// Slot of partner g among the first n entries of the slot-major list row kp
-// (outer oj or inner ik), or -1; the first LIST_PEEK entries are requested
-// together (as find_partner), the rest read one by one.
-__device__ __forceinline__ int find_entry(const int64_t* list, int64_t SS, int kp, int n, int g) {
-    int id[LIST_PEEK];
+// The first LIST_PEEK of n entries of the slot-major list row kp (outer oj or
+// inner ik), requested together (entries past n stand in for the last one).
+struct Peek { int64_t e[LIST_PEEK]; };
+__device__ __forceinline__ Peek peek_entries(const int64_t* list, int64_t SS, int kp, int n) {
+    Peek p;
 #pragma unroll
-    for (int s = 0; s < LIST_PEEK; ++s) id[s] = -1;
+    for (int s = 0; s < LIST_PEEK; ++s) p.e[s] = -1;
     if (n > 0) {
 #pragma unroll
-        for (int s = 0; s < LIST_PEEK; ++s) id[s] = ent_id(list[(int64_t)min(s, n - 1) * SS + kp]);
+        for (int s = 0; s < LIST_PEEK; ++s) p.e[s] = list[(int64_t)min(s, n - 1) * SS + kp];
     }
+    return p;
+}
+// Slot of partner g among the n entries, or -1, and its entry; the rest of a
+// long list LIST_PEEK entries a round.
+__device__ __forceinline__ int find_peeked(const Peek& p, const int64_t* list, int64_t SS, int kp,
+                                           int n, int g, int64_t& e) {
     int r = -1;
+    e = -1;
 #pragma unroll
-    for (int s = LIST_PEEK - 1; s >= 0; --s) r = (s < n && id[s] == g) ? s : r;
-    // (long lists: LIST_PEEK entries a round)
+    for (int s = LIST_PEEK - 1; s >= 0; --s) {
+        const bool is = s < n && ent_id(p.e[s]) == g;
+        r = is ? s : r;
+        e = is ? p.e[s] : e;
+    }
     for (int s0 = LIST_PEEK; r < 0 && s0 < n; s0 += LIST_PEEK) {
+        Peek q;
 #pragma unroll
-        for (int s = 0; s < LIST_PEEK; ++s) id[s] = ent_id(list[(int64_t)min(s0 + s, n - 1) * SS + kp]);
+        for (int s = 0; s < LIST_PEEK; ++s) q.e[s] = list[(int64_t)min(s0 + s, n - 1) * SS + kp];
 #pragma unroll
-        for (int s = LIST_PEEK - 1; s >= 0; --s) r = (s0 + s < n && id[s] == g) ? s0 + s : r;
+        for (int s = LIST_PEEK - 1; s >= 0; --s) {
+            const bool is = s0 + s < n && ent_id(q.e[s]) == g;
+            r = is ? s0 + s : r;
+            e = is ? q.e[s] : e;
+        }
     }
     return r;
 }
+__device__ __forceinline__ int find_entry(const int64_t* list, int64_t SS, int kp, int n, int g) {
+    int64_t e;
+    return find_peeked(peek_entries(list, SS, kp, n), list, SS, kp, n, g, e);
+}
+
+// Old contact history and bond records of the floe at position k (what its
+// storage slot's counts say, which are one load further away).
+__device__ __forceinline__ int2 record_counts(uint32_t w) { return make_int2((int)(w & 0xFFFF), (int)(w >> 16)); }
 
 __device__ __forceinline__ BondRec bond_from(const PairState& ps, int j) {
     BondRec b;
@@ -787,7 +825,7 @@ __device__ __forceinline__ void cand_single(const DS& S, int k, int m, bool bond
 }
 
 template <bool MIXED>
-__device__ __forceinline__ void cand_thread(const DS& S, int k, const GeoRec& me, const CandPre& pre,
+__device__ __forceinline__ void cand_thread(const DS& S, int k0, int k, const GeoRec& me, const CandPre& pre,
                                             int m, bool act, bool& qc, bool& qb, bool& qw,
                                             unsigned char* lds) {
     using T = typename Prec<MIXED>::T;
@@ -968,7 +1006,7 @@ __device__ __forceinline__ void cand_thread(const DS& S, int k, const GeoRec& me
                 for (int t = b; t < b + n; ++t) before += td[t] < 0.0 && ent_id(te[t]) < id;
             }
             if (c0 + lane < atotal) {
-                const int64_t at = before * SS + (k - lane + ow);
+                const int64_t at = before * SS + (k0 + ow);
                 if (d >= 0.0) {
                     if (before < S.CO) {
                         S.oj[at] = en;
@@ -995,7 +1033,7 @@ __device__ __forceinline__ void cand_thread(const DS& S, int k, const GeoRec& me
             if (valid) { en = te[idx]; d = td[idx]; ow = to[idx]; }
             // (the member parameters are read again: kept for this pass they
             // cost the search its fourth wavefront per SIMD)
-            const int ko = k - lane + ow;
+            const int ko = k0 + ow;
             const int om = __shfl(m, ow), fl_o = __shfl(pflags, ow);
             T ta = T(1), tw = T(1);
             uint32_t fl = 0;
@@ -1067,6 +1105,7 @@ __device__ __forceinline__ void cand_thread(const DS& S, int k, const GeoRec& me
     S.bgat[k] = 0;
     S.rhead[k] = -1;
     S.cls[k] = qc ? CLS_CONTACT : 0;   // the fix-up sets CLS_BOND
+    S.rcnt[k] = (uint32_t)pre.hc | ((uint32_t)pre.bc << 16);
 }
 
 // Superset build, thread per floe (members that are not dense; span 1 or
@@ -1167,12 +1206,15 @@ __global__ __launch_bounds__(SCAN_TILE) void k_scan_offsets(DS S) {
 // does nothing else: every later kernel of the step returns at once and the
 // host runs the step again with them.)
 template <bool MIXED>
-__global__ __launch_bounds__(FLOE_BLOCK) void k_cand(DS S, int lean, int nmembers) {
-    const int k = xcd_block() * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(FLOE_BLOCK) void k_cand(DS S, int lean, int nmembers, int floes) {
+    // (the wavefront's floes: lanes past them only help with the pairs)
+    const int lane = (int)(threadIdx.x & 63);
+    const int k0 = (xcd_block() * (int)(blockDim.x >> 6) + (int)(threadIdx.x >> 6)) * floes;
+    const int k = k0 + lane;
     bool qc = false, qb = false, qw = false;
     // every row the search starts from is requested before anything is
     // tested (reads only: harmless for free slots and failed steps)
-    const bool inr = k < S.N;
+    const bool inr = lane < floes && k < S.N;
     GeoRec me;
     CandPre pre;
     if (inr) {
@@ -1190,7 +1232,7 @@ __global__ __launch_bounds__(FLOE_BLOCK) void k_cand(DS S, int lean, int nmember
     }
     extern __shared__ unsigned char cand_lds[];
     const bool act = slot_used & ok;
-    cand_thread<MIXED>(S, k, me, pre, m, act, qc, qb, qw,
+    cand_thread<MIXED>(S, k0, k, me, pre, m, act, qc, qb, qw,
                        cand_lds + (threadIdx.x >> 6) * CAND_LDS_PER_WAVE);
     if (inr && ok && !slot_used) {
         S.ocnt[k] = 0;
@@ -1279,16 +1321,15 @@ __global__ __launch_bounds__(64) void k_sup_dense(DS S) {
 // Contact state of pair (i, j), owner i by storage slot, partner j by
 // identity: history, last contact forces and whether it is bonded.  Returns
 // whether it has a history.
-__device__ __forceinline__ bool load_contact_state(const DS& S, int i, int j, PairState& ps) {
+__device__ __forceinline__ bool load_contact_state(const DS& S, int i, int j, int2 counts, PairState& ps) {
     ps.deltat = 0.0; ps.thetarelc = 0.0; ps.fcn = 0.0; ps.fct = 0.0;
     ps.bond = 0; ps.has_bond_rec = false;
     ps.damage = ps.deltanb = ps.deltatb = ps.trb_ji = ps.trb_ij = 0.0;
     ps.rb = ps.hb = ps.lb = ps.sb = ps.ib = 0.0;
     // both lists are searched at once, the first two records of each
     // requested together
-    const int hc = S.hcnt_old[i], bc = S.bcnt_old[i];
-    const int hq = find_partner<2>(S.hist_old, S.S, i, hc, j);
-    const int bq = find_partner<2>(S.bond_old, S.S, i, bc, j);
+    const int hq = find_partner<2>(S.hist_old, S.S, i, counts.x, j);
+    const int bq = find_partner<2>(S.bond_old, S.S, i, counts.y, j);
     if (hq >= 0) {
         const HistRec& hr = S.hist_old[(int64_t)hq * S.S + i];
         ps.deltat = hr.deltat; ps.thetarelc = hr.thetarelc; ps.fcn = hr.fcn; ps.fct = hr.fct;
@@ -1331,6 +1372,7 @@ __device__ __forceinline__ void contacts(const DS& S, const QueueBlocks& qb, Con
         const bool act = k >= 0;
         const int64_t SS = S.S;
         int m = 0, f = 0, fs = 0, ni = 0, no = 0;
+        uint32_t rc = 0;
         if (act) {
             const GeoRec me = S.geo[k];
             m = me.member;
@@ -1338,6 +1380,7 @@ __device__ __forceinline__ void contacts(const DS& S, const QueueBlocks& qb, Con
             fs = S.cval[k];             // storage slot of the floe's pair state
             ni = S.icnt[k];
             no = S.ocnt[k];
+            rc = S.rcnt[k];
         }
         const int cnt = ni + no;
         int incl = cnt;
@@ -1358,6 +1401,7 @@ __device__ __forceinline__ void contacts(const DS& S, const QueueBlocks& qb, Con
                 if (__shfl(start, own + step) <= idx) own += step;
             const int ko = __shfl(k, own), om = __shfl(m, own), of = __shfl(f, own);
             const int ofs = __shfl(fs, own), oni = __shfl(ni, own), ostart = __shfl(start, own);
+            const uint32_t orc = (uint32_t)__shfl((int)rc, own);
             ContactOut r;
             r.kind = 0;
             if (idx < total) {
@@ -1374,6 +1418,8 @@ __device__ __forceinline__ void contacts(const DS& S, const QueueBlocks& qb, Con
                     const int64_t e = S.ik[(int64_t)local * SS + ko];
                     const int i = ent_id(e), qi = ent_pos(e);
                     const GeoRec gi = S.geo[qi];
+                    const int si = S.cval[qi];
+                    const uint32_t irc = S.rcnt[qi];
                     const double dx = gi.x - gf.x, dy = gi.y - gf.y;
                     const double dn = gi.r + gf.r - sqrt(dx * dx + dy * dy);
                     if (dn > 0) {
@@ -1382,7 +1428,7 @@ __device__ __forceinline__ void contacts(const DS& S, const QueueBlocks& qb, Con
                         Kin kn;
                         kinematics(Fi, Fj, kn);
                         PairState ps;
-                        load_contact_state(S, S.cval[qi], of, ps);
+                        load_contact_state(S, si, of, record_counts(irc), ps);
                         bond_create(P, tstep, i - first, of - first, Fi, Fj, kn, ps);
                         EventOut o;
                         o.flags = 0;
@@ -1404,7 +1450,7 @@ __device__ __forceinline__ void contacts(const DS& S, const QueueBlocks& qb, Con
                     if (!(dn > 0)) {
                         // reset_contact (reset.f90:1-15): the history goes, the
                         // last contact forces stay
-                        const int q = find_partner<2>(S.hist_old, SS, ofs, S.hcnt_old[ofs], j);
+                        const int q = find_partner<2>(S.hist_old, SS, ofs, record_counts(orc).x, j);
                         if (q >= 0) {
                             const HistRec& h0 = S.hist_old[(int64_t)q * SS + ofs];
                             if (h0.fcn != 0.0 || h0.fct != 0.0) {
@@ -1423,7 +1469,7 @@ __device__ __forceinline__ void contacts(const DS& S, const QueueBlocks& qb, Con
                         Kin kn;
                         kinematics(Fi, Fj, kn);
                         PairState ps;
-                        const bool had = load_contact_state(S, ofs, j, ps);
+                        const bool had = load_contact_state(S, ofs, j, record_counts(orc), ps);
                         bond_create(P, tstep, of - first, j - first, Fi, Fj, kn, ps);
                         EventOut o;
                         o.flags = 0;
@@ -1488,11 +1534,13 @@ __device__ __forceinline__ void contacts(const DS& S, const QueueBlocks& qb, Con
         if (act) {
             // contact histories of pairs that are not candidates this step
             // persist (the reference only resets a candidate pair, reset_contact)
-            const int hco = S.hcnt_old[fs];
+            const int hco = record_counts(rc).x;
+            const Peek po = peek_entries(S.oj, SS, k, hco > 0 ? no : 0);
             for (int q = 0; q < hco; ++q) {
                 HistRec hr = S.hist_old[(int64_t)q * SS + fs];
                 if (hr.j < 0) continue;
-                const bool cand = find_entry(S.oj, SS, k, no, hr.j) >= 0;
+                int64_t e;
+                const bool cand = find_peeked(po, S.oj, SS, k, no, hr.j, e) >= 0;
                 if (!cand) {
                     if (nh < S.HC) S.hist_new[(int64_t)nh * SS + fs] = hr, ++nh;
                     else over |= ERR_HIST_CAP;
@@ -1515,15 +1563,17 @@ __device__ __forceinline__ void contacts(const DS& S, const QueueBlocks& qb, Con
 // it (the floes then have bond terms to gather).
 template <bool MIXED>
 __device__ __forceinline__ bool bond_event(const DS& S, const DevParams& P, int tstep, int first,
-                                           int f, int k, int fs, const Floe& F0, int s, int rq,
-                                           int& nb, PairState& ps, uint32_t& over) {
+                                           int f, int k, int fs, const Floe& F0, int s, int64_t e,
+                                           int rq, int& nb, PairState& ps, uint32_t& over) {
     const int64_t SS = S.S;
-    const int64_t e = S.oj[s * SS + k];
     const int j = ent_id(e), qj = ent_pos(e);
     Floe Fi = F0;
     Floe Fj = floe_at(S, qj);
+    const int nij = S.icnt[qj];
     Kin kn;
     kinematics(Fi, Fj, kn);
+    // (the partner's inner list, searched at the end, arrives meanwhile)
+    const Peek pij = peek_entries(S.ik, SS, qj, nij);
     bond_create(P, tstep, f - first, j - first, Fi, Fj, kn, ps);
     if (!ps.has_bond_rec) return false;
     EventOut o;
@@ -1546,7 +1596,8 @@ __device__ __forceinline__ bool bond_event(const DS& S, const DevParams& P, int 
     S.bterm[(int64_t)rq * SS + k] = bt;          // (by the owner's position)
     atomicOr(&S.evf[s * SS + k], EV_BONDED | ((uint32_t)(rq + 1) << 16));   // (as k_contact)
     // tell the partner where its terms are: its inner slot of f
-    const int qi = find_entry(S.ik, SS, qj, S.icnt[qj], f);
+    int64_t eij;
+    const int qi = find_peeked(pij, S.ik, SS, qj, nij, f, eij);
     if (qi >= 0) S.ibond[(int64_t)qi * SS + qj] = rq + 1;
     S.bgat[qj] = 1;
     return true;
@@ -1558,8 +1609,10 @@ __device__ __forceinline__ bool bond_event(const DS& S, const DevParams& P, int 
 template <bool MIXED>
 __device__ __forceinline__ bool bond_record(const DS& S, const DevParams& P, int tstep, int first,
                                             int f, int k, int fs, const Floe& F0, int no,
-                                            const BondRec& b, int rq, int& nb, uint32_t& over) {
-    const int s = find_entry(S.oj, S.S, k, no, b.j);
+                                            const Peek& po, const BondRec& b, int rq, int& nb,
+                                            uint32_t& over) {
+    int64_t e;
+    const int s = find_peeked(po, S.oj, S.S, k, no, b.j, e);
     if (s < 0) {
         S.bond_new[(int64_t)rq * S.S + fs] = b;
         return false;
@@ -1569,7 +1622,7 @@ __device__ __forceinline__ bool bond_record(const DS& S, const DevParams& P, int
     ps.has_bond_rec = true; ps.bond = b.bond; ps.damage = b.damage;
     ps.deltanb = b.deltanb; ps.deltatb = b.deltatb; ps.trb_ji = b.trb_ji; ps.trb_ij = b.trb_ij;
     ps.rb = b.rb; ps.hb = b.hb; ps.lb = b.lb; ps.sb = b.sb; ps.ib = b.ib;
-    return bond_event<MIXED>(S, P, tstep, first, f, k, fs, F0, s, rq, nb, ps, over);
+    return bond_event<MIXED>(S, P, tstep, first, f, k, fs, F0, s, e, rq, nb, ps, over);
 }
 
 // (owner lane, record, new record index) triples of one wavefront, evaluated
@@ -1591,10 +1644,10 @@ __device__ __forceinline__ void bonds(const DS& S, const QueueBlocks& qb, uint32
     const QueueView qv = queue_view(S, 1);
     // (the wavefront loops while any lane has an entry: its lanes share LDS
     // and shuffles)
-    for (int it = 0;; ++it) {
-        const int qt = queue_slot_it(qb, qv.total, it);
-        if (__ballot(qt >= 0) == 0) break;
-        const int k = qt >= 0 ? queue_at(S, 1, qv, qt) : -1;
+    const QueueShare qs = bond_share(qb, qv.total);
+    for (int t0 = qs.begin; t0 < qs.end; t0 += qs.stride) {
+        const int qt = t0 + (int)(threadIdx.x & 63);
+        const int k = qt < min(t0 + qs.floes, qs.end) ? queue_at(S, 1, qv, qt) : -1;
         const bool act = k >= 0;
         const int lane = (int)(threadIdx.x & 63);
         const int64_t SS = S.S;
@@ -1606,7 +1659,7 @@ __device__ __forceinline__ void bonds(const DS& S, const QueueBlocks& qb, uint32
             const GeoRec g = S.geo[k];
             fs = S.cval[k];
             no = S.ocnt[k];
-            bco = S.bcnt_old[fs];
+            bco = record_counts(S.rcnt[k]).y;
             // (a queued owner has at least one record)
 #pragma unroll
             for (int q = 0; q < LIST_PEEK; ++q) id[q] = S.bond_old[(int64_t)min(q, max(bco - 1, 0)) * SS + fs].j;
@@ -1667,8 +1720,9 @@ __device__ __forceinline__ void bonds(const DS& S, const QueueBlocks& qb, uint32
                     const DevParams& P = S.params[mo];
                     const Floe F0 = floe_at(S, ko);
                     const BondRec b = S.bond_old[(int64_t)q * SS + fso];
+                    const Peek po = peek_entries(S.oj, SS, ko, noo);
                     int nb = 0;
-                    if (bond_record<MIXED>(S, P, tso, fro, fo, ko, fso, F0, noo, b, rq, nb, over))
+                    if (bond_record<MIXED>(S, P, tso, fro, fo, ko, fso, F0, noo, po, b, rq, nb, over))
                         S.bgat[ko] = 1;
                 }
             }
@@ -1680,19 +1734,21 @@ __device__ __forceinline__ void bonds(const DS& S, const QueueBlocks& qb, uint32
             const int first = S.members[m].first;
             const int f = me.id;
             const Floe F0 = floe_at(S, k);
+            const Peek po = peek_entries(S.oj, SS, k, no);
             bool any = false;
             int nb = 0;                     // records written so far
             for (int q = 0; q < bco; ++q) {
                 const BondRec b = S.bond_old[q * SS + fs];
                 if (b.j < 0) continue;
                 const int rq = nb++;
-                any |= bond_record<MIXED>(S, P, tstep, first, f, k, fs, F0, no, b, rq, nb, over);
+                any |= bond_record<MIXED>(S, P, tstep, first, f, k, fs, F0, no, po, b, rq, nb, over);
             }
             // bonds that form this step (bond_create), in candidate order, appended
             if (bond_step) {
                 const int nb_old = nb;
                 for (int s = 0; s < no; ++s) {
-                    const int j = ent_id(S.oj[s * SS + k]);
+                    const int64_t e = S.oj[s * SS + k];
+                    const int j = ent_id(e);
                     bool has = false;
                     for (int q = 0; q < nb_old; ++q)
                         if (S.bond_new[(int64_t)q * SS + fs].j == j) { has = true; break; }
@@ -1702,7 +1758,7 @@ __device__ __forceinline__ void bonds(const DS& S, const QueueBlocks& qb, uint32
                     ps.bond = 0; ps.has_bond_rec = false;
                     ps.damage = ps.deltanb = ps.deltatb = ps.trb_ji = ps.trb_ij = 0.0;
                     ps.rb = ps.hb = ps.lb = ps.sb = ps.ib = 0.0;
-                    any |= bond_event<MIXED>(S, P, tstep, first, f, k, fs, F0, s, -1, nb, ps, over);
+                    any |= bond_event<MIXED>(S, P, tstep, first, f, k, fs, F0, s, e, -1, nb, ps, over);
                 }
             }
             if (any) S.bgat[k] = 1;
@@ -2985,8 +3041,8 @@ template __global__ void k_sup<false>(DS);
 template __global__ void k_sup<true>(DS);
 template __global__ void k_sup_dense<false>(DS);
 template __global__ void k_sup_dense<true>(DS);
-template __global__ void k_cand<false>(DS, int, int);
-template __global__ void k_cand<true>(DS, int, int);
+template __global__ void k_cand<false>(DS, int, int, int);
+template __global__ void k_cand<true>(DS, int, int, int);
 template __global__ void k_events<false>(DS, int, int, int);
 template __global__ void k_events<true>(DS, int, int, int);
 template __global__ void k_contact<false>(DS);
