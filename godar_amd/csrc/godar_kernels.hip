@@ -1987,7 +1987,8 @@ template <bool MIXED>
 __global__ __launch_bounds__(REPAIR_THREADS) void k_repair(DS S, int nmembers) {
     __shared__ uint64_t wl[REPAIR_LIST];   // events to evaluate: outer position << 16 | slot
     __shared__ int cl[REPAIR_LIST];        // records that changed
-    __shared__ int nw_, nc_, nn_, rep_, ns_;
+    __shared__ int nw_, nc_, nn_, rep_, ns_, nt_, first_, nmem_, tstep_;
+    __shared__ int64_t mean_;
     __shared__ uint32_t over_;
     // the member's parameters: the physics reads them at LDS latency
     __shared__ uint64_t pbuf[sizeof(DevParams) / 8];
@@ -1995,6 +1996,11 @@ __global__ __launch_bounds__(REPAIR_THREADS) void k_repair(DS S, int nmembers) {
     const int m = blockIdx.x;
     const int tid = (int)threadIdx.x, lane = tid & 63;
     if (m >= nmembers) return;
+    // (the parameters and the mean superset length of the last build are
+    // requested beside the seed count)
+    if (tid >= 64 && tid < 64 + (int)(sizeof(DevParams) / 8))
+        pbuf[tid - 64] = reinterpret_cast<const uint64_t*>(S.params + m)[tid - 64];
+    if (tid == 128) mean_ = 1 + S.sblk[(S.N + SCAN_TILE - 1) / SCAN_TILE] / S.N;
     // (the error word is read once for the block: all its wavefronts take the
     // barriers below or none does)
     if (tid == 0) {
@@ -2003,8 +2009,9 @@ __global__ __launch_bounds__(REPAIR_THREADS) void k_repair(DS S, int nmembers) {
         const Member M = S.members[m];
         ns_ = err || !member_live(M) ? 0 : min(n, S.SEEDK * M.n);
         nn_ = ns_;
-        nw_ = nc_ = rep_ = 0;
+        nw_ = nc_ = rep_ = nt_ = 0;
         over_ = 0;
+        first_ = M.first; nmem_ = M.n; tstep_ = M.tstep;
     }
     __syncthreads();
     const int ns = ns_;
@@ -2015,18 +2022,14 @@ __global__ __launch_bounds__(REPAIR_THREADS) void k_repair(DS S, int nmembers) {
     const int lanes = min(max(S.repair_lanes, 1), 64);
     int waves = 1;
     if (lanes == 64) {
-        const int64_t mean = 1 + S.sblk[(S.N + SCAN_TILE - 1) / SCAN_TILE] / S.N;
-        waves = (int)min((int64_t)(REPAIR_THREADS / 64), ((int64_t)ns * mean + 63) / 64);
+        waves = (int)min((int64_t)(REPAIR_THREADS / 64), ((int64_t)ns * mean_ + 63) / 64);
     }
     const int width = lanes < 64 ? lanes : waves * 64;
     if (tid >= waves * 64) return;
     // records a wavefront takes at once from a list of n
     auto share = [&](int n) { return min(lanes, (n + waves - 1) / waves); };
-    if (tid < (int)(sizeof(DevParams) / 8))
-        pbuf[tid] = reinterpret_cast<const uint64_t*>(S.params + m)[tid];
-    __syncthreads();
     const DevParams& P = *reinterpret_cast<const DevParams*>(pbuf);
-    const int first = S.members[m].first, nmem = S.members[m].n, tstep = S.members[m].tstep;
+    const int first = first_, nmem = nmem_, tstep = tstep_;
     const int64_t SS = S.S;
     Reshape* rec = S.shape + (int64_t)S.SEEDK * first;
     const int reccap = S.SEEDK * nmem;
@@ -2042,6 +2045,14 @@ __global__ __launch_bounds__(REPAIR_THREADS) void k_repair(DS S, int nmembers) {
         if (at < cap) wl[at] = w;
         else if (at - cap < hcap) whbm[at - cap] = w;
         else over |= ERR_REPAIR_CAP;
+    };
+    // floes for the fix-up queue: listed in LDS (the event list's room, which
+    // the rounds have done with) and queued together at the end, two atomics
+    // one behind the other once instead of for every floe
+    auto touch = [&](int k) {
+        const int at = atomicAdd(&nt_, 1);
+        if (at < REPAIR_LIST) wl[at] = (uint64_t)(uint32_t)k;
+        else touch_floe(S, k);
     };
     auto put_change = [&](int p) {
         const int at = atomicAdd(&nc_, 1);
@@ -2237,26 +2248,27 @@ __global__ __launch_bounds__(REPAIR_THREADS) void k_repair(DS S, int nmembers) {
             const int64_t key = rec[p].key;
             kg = rec[p].pos;
             const int kf = rec[p].kf, kj = rec[p].kj;
-            touch_floe(S, kf);
-            if (kj >= 0) touch_floe(S, kj);
+            const bool live = rec[p].live != 0;
+            const int ko = kg == kf ? kj : kf;
+            // (what follows reads, requested at once)
             gg = S.geo[kg];
+            const int h0 = rhead_at(S, kg), h1 = ko >= 0 ? rhead_at(S, ko) : -1;
+            const GeoRec gj = S.geo[max(kj, 0)];
+            const int scnt = S.scnt[kg];
+            soff = S.soff[kg];
+            bown = record_counts(S.rcnt[kg]).y;
+            touch(kf);
+            if (kj >= 0) touch(kj);
             gid = gg.id;
-            const int64_t k0 = first_reshape(rec, rhead_at(S, kg));
-            if (p < ns) {
-                // a seed that is not after a reshape of either floe
-                const int ko = kg == kf ? kj : kf;
-                const int64_t ko0 = ko >= 0 ? first_reshape(rec, rhead_at(S, ko)) : INT64_MAX;
-                if (!(k0 < key) && !(ko0 < key)) ++counted;
-            }
+            const int64_t k0 = first_reshape(rec, h0);
+            // a seed that is not after a reshape of either floe
+            if (p < ns && !(k0 < key) && !(first_reshape(rec, h1) < key)) ++counted;
             // (a floe's walls are its last event)
-            if (rec[p].live && k0 == key && (key & 0xFFFF) != WALL_SLOT) {
+            if (live && k0 == key && (key & 0xFFFF) != WALL_SLOT) {
                 ++counted;           // its walls come after
-                cnt = S.scnt[kg];
-                soff = S.soff[kg];
+                cnt = scnt;
                 fr = (int)(key >> 16);
-                bown = S.bcnt_old[S.cval[kg]];
                 if (kg == kf) {
-                    const GeoRec gj = S.geo[kj];
                     const double dx = gg.x - gj.x, dy = gg.y - gj.y;
                     dr = sqrt(dx * dx + dy * dy);
                     idr = gj.id;
@@ -2281,7 +2293,7 @@ __global__ __launch_bounds__(REPAIR_THREADS) void k_repair(DS S, int nmembers) {
             if (!later) return;
             const ShelRec sh = S.shel[q];
             const int hq = rhead_at(S, q);
-            const int bc = inner ? S.bcnt_old[S.cval[q]] : bo;
+            const int bc = inner ? record_counts(S.rcnt[q]).y : bo;
             // the partner's own reshape may come before the event too: counted
             // from the outer floe's side
             bool both = false;
@@ -2307,11 +2319,12 @@ __global__ __launch_bounds__(REPAIR_THREADS) void k_repair(DS S, int nmembers) {
             const T lim = sizeof(T) == 4 ? T(20) : T(40), dnt = T(dn);
             const bool far = dnt < T(0) && T((double)0.18f) * -dnt >= lim * T(sh.hfa) &&
                              T((double)0.18f) * -dnt >= lim * T(sh.hfw);
-            if (dn > 0 || bc > 0 || (bond_step && dn >= -P.bond_lim) || (P.shelter && !far)) touch_floe(S, q);
+            if (dn > 0 || bc > 0 || (bond_step && dn >= -P.bond_lim) || (P.shelter && !far)) touch(q);
         });
     }
     atomicAdd(&rep_, counted);
     __syncthreads();
+    for (int t = tid; t < min(nt_, REPAIR_LIST); t += waves * 64) touch_floe(S, (int)wl[t]);
     if (tid == 0) {
         S.stats[4 * m + 2] = ns;
         S.stats[4 * m + 3] = rep_;
@@ -2375,6 +2388,51 @@ __device__ __forceinline__ void pair_state_at(const DS& S, int i, const PairRefs
     }
 }
 
+// The touched floes that a reshape changed, one per lane: their walls, with
+// the properties they have when their turn comes, and the properties the step
+// leaves them with.  Wavefront w of nw takes every nw-th share of the queue.
+template <bool MIXED>
+__device__ __forceinline__ void reshaped_floes(const DS& S, const QueueView& qv, int w, int nw) {
+    const int F = min(64, max(1, (qv.total + nw - 1) / nw));
+    for (int t0 = w * F; t0 < qv.total; t0 += nw * F) {
+        const int lane = (int)(threadIdx.x & 63), t = t0 + lane;
+        if (lane >= F || t >= qv.total || *S.err) continue;
+        const int k = queue_at(S, 4, qv, t);
+        const GeoRec me = S.geo[k];
+        const int hk = S.rhead[k], fs = S.cval[k];
+        const uint8_t wf = S.wflag[k];
+        const float nb = S.nb[k];
+        const int m = me.member;
+        if (m < 0 || hk < 0) continue;
+        const int first = S.members[m].first;
+        const Reshape* rec = S.shape + (int64_t)S.SEEDK * first;
+        const DevParams& P = S.params[m];
+        if (wf & WF_WALL) {
+            Floe Fw = floe_at(S, k);
+            floe_at_event(rec, hk, ((int64_t)(me.id - first) << 16) | WALL_SLOT, Fw);
+            double hist[4] = {S.wbc[0 * S.S + fs], S.wbc[1 * S.S + fs], S.wbc[2 * S.S + fs], S.wbc[3 * S.S + fs]};
+            WallOut W;
+            walls<MIXED>(P, Fw, hist, W);
+            if (W.flags & 1u) S.wout[k] = W;
+            else wflag_clear(S, k, WF_WALL);
+        }
+        if (first_reshape(rec, hk) == INT64_MAX) continue;
+        Floe Fn;
+        floe_at_event(rec, hk, INT64_MAX, Fn);
+        S.cur[0 * S.S + fs] = Fn.r; S.cur[1 * S.S + fs] = Fn.h; S.cur[2 * S.S + fs] = Fn.mass;
+        S.cur[3 * S.S + fs] = Fn.inertia; S.cur[4 * S.S + fs] = Fn.hfa; S.cur[5 * S.S + fs] = Fn.hfw;
+        S.dirty[fs] = 1;
+        // drafts that outgrew the floe's bound: its lists may lack a
+        // pair, so the step runs again with a build and more room
+        const double reach = P.shelter ? near_reach(S.near_lim, Fn.hfa, Fn.hfw) : 0.0;
+        if (1.01 * reach > (double)nb) {
+            S.nbmin[fs] = (float)fmin(NEAR_ROOM * reach, 1e30);
+            atomicOr(S.rebuild, BUILD_DUE);
+            set_err(S, ERR_NEED_BUILD);
+        }
+    }
+}
+
 // The floes the repair touched re-gather every event of theirs, in the
 // reference's order (inner pairs by ascending outer index, then their own
 // candidates in distance order), each event with the properties its floes
@@ -2403,8 +2461,16 @@ __global__ __launch_bounds__(FLOE_BLOCK, 2) void k_fixup(DS S) {
     // wavefronts.
     const int lane = (int)(threadIdx.x & 63);
     const QueueView qv = queue_view(S, 4);
-    const int nw = (int)(gridDim.x * blockDim.x) >> 6;
-    const int w = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+    const int waves = (int)(gridDim.x * blockDim.x) >> 6;
+    const int wave = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+    // every eighth wavefront leaves the reshaped floes with their final
+    // properties instead, beside the events (behind them it was a fifth of a
+    // small field's chain of loads)
+    if ((wave & 7) == 7) {
+        reshaped_floes<MIXED>(S, qv, wave >> 3, waves >> 3);
+        return;
+    }
+    const int nw = waves - (waves >> 3), w = wave - (wave >> 3);
     const int F = min(64, max(1, (qv.total + nw - 1) / nw));
     for (int t0 = w * F; t0 < qv.total; t0 += nw * F) {     // (the same for all lanes)
         const int t = t0 + lane;
@@ -2599,37 +2665,6 @@ __global__ __launch_bounds__(FLOE_BLOCK, 2) void k_fixup(DS S) {
 #pragma unroll
             for (int a = 0; a < NACC; ++a) S.acc[a * SS + k] = acc[a];
             S.cls[k] = CLS_CONTACT | CLS_BOND;
-            if (hk >= 0) {
-                const Member Mb = S.members[m];
-                const Reshape* rec = S.shape + (int64_t)S.SEEDK * Mb.first;
-                const DevParams& P = S.params[m];
-                if (S.wflag[k] & WF_WALL) {
-                    // its walls, with the properties it has when their turn comes
-                    Floe Fw = floe_at(S, k);
-                    floe_at_event(rec, hk, ((int64_t)(f - Mb.first) << 16) | WALL_SLOT, Fw);
-                    double hist[4] = {S.wbc[0 * SS + fs], S.wbc[1 * SS + fs], S.wbc[2 * SS + fs], S.wbc[3 * SS + fs]};
-                    WallOut W;
-                    walls<MIXED>(P, Fw, hist, W);
-                    if (W.flags & 1u) S.wout[k] = W;
-                    else wflag_clear(S, k, WF_WALL);
-                }
-                // the properties the step leaves it with
-                if (first_reshape(rec, hk) != INT64_MAX) {
-                    Floe Fn;
-                    floe_at_event(rec, hk, INT64_MAX, Fn);
-                    S.cur[0 * SS + fs] = Fn.r; S.cur[1 * SS + fs] = Fn.h; S.cur[2 * SS + fs] = Fn.mass;
-                    S.cur[3 * SS + fs] = Fn.inertia; S.cur[4 * SS + fs] = Fn.hfa; S.cur[5 * SS + fs] = Fn.hfw;
-                    S.dirty[fs] = 1;
-                    // drafts that outgrew the floe's bound: its lists may lack a
-                    // pair, so the step runs again with a build and more room
-                    const double reach = P.shelter ? near_reach(S.near_lim, Fn.hfa, Fn.hfw) : 0.0;
-                    if (1.01 * reach > (double)S.nb[k]) {
-                        S.nbmin[fs] = (float)fmin(NEAR_ROOM * reach, 1e30);
-                        atomicOr(S.rebuild, BUILD_DUE);
-                        set_err(S, ERR_NEED_BUILD);
-                    }
-                }
-            }
         }
         if (over) set_err(S, over);
     }
