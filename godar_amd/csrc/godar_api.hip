@@ -808,11 +808,13 @@ int godar_create(int64_t max_floes, int32_t max_members, int32_t precision, goda
     *out = nullptr;
     godar_ctx* c = new godar_ctx();
     c->precision = precision;
-    // default block sizes: 256 threads, except the bond and wall stages (64)
-    // and the integration (128);
-    // measured on the 512-field ensemble and the served mix
+    // default block sizes: 256 threads for the build's kernels and contacts
+    // (timed stage by stage), 64 for the search, bonds, walls, fix-up and
+    // stresses, whose few busy wavefronts end sooner on CUs of their own than
+    // four to a CU (1,000 floes: fix-up 20 -> 16 us, stresses 11.4 -> 8.5; the
+    // search 1 to 2% at every size), 128 for the integration
     for (int k = 0; k < GODAR_NSTAGES; ++k) c->sblock[k] = FLOE_BLOCK;
-    c->sblock[5] = c->sblock[7] = 64;
+    for (int k : {3, 5, 7, 9, 10}) c->sblock[k] = 64;
     c->sblock[11] = 128;
     c->S = max_floes;
     c->Mcap = max_members;

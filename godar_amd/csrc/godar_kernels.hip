@@ -2446,9 +2446,9 @@ __device__ __forceinline__ void reshaped_floes(const DS& S, const QueueView& qv,
 // in order, so that a floe with many candidates does not hold one lane
 // through all of them.  It is bound by the chain of loads of one event (queue
 // -> list entry -> rows -> the owner's lists -> records), so each round of
-// that chain requests all it can at once.  (One MI355X: 0.025-0.028 ms with a
-// few to a few thousand touched floes of sparse fields, 0.033 for 24 dense
-// fields, 0.10 when every partner of a reshaped floe was gathered again.)
+// that chain requests all it can at once.  (One MI355X: 0.016 ms for 1,000
+// sparse floes, 0.021 for a few thousand touched ones, 0.017 for 24 dense
+// fields; 0.10 when every partner of a reshaped floe was gathered again.)
 template <bool MIXED>
 __global__ __launch_bounds__(FLOE_BLOCK, 2) void k_fixup(DS S) {
     using T = typename Prec<MIXED>::T;
