@@ -33,6 +33,7 @@ template <bool M> __global__ void k_fixup(DS);
 template <bool M, bool R> __global__ void k_final(DS);
 __global__ void k_totals(DS, int64_t*);
 __global__ void k_status(DS, int, HostStatus*);
+__global__ void k_admit(DS, int, int, int, int, const FloeRec*, const int32_t*);
 template <int W> __global__ void k_read(DS, int, int, int, double*);
 template <int K> __global__ void k_pairs(DS, int, PairOut*, int);
 __global__ void k_take_count(int32_t*, int32_t*);
@@ -396,6 +397,8 @@ int download_members(godar_ctx* c) { return read_status(c); }
 // out while the GPU fills the other.  4 MiB keep a half (2 MiB) above the
 // size where the launch and the wait still count and within a core's caches.
 constexpr size_t STAGE_BYTES = 4u << 20;
+// wind values beyond twice the members' own that the pool may hold
+constexpr int64_t WIND_SLACK = 1 << 16;
 
 int ensure_stage(godar_ctx* c) {
     for (hipEvent_t& e : c->estage)
@@ -1122,42 +1125,49 @@ int godar_member_add(godar_ctx* c, const godar_params* p, int32_t n, const doubl
         };
         for (int i = 0; i < n; ++i)
             key[i] = (uint32_t)(coord(y[i], dp.cell, dp.gy) * dp.gx + coord(x[i], dp.cell, dp.gx));
-        for (int i = 0; i < n; ++i) order[i] = i;
-        std::stable_sort(order.begin(), order.end(),
-                         [&](int32_t a, int32_t b) { return key[a] < key[b]; });
+        // (stable either way: a count per cell unless cells outnumber floes)
+        if (ncell <= 4 * (int64_t)n) {
+            std::vector<int32_t> at(ncell + 1, 0);
+            for (int i = 0; i < n; ++i) ++at[key[i] + 1];
+            for (int32_t k = 0; k < ncell; ++k) at[k + 1] += at[k];
+            for (int i = 0; i < n; ++i) order[at[key[i]]++] = i;
+        } else {
+            for (int i = 0; i < n; ++i) order[i] = i;
+            std::stable_sort(order.begin(), order.end(),
+                             [&](int32_t a, int32_t b) { return key[a] < key[b]; });
+        }
     }
-    // floe state and floe_properties (physics.f90:179-197), as ini_get does
-    std::vector<FloeRec> recs(n);
-    std::vector<int32_t> gid(n), sid(n);
-    for (int t = 0; t < n; ++t) {
-        const int i = order[t];
-        FloeRec& q = recs[t];
-        q.x = x[i]; q.y = y[i]; q.u = u[i]; q.v = v[i]; q.omega = omega[i]; q.theta = theta[i];
-        q.r = r[i]; q.h = h[i];
-        q.mass = dp.rhoice * dp.pi * h[i] * (r[i] * r[i]);
-        q.inertia = 0.5 * q.mass * (r[i] * r[i]);
-        q.hfa = h[i] * (dp.rhowater - dp.rhoice) / dp.rhowater;
-        q.hfw = h[i] * dp.rhoice / dp.rhowater;
-        gid[t] = (int32_t)(first + i);
-        sid[i] = (int32_t)(first + t);
-    }
+    rc = ensure_stage(c);
+    if (rc != GODAR_OK) return rc;
     spill(c);
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    DS& d = c->d;
-    HIPCHK(c, hipMemcpy(d.rec + first, recs.data(), sizeof(FloeRec) * n, hipMemcpyHostToDevice));
-    HIPCHK(c, hipMemcpy(d.gid_of + first, gid.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice));
-    HIPCHK(c, hipMemcpy(d.sid_of + first, sid.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice));
-    c->perm[m] = order;
-    for (int k = 0; k < 4; ++k) HIPCHK(c, hipMemset(d.wbc + k * c->S + first, 0, sizeof(double) * n));
-    for (int k = 0; k < 2; ++k) {
-        HIPCHK(c, hipMemset(c->hcnt[k] + first, 0, sizeof(int32_t) * n));
-        HIPCHK(c, hipMemset(c->bcnt[k] + first, 0, sizeof(int32_t) * n));
+    sync_ds(c);
+    // floe state and floe_properties (physics.f90:179-197), as ini_get does,
+    // in parts that k_admit takes from the staging area
+    const int part = (int)(STAGE_BYTES / 2 / (sizeof(FloeRec) + sizeof(int32_t))) & ~63;
+    for (int b = 0, p = 0; b < n; b += part, ++p) {
+        const int cnt = std::min(part, n - b);
+        FloeRec* recs = reinterpret_cast<FloeRec*>(c->stage + (p & 1) * (STAGE_BYTES / 2));
+        int32_t* ord = reinterpret_cast<int32_t*>(recs + part);
+        // (the half's last part has been taken; the first two wait for
+        // nothing, every call ends with the stream idle)
+        if (p >= 2) HIPCHK(c, hipEventSynchronize(c->estage[p & 1]));
+        for (int t = 0; t < cnt; ++t) {
+            const int i = order[b + t];
+            FloeRec q;
+            q.x = x[i]; q.y = y[i]; q.u = u[i]; q.v = v[i]; q.omega = omega[i]; q.theta = theta[i];
+            q.r = r[i]; q.h = h[i];
+            q.mass = dp.rhoice * dp.pi * h[i] * (r[i] * r[i]);
+            q.inertia = 0.5 * q.mass * (r[i] * r[i]);
+            q.hfa = h[i] * (dp.rhowater - dp.rhoice) / dp.rhowater;
+            q.hfw = h[i] * dp.rhoice / dp.rhowater;
+            recs[t] = q;
+            ord[t] = i;
+        }
+        hipLaunchKernelGGL(k_admit, dim3((cnt + 63) / 64), dim3(64), 0, c->stream, c->d, m, (int)first, b, cnt, recs, ord);
+        HIPCHK(c, hipGetLastError());
+        HIPCHK(c, hipEventRecord(c->estage[p & 1], c->stream));
     }
-    HIPCHK(c, hipMemset(d.dirty + first, 0, n));
-    HIPCHK(c, hipMemset(d.nbmin + first, 0, sizeof(float) * n));
-    HIPCHK(c, hipMemset(d.wnz + first, 0, n));        // wall history rows zeroed above
-    std::vector<int32_t> mo(n, m);
-    HIPCHK(c, hipMemcpy(d.member_of + first, mo.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice));
+    c->perm[m] = std::move(order);
     c->dparams[m] = dp;
     c->rmax[m] = rmax;
     c->members[m].first = (int32_t)first;
@@ -1474,6 +1484,39 @@ int godar_set_forcing(godar_ctx* c, int32_t m, double ua, double va, double uw, 
     return GODAR_OK;
 }
 
+// Once more than half of the wind pool is of no member any more (members that
+// left, winds replaced), the others' winds move together, so that a context
+// that admits and frees members for ever keeps about twice what its members
+// use and not every wind it was ever given.  The stream is idle.
+static int drop_unused_winds(godar_ctx* c) {
+    auto size = [](const WindGridDesc& g) { return (int64_t)2 * g.nxn * g.nyn * g.nframes; };
+    int64_t used = 0;
+    for (int k = 0; k < c->Mcap; ++k)
+        if (c->members[k].active && c->dparams[k].wind_grid >= 0) used += size(c->wgrids[c->dparams[k].wind_grid]);
+    if ((int64_t)c->wpool.size() <= 2 * used + WIND_SLACK) return GODAR_OK;
+    std::vector<WindGridDesc> grids;
+    std::vector<double> pool;
+    pool.reserve((size_t)used);
+    for (int k = 0; k < c->Mcap; ++k) {
+        int32_t& w = c->dparams[k].wind_grid;
+        if (!c->members[k].active || w < 0) continue;
+        WindGridDesc g = c->wgrids[w];
+        const int64_t from = g.offset;
+        g.offset = (int64_t)pool.size();
+        pool.insert(pool.end(), c->wpool.begin() + from, c->wpool.begin() + from + size(g));
+        w = (int32_t)grids.size();
+        grids.push_back(g);
+    }
+    c->wgrids.swap(grids);
+    c->wpool.swap(pool);
+    if (!c->wpool.empty()) {
+        HIPCHK(c, hipMemcpy((void*)c->d.wpool, c->wpool.data(), sizeof(double) * c->wpool.size(), hipMemcpyHostToDevice));
+        HIPCHK(c, hipMemcpy((void*)c->d.wgrids, c->wgrids.data(), sizeof(WindGridDesc) * c->wgrids.size(), hipMemcpyHostToDevice));
+    }
+    HIPCHK(c, hipMemcpy((void*)c->d.params, c->dparams.data(), sizeof(DevParams) * c->Mcap, hipMemcpyHostToDevice));
+    return GODAR_OK;
+}
+
 int godar_set_wind_frames(godar_ctx* c, int32_t m, int32_t nxn, int32_t nyn, double x0, double y0,
                           double dx, double dy, int32_t nframes, double t0, double frame_dt,
                           int32_t disc_average, const double* ua, const double* va) {
@@ -1482,46 +1525,46 @@ int godar_set_wind_frames(godar_ctx* c, int32_t m, int32_t nxn, int32_t nyn, dou
         return fail(c, GODAR_ERR_ARG, "set_wind_frames: bad argument");
     WindGridDesc g;
     g.nxn = nxn; g.nyn = nyn; g.x0 = x0; g.y0 = y0; g.dx = dx; g.dy = dy;
-    g.offset = (int64_t)c->wpool.size();
     g.nframes = nframes; g.avg = disc_average ? 1 : 0;
     g.t0 = t0; g.fdt = nframes > 1 ? frame_dt : 1.0;
     const int64_t cnt = (int64_t)nxn * nyn;
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    int rc = drop_unused_winds(c);
+    if (rc != GODAR_OK) return rc;
+    g.offset = (int64_t)c->wpool.size();
     for (int32_t f = 0; f < nframes; ++f) {
         c->wpool.insert(c->wpool.end(), ua + f * cnt, ua + (f + 1) * cnt);
         c->wpool.insert(c->wpool.end(), va + f * cnt, va + (f + 1) * cnt);
     }
     c->wgrids.push_back(g);
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    if ((int64_t)c->wpool.size() > c->wpool_dev_cap) {
-        double* wp = nullptr;
-        const int64_t cap = std::max<int64_t>((int64_t)c->wpool.size(), 2 * c->wpool_dev_cap);
-        if (dalloc(&wp, cap) != hipSuccess) {
-            (void)hipGetLastError();
-            c->wgrids.pop_back();
-            c->wpool.resize((size_t)g.offset);
-            return fail(c, GODAR_ERR_NOMEM, "set_wind_frames: out of device memory");
-        }
+    int64_t from = g.offset;            // the device's pool holds what is before
+    double* wp = nullptr;
+    WindGridDesc* wg = nullptr;
+    const int64_t pcap = std::max<int64_t>((int64_t)c->wpool.size(), 2 * c->wpool_dev_cap);
+    const int gcap = std::max<int>((int)c->wgrids.size(), 2 * c->wgrids_dev_cap);
+    const bool grow_p = (int64_t)c->wpool.size() > c->wpool_dev_cap, grow_g = (int)c->wgrids.size() > c->wgrids_dev_cap;
+    if ((grow_p && dalloc(&wp, pcap) != hipSuccess) || (grow_g && dalloc(&wg, gcap) != hipSuccess)) {
+        dfree(wp); dfree(wg);
+        (void)hipGetLastError();
+        c->wgrids.pop_back();
+        c->wpool.resize((size_t)g.offset);
+        return fail(c, GODAR_ERR_NOMEM, "set_wind_frames: out of device memory");
+    }
+    if (grow_p) {
         double* old = const_cast<double*>(c->d.wpool);
         dfree(old);
         c->d.wpool = wp;
-        c->wpool_dev_cap = cap;
+        c->wpool_dev_cap = pcap;
+        from = 0;
     }
-    if ((int)c->wgrids.size() > c->wgrids_dev_cap) {
-        WindGridDesc* wg = nullptr;
-        const int cap = std::max<int>((int)c->wgrids.size(), 2 * c->wgrids_dev_cap);
-        if (dalloc(&wg, cap) != hipSuccess) {
-            (void)hipGetLastError();
-            c->wgrids.pop_back();
-            c->wpool.resize((size_t)g.offset);
-            return fail(c, GODAR_ERR_NOMEM, "set_wind_frames: out of device memory");
-        }
+    if (grow_g) {
         WindGridDesc* old = const_cast<WindGridDesc*>(c->d.wgrids);
         dfree(old);
         c->d.wgrids = wg;
-        c->wgrids_dev_cap = cap;
+        c->wgrids_dev_cap = gcap;
     }
-    HIPCHK(c, hipMemcpy((void*)c->d.wpool, c->wpool.data(), sizeof(double) * c->wpool.size(),
-                        hipMemcpyHostToDevice));
+    HIPCHK(c, hipMemcpy((void*)(c->d.wpool + from), c->wpool.data() + from,
+                        sizeof(double) * (c->wpool.size() - from), hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy((void*)c->d.wgrids, c->wgrids.data(), sizeof(WindGridDesc) * c->wgrids.size(),
                         hipMemcpyHostToDevice));
     c->dparams[m].wind_grid = (int32_t)c->wgrids.size() - 1;

@@ -3047,6 +3047,28 @@ __global__ void k_pairs(DS S, int m, PairOut* out, int cap) {
     }
 }
 
+// Floes [b, b + count) in storage order of a new member m from storage slot
+// `first` on: their records and their indices in the caller's arrays, from
+// pinned host memory, and empty pair and wall state (one launch for eleven
+// clears and four copies, each of which waited: adding 5,000 floes 0.70 ->
+// 0.15 ms).
+__global__ __launch_bounds__(64) void k_admit(DS S, int m, int first, int b, int count, const FloeRec* recs,
+                                              const int32_t* order) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= count) return;
+    const int f = first + b + t, id = first + order[t];
+    S.rec[f] = recs[t];
+    S.gid_of[f] = id;
+    S.sid_of[id] = f;
+    S.member_of[f] = m;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) S.wbc[k * S.S + f] = 0.0;
+    S.hcnt_old[f] = S.hcnt_new[f] = S.bcnt_old[f] = S.bcnt_new[f] = 0;
+    S.nbmin[f] = 0.0f;
+    S.dirty[f] = 0;
+    S.wnz[f] = 0;                  // (the wall history rows are all +0.0)
+}
+
 // The pair count to the host, and back to 0 for the next list.
 __global__ void k_take_count(int32_t* n, int32_t* out) {
     *out = *n;

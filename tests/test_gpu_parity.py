@@ -623,6 +623,64 @@ def test_search_takes_floes_in_groups(n):
     ctx.close()
 
 
+@pytest.mark.parametrize("n", [1, 20928, 62789])
+def test_member_add_in_parts(n):
+    """A member's floes reach the device as given, whatever their order, where
+    the staging area takes them in one part, just fills one, and takes a fourth
+    (which waits for a half to be free again), beside another member and in the
+    slots of one that was removed."""
+    rng = np.random.default_rng(n)
+    mate = g.config0_member(52, 100)
+    keys = ["x", "y", "r", "h", "theta", "omega", "u", "v"]
+    ctx = _ctx(2 * n + mate.n, 3)
+    pm = config0_params(mate)
+    a = ctx.add_field(pm, mate)
+    for rep in range(2):
+        v = {k: rng.uniform(1.0, 1e5 if k in "xy" else 2.0, n) for k in keys}
+        p = config0_params(mate, nx=1e5, ny=1e5)
+        m = ctx.add(p, *[v[k] for k in keys])
+        got = ctx.floes(m)
+        for k in keys:
+            assert np.array_equal(got[k], v[k]), (rep, k)
+        assert np.array_equal(got["mass"], p.rhoice * np.pi * v["h"] * (v["r"] * v["r"]))
+        assert np.array_equal(ctx.floes(a)["x"], mate.x)
+        ctx.remove(m)
+    ctx.close()
+
+
+def test_winds_of_members_that_left_are_dropped():
+    """Members come and go, each with a gridded wind of 2 x 72 x 72 values (the
+    pool drops unused ones past 65,536): two members that stay, with winds of
+    their own, and each of the guests take the steps they take alone."""
+    def wind(seed, n=72):
+        rng = np.random.default_rng(seed)
+        return g.WindGrid(rng.normal(5, 3, (n, n)), rng.normal(0, 3, (n, n)), 0.0, 0.0, 1000.0, 1000.0)
+    stay = [g.config0_member(61 + k, 60) for k in range(2)]
+    guest = g.config0_member(70, 50)
+    alone = []
+    for k, f in enumerate(stay + [guest]):
+        f.wind_grid = wind(k)
+        c = _ctx(f.n)
+        m = c.add_field(config0_params(f), f)
+        c.step(4 if f is guest else 48)
+        alone.append(c.floes(m))
+        c.close()
+    ctx = _ctx(sum(f.n for f in stay) + guest.n, 3)
+    ms = [ctx.add_field(config0_params(f), f) for f in stay]
+    for _ in range(12):
+        m = ctx.add_field(config0_params(guest), guest)
+        ctx.step(4)
+        got = ctx.floes(m)
+        for k in STATE:
+            assert np.array_equal(got[k], alone[2][k]), k
+        ctx.remove(m)
+    for m, want in zip(ms, alone):
+        got = ctx.floes(m)
+        for k in STATE:
+            assert np.array_equal(got[k], want[k]), k
+    ctx.close()
+
+
 def test_checkpoint_restore_continues_exactly():
     """A member restored from a checkpoint (floes, walls, contact histories
     with last contact forces, bond strain state, step number) continues
