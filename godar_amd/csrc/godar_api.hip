@@ -154,9 +154,9 @@ struct godar_ctx {
     std::vector<double> rmax;           // largest radius of each member when it was added
     int64_t sup_cap = 0;                // superset pool entries
     int32_t built_qseg = -1;            // queue share the dense list was built with
-    // captured step graphs by [parity][lean]
-    hipGraphExec_t gexec[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
-    std::vector<unsigned char> gsig[2][2];
+    // captured graphs of the step with the build kernels, by parity
+    hipGraphExec_t gexec[2] = {nullptr, nullptr};
+    std::vector<unsigned char> gsig[2];
     // Steps without a build launch no build kernels (lean steps): the host
     // launches the full sequence when it forced a build or refresh itself,
     // after LEAN_RUN lean steps in a row (the device builds early there once
@@ -725,26 +725,29 @@ std::vector<unsigned char> launch_signature(godar_ctx* c) {
 }
 
 void drop_graphs(godar_ctx* c) {
-    for (int k = 0; k < 2; ++k)
-        for (int l = 0; l < 2; ++l) {
-            if (c->gexec[k][l]) (void)hipGraphExecDestroy(c->gexec[k][l]);
-            c->gexec[k][l] = nullptr;
-            c->gsig[k][l].clear();
-        }
+    for (int k = 0; k < 2; ++k) {
+        if (c->gexec[k]) (void)hipGraphExecDestroy(c->gexec[k]);
+        c->gexec[k] = nullptr;
+        c->gsig[k].clear();
+    }
 }
 
-// One step as a replay of the captured graph of the current parity; the
-// graph is (re)captured when the launch signature changed.
-int graph_step(godar_ctx* c, bool lean) {
+// One step with the build kernels as a replay of the captured graph of the
+// current parity; the graph is (re)captured when the launch signature
+// changed.  (The steps without them are five launches, which a replay made 3
+// to 9% of a step slower: 1,000 floes 64.6 -> 59.6 us a step launched one by
+// one, 24 members of 2,700 floes 87 -> 78, 24 power-law requests 150 -> 147;
+// nor do they need two captures of their own each time members change.)
+int graph_step(godar_ctx* c) {
     if (c->N_used == 0) return GODAR_OK;
-    const int par = c->parity, l = lean ? 1 : 0;
+    const int par = c->parity;
     std::vector<unsigned char> sig = launch_signature(c);
-    if (!c->gexec[par][l] || sig != c->gsig[par][l]) {
-        if (c->gexec[par][l]) (void)hipGraphExecDestroy(c->gexec[par][l]);
-        c->gexec[par][l] = nullptr;
-        c->gsig[par][l].clear();
+    if (!c->gexec[par] || sig != c->gsig[par]) {
+        if (c->gexec[par]) (void)hipGraphExecDestroy(c->gexec[par]);
+        c->gexec[par] = nullptr;
+        c->gsig[par].clear();
         HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-        int rc = launch_step(c, lean);
+        int rc = launch_step(c, false);
         hipGraph_t g = nullptr;
         hipError_t e = hipStreamEndCapture(c->stream, &g);
         c->parity = par;   // the captured step has not run yet
@@ -758,10 +761,10 @@ int graph_step(godar_ctx* c, bool lean) {
         e = hipGraphInstantiate(&x, g, nullptr, nullptr, 0);
         (void)hipGraphDestroy(g);
         HIPCHK(c, e);
-        c->gexec[par][l] = x;
-        c->gsig[par][l] = std::move(sig);
+        c->gexec[par] = x;
+        c->gsig[par] = std::move(sig);
     }
-    HIPCHK(c, hipGraphLaunch(c->gexec[par][l], c->stream));
+    HIPCHK(c, hipGraphLaunch(c->gexec[par], c->stream));
     c->parity ^= 1;
     return GODAR_OK;
 }
@@ -1921,7 +1924,7 @@ int godar_step_async(godar_ctx* c, int32_t nsteps) {
             c->built_qseg = q;
         }
         const bool lean = !c->need_full && c->full_hold == 0 && c->lean_run < LEAN_RUN;
-        int rc = graphs ? graph_step(c, lean) : launch_step(c, lean);
+        int rc = graphs && !lean ? graph_step(c) : launch_step(c, lean);
         if (rc != GODAR_OK) return rc;
         c->need_full = false;
         c->lean_run = lean ? c->lean_run + 1 : 0;

@@ -220,7 +220,8 @@ class Context:
         return self.stage_blocks()
 
     def use_graphs(self, on: bool = True):
-        """Replay a captured HIP graph per step (default) or launch kernels one by one."""
+        """Replay a captured HIP graph for the steps that launch the build kernels
+        (default) or launch every kernel one by one."""
         self._chk(self.L.godar_use_graphs(self.h, int(bool(on))))
 
     def graphs_on(self) -> bool:

@@ -263,10 +263,11 @@ int godar_get_stage_blocks(const godar_ctx *ctx, int32_t *threads);   /* GODAR_N
  * the search shape and 4 (1 + max(32, 16 trial)) for the launch mode. */
 int godar_autotune(godar_ctx *ctx, int32_t trial);
 /* Step launch mode (no counterpart in the reference): on (the default), each
- * step replays a captured HIP graph of the whole kernel sequence, recaptured
- * whenever members, capacities or the block size change; off, the kernels are
- * launched one by one.  Results are identical.  Steps timed by godar_profile
- * are always launched one by one. */
+ * step with the build kernels (about 20 launches) replays a captured HIP graph
+ * of its kernel sequence, recaptured whenever members, capacities or the block
+ * size change, and the other steps, five launches, are launched one by one;
+ * off, every kernel is launched one by one.  Results are identical.  Steps
+ * timed by godar_profile are always launched one by one. */
 int godar_use_graphs(godar_ctx *ctx, int32_t on);
 int godar_graphs_on(const godar_ctx *ctx, int32_t *on);   /* the current launch mode */
 
