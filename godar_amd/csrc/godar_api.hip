@@ -159,12 +159,21 @@ struct godar_ctx {
     std::vector<unsigned char> gsig[2];
     // Steps without a build launch no build kernels (lean steps): the host
     // launches the full sequence when it forced a build or refresh itself,
-    // after LEAN_RUN lean steps in a row (the device builds early there once
-    // a floe has moved 0.3 skin), and for a while after a lean step found a
-    // build due (ERR_NEED_BUILD; godar_sync runs such steps again).
+    // when the last godar_sync found one due or near (a floe past 0.3 skin),
+    // after a run of lean steps in one go that grows with the steps since the
+    // last build (godar_step_async), and for a while after a lean step found a
+    // build due (ERR_NEED_BUILD; godar_sync runs such steps again).  (The 16
+    // build kernels of a full step that builds nothing take 70 us: with one
+    // such step in 16, 1,000 power-law floes took 51 us a step, without 45; 64
+    // floes called step by step 4% longer.)
     bool need_full = true;
     int lean_run = 0;                   // lean steps since the last full one
     int full_hold = 0;                  // full steps still to launch after a missed build
+    // as of the last godar_sync: a build or refresh is due or comes near, the
+    // builds so far, the steps since the last of them
+    bool soon = false;
+    int32_t builds = 0;
+    int64_t since_build = 0;
     int64_t pend_launched = 0;          // steps launched since the last sync
     int device = 0;                     // the GPU the context lives on
     int ncu = 256;                      // its compute units
@@ -598,7 +607,8 @@ static dim3 grid_queue(int N, int B) {
     return dim3(std::max(XCD_COUNT, std::min((int)g.x, cap)));
 }
 
-constexpr int LEAN_RUN = 15;       // lean steps between two full ones
+constexpr int LEAN_RUN = 15;       // lean steps between two full ones, at least
+constexpr int LEAN_RUN_MAX = 255;  // and at most
 constexpr int FULL_HOLD = 64;      // full steps after a lean step found a build due
 
 int launch_step(godar_ctx* c, bool lean) {
@@ -908,7 +918,7 @@ int godar_create(int64_t max_floes, int32_t max_members, int32_t precision, goda
     ACHK(dalloc(&d.soff, S));
     ACHK(dalloc(&d.sblk, S / SCAN_TILE + 2));
     ACHK(dalloc(&d.x0, S));
-    ACHK(dalloc(&d.rebuild, 3));
+    ACHK(dalloc(&d.rebuild, 4));
     ACHK(radix_alloc(c->rs, S));
 #undef ACHK
     (void)hipMemsetAsync(d.err, 0, sizeof(uint32_t), c->stream);
@@ -921,7 +931,7 @@ int godar_create(int64_t max_floes, int32_t max_members, int32_t precision, goda
     for (int k = 0; k < 2; ++k)
         (void)hipMemsetAsync(c->qn[k], 0, sizeof(int32_t) * NQUEUE * XCD_COUNT * QN_STRIDE, c->stream);
     hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, c->stream, d.rebuild, 2, 1);
-    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, c->stream, d.rebuild + 2, 1, 0);
+    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, c->stream, d.rebuild + 2, 2, 0);
     (void)hipMemsetAsync(d.dirty, 0, (S + 3) / 4 * 4, c->stream);
     (void)hipMemsetAsync(d.wnz, 1, S, c->stream);
     (void)hipMemsetAsync(d.stats, 0, sizeof(int64_t) * 4 * max_members, c->stream);
@@ -1915,6 +1925,10 @@ int godar_step_async(godar_ctx* c, int32_t nsteps) {
         c->pend_launched = 0;
     }
     const bool graphs = c->use_graphs && !c->prof;
+    // a run of lean steps ends in a full one that builds early if it must: no
+    // floe has moved 0.3 skin in the steps since the last build, and a fifth as
+    // many more keep one that speeds up steadily from rest below 0.45
+    const int run = (int)std::min<int64_t>(std::max<int64_t>(c->since_build / 5, LEAN_RUN), LEAN_RUN_MAX);
     for (int k = 0; k < nsteps; ++k) {
         // the dense-search list is laid out by the candidate search's XCD
         // shares: a new block size or floe count needs a build
@@ -1923,10 +1937,10 @@ int godar_step_async(godar_ctx* c, int32_t nsteps) {
             force_rebuild(c);
             c->built_qseg = q;
         }
-        const bool lean = !c->need_full && c->full_hold == 0 && c->lean_run < LEAN_RUN;
+        const bool lean = !c->need_full && !c->soon && c->full_hold == 0 && c->lean_run < run;
         int rc = graphs && !lean ? graph_step(c) : launch_step(c, lean);
         if (rc != GODAR_OK) return rc;
-        c->need_full = false;
+        c->need_full = c->soon = false;
         c->lean_run = lean ? c->lean_run + 1 : 0;
         if (c->full_hold > 0 && !lean) --c->full_hold;
         ++c->pend_launched;
@@ -1955,6 +1969,10 @@ int godar_sync(godar_ctx* c) {
     collect_events(c);
     const uint32_t e = c->status->err;
     const int64_t now = c->status->steps_done;
+    c->since_build = c->status->builds == c->builds ? c->since_build + now - c->done : 0;
+    c->builds = c->status->builds;
+    c->soon = c->status->due != 0;
+    if (!c->soon) c->lean_run = 0;
     c->done = now;
     bool was_pending = c->pending;
     c->pending = false;

@@ -142,8 +142,8 @@ struct DS {
     int64_t* soff;             // [S] by pos
     int64_t* sblk;             // [S / SCAN_TILE + 2] scan of per-tile totals
     double2* x0;               // [S] by pos (positions stand between builds)
-    int32_t* rebuild;          // [3] 0: build the supersets; 1: refresh the ordered copies;
-                               //     2: the copies are newer than rec
+    int32_t* rebuild;          // [4] 0: build the supersets; 1: refresh the ordered copies;
+                               //     2: the copies are newer than rec; 3: builds so far
     // Work queues (contact, bond, wall, dense search, fixup), each in XCD_COUNT
     // segments: the candidate search's blocks on XCD x cover positions
     // [x qseg, (x+1) qseg) and queue them into segment x, at
@@ -177,6 +177,8 @@ struct DS {
 struct HostStatus {
     int64_t steps_done;
     uint32_t err;
+    int32_t due;               // rebuild[0] | rebuild[1]
+    int32_t builds;
     int32_t npairs;            // the last pair list's length (k_take_count)
     __host__ __device__ Member* members() { return reinterpret_cast<Member*>(this + 1); }
     static size_t bytes(int nmembers) { return sizeof(HostStatus) + sizeof(Member) * nmembers; }

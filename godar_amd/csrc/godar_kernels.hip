@@ -465,7 +465,10 @@ __global__ void k_begin(DS S, int nmembers) {
     const bool newer = S.rebuild[2] != 0;
     if (i < NQUEUE * XCD_COUNT) S.qn[i * QN_STRIDE] = 0;
     if (build && i <= S.ncells) S.crange[i] = make_int2(0, 0);
-    if (build && i == 0) *S.nearsum = 0;
+    if (build && i == 0) {
+        *S.nearsum = 0;
+        ++S.rebuild[3];
+    }
     member_resets(S, i, (int)(gridDim.x * blockDim.x), nmembers);
     if (i >= S.N) return;
     if (newer && (build || refresh)) {
@@ -3080,6 +3083,8 @@ __global__ void k_status(DS S, int nmembers, HostStatus* out) {
     if (threadIdx.x == 0) {
         out->steps_done = *S.steps_done;
         out->err = *S.err;
+        out->due = S.rebuild[0] | S.rebuild[1];
+        out->builds = S.rebuild[3];
     }
     const int32_t* src = reinterpret_cast<const int32_t*>(S.members);
     int32_t* dst = reinterpret_cast<int32_t*>(out->members());

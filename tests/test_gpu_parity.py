@@ -623,6 +623,34 @@ def test_search_takes_floes_in_groups(n):
     ctx.close()
 
 
+@pytest.mark.parametrize("batch", [1, 7, 100, 600])
+def test_lean_runs_do_not_change_the_steps(batch):
+    """However many steps a call takes, and so however many go by between two
+    looks at whether the supersets need building: 600 steps of floes that start
+    from rest under a strong wind (the longest lean runs come just before the
+    builds become frequent) and of floes that move from the start equal those
+    with a build at every step (skin 0)."""
+    fields = [g.config0_member(81, 120), kick(g.config0_member(82, 90), 2, speed=3.0)]
+    fields[0].wind = (60.0, 20.0)
+    want = None
+    for skin, nb in ((0.0, 600), (0.02, batch)):
+        ctx = _ctx(sum(f.n for f in fields), 2)
+        ctx.set_skin(skin)
+        ms = [ctx.add_field(config0_params(f), f) for f in fields]
+        left = 600
+        while left > 0:
+            ctx.step(min(nb, left))
+            left -= nb
+        got = [ctx.floes(m) for m in ms]
+        ctx.close()
+        if want is None:
+            want = got
+            continue
+        for a, b in zip(got, want):
+            for k in STATE:
+                assert np.array_equal(a[k], b[k]), k
+
+
 @pytest.mark.parametrize("n", [1, 20928, 62789])
 def test_member_add_in_parts(n):
     """A member's floes reach the device as given, whatever their order, where
