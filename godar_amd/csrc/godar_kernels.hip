@@ -294,8 +294,13 @@ __device__ __forceinline__ int cell_coord(double p, double cell, int g) {
 
 // Old pair state of (i, j): owner i by storage slot, partner j by identity.
 // Lists are searched with their first LIST_PEEK entries read at once (a
-// floe's lists are short): one round of loads instead of one per entry.
-constexpr int LIST_PEEK = 4;
+// floe's lists are short): one round of loads instead of one per entry.  Two:
+// with four, most loads of a sparse field repeat a list's last entry, 64
+// scattered lines each (512 members of 2,700 floes: events 190 -> 181 us).
+constexpr int LIST_PEEK = 2;
+// The bond gather reads both sides' words of a floe: with two, k_final waits
+// for a second round in most wavefronts (114 -> 118 us there).
+constexpr int GATHER_PEEK = 4;
 
 // Index of the first of owner i's n records (slot-major rows of stride SS)
 // whose partner is j (j >= 0; empty records hold -1), or -1.
@@ -1792,14 +1797,14 @@ __device__ __forceinline__ void bonds(const DS& S, const QueueBlocks& qb, uint32
 // repair left alone: their flags and terms are k_bond's.
 __device__ __forceinline__ void gather_bonds(const DS& S, int k, int ni, int no, double* a) {
     const int64_t SS = S.S;
-    // the first LIST_PEEK slots' bond words and inner partners of both sides
+    // the first GATHER_PEEK slots' bond words and inner partners of both sides
     // are requested together (slots past a count stand in for its last one)
-    int rqi[LIST_PEEK], rqo[LIST_PEEK], pki[LIST_PEEK];
+    int rqi[GATHER_PEEK], rqo[GATHER_PEEK], pki[GATHER_PEEK];
 #pragma unroll
-    for (int q = 0; q < LIST_PEEK; ++q) rqi[q] = rqo[q] = pki[q] = 0;
+    for (int q = 0; q < GATHER_PEEK; ++q) rqi[q] = rqo[q] = pki[q] = 0;
     if (ni > 0) {
 #pragma unroll
-        for (int q = 0; q < LIST_PEEK; ++q) {
+        for (int q = 0; q < GATHER_PEEK; ++q) {
             const int64_t r = (int64_t)min(q, ni - 1) * SS + k;
             rqi[q] = S.ibond[r];
             pki[q] = ent_pos(S.ik[r]);
@@ -1807,10 +1812,10 @@ __device__ __forceinline__ void gather_bonds(const DS& S, int k, int ni, int no,
     }
     if (no > 0) {
 #pragma unroll
-        for (int q = 0; q < LIST_PEEK; ++q) rqo[q] = (int)S.evf[(int64_t)min(q, no - 1) * SS + k];
+        for (int q = 0; q < GATHER_PEEK; ++q) rqo[q] = (int)S.evf[(int64_t)min(q, no - 1) * SS + k];
     }
 #pragma unroll
-    for (int q = 0; q < LIST_PEEK; ++q) {
+    for (int q = 0; q < GATHER_PEEK; ++q) {
         rqi[q] = q < ni ? rqi[q] : 0;
         rqo[q] = q < no ? rqo[q] : 0;
     }
@@ -1822,11 +1827,11 @@ __device__ __forceinline__ void gather_bonds(const DS& S, int k, int ni, int no,
         if ((fl & EV_BONDED) && rq >= 1 && rq <= S.BC) add_bond_i(a, S.bterm[(int64_t)(rq - 1) * SS + k]);
     };
 #pragma unroll
-    for (int q = 0; q < LIST_PEEK; ++q) inner(pki[q], rqi[q]);
-    for (int q = LIST_PEEK; q < ni; ++q) inner(ent_pos(S.ik[q * SS + k]), S.ibond[q * SS + k]);
+    for (int q = 0; q < GATHER_PEEK; ++q) inner(pki[q], rqi[q]);
+    for (int q = GATHER_PEEK; q < ni; ++q) inner(ent_pos(S.ik[q * SS + k]), S.ibond[q * SS + k]);
 #pragma unroll
-    for (int s = 0; s < LIST_PEEK; ++s) outer((uint32_t)rqo[s]);
-    for (int s = LIST_PEEK; s < no; ++s) outer(S.evf[s * SS + k]);
+    for (int s = 0; s < GATHER_PEEK; ++s) outer((uint32_t)rqo[s]);
+    for (int s = GATHER_PEEK; s < no; ++s) outer(S.evf[s * SS + k]);
 }
 
 // Walls of the queued floes (verify_bc, boundaries.f90:1-97).
