@@ -575,6 +575,7 @@ __global__ void k_ranges(DS S) {
             if (P.cohesion) nb = fmax(nb, P.bond_lim);
             nb = fmax(nb, (double)S.nbmin[f]) * (1.0 + 1e-6);
             S.nb[k] = nb < 1e30 ? (float)nb : SUP_KEEP;
+            S.rcnt[k] = (uint32_t)S.hcnt_old[f] | ((uint32_t)S.bcnt_old[f] << 16);
             const uint32_t key = S.ckey[k];
             if (k == 0 || S.ckey[k - 1] != key) S.crange[key].x = k;
             if (k == S.N - 1 || S.ckey[k + 1] != key) S.crange[key].y = k + 1;
@@ -644,15 +645,17 @@ constexpr int SCAN_BATCH = 4;
 // many events a reshape came before (k_repair).  A reshape whose drafts
 // outgrow their room ends the step, which is run again with a build and more
 // room (k_fixup).
-__device__ __forceinline__ bool has_records(const DS& S, int i, int j) {
-    const int hc = S.hcnt_old[i], bc = S.bcnt_old[i];
-    if (hc == 0 && bc == 0) return false;
-    return find_partner(S.hist_old, S.S, i, hc, j) >= 0 || find_partner(S.bond_old, S.S, i, bc, j) >= 0;
+__device__ __forceinline__ bool has_records(const DS& S, int i, uint32_t rc, int j) {
+    const int2 n = record_counts(rc);
+    return find_partner(S.hist_old, S.S, i, n.x, j) >= 0 || find_partner(S.bond_old, S.S, i, n.y, j) >= 0;
 }
-// bound of the pair of floe f (storage slot fs, bound nbf) and floe j at q
-__device__ __forceinline__ float sup_bound_of(const DS& S, int f, int fs, float nbf, int j, int q) {
-    const bool keep = j > f ? has_records(S, fs, j) : has_records(S, S.cval[q], f);
-    return keep ? SUP_KEEP : fmaxf(nbf, S.nb[q]);
+// bound of the pair of floe f (storage slot fs, bound nbf, record counts rcf)
+// and floe j at q (bound nbq, record counts rcq)
+__device__ __forceinline__ float sup_bound_of(const DS& S, int f, int fs, float nbf, uint32_t rcf, int j,
+                                              int q, float nbq, uint32_t rcq) {
+    const bool keep = j > f ? rcf != 0 && has_records(S, fs, rcf, j)
+                            : rcq != 0 && has_records(S, S.cval[q], rcq, f);
+    return keep ? SUP_KEEP : fmaxf(nbf, nbq);
 }
 
 // Candidate superset of one floe by one thread over its (2 SPAN + 1)^2 cell
@@ -700,6 +703,7 @@ __device__ __forceinline__ int2 sup_thread(const DS& S, int k, const GeoRec& me,
     const double rad = me.r + P.rtree + P.skin, reach = P.rtree + P.skin;
     const int fs = S.cval[k];
     const float nbme = S.nb[k];
+    const uint32_t rcme = S.rcnt[k];
     int n = 0, nn = 0;
     for (int v0 = 0; v0 < L; v0 += SCAN_BATCH) {
         GeoRec g[SCAN_BATCH];
@@ -726,7 +730,7 @@ __device__ __forceinline__ int2 sup_thread(const DS& S, int k, const GeoRec& me,
             // a superset: the margin only adds entries
             const double d2 = dx * dx + dy * dy;
             if (d2 <= thr * thr * (1.0 + 1e-12)) {
-                const float bound = sup_bound_of(S, f, fs, nbme, g[u].id, q);
+                const float bound = sup_bound_of(S, f, fs, nbme, rcme, g[u].id, q, S.nb[q], S.rcnt[q]);
                 const double w = me.r + g[u].r + (double)bound + P.skin;
                 const bool near = d2 <= w * w * (1.0 + 1e-12);
                 if (FILL) out[near ? nn : snear + n - nn] = sup_ent(bound, q);
@@ -1149,7 +1153,6 @@ __global__ __launch_bounds__(FLOE_BLOCK) void k_sup(DS S) {
     if (!*S.rebuild || *S.err) return;
     const int k = xcd_block() * blockDim.x + threadIdx.x;
     bool qd = false;
-    int n = 0;
     if (k < S.N) {
         const GeoRec me = S.geo[k];
         if (me.member < 0) {
@@ -1167,16 +1170,11 @@ __global__ __launch_bounds__(FLOE_BLOCK) void k_sup(DS S) {
                 const int2 c = P.span == 2 ? sup_thread<2, false>(S, k, me, P, nullptr, 0)
                                            : sup_thread<1, false>(S, k, me, P, nullptr, 0);
                 S.scnt[k] = c.x;
-                S.snear[k] = n = c.y;
+                S.snear[k] = c.y;
             }
         }
     }
-    if (!FILL) {
-        enqueue(S, qd, 3, k);
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off);
-        if ((threadIdx.x & 63) == 0 && n) atomicAdd((unsigned long long*)S.nearsum, (unsigned long long)n);
-    }
+    if (!FILL) enqueue(S, qd, 3, k);
 }
 
 // Superset offsets: per-tile totals, their exclusive scan (one workgroup;
@@ -1199,11 +1197,21 @@ __device__ __forceinline__ int64_t block_exclusive_scan(int64_t v, int64_t* tmp,
 
 __global__ __launch_bounds__(SCAN_TILE) void k_scan_tiles(DS S) {
     __shared__ int64_t tmp[SCAN_TILE];
+    __shared__ int near;
     if (!*S.rebuild || *S.err) return;
     const int k = blockIdx.x * SCAN_TILE + threadIdx.x;
+    if (threadIdx.x == 0) near = 0;
     int64_t tot;
     block_exclusive_scan(k < S.N ? S.scnt[k] : 0, tmp, tot);
-    if (threadIdx.x == 0) S.sblk[blockIdx.x] = tot;
+    // the near entries' sum: one global atomic per tile (one per wavefront of
+    // the counting kernels, 8,192 on one word, took 60 us by themselves)
+    const int sum = wave_last(wave_scan(k < S.N ? S.snear[k] : 0));
+    if ((threadIdx.x & 63) == 0) atomicAdd(&near, sum);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        S.sblk[blockIdx.x] = tot;
+        atomicAdd((unsigned long long*)S.nearsum, (unsigned long long)near);
+    }
 }
 
 __global__ __launch_bounds__(SCAN_TILE) void k_scan_total(DS S, int ntiles) {
@@ -1276,8 +1284,17 @@ __global__ __launch_bounds__(FLOE_BLOCK) void k_cand(DS S, int lean, int nmember
 }
 
 // Superset build of the dense members' floes (queue 3), one wavefront per
-// floe over its (2 span + 1)^2 cell block, 64 entries at a time: counts, or
-// the entries and the build positions.  Only on build steps.
+// floe over its (2 span + 1)^2 cell block: counts, or the entries and the build
+// positions.  Only on build steps.  A lane per cell reads the ranges at once,
+// and the rows of the block, each one range of positions (the cells of a row
+// are consecutive in the cell order), are taken as one sequence, SUP_AHEAD
+// rounds of 64 positions requested together: the kernel is bound by its chain
+// of loads, six of them instead of about 25 with the rows one after the other
+// and the record counts behind the storage slots (count + fill of a build:
+// 320,000 power-law floes 0.79 + 0.87 -> 0.40 + 0.44 ms, 106,000 0.29 + 0.27 ->
+// 0.14 + 0.15, 262,144 in FP64 0.67 + 0.74 -> 0.33 + 0.38; the next floe's rows
+// requested ahead as well: the same).
+constexpr int SUP_AHEAD = 2;
 template <bool FILL>
 __global__ __launch_bounds__(64) void k_sup_dense(DS S) {
     if (!*S.rebuild || *S.err) return;
@@ -1289,40 +1306,63 @@ __global__ __launch_bounds__(64) void k_sup_dense(DS S) {
     const int per = (nq + XCD_COUNT - 1) / XCD_COUNT;
     const int t1 = min(nq, xcd * per + per);
     const uint64_t lt = lane ? ((~0ull) >> (64 - lane)) : 0ull;
-    int64_t sum = 0;
     for (int t = xcd * per + bi; t < t1; t += nb) {
         const int k = queue_at(S, 3, qv, t);
         const GeoRec me = S.geo[k];
-        const DevParams& P = S.params[me.member];
-        const double rad = me.r + P.rtree + P.skin, reach = P.rtree + P.skin;
         const int f = me.id, fs = S.cval[k];
         const float nbme = S.nb[k];
-        const int sp = P.span;
-        const int cx = cell_coord(me.x, P.cell, P.gx), cy = cell_coord(me.y, P.cell, P.gy);
-        int64_t* out = FILL ? S.sup + S.soff[k] : nullptr;
+        const uint32_t rcme = S.rcnt[k];
+        const int64_t soff = FILL ? S.soff[k] : 0;
         const int snear = FILL ? S.snear[k] : 0;
+        const DevParams& P = S.params[me.member];
+        const double skin = P.skin, rad = me.r + P.rtree + skin, reach = P.rtree + skin;
+        const int sp = P.span, gx = P.gx, gy = P.gy, cell_base = P.cell_base;
+        const int cx = cell_coord(me.x, P.cell, gx), cy = cell_coord(me.y, P.cell, gy);
+        // the block's cells by row, a lane each (span 1 or 2: at most 25)
+        const int R = 2 * sp + 1;
+        const int lr = R == 3 ? lane / 3 : lane / 5;
+        const int ca = cx - sp + (lane - lr * R), cb = cy - sp + lr;
+        int2 rg = make_int2(0, 0);
+        if (lane < R * R && ca >= 0 && ca < gx && cb >= 0 && cb < gy) rg = S.crange[cell_base + cb * gx + ca];
+        const uint64_t cells = __ballot(rg.y > rg.x);
+        int lo[5], end[5], L = 0;       // row r holds the sequence's entries up to end[r]
+#pragma unroll
+        for (int r = 0; r < 5; ++r) {
+            const uint32_t row = r < R ? (uint32_t)(cells >> (r * R)) & ((1u << R) - 1) : 0u;
+            lo[r] = row ? __builtin_amdgcn_readlane(rg.x, r * R + __ffs((int)row) - 1) : 0;
+            if (row) L += __builtin_amdgcn_readlane(rg.y, r * R + 31 - __clz((int)row)) - lo[r];
+            end[r] = L;
+        }
+        int64_t* out = FILL ? S.sup + soff : nullptr;
         int n = 0, nn = 0;
-        const int a0 = max(cx - sp, 0), a1 = min(cx + sp, P.gx - 1);
-        for (int b = cy - sp; b <= cy + sp; ++b) {
-            if (b < 0 || b >= P.gy) continue;
-            // the cells of one row are consecutive in the cell order
-            int lo = INT_MAX, hi = 0;
-            for (int a = a0; a <= a1; ++a) {
-                const int2 rg = S.crange[P.cell_base + b * P.gx + a];
-                if (rg.y > rg.x) { lo = min(lo, rg.x); hi = max(hi, rg.y); }
+        for (int c0 = 0; c0 < L; c0 += 64 * SUP_AHEAD) {
+            GeoRec o[SUP_AHEAD];
+            int qq[SUP_AHEAD];
+            float nbq[SUP_AHEAD];
+            uint32_t rcq[SUP_AHEAD];
+#pragma unroll
+            for (int u = 0; u < SUP_AHEAD; ++u) {
+                const int v = min(c0 + 64 * u + lane, L - 1);    // (the last entry stands in past the end)
+                int q = lo[0] + v;
+#pragma unroll
+                for (int r = 1; r < 5; ++r) q = v >= end[r - 1] ? lo[r] + v - end[r - 1] : q;
+                qq[u] = q;
+                o[u] = S.geo[q];
+                nbq[u] = S.nb[q];
+                rcq[u] = S.rcnt[q];
             }
-            for (int base = lo; base < hi; base += 64) {
-                const int q = base + lane;
+#pragma unroll
+            for (int u = 0; u < SUP_AHEAD; ++u) {
+                const int q = qq[u];
                 bool in = false, near = false;
                 float bound = 0.0f;
-                if (q < hi && q != k) {
-                    const GeoRec o = S.geo[q];
-                    const double dx = me.x - o.x, dy = me.y - o.y, d2 = dx * dx + dy * dy;
-                    const double thr = o.id > f ? rad : o.r + reach;
+                if (c0 + 64 * u + lane < L && q != k) {
+                    const double dx = me.x - o[u].x, dy = me.y - o[u].y, d2 = dx * dx + dy * dy;
+                    const double thr = o[u].id > f ? rad : o[u].r + reach;
                     in = d2 <= thr * thr * (1.0 + 1e-12);
                     if (in) {
-                        bound = sup_bound_of(S, f, fs, nbme, o.id, q);
-                        const double w = me.r + o.r + (double)bound + P.skin;
+                        bound = sup_bound_of(S, f, fs, nbme, rcme, o[u].id, q, nbq[u], rcq[u]);
+                        const double w = me.r + o[u].r + (double)bound + skin;
                         near = d2 <= w * w * (1.0 + 1e-12);
                     }
                 }
@@ -1342,9 +1382,7 @@ __global__ __launch_bounds__(64) void k_sup_dense(DS S) {
                 S.snear[k] = nn;
             }
         }
-        sum += nn;
     }
-    if (!FILL && lane == 0 && sum) atomicAdd((unsigned long long*)S.nearsum, (unsigned long long)sum);
 }
 
 // ---------------------------------------------------------------------
