@@ -153,7 +153,7 @@ struct godar_ctx {
     double tuned_cost_ms = 0.0;         // the autotuner's price of the chosen search shape
     std::vector<double> rmax;           // largest radius of each member when it was added
     int64_t sup_cap = 0;                // superset pool entries
-    int32_t built_qseg = -1;            // queue share the dense list was built with
+    int32_t built_qseg = -1;            // queue share of the last step launched
     // captured graphs of the step with the build kernels, by parity
     hipGraphExec_t gexec[2] = {nullptr, nullptr};
     std::vector<unsigned char> gsig[2];
@@ -643,7 +643,7 @@ int launch_step(godar_ctx* c, bool lean) {
         StageTimer t(c, 2);
         hipLaunchKernelGGL(k_ranges, grid_for(N, B[2], false), dim3(B[2]), 0, s, d);
         // superset build: counts, offsets, entries (k_sup shares k_cand's
-        // grid, whose XCD shares lay out the dense-search list)
+        // grid)
         const int ntiles = (N + SCAN_TILE - 1) / SCAN_TILE;
         hipLaunchKernelGGL(k_sup<false>, grid_for(N, B[3], true), dim3(B[3]), 0, s, d);
         if (any_dense) hipLaunchKernelGGL(k_sup_dense<false>, dim3(XCD_COUNT * 1024), dim3(64), 0, s, d);
@@ -1012,8 +1012,8 @@ static int64_t bytes_per_floe(const godar_ctx* c) {
 // only shrink, by ridging): the superset skin is skin_frac (rmax + rtree);
 // the member is dense when the 3x3 cells around a floe on a grid of cells
 // >= rmax + rtree + skin hold dense_scan floes or more (on average); the
-// cells are >= (rmax + rtree + skin) / span, span = 2 for the dense search
-// and thread_span for the thread search, so that the (2 span + 1)^2 cells
+// cells are >= (rmax + rtree + skin) / span, span = 2 for dense members
+// and thread_span for the others, so that the (2 span + 1)^2 cells
 // around a floe hold its whole superset.  Grids are coarsened to at most
 // 4n + 64 cells.
 void member_search(const godar_ctx* c, DevParams& dp, int n, double rmax, int64_t& gx, int64_t& gy) {
@@ -1785,7 +1785,7 @@ int build_period(godar_ctx* c, double frac, double* period) {
 }
 
 // Search shape: the superset skin (so the cell size), the thread search's
-// cell span and the dense-search threshold, one after the other.  Each
+// cell span and the dense threshold, one after the other.  Each
 // candidate is priced as a build step plus `4 trial` steps after it: the
 // mean step cost over a build and the steps until the next one,
 // t_step + (t_build - t_step) / period.  The settings stay where they were
@@ -1930,7 +1930,7 @@ int godar_step_async(godar_ctx* c, int32_t nsteps) {
     // many more keep one that speeds up steadily from rest below 0.45
     const int run = (int)std::min<int64_t>(std::max<int64_t>(c->since_build / 5, LEAN_RUN), LEAN_RUN_MAX);
     for (int k = 0; k < nsteps; ++k) {
-        // the dense-search list is laid out by the candidate search's XCD
+        // the queues are laid out by the candidate search's XCD
         // shares: a new block size or floe count needs a build
         const int32_t q = qseg_of(c);
         if (q != c->built_qseg) {

@@ -20,7 +20,7 @@ constexpr int WALL_SLOT = 0xFFFF;
 constexpr uint8_t CLS_CONTACT = 1, CLS_BOND = 2;
 constexpr int FLOE_BLOCK = 256;   // upper bound of the per-floe kernels' block size
 constexpr int XCD_COUNT = 8;      // accelerator complex dies of an MI355X
-constexpr int NQUEUE = 5;         // work queues: contact, bond, wall, dense search, fixup
+constexpr int NQUEUE = 5;         // work queues: contact, bond, wall, dense superset build, fixup
 constexpr int QN_STRIDE = 64;     // ints between queue counters (256 B)
 constexpr int SCAN_TILE = 1024;   // positions per tile of the superset offset scan
 constexpr int QUEUE_GRID_WAVES = 4096;   // wavefronts launched for a queue kernel at most
@@ -144,7 +144,7 @@ struct DS {
     double2* x0;               // [S] by pos (positions stand between builds)
     int32_t* rebuild;          // [4] 0: build the supersets; 1: refresh the ordered copies;
                                //     2: the copies are newer than rec; 3: builds so far
-    // Work queues (contact, bond, wall, dense search, fixup), each in XCD_COUNT
+    // Work queues (contact, bond, wall, dense superset build, fixup), each in XCD_COUNT
     // segments: the candidate search's blocks on XCD x cover positions
     // [x qseg, (x+1) qseg) and queue them into segment x, at
     // qlist[c S + x qseg + i], counted by their own counter (one per

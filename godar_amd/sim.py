@@ -184,7 +184,7 @@ class Context:
 
     def set_search(self, skin_frac: float = 0.1, thread_span: int = 1, dense_scan: int = 96):
         """Search shape of the current members (and later ones): superset
-        skin, cells the thread search scans on each side, dense-search
+        skin, cells the thread search scans on each side, dense
         threshold.  The next step builds the supersets; results do not depend
         on any of them."""
         self._chk(self.L.godar_set_search(self.h, float(skin_frac), int(thread_span), int(dense_scan)))

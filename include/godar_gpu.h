@@ -240,7 +240,7 @@ int godar_set_skin(godar_ctx *ctx, double frac);
 /* Search shape of the current members and of those added afterwards: the
  * superset skin `skin_frac` x (max r + rtree) (0-1), the cells the thread
  * search scans on each side of a floe at a build (1 or 2: cells of 1/span of
- * the superset reach) and the dense-search threshold (as
+ * the superset reach) and the dense threshold (as
  * godar_set_dense_search).  The next step builds the supersets.  Results do
  * not depend on any of them. */
 int godar_set_search(godar_ctx *ctx, double skin_frac, int32_t thread_span, int32_t dense_scan);
