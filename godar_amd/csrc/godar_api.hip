@@ -315,10 +315,37 @@ void force_refresh(godar_ctx* c) {
     c->need_full = true;
 }
 
+// Floes per wavefront of the candidate search.  Its passes over the floes'
+// pairs take 64 pairs a round, one round behind the other, so with room on the
+// chip fewer floes per wavefront end sooner: 1,000 floes 17 -> 10 us, 40,015
+// power-law floes 33 -> 19, 100,000 38 -> 28; with 2,048 wavefronts on the way,
+// twice as many cost 65,000 floes on [500, 2000] m 17 -> 26 us and 320,000
+// power-law ones 61 -> 62.  Past the wavefronts the chip holds at once (16 a
+// CU), the last of a few rounds is nearly empty; the long wavefronts of dense
+// members (10 superset entries a floe) end sooner spread over full rounds:
+// 270,000 power-law floes 52 -> 45 us, 320,000 57 -> 51, 400,000 63 -> 60,
+// 800,000 123 -> 118.  The short ones of sparse members do not (270,000 floes
+// on [500, 2000] m 27.5 -> 30.7 us, 330,000 32.1 -> 31.6, 810,000 66 -> 69).
+static int cand_floes(const godar_ctx* c) {
+    const int N = std::max(c->N_used, 1);
+    const int64_t slots = (int64_t)CAND_RESIDENT * c->ncu, waves = (N + 63) / 64;
+    int64_t dense = 0;
+    for (int k = 0; k < c->Mcap; ++k)
+        if (c->members[k].active && c->dparams[k].dense) dense += c->members[k].n;
+    if (2 * dense >= N && waves > slots && waves <= CAND_ROUNDS * slots) {
+        const int64_t rounds = (waves + slots - 1) / slots;
+        return (int)std::min<int64_t>(64, ((N + rounds * slots - 1) / (rounds * slots) + 3) / 4 * 4);
+    }
+    int f = 64;
+    while (f > CAND_MIN_FLOES && N / f < CAND_WAVES) f /= 2;
+    return f;
+}
+
+// Floe positions per XCD share of the candidate search's grid.
 int32_t qseg_of(const godar_ctx* c) {
-    const int bc = c->sblock[3];
-    const int gc = ((std::max(c->N_used, 1) + bc - 1) / bc + XCD_COUNT - 1) / XCD_COUNT * XCD_COUNT;
-    return gc / XCD_COUNT * bc;
+    const int N = std::max(c->N_used, 1), wpb = c->sblock[3] / 64, f = cand_floes(c);
+    const int blocks = (N + wpb * f - 1) / (wpb * f);
+    return (blocks + XCD_COUNT - 1) / XCD_COUNT * wpb * f;
 }
 
 void sync_ds(godar_ctx* c) {
@@ -590,17 +617,6 @@ static dim3 grid_for(int N, int B, bool xcd) {
 // Queue kernels loop over their entries: at most QUEUE_GRID_WAVES
 // wavefronts (about one round of resident wavefronts), so that short queues
 // do not launch a wavefront per 64 floes that finds nothing to do.
-// Floes per wavefront of the candidate search: its passes over the floes'
-// pairs take 64 pairs a round, one round behind the other, so with room on the
-// chip fewer floes per wavefront end sooner (a power of two, as the queues'
-// shares are made of 64s): 1,000 floes 17 -> 10 us, 40,015 power-law floes 33 ->
-// 19, 100,000 38 -> 28; with 2,048 wavefronts on the way, twice as many cost
-// 65,000 floes on [500, 2000] m 17 -> 26 us and 320,000 power-law ones 61 -> 62.
-static int cand_floes(int N) {
-    int f = 64;
-    while (f > CAND_MIN_FLOES && N / f < CAND_WAVES) f /= 2;
-    return f;
-}
 static dim3 grid_queue(int N, int B) {
     const int cap = QUEUE_GRID_WAVES * 64 / B / XCD_COUNT * XCD_COUNT;
     const dim3 g = grid_for(N, B, true);
@@ -656,7 +672,7 @@ int launch_step(godar_ctx* c, bool lean) {
     {
         StageTimer t(c, 3);
         // LDS: one list of (floe, candidate) pairs per wavefront
-        const int floes = cand_floes(N);
+        const int floes = cand_floes(c);
         hipLaunchKernelGGL(mixed ? k_cand<true> : k_cand<false>, grid_for(N, B[3] / 64 * floes, true),
                            dim3(B[3]), (B[3] / 64) * CAND_LDS_PER_WAVE, s, d, lean ? 1 : 0, nm, floes);
     }

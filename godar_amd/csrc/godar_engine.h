@@ -26,6 +26,8 @@ constexpr int SCAN_TILE = 1024;   // positions per tile of the superset offset s
 constexpr int QUEUE_GRID_WAVES = 4096;   // wavefronts launched for a queue kernel at most
 constexpr int CAND_WAVES = 2048;           // wavefronts below which the search takes fewer floes each
 constexpr int CAND_MIN_FLOES = 8;
+constexpr int CAND_RESIDENT = 16;          // wavefronts of the search a CU holds (registers, LDS)
+constexpr int CAND_ROUNDS = 4;             // rounds of them up to which the floes are spread evenly
 constexpr int WALL_GRID_WAVES = 256;     // wavefronts of the walls beside contacts and bonds at most
 constexpr int FIXUP_GRID_WAVES = 2048;   // wavefronts of the fix-up (about one resident round)
 

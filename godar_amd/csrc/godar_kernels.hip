@@ -596,17 +596,23 @@ __global__ void k_ranges(DS S) {
 // of the wavefront must call it; the wavefront's positions lie in one XCD
 // share of the candidate search.
 __device__ __forceinline__ void enqueue(const DS& S, bool want, int c, int k) {
-    const uint64_t mask = __ballot(want);
-    if (!mask) return;
+    uint64_t mask = __ballot(want);
     const int lane = threadIdx.x & 63;
-    const int leader = __ffsll((long long)mask) - 1;
-    const int x = __shfl(k, leader) / S.qseg;
-    int base = 0;
-    if (lane == leader) base = atomicAdd(qcount(S, c, x), __popcll(mask));
-    base = __shfl(base, leader);
-    if (want) {
-        const uint64_t below = lane ? mask & ((~0ull) >> (64 - lane)) : 0ull;
-        S.qlist[(int64_t)c * S.S + x * S.qseg + base + __popcll(below)] = k;
+    // (once, unless the wavefront's positions lie on either side of a segment
+    // boundary, which the candidate search's never do)
+    while (mask) {
+        const int leader = __ffsll((long long)mask) - 1;
+        const int x = __builtin_amdgcn_readlane(k, leader) / S.qseg;
+        const uint64_t mine = __ballot(want && k < (x + 1) * S.qseg);
+        int base = 0;
+        if (lane == leader) base = atomicAdd(qcount(S, c, x), __popcll(mine));
+        base = __builtin_amdgcn_readlane(base, leader);
+        if (mine >> lane & 1) {
+            const uint64_t below = lane ? mine & ((~0ull) >> (64 - lane)) : 0ull;
+            S.qlist[(int64_t)c * S.S + x * S.qseg + base + __popcll(below)] = k;
+            want = false;
+        }
+        mask &= ~mine;
     }
 }
 

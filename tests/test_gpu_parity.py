@@ -709,6 +709,35 @@ def test_winds_of_members_that_left_are_dropped():
     ctx.close()
 
 
+@pytest.mark.parametrize("copies,dense", [(91, True), (91, False), (175, True)])
+def test_search_spread_over_full_rounds(copies, dense):
+    """More floes than the search's wavefronts on the chip at 64 each (273,000
+    and 525,000 where that is 262,144): the floes are spread over them in
+    shares that are no multiple of 64, and the work queues' segments with them,
+    if the members are dense.  Every copy of a member takes the steps it takes
+    alone."""
+    f = kick(squeeze(g.config0_member(91, 3000), 0.998), 4)
+    p = config0_params(f)
+    out = []
+    for n in (1, copies):
+        ctx = _ctx(n * f.n, n, "mixed")
+        ctx.record_forces(False)
+        if dense:
+            ctx.set_dense_search(0)
+        ms = [ctx.add_field(p, f) for _ in range(n)]
+        ctx.step(6)
+        out.append([ctx.floes(m) for m in ms])
+        tot = ctx.totals()
+        out[-1].append({k: v // n for k, v in tot.items()})
+        assert all(v % n == 0 for v in tot.values())
+        ctx.close()
+    alone, tot = out[0]
+    assert out[1].pop() == tot and tot["contacts"] > 0 and tot["bonds"] > 0
+    for got in out[1]:
+        for k in STATE:
+            assert np.array_equal(got[k], alone[k]), k
+
+
 def test_checkpoint_restore_continues_exactly():
     """A member restored from a checkpoint (floes, walls, contact histories
     with last contact forces, bond strain state, step number) continues
