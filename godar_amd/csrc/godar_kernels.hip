@@ -748,8 +748,8 @@ __device__ __forceinline__ int2 sup_thread(const DS& S, int k, const GeoRec& me,
     return make_int2(n, nn);
 }
 
-// (floe, candidate) pairs of one wavefront in LDS: entry, distance (inner:
-// -1) and owner lane, the per-lane pair counts and the pairs whose terms are
+// (floe, candidate) pairs of one wavefront in LDS: entry, distance (inner: -1 -
+// identity) and owner lane, the per-lane pair counts and the pairs whose terms are
 // evaluated
 constexpr int CAND_TCAP = 512;
 constexpr int CAND_LDS_PER_WAVE = CAND_TCAP * (8 + 8 + 1) + 64 * 4 + CAND_TCAP * 2 + 64;
@@ -771,8 +771,9 @@ static_assert(CAND_TCAP < 1 << 10, "the per-lane counts are packed 10 bits each"
 // place (inserting them one after the other, a lane per floe, held the
 // wavefront for its longest list, whose part past a few entries in registers
 // went through memory: 320,000 power-law floes mixed 109 -> 60 us, 40,015 57
-// -> 33, 262,144 FP64 164 -> 76; radii on [500, 2000] m, 1.7 pairs a floe, the
-// same), and the
+// -> 33, 262,144 FP64 164 -> 76; with one comparison for both lists and the
+// equal distances apart, of 320,000 51 -> 46, 262,144 FP64 72 -> 61, 1.38 M on
+// [500, 2000] m 111 -> 105), and the
 // sheltering and classification terms of the pairs that need them are
 // evaluated together, 64 at a time; each floe then takes the minimum of its
 // own terms (a minimum of fmin terms does not depend on which lane computed
@@ -903,7 +904,7 @@ __device__ __forceinline__ void cand_thread(const DS& S, int k0, int k, const Ge
         soff = pre.soff;
     }
     int64_t* te = reinterpret_cast<int64_t*>(lds);                      // entry, then the water term
-    double* td = reinterpret_cast<double*>(lds + 8 * CAND_TCAP);         // distance (inner: -1), then the air term
+    double* td = reinterpret_cast<double*>(lds + 8 * CAND_TCAP);         // distance (inner: -1 - identity), then the air term
     uint8_t* to = lds + 16 * CAND_TCAP;                                   // owner lane, then flags
     // per lane: pairs, outer ones << 10, pairs whose terms are needed << 20
     int32_t* tn = reinterpret_cast<int32_t*>(lds + 17 * CAND_TCAP);
@@ -1003,7 +1004,7 @@ __device__ __forceinline__ void cand_thread(const DS& S, int k0, int k, const Ge
             if (hit) {
                 const int at = atotal + __popcll(mh & lt);
                 te[at] = ent(j, q);
-                td[at] = j > of ? d : -1.0;
+                td[at] = j > of ? d : -(double)j - 1.0;
                 to[at] = (uint8_t)own;
                 atomicAdd(&tn[own], 1 + (j > of ? 1 << 10 : 0) + (need ? 1 << 20 : 0));
                 if (need) tx[nneed + __popcll(mn & lt)] = (uint16_t)at;
@@ -1038,15 +1039,17 @@ __device__ __forceinline__ void cand_thread(const DS& S, int k0, int k, const Ge
             const int64_t en = te[idx];
             const double d = td[idx];
             const int id = ent_id(en);
-            int before = 0;
-            if (d >= 0.0) {
-                for (int t = b; t < b + n; ++t) {
-                    const double dt = td[t];
-                    before += dt >= 0.0 && (dt < d || (dt == d && ent_id(te[t]) < id));
-                }
-            } else {
-                for (int t = b; t < b + n; ++t) before += td[t] < 0.0 && ent_id(te[t]) < id;
+            // outer entries below the distance, inner ones with a smaller
+            // identity; equal distances, which next to never meet, by identity
+            const double above = d >= 0.0 ? -0.5 : d, below = d >= 0.0 ? d : -0.5;
+            int before = 0, same = 0;
+            for (int t = b; t < b + n; ++t) {
+                const double dt = td[t];
+                before += (dt > above) & (dt < below);
+                same += dt == d;
             }
+            if (same > 1)
+                for (int t = b; t < b + n; ++t) before += td[t] == d && ent_id(te[t]) < id;
             if (c0 + lane < atotal) {
                 const int64_t at = before * SS + (k0 + ow);
                 if (d >= 0.0) {

@@ -592,6 +592,42 @@ def test_dense_search_long_lists_and_unordered_supersets():
             assert np.array_equal(ha, hb)
 
 
+def test_candidates_at_equal_distances_go_by_identity():
+    """Equal floes on a lattice, in shuffled order: each has up to four
+    neighbours at every one of five distances, exactly (the coordinates are
+    whole numbers), all bonded to the nearest ones and sheltering the others.
+    The order among equals is the identities', as the oracle's: lists, state and
+    force sums agree from the first step on."""
+    from oracle_py import OracleSim
+    side = 9
+    n = side * side
+    rng = np.random.default_rng(7)
+    f = g.config0_member(51, 100)
+    site = rng.permutation(n)
+    f.x, f.y = 2000.0 * (site % side) + 1000.0, 2000.0 * (site // side) + 1000.0
+    f.r, f.h = np.full(n, 995.0), np.full(n, 40.0)
+    f.theta, f.omega = np.zeros(n), rng.normal(0, 1e-4, n)
+    f.u, f.v = rng.normal(0, 0.5, n), rng.normal(0, 0.5, n)
+    f.box = 2000.0 * side
+    p = config0_params(f, bond_lim=20.0, bond_frac=1.0, rtree=3500.0)
+    ctx = _ctx(n)
+    ctx.reserve(outer=64, inner=64)
+    m = ctx.add_field(p, f)
+    O = OracleSim(p, f)
+    for t in range(1, 4):
+        ctx.step(1)
+        O.step()
+        cand, cont = _oracle_pairs(O)
+        assert _pairs(ctx, m, "candidate") == cand and _pairs(ctx, m, "contact") == cont, t
+        a, b = ctx.floes(m), O.state()
+        for k in STATE:
+            assert np.array_equal(a[k], b[k]), (t, k)
+        fa, fb = ctx.forces(m), O.forces()
+        for k in ("fbx", "fby", "mb"):
+            assert np.array_equal(fa[k], fb[k]), (t, k)
+    ctx.close()
+
+
 @pytest.mark.parametrize("n", [9, 200, 700])
 def test_search_takes_floes_in_groups(n):
     """Small floes of such draft that all of them matter to each other: 64
