@@ -2948,11 +2948,24 @@ __global__ __launch_bounds__(FLOE_BLOCK, (MIXED && !REC) ? 5 : 4) void k_final(D
     }
 }
 
-// The candidate pairs of the floe at position k in the last step (the
-// reference's kNearest within r(i) + rtree): those of its superset within the
-// query radius, by the positions the step started from (the other of the two
-// position buffers) and its radius at the top of its iteration; fn(partner's
-// identity) for each.
+// Whether the row at position k of the last step's order is a floe that is
+// still there.  Positions, and with them the lists and the reshape records,
+// stand until the next build while members leave and others take their slots
+// and storage: rows of a member that left have no member at their storage slot
+// any more, and floes added since the step have no position (k_admit).  Lists
+// are walked for such rows only: a new member in an old one's slot has another
+// first floe, and the old one's record indices lead anywhere from there.
+__device__ __forceinline__ bool still_there(const DS& S, const GeoRec& g, int k) {
+    if (g.member < 0) return false;
+    const int f = S.sid_of[g.id];
+    return S.member_of[f] == g.member && S.pos_of[f] == k;
+}
+
+// The candidate pairs of the floe at position k (still_there) in the last step
+// (the reference's kNearest within r(i) + rtree): those of its superset within
+// the query radius, by the positions the step started from (the other of the
+// two position buffers) and its radius at the top of its iteration;
+// fn(partner's identity) for each.
 template <typename F>
 __device__ __forceinline__ void each_candidate(const DS& S, int k, const GeoRec& me, F&& fn) {
     const int m = me.member;
@@ -2981,17 +2994,16 @@ __device__ __forceinline__ void each_candidate(const DS& S, int k, const GeoRec&
 __global__ void k_totals(DS S, int64_t* out) {
     int k = blockIdx.x * blockDim.x + threadIdx.x;
     int64_t c = 0, ct = 0, bd = 0;
-    if (k < S.N && S.geo[k].member >= 0) {
-        const GeoRec me = S.geo_new[k];
-        int no = S.ocnt[k];
-        if (me.member >= 0) each_candidate(S, k, me, [&](int) { ++c; });
-        else no = 0;
+    const GeoRec me = k < S.N ? S.geo_new[k] : GeoRec{0.0, 0.0, 0.0, 0, -1};
+    if (still_there(S, me, k)) {
+        const int no = S.ocnt[k];
+        each_candidate(S, k, me, [&](int) { ++c; });
         for (int s = 0; s < no; ++s) {
             uint32_t fl = S.evf[(int64_t)s * S.S + k];
             if (fl & EV_REMOVED) continue;
             if (fl & EV_CONTACT) ++ct;
         }
-        int f = S.cval[k];
+        const int f = S.sid_of[me.id];
         int nb = S.bcnt_old[f];
         for (int q = 0; q < nb; ++q) {
             const BondRec& b = S.bond_old[(int64_t)q * S.S + f];
@@ -3068,7 +3080,7 @@ __global__ void k_pairs(DS S, int m, PairOut* out, int cap) {
     if (K == PAIRS_CANDIDATE) {
         if (k >= S.N) return;
         const GeoRec me = S.geo_new[k];
-        if (me.member != m) return;
+        if (me.member != m || !still_there(S, me, k)) return;
         each_candidate(S, k, me, [&](int j) {
             const int at = atomicAdd(S.npairs, 1);
             if (at < cap) { out[at].i = me.id - mb.first; out[at].j = j - mb.first; }
@@ -3079,7 +3091,7 @@ __global__ void k_pairs(DS S, int m, PairOut* out, int cap) {
     const int f = mb.first + k, i = S.gid_of[f] - mb.first;
     if (K == PAIRS_CONTACT) {
         const int q = S.pos_of[f];
-        if ((uint32_t)q >= (uint32_t)S.N) return;
+        if ((uint32_t)q >= (uint32_t)S.N) return;      // (-1: the member's first step is to come)
         const int no = min(S.ocnt[q], S.CO);
         for (int s = 0; s < no; ++s) {
             const int64_t at0 = (int64_t)s * S.S + q;
@@ -3119,6 +3131,7 @@ __global__ __launch_bounds__(64) void k_admit(DS S, int m, int first, int b, int
     S.rec[f] = recs[t];
     S.gid_of[f] = id;
     S.sid_of[id] = f;
+    S.pos_of[f] = -1;              // (none before the next build)
     S.member_of[f] = m;
 #pragma unroll
     for (int k = 0; k < 4; ++k) S.wbc[k * S.S + f] = 0.0;

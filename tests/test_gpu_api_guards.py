@@ -133,3 +133,51 @@ def test_restore_refuses_foreign_blocks():
     _same(a, b, m, mb)
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("n", [64, 40, 200])
+def test_lists_of_a_member_that_left_are_not_walked(n):
+    """A member that was reshaping floes leaves and another takes its slot,
+    in the same storage (64 and 40 floes fit the gap) or past the others' (200):
+    before the next step the totals, pair lists and statistics are those of
+    the member that stayed, and the new one has none; after a step every
+    member's are those it has alone."""
+    f, p = _box()
+    mate = kick(squeeze(packed_box(64, 11)), 4)
+    pm = config0_params(mate, sigmanc_crit=1e5)
+    new = kick(squeeze(packed_box(n, 7, box=2.0e4 * np.sqrt(n / 64))), 2)
+    pn = config0_params(new, sigmanc_crit=1e5)
+    a = _ctx(f.n + mate.n + 200, 2)
+    ma, mb = a.add_field(p, f), a.add_field(pm, mate)
+    for _ in range(40):
+        a.step(1)
+        if a.stats(ma)["seeds"] > 0:
+            break
+    assert a.stats(ma)["seeds"] > 0
+    steps = a.tstep(mb) - 1
+    kinds = ("candidate", "contact", "bond")
+    of_mate = {k: [x.tolist() for x in a.pairs(mb, k)] for k in kinds}
+    a.remove(ma)
+    mc = a.add_field(pn, new)
+    assert mc == ma
+    t = a.totals()
+    assert (t["candidates"], t["contacts"], t["bonds"]) == tuple(len(of_mate[k][0]) for k in kinds)
+    s = a.stats(mc)
+    assert (s["candidates"], s["contacts"]) == (0, 0)
+    for k in kinds:
+        assert a.pairs(mc, k)[0].size == 0, k
+        assert [x.tolist() for x in a.pairs(mb, k)] == of_mate[k], k
+    a.step(1)
+    t = a.totals()
+    want = dict.fromkeys(kinds, 0)
+    for m, fld, par, done in ((mb, mate, pm, steps + 1), (mc, new, pn, 1)):
+        b = _ctx(fld.n)
+        m1 = b.add_field(par, fld)
+        b.step(done)
+        for k in kinds:
+            pair = [x.tolist() for x in b.pairs(m1, k)]
+            assert [x.tolist() for x in a.pairs(m, k)] == pair, k
+            want[k] += len(pair[0])
+        b.close()
+    assert (t["candidates"], t["contacts"], t["bonds"]) == tuple(want[k] for k in kinds)
+    a.close()
