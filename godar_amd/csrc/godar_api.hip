@@ -159,22 +159,22 @@ struct godar_ctx {
     std::vector<unsigned char> gsig[2];
     // Steps without a build launch no build kernels (lean steps): the host
     // launches the full sequence when it forced a build or refresh itself,
-    // when the last godar_sync found one due or near (a floe past 0.3 skin),
+    // when the last settle found one due or near (a floe past 0.3 skin),
     // after a run of lean steps in one go that grows with the steps since the
     // last build (godar_step_async), and for a while after a lean step found a
-    // build due (ERR_NEED_BUILD; godar_sync runs such steps again).  (The 16
+    // build due (ERR_NEED_BUILD; settle runs such steps again).  (The 16
     // build kernels of a full step that builds nothing take 70 us: with one
     // such step in 16, 1,000 power-law floes took 51 us a step, without 45; 64
     // floes called step by step 4% longer.)
     bool need_full = true;
     int lean_run = 0;                   // lean steps since the last full one
     int full_hold = 0;                  // full steps still to launch after a missed build
-    // as of the last godar_sync: a build or refresh is due or comes near, the
+    // as of the last settle: a build or refresh is due or comes near, the
     // builds so far, the steps since the last of them
     bool soon = false;
     int32_t builds = 0;
     int64_t since_build = 0;
-    int64_t pend_launched = 0;          // steps launched since the last sync
+    int64_t pend_launched = 0;          // steps launched since then
     int device = 0;                     // the GPU the context lives on
     int ncu = 256;                      // its compute units
     int64_t* totals_scratch = nullptr;  // device address of that GPU's `scratch`
@@ -183,7 +183,7 @@ struct godar_ctx {
     HostStatus* status = nullptr;
     unsigned char* stage = nullptr;
     hipEvent_t estage[2] = {nullptr, nullptr};
-    int64_t done = 0;                   // steps completed, as of the last godar_sync
+    int64_t done = 0;                   // steps completed, as of the last settle
 };
 
 namespace {
@@ -404,6 +404,10 @@ int upload_members_only(godar_ctx* c) {
     return GODAR_OK;
 }
 
+constexpr int LEAN_RUN = 15;       // lean steps between two full ones, at least
+constexpr int LEAN_RUN_MAX = 255;  // and at most
+constexpr int FULL_HOLD = 64;      // full steps after a lean step found a build due
+
 // Waits for the context's stream and brings the step status back: the error
 // word, the steps completed and the members (their step numbers).
 int read_status(godar_ctx* c) {
@@ -415,19 +419,49 @@ int read_status(godar_ctx* c) {
     return GODAR_OK;
 }
 
-// steps completed without error since the context was created
-int steps_done(godar_ctx* c, int64_t* out) {
-    if (c->pending) {
+// Ends the steps under way, before the host reads or writes device state: waits
+// for them, runs those that a missed build kept from running, and binds the
+// buffers of the last complete step.  (The host counts a step, after which the
+// positions and the pair state change buffers, when it launches it; the launches
+// behind a missed build or an error do nothing.)  Errors other than a missed
+// build stay on the device for godar_sync to report, and the state of the last
+// complete step is what is read and written meanwhile.
+int settle(godar_ctx* c) {
+    while (c->pending) {
         int rc = read_status(c);
         if (rc != GODAR_OK) return rc;
-        *out = c->status->steps_done;
-    } else {
-        *out = c->done;
+        const uint32_t e = c->status->err;
+        const int64_t now = c->status->steps_done;
+        c->since_build = c->status->builds == c->builds ? c->since_build + now - c->done : 0;
+        c->builds = c->status->builds;
+        c->soon = c->status->due != 0;
+        if (!c->soon) c->lean_run = 0;
+        c->done = now;
+        if (!e) {
+            c->pending = false;
+            return GODAR_OK;
+        }
+        c->parity = c->pend_parity ^ (int)((now - c->pend_done0) & 1);
+        bind_parity(c);
+        if (e != ERR_NEED_BUILD) return GODAR_OK;
+        // a lean step found a build due, or a floe's drafts outgrew its lists:
+        // that step and the ones after it did nothing; they run again from
+        // here, with the build kernels
+        HIPCHK(c, hipMemsetAsync(c->d.dirty, 0, c->S, c->stream));
+        HIPCHK(c, hipMemsetAsync(c->d.err, 0, sizeof(uint32_t), c->stream));
+        const int64_t left = c->pend_launched - (now - c->pend_done0);
+        c->pend_parity = c->parity;
+        c->pend_done0 = now;
+        c->pend_launched = 0;
+        c->need_full = true;
+        c->full_hold = FULL_HOLD;
+        rc = godar_step_async(c, (int32_t)std::max<int64_t>(left, 0));
+        if (rc != GODAR_OK) return rc;
     }
     return GODAR_OK;
 }
 
-int download_members(godar_ctx* c) { return read_status(c); }
+int download_members(godar_ctx* c) { return c->pending ? settle(c) : read_status(c); }
 
 // The staging area of the read-backs: two halves, so that the host copies one
 // out while the GPU fills the other.  4 MiB keep a half (2 MiB) above the
@@ -455,7 +489,8 @@ int ensure_stage(godar_ctx* c) {
 // rows) into dst[row] (null: not wanted), by way of the staging area.
 template <int W>
 int read_rows(godar_ctx* c, int32_t m, int rows, double* const* dst) {
-    int rc = ensure_stage(c);
+    int rc = settle(c);
+    if (rc == GODAR_OK) rc = ensure_stage(c);
     if (rc != GODAR_OK) return rc;
     sync_ds(c);
     const int n = c->members[m].n;
@@ -483,7 +518,8 @@ int read_rows(godar_ctx* c, int32_t m, int rows, double* const* dst) {
 // listed, in no order, in the staging area or, past its room, in `more`.
 template <int K>
 int read_pairs(godar_ctx* c, int32_t m, bool want, const PairOut** list, std::vector<PairOut>& more, int* n) {
-    int rc = ensure_stage(c);
+    int rc = settle(c);
+    if (rc == GODAR_OK) rc = ensure_stage(c);
     if (rc != GODAR_OK) return rc;
     sync_ds(c);
     auto pass = [&](PairOut* out, int cap) -> hipError_t {
@@ -622,10 +658,6 @@ static dim3 grid_queue(int N, int B) {
     const dim3 g = grid_for(N, B, true);
     return dim3(std::max(XCD_COUNT, std::min((int)g.x, cap)));
 }
-
-constexpr int LEAN_RUN = 15;       // lean steps between two full ones, at least
-constexpr int LEAN_RUN_MAX = 255;  // and at most
-constexpr int FULL_HOLD = 64;      // full steps after a lean step found a build due
 
 int launch_step(godar_ctx* c, bool lean) {
     DS& d = c->d;
@@ -1053,6 +1085,8 @@ void member_search(const godar_ctx* c, DevParams& dp, int n, double rmax, int64_
 // other; the next step builds the supersets.  Nothing changes if the cell
 // table cannot grow.
 int research_all(godar_ctx* c) {
+    int rc = settle(c);
+    if (rc != GODAR_OK) return rc;
     HIPCHK(c, hipStreamSynchronize(c->stream));
     std::vector<DevParams> dps = c->dparams;
     std::vector<int32_t> cn(c->Mcap, 0);
@@ -1066,7 +1100,7 @@ int research_all(godar_ctx* c) {
         base += gx * gy;
         if (base >= ((int64_t)1 << 30)) return fail(c, GODAR_ERR_NOMEM, "search: too many cells");
     }
-    int rc = ensure_cells(c, (int32_t)base);
+    rc = ensure_cells(c, (int32_t)base);
     if (rc != GODAR_OK) return rc;
     c->dparams = dps;
     c->cell_n = cn;
@@ -1110,6 +1144,8 @@ int godar_member_add(godar_ctx* c, const godar_params* p, int32_t n, const doubl
     if (p->ntree != 1)
         return fail(c, GODAR_ERR_ARG, "member_add: ntree must be 1 (the neighbour search uses the "
                                       "current positions every step)");
+    int rc = settle(c);
+    if (rc != GODAR_OK) return rc;
     int m = -1;
     for (int k = 0; k < c->Mcap; ++k)
         if (!c->members[k].active) { m = k; break; }
@@ -1137,7 +1173,7 @@ int godar_member_add(godar_ctx* c, const godar_params* p, int32_t n, const doubl
         if (c->members[k].active) cused.push_back({c->dparams[k].cell_base, c->cell_n[k]});
     int64_t cbase;
     find_range(c, ncell, (int64_t)1 << 30, cused, cbase);
-    int rc = ensure_cells(c, (int32_t)(cbase + ncell));
+    rc = ensure_cells(c, (int32_t)(cbase + ncell));
     if (rc != GODAR_OK) return rc;
     dp.cell_base = (int32_t)cbase;
     c->cell_n[m] = ncell;
@@ -1238,6 +1274,8 @@ struct MemberState {
 };
 
 int read_member_state(godar_ctx* c, int32_t m, MemberState& out) {
+    int rc = settle(c);
+    if (rc != GODAR_OK) return rc;
     spill(c);
     HIPCHK(c, hipStreamSynchronize(c->stream));
     const Member& mm = c->members[m];
@@ -1483,8 +1521,10 @@ int godar_member_restore(godar_ctx* c, const void* buf, int64_t size, int32_t* m
 
 int godar_member_remove(godar_ctx* c, int32_t m) {
     if (!valid_member(c, m)) return fail(c, GODAR_ERR_ARG, "member_remove: bad member");
+    int rc = settle(c);
+    if (rc != GODAR_OK) return rc;
     spill(c);                       // before the floe count changes
-    int rc = download_members(c);   // keep device-side step counters
+    rc = download_members(c);       // keep device-side step counters
     if (rc != GODAR_OK) return rc;
     Member& mm = c->members[m];
     hipLaunchKernelGGL(k_fill_i32, dim3((mm.n + 255) / 256), dim3(256), 0, c->stream,
@@ -1504,6 +1544,8 @@ int godar_member_remove(godar_ctx* c, int32_t m) {
 
 int godar_set_forcing(godar_ctx* c, int32_t m, double ua, double va, double uw, double vw) {
     if (!valid_member(c, m)) return fail(c, GODAR_ERR_ARG, "set_forcing: bad member");
+    int rc = settle(c);
+    if (rc != GODAR_OK) return rc;
     DevParams& d = c->dparams[m];
     d.ua = ua; d.va = va; d.uw = uw; d.vw = vw;
     HIPCHK(c, hipMemcpyAsync((void*)(c->d.params + m), &d, sizeof(DevParams), hipMemcpyHostToDevice,
@@ -1557,8 +1599,10 @@ int godar_set_wind_frames(godar_ctx* c, int32_t m, int32_t nxn, int32_t nyn, dou
     g.nframes = nframes; g.avg = disc_average ? 1 : 0;
     g.t0 = t0; g.fdt = nframes > 1 ? frame_dt : 1.0;
     const int64_t cnt = (int64_t)nxn * nyn;
+    int rc = settle(c);
+    if (rc != GODAR_OK) return rc;
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    int rc = drop_unused_winds(c);
+    rc = drop_unused_winds(c);
     if (rc != GODAR_OK) return rc;
     g.offset = (int64_t)c->wpool.size();
     for (int32_t f = 0; f < nframes; ++f) {
@@ -1612,6 +1656,8 @@ int godar_set_bonds(godar_ctx* c, int32_t m, int32_t nb, const int32_t* bi, cons
                     const double* st) {
     if (!valid_member(c, m) || nb < 0 || (nb > 0 && (!bi || !bj || !st)))
         return fail(c, GODAR_ERR_ARG, "set_bonds: bad argument");
+    int rc = settle(c);
+    if (rc != GODAR_OK) return rc;
     const Member& mm = c->members[m];
     int64_t S = c->S;
     HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -1642,6 +1688,8 @@ int godar_reserve(godar_ctx* c, int32_t outer, int32_t inner, int32_t histc, int
     if (!c || outer < 0 || inner < 0 || histc < 0 || bonds < 0 || outer > 0xFFFE ||
         inner > (1 << 15) || histc > (1 << 12) || bonds > (1 << 12))
         return fail(c, GODAR_ERR_ARG, "reserve: bad argument");
+    int rc = settle(c);
+    if (rc != GODAR_OK) return rc;
     HIPCHK(c, hipStreamSynchronize(c->stream));
     const int nCO = outer ? outer : c->CO, nCI = inner ? inner : c->CI;
     const int nHC = histc ? histc : c->HC, nBC = bonds ? bonds : c->BC;
@@ -1660,7 +1708,6 @@ int godar_reserve(godar_ctx* c, int32_t outer, int32_t inner, int32_t histc, int
         return GODAR_OK;
     };
     int32_t mo = 0, mi = 0, mh = 0, mb = 0;
-    int rc;
     if (nCO < c->CO && (rc = longest(c->d.ocnt, mo)) != GODAR_OK) return rc;
     if (nCI < c->CI && (rc = longest(c->d.icnt, mi)) != GODAR_OK) return rc;
     if (nHC < c->HC && (rc = longest(c->hcnt[o], mh)) != GODAR_OK) return rc;
@@ -1934,8 +1981,7 @@ int godar_record_forces(godar_ctx* c, int32_t on) {
 int godar_step_async(godar_ctx* c, int32_t nsteps) {
     if (!c || nsteps < 0) return GODAR_ERR_ARG;
     if (!c->pending) {
-        int rc = steps_done(c, &c->pend_done0);
-        if (rc != GODAR_OK) return rc;
+        c->pend_done0 = c->done;
         c->pend_parity = c->parity;
         c->pending = true;
         c->pend_launched = 0;
@@ -1980,43 +2026,16 @@ int godar_use_graphs(godar_ctx* c, int32_t on) {
 
 int godar_sync(godar_ctx* c) {
     if (!c) return GODAR_ERR_ARG;
-    int rc = read_status(c);
+    const bool was_pending = c->pending;
+    int rc = was_pending ? settle(c) : read_status(c);
     if (rc != GODAR_OK) return rc;
     collect_events(c);
-    const uint32_t e = c->status->err;
-    const int64_t now = c->status->steps_done;
-    c->since_build = c->status->builds == c->builds ? c->since_build + now - c->done : 0;
-    c->builds = c->status->builds;
-    c->soon = c->status->due != 0;
-    if (!c->soon) c->lean_run = 0;
-    c->done = now;
-    bool was_pending = c->pending;
     c->pending = false;
-    if (e == ERR_NEED_BUILD && was_pending) {
-        // a lean step found a build due, or a floe's drafts outgrew its lists:
-        // that step and the ones after it did nothing; back to the last
-        // complete step, and the rest again with the build kernels
-        c->parity = c->pend_parity ^ (int)((now - c->pend_done0) & 1);
-        bind_parity(c);
-        HIPCHK(c, hipMemsetAsync(c->d.dirty, 0, c->S, c->stream));
-        HIPCHK(c, hipMemsetAsync(c->d.err, 0, sizeof(uint32_t), c->stream));
-        const int64_t left = c->pend_launched - (now - c->pend_done0);
-        c->need_full = true;
-        c->full_hold = FULL_HOLD;
-        if (left <= 0) return GODAR_OK;
-        rc = godar_step_async(c, (int32_t)left);
-        if (rc != GODAR_OK) return rc;
-        return godar_sync(c);
-    }
+    const uint32_t e = c->status->err;
     if (e) {
-        // Roll back to the last complete step.  Steps after the failing one
-        // were no-ops; the device step counters tell how many completed, which
-        // fixes the pair-state parity.  Repair flags and the error word are
+        // Rolled back to the last complete step (settle).  Steps after the
+        // failing one were no-ops.  Repair flags and the error word are
         // cleared so the caller can reserve more room and step again.
-        if (was_pending) {
-            c->parity = c->pend_parity ^ (int)((now - c->pend_done0) & 1);
-            bind_parity(c);
-        }
         HIPCHK(c, hipMemsetAsync(c->d.dirty, 0, c->S, c->stream));
         HIPCHK(c, hipMemsetAsync(c->d.err, 0, sizeof(uint32_t), c->stream));
         HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -2073,9 +2092,9 @@ static bool grow_for(godar_ctx* c, uint32_t bits) {
 
 int godar_step(godar_ctx* c, int32_t nsteps) {
     if (!c || nsteps < 0) return GODAR_ERR_ARG;
-    int64_t start = 0, now = 0;
-    int rc = steps_done(c, &start);
+    int rc = settle(c);
     if (rc != GODAR_OK) return rc;
+    const int64_t start = c->done;
     int32_t left = nsteps;
     for (int attempt = 0; attempt < 64; ++attempt) {
         rc = godar_step_async(c, left);
@@ -2083,9 +2102,7 @@ int godar_step(godar_ctx* c, int32_t nsteps) {
         rc = godar_sync(c);
         if (rc != GODAR_ERR_CAPACITY || !c->auto_grow) return rc;
         // some steps completed before the overflow: only the rest is retried
-        rc = steps_done(c, &now);
-        if (rc != GODAR_OK) return rc;
-        left = nsteps - (int32_t)(now - start);
+        left = nsteps - (int32_t)(c->done - start);
         std::string why = c->err;
         if (!grow_for(c, c->last_err_bits))
             return fail(c, GODAR_ERR_CAPACITY, why + " (capacity limit reached)");
@@ -2172,6 +2189,8 @@ int godar_get_bond_state(godar_ctx* c, int32_t m, int32_t cap, double* st, int32
 
 int godar_get_totals(godar_ctx* c, int64_t* out) {
     if (!c || !out) return GODAR_ERR_ARG;
+    int rc = settle(c);
+    if (rc != GODAR_OK) return rc;
     HIPCHK(c, hipStreamSynchronize(c->stream));
     int64_t* dout = nullptr;
     HIPCHK(c, hipMalloc(&dout, 5 * sizeof(int64_t)));
@@ -2209,6 +2228,8 @@ int godar_get_totals_noalloc(godar_ctx* c, int64_t* out) {
         return fail(c, GODAR_ERR_STATE, "get_totals_noalloc: call with the context's GPU current (" +
                                             std::to_string(c->device) + ")");
     int64_t* w = c->totals_scratch;
+    int rc = settle(c);
+    if (rc != GODAR_OK) return rc;
     HIPCHK(c, hipStreamSynchronize(c->stream));
     sync_ds(c);
     hipLaunchKernelGGL(k_zero_i64, dim3(1), dim3(64), 0, c->stream, w, GODAR_NTOTALS);

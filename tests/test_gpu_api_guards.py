@@ -181,3 +181,91 @@ def test_lists_of_a_member_that_left_are_not_walked(n):
         b.close()
     assert (t["candidates"], t["contacts"], t["bonds"]) == tuple(want[k] for k in kinds)
     a.close()
+
+
+def _copy_bonds(ctx, m, f):
+    i, j = ctx.pairs(m, "bond")
+    s = ctx.bond_state(m)
+    ctx.set_bonds(m, i, j, np.stack([s[k] for k in s], axis=1))
+
+
+UNSYNCED = {
+    "floes": lambda c, m, f, p: c.floes(m),
+    "forces": lambda c, m, f, p: c.forces(m),
+    "walls": lambda c, m, f, p: c.walls(m),
+    "pairs": lambda c, m, f, p: {str(k): v for k in ("candidate", "contact", "bond")
+                                 for k, v in enumerate(c.pairs(m, k))},
+    "totals": lambda c, m, f, p: c.totals(),
+    "stats": lambda c, m, f, p: c.stats(m),
+    "tstep": lambda c, m, f, p: {"t": c.tstep(m), "all": c.tsteps()},
+    "checkpoint": lambda c, m, f, p: {"block": np.frombuffer(c.checkpoint(m, p), np.uint8)},
+    "remove": lambda c, m, f, p: c.remove(m) or {},
+    "add": lambda c, m, f, p: {"m": c.add_field(p, f)},
+    "restore": lambda c, m, f, p: {"m": c.restore(c.checkpoint(m, p))},
+    "run_until": lambda c, m, f, p: c.run_until(m, 12) or {},
+    "set_forcing": lambda c, m, f, p: c.set_forcing(m, -9.0, 4.0, 0.1, -0.2) or {},
+    "set_bonds": lambda c, m, f, p: _copy_bonds(c, m, f) or {},
+    "reserve": lambda c, m, f, p: c.reserve(hist=48) or {},
+    "search": lambda c, m, f, p: c.set_search(0.05, 2, 0) or {},
+    "step": lambda c, m, f, p: c.step(3) or {},
+}
+
+
+@pytest.mark.parametrize("k", [2, 3, 8])
+@pytest.mark.parametrize("call", list(UNSYNCED))
+def test_calls_after_step_async_see_its_steps(call, k):
+    """With no skin every step needs a build, so the launches behind the second
+    step of a run do nothing (an odd or an even number of them) until
+    they are run again: every call that reads or writes state in between gives
+    and leaves what it does after godar_sync."""
+    f, p = _box()
+    mate = kick(squeeze(packed_box(50, 11)), 4)
+    pm = config0_params(mate, sigmanc_crit=1e5)
+    out = []
+    for sync in (True, False):
+        c = _ctx(2 * f.n + mate.n, 3)
+        c.set_skin(0.0)
+        m, mm = c.add_field(p, f), c.add_field(pm, mate)
+        c.step(1)
+        c.step_async(k)
+        if sync:
+            c.sync()
+        got = UNSYNCED[call](c, m, f, p)
+        c.sync()
+        c.step(5)
+        out.append([got, c.tsteps()] + [c.floes(x) for x in (m, mm) if c.tsteps()[x] > 0])
+        c.close()
+    for a, b in zip(*out):
+        if isinstance(a, dict):
+            assert a.keys() == b.keys()
+            for key in a:
+                assert np.array_equal(a[key], b[key]), key
+        else:
+            assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("k", [30, 31])
+def test_state_after_an_unsynced_capacity_error(k):
+    """An asynchronous run that ends at a full history list: the state read
+    before godar_sync is that of its last complete step, and godar_sync still
+    reports the error."""
+    f = kick(packed_box(64, 3), 1)      # (gaps of half a metre: no contact in the first step)
+    p = config0_params(f, sigmanc_crit=1e5)
+    a, b = _ctx(f.n), _ctx(f.n)
+    ma, mb = a.add_field(p, f), b.add_field(p, f)
+    a.reserve(hist=1)
+    a.step_async(k)
+    got, t = a.floes(ma), a.tstep(ma)
+    with pytest.raises(_lib.GodarError) as e:
+        a.sync()
+    assert e.value.code == _lib.GODAR_ERR_CAPACITY and 1 < t <= k
+    b.step(t - 1)
+    want = b.floes(mb)
+    for key in STATE:
+        assert np.array_equal(got[key], want[key]), key
+    a.reserve(hist=16)
+    a.step(k + 1 - t)
+    b.step(k + 1 - t)
+    _same(a, b, ma, mb)
+    a.close()
+    b.close()
