@@ -31,7 +31,7 @@ template <bool M> __global__ void k_walls(DS);
 template <bool M> __global__ void k_repair(DS, int);
 template <bool M> __global__ void k_fixup(DS);
 template <bool M, bool R> __global__ void k_final(DS);
-__global__ void k_totals(DS, int64_t*);
+__global__ void k_totals(DS, int, int64_t*);
 __global__ void k_status(DS, int, HostStatus*);
 __global__ void k_admit(DS, int, int, int, int, const FloeRec*, const int32_t*);
 template <int W> __global__ void k_read(DS, int, int, int, double*);
@@ -184,6 +184,11 @@ struct godar_ctx {
     unsigned char* stage = nullptr;
     hipEvent_t estage[2] = {nullptr, nullptr};
     int64_t done = 0;                   // steps completed, as of the last settle
+    // The candidate and contact lists, the supersets and the reshape records
+    // are those of one step that completed.  A step that fails leaves parts of
+    // its own (and the host may replace the pools they are in), in an order
+    // that may differ from the positions': nothing follows them then.
+    bool lists = false;
 };
 
 namespace {
@@ -436,6 +441,8 @@ int settle(godar_ctx* c) {
         c->builds = c->status->builds;
         c->soon = c->status->due != 0;
         if (!c->soon) c->lean_run = 0;
+        if (now > c->done) c->lists = true;
+        if (e && e != ERR_NEED_BUILD) c->lists = false;
         c->done = now;
         if (!e) {
             c->pending = false;
@@ -522,6 +529,9 @@ int read_pairs(godar_ctx* c, int32_t m, bool want, const PairOut** list, std::ve
     if (rc == GODAR_OK) rc = ensure_stage(c);
     if (rc != GODAR_OK) return rc;
     sync_ds(c);
+    *list = nullptr;
+    *n = 0;
+    if (K != PAIRS_BOND && !c->lists) return GODAR_OK;
     auto pass = [&](PairOut* out, int cap) -> hipError_t {
         if (c->N_used > 0)
             hipLaunchKernelGGL(k_pairs<K>, dim3((c->N_used + 255) / 256), dim3(256), 0, c->stream, c->d, m, out, cap);
@@ -2198,7 +2208,7 @@ int godar_get_totals(godar_ctx* c, int64_t* out) {
     // (on the context's stream, which the null stream's memset would not wait for)
     hipLaunchKernelGGL(k_zero_i64, dim3(1), dim3(64), 0, c->stream, dout, 5);
     if (c->N_used > 0)
-        hipLaunchKernelGGL(k_totals, dim3((c->N_used + 255) / 256), dim3(256), 0, c->stream, c->d, dout);
+        hipLaunchKernelGGL(k_totals, dim3((c->N_used + 255) / 256), dim3(256), 0, c->stream, c->d, c->lists ? 1 : 0, dout);
     hipLaunchKernelGGL(k_member_totals, dim3(1), dim3(256), 0, c->stream, c->d, c->Mcap, dout + 3);
     hipError_t e = hipStreamSynchronize(c->stream);
     if (e == hipSuccess) e = hipMemcpy(out, dout, 3 * sizeof(int64_t), hipMemcpyDeviceToHost);
@@ -2234,7 +2244,7 @@ int godar_get_totals_noalloc(godar_ctx* c, int64_t* out) {
     sync_ds(c);
     hipLaunchKernelGGL(k_zero_i64, dim3(1), dim3(64), 0, c->stream, w, GODAR_NTOTALS);
     if (c->N_used > 0)
-        hipLaunchKernelGGL(k_totals, dim3((c->N_used + 255) / 256), dim3(256), 0, c->stream, c->d, w);
+        hipLaunchKernelGGL(k_totals, dim3((c->N_used + 255) / 256), dim3(256), 0, c->stream, c->d, c->lists ? 1 : 0, w);
     hipLaunchKernelGGL(k_queue_totals, dim3(1), dim3(64), 0, c->stream, c->d.qn_next, w + 3);
     hipLaunchKernelGGL(k_member_totals, dim3(1), dim3(256), 0, c->stream, c->d, c->Mcap, w + 6);
     HIPCHK(c, hipGetLastError());

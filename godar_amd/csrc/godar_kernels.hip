@@ -2989,12 +2989,14 @@ __device__ __forceinline__ void each_candidate(const DS& S, int k, const GeoRec&
     }
 }
 
-// totals of the last step: candidates, contacts (evf flags) and current
-// bonds; diagnostics only
-__global__ void k_totals(DS S, int64_t* out) {
+// totals of the last step: candidates, contacts (evf flags; `lists`: the
+// step's lists are there to read) and current bonds, of the members that take
+// steps; diagnostics only.  Thread k: position k's lists, storage slot k's
+// bonds.
+__global__ void k_totals(DS S, int lists, int64_t* out) {
     int k = blockIdx.x * blockDim.x + threadIdx.x;
     int64_t c = 0, ct = 0, bd = 0;
-    const GeoRec me = k < S.N ? S.geo_new[k] : GeoRec{0.0, 0.0, 0.0, 0, -1};
+    const GeoRec me = lists && k < S.N ? S.geo_new[k] : GeoRec{0.0, 0.0, 0.0, 0, -1};
     if (still_there(S, me, k)) {
         const int no = S.ocnt[k];
         each_candidate(S, k, me, [&](int) { ++c; });
@@ -3003,10 +3005,11 @@ __global__ void k_totals(DS S, int64_t* out) {
             if (fl & EV_REMOVED) continue;
             if (fl & EV_CONTACT) ++ct;
         }
-        const int f = S.sid_of[me.id];
-        int nb = S.bcnt_old[f];
+    }
+    if (k < S.N && S.member_of[k] >= 0 && S.pos_of[k] >= 0 && S.geo[S.pos_of[k]].member == S.member_of[k]) {
+        int nb = S.bcnt_old[k];
         for (int q = 0; q < nb; ++q) {
-            const BondRec& b = S.bond_old[(int64_t)q * S.S + f];
+            const BondRec& b = S.bond_old[(int64_t)q * S.S + k];
             if (b.j >= 0 && b.bond == 1) ++bd;
         }
     }

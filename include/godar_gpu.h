@@ -185,7 +185,9 @@ int godar_get_forces(godar_ctx *ctx, int32_t member, double *f);
 /* Wall histories (4, n): deltat_bc1 deltat_bc2 theta_bc1 theta_bc2. */
 int godar_get_walls(godar_ctx *ctx, int32_t member, double *w);
 /* Pair lists of a member, canonically sorted by (i, j), 0-based member-local
- * indices.  Writes up to cap pairs, *count gets the total. */
+ * indices.  Writes up to cap pairs, *count gets the total.  Candidates and
+ * contacts are those of the last step; after a step that failed there are
+ * none (here and in the statistics and totals) until a step completes. */
 int godar_get_pairs(godar_ctx *ctx, int32_t member, int32_t kind, int32_t cap, int32_t *pi,
                     int32_t *pj, int32_t *count);
 /* Bond state of the member's bonds (same order as GODAR_PAIRS_BOND),

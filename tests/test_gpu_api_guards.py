@@ -269,3 +269,52 @@ def test_state_after_an_unsynced_capacity_error(k):
     _same(a, b, ma, mb)
     a.close()
     b.close()
+
+
+def test_lists_after_a_step_that_failed():
+    """A step that ends at a full superset pool (the context's first, before
+    any lists are built) or history list (after steps that completed) leaves
+    no candidates or contacts to read until a step completes; bonds are those
+    of the last complete step; the run then goes on as a twin's."""
+    f, p = _box()
+    p.rtree = 1.0e5                     # every floe is a candidate of every other: 63 a floe, room for 8
+    a, b = _ctx(f.n), _ctx(f.n)
+    ma, mb = a.add_field(p, f), b.add_field(p, f)
+    a.step_async(3)
+    for _ in range(2):
+        t = a.totals()
+        assert (t["candidates"], t["contacts"], t["bonds"]) == (0, 0, 0)
+        for k in ("candidate", "contact", "bond"):
+            assert a.pairs(ma, k)[0].size == 0, k
+        if _ == 0:
+            with pytest.raises(_lib.GodarError) as e:
+                a.sync()
+            assert "superset" in str(e.value)
+    a.step(3)
+    b.step(3)
+    assert a.totals() == b.totals() and a.totals()["candidates"] > 0
+    _same(a, b, ma, mb)
+    a.close()
+    b.close()
+    f = kick(packed_box(64, 3), 1)
+    p = config0_params(f, sigmanc_crit=1e5, bond_lim=50.0, bond_frac=0.1)
+    a, b = _ctx(f.n), _ctx(f.n)
+    ma, mb = a.add_field(p, f), b.add_field(p, f)
+    a.reserve(hist=1)
+    a.step_async(200)
+    with pytest.raises(_lib.GodarError):
+        a.sync()
+    done = a.tstep(ma) - 1
+    assert 0 < done < 200
+    b.step(done)
+    t = a.totals()
+    assert (t["candidates"], t["contacts"]) == (0, 0)
+    assert a.stats(ma)["candidates"] == 0 and a.pairs(ma, "contact")[0].size == 0
+    assert t["bonds"] == b.totals()["bonds"] > 0
+    assert [x.tolist() for x in a.pairs(ma, "bond")] == [x.tolist() for x in b.pairs(mb, "bond")]
+    a.step(5)                            # (the list grows)
+    b.step(5)
+    assert a.totals() == b.totals() and a.totals()["contacts"] > 0
+    _same(a, b, ma, mb)
+    a.close()
+    b.close()
