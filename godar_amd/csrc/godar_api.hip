@@ -35,7 +35,7 @@ __global__ void k_totals(DS, int, int64_t*);
 __global__ void k_status(DS, int, HostStatus*);
 __global__ void k_admit(DS, int, int, int, int, const FloeRec*, const int32_t*);
 template <int W> __global__ void k_read(DS, int, int, int, double*);
-template <int K> __global__ void k_pairs(DS, int, PairOut*, int);
+template <int K> __global__ void k_pairs(DS, int, int, PairOut*, int);
 __global__ void k_take_count(int32_t*, int32_t*);
 
 __global__ void k_fill_u8(uint8_t* p, int64_t n, uint8_t v) {
@@ -109,6 +109,9 @@ struct godar_ctx {
     int record = 0;
     int parity = 0;
     int32_t N_used = 0;
+    // floe slots in use at the last step launched: its positions, which stand
+    // until the next build whatever N_used becomes
+    int32_t N_pos = 0;
     int32_t ncells_cap = 0;
     std::vector<Member> members;
     std::vector<DevParams> dparams;
@@ -533,8 +536,8 @@ int read_pairs(godar_ctx* c, int32_t m, bool want, const PairOut** list, std::ve
     *n = 0;
     if (K != PAIRS_BOND && !c->lists) return GODAR_OK;
     auto pass = [&](PairOut* out, int cap) -> hipError_t {
-        if (c->N_used > 0)
-            hipLaunchKernelGGL(k_pairs<K>, dim3((c->N_used + 255) / 256), dim3(256), 0, c->stream, c->d, m, out, cap);
+        const int nt = std::max(c->N_pos, c->members[m].n);      // (a thread per position, or floe)
+        hipLaunchKernelGGL(k_pairs<K>, dim3((nt + 255) / 256), dim3(256), 0, c->stream, c->d, m, c->N_pos, out, cap);
         hipLaunchKernelGGL(k_take_count, dim3(1), dim3(1), 0, c->stream, c->d.npairs, &c->status->npairs);
         hipError_t e = hipGetLastError();
         if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
@@ -1709,19 +1712,19 @@ int godar_reserve(godar_ctx* c, int32_t outer, int32_t inner, int32_t histc, int
     // The kernels walk a floe's records up to its count, and the last step's
     // candidate lists stay readable (godar_get_pairs): a list may shrink only
     // down to the longest one in use.
-    auto longest = [&](const int32_t* cnt, int32_t& mx) -> int {
+    auto longest = [&](const int32_t* cnt, int32_t n, int32_t& mx) -> int {
         mx = 0;
-        if (c->N_used == 0) return GODAR_OK;
-        std::vector<int32_t> h(c->N_used);
-        HIPCHK(c, hipMemcpy(h.data(), cnt, sizeof(int32_t) * c->N_used, hipMemcpyDeviceToHost));
+        if (n == 0) return GODAR_OK;
+        std::vector<int32_t> h(n);
+        HIPCHK(c, hipMemcpy(h.data(), cnt, sizeof(int32_t) * n, hipMemcpyDeviceToHost));
         for (int32_t v : h) mx = std::max(mx, v);
         return GODAR_OK;
     };
     int32_t mo = 0, mi = 0, mh = 0, mb = 0;
-    if (nCO < c->CO && (rc = longest(c->d.ocnt, mo)) != GODAR_OK) return rc;
-    if (nCI < c->CI && (rc = longest(c->d.icnt, mi)) != GODAR_OK) return rc;
-    if (nHC < c->HC && (rc = longest(c->hcnt[o], mh)) != GODAR_OK) return rc;
-    if (nBC < c->BC && (rc = longest(c->bcnt[o], mb)) != GODAR_OK) return rc;
+    if (nCO < c->CO && (rc = longest(c->d.ocnt, c->N_pos, mo)) != GODAR_OK) return rc;
+    if (nCI < c->CI && (rc = longest(c->d.icnt, c->N_pos, mi)) != GODAR_OK) return rc;
+    if (nHC < c->HC && (rc = longest(c->hcnt[o], c->N_used, mh)) != GODAR_OK) return rc;
+    if (nBC < c->BC && (rc = longest(c->bcnt[o], c->N_used, mb)) != GODAR_OK) return rc;
     if (nCO < mo || nCI < mi || nHC < mh || nBC < mb)
         return fail(c, GODAR_ERR_ARG,
                     "reserve: a capacity is below the entries a floe holds (outer " + std::to_string(mo) +
@@ -2015,6 +2018,7 @@ int godar_step_async(godar_ctx* c, int32_t nsteps) {
         c->need_full = c->soon = false;
         c->lean_run = lean ? c->lean_run + 1 : 0;
         if (c->full_hold > 0 && !lean) --c->full_hold;
+        if (c->N_used > 0) c->N_pos = c->N_used;
         ++c->pend_launched;
     }
     return GODAR_OK;
@@ -2207,8 +2211,9 @@ int godar_get_totals(godar_ctx* c, int64_t* out) {
     sync_ds(c);
     // (on the context's stream, which the null stream's memset would not wait for)
     hipLaunchKernelGGL(k_zero_i64, dim3(1), dim3(64), 0, c->stream, dout, 5);
-    if (c->N_used > 0)
-        hipLaunchKernelGGL(k_totals, dim3((c->N_used + 255) / 256), dim3(256), 0, c->stream, c->d, c->lists ? 1 : 0, dout);
+    const int nt = std::max(c->N_pos, c->N_used);      // (a thread per position and storage slot)
+    if (nt > 0)
+        hipLaunchKernelGGL(k_totals, dim3((nt + 255) / 256), dim3(256), 0, c->stream, c->d, c->lists ? c->N_pos : 0, dout);
     hipLaunchKernelGGL(k_member_totals, dim3(1), dim3(256), 0, c->stream, c->d, c->Mcap, dout + 3);
     hipError_t e = hipStreamSynchronize(c->stream);
     if (e == hipSuccess) e = hipMemcpy(out, dout, 3 * sizeof(int64_t), hipMemcpyDeviceToHost);
@@ -2243,8 +2248,9 @@ int godar_get_totals_noalloc(godar_ctx* c, int64_t* out) {
     HIPCHK(c, hipStreamSynchronize(c->stream));
     sync_ds(c);
     hipLaunchKernelGGL(k_zero_i64, dim3(1), dim3(64), 0, c->stream, w, GODAR_NTOTALS);
-    if (c->N_used > 0)
-        hipLaunchKernelGGL(k_totals, dim3((c->N_used + 255) / 256), dim3(256), 0, c->stream, c->d, c->lists ? 1 : 0, w);
+    const int nt = std::max(c->N_pos, c->N_used);      // (a thread per position and storage slot)
+    if (nt > 0)
+        hipLaunchKernelGGL(k_totals, dim3((nt + 255) / 256), dim3(256), 0, c->stream, c->d, c->lists ? c->N_pos : 0, w);
     hipLaunchKernelGGL(k_queue_totals, dim3(1), dim3(64), 0, c->stream, c->d.qn_next, w + 3);
     hipLaunchKernelGGL(k_member_totals, dim3(1), dim3(256), 0, c->stream, c->d, c->Mcap, w + 6);
     HIPCHK(c, hipGetLastError());

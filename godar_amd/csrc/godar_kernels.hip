@@ -2989,14 +2989,14 @@ __device__ __forceinline__ void each_candidate(const DS& S, int k, const GeoRec&
     }
 }
 
-// totals of the last step: candidates, contacts (evf flags; `lists`: the
-// step's lists are there to read) and current bonds, of the members that take
-// steps; diagnostics only.  Thread k: position k's lists, storage slot k's
-// bonds.
-__global__ void k_totals(DS S, int lists, int64_t* out) {
+// totals of the last step: candidates, contacts (evf flags) and current bonds,
+// of the members that take steps; diagnostics only.  Thread k: position k's
+// lists (of the step's np positions; 0: there are no lists to read), storage
+// slot k's bonds.
+__global__ void k_totals(DS S, int np, int64_t* out) {
     int k = blockIdx.x * blockDim.x + threadIdx.x;
     int64_t c = 0, ct = 0, bd = 0;
-    const GeoRec me = lists && k < S.N ? S.geo_new[k] : GeoRec{0.0, 0.0, 0.0, 0, -1};
+    const GeoRec me = k < np ? S.geo_new[k] : GeoRec{0.0, 0.0, 0.0, 0, -1};
     if (still_there(S, me, k)) {
         const int no = S.ocnt[k];
         each_candidate(S, k, me, [&](int) { ++c; });
@@ -3074,14 +3074,15 @@ __global__ __launch_bounds__(64) void k_read(DS S, int m, int begin, int count, 
 
 // Member m's pairs of the last step, in the caller's indices, in no order:
 // counted in *S.npairs, the first `cap` written to `out`.  Candidates come
-// from the supersets (thread k: position k), contacts from the step's lists
-// and bonds from the owners' records (thread k: the member's k-th floe).
+// from the supersets (thread k: position k of the step's np, which may be more
+// than the floe slots in use now), contacts from the step's lists and bonds
+// from the owners' records (thread k: the member's k-th floe).
 template <int K>
-__global__ void k_pairs(DS S, int m, PairOut* out, int cap) {
+__global__ void k_pairs(DS S, int m, int np, PairOut* out, int cap) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     const Member mb = S.members[m];
     if (K == PAIRS_CANDIDATE) {
-        if (k >= S.N) return;
+        if (k >= np) return;
         const GeoRec me = S.geo_new[k];
         if (me.member != m || !still_there(S, me, k)) return;
         each_candidate(S, k, me, [&](int j) {
@@ -3094,7 +3095,7 @@ __global__ void k_pairs(DS S, int m, PairOut* out, int cap) {
     const int f = mb.first + k, i = S.gid_of[f] - mb.first;
     if (K == PAIRS_CONTACT) {
         const int q = S.pos_of[f];
-        if ((uint32_t)q >= (uint32_t)S.N) return;      // (-1: the member's first step is to come)
+        if ((uint32_t)q >= (uint32_t)np) return;       // (-1: the member's first step is to come)
         const int no = min(S.ocnt[q], S.CO);
         for (int s = 0; s < no; ++s) {
             const int64_t at0 = (int64_t)s * S.S + q;
@@ -3168,9 +3169,9 @@ __global__ void k_status(DS S, int nmembers, HostStatus* out) {
 template __global__ void k_read<READ_FLOES>(DS, int, int, int, double*);
 template __global__ void k_read<READ_FORCES>(DS, int, int, int, double*);
 template __global__ void k_read<READ_WALLS>(DS, int, int, int, double*);
-template __global__ void k_pairs<PAIRS_CANDIDATE>(DS, int, PairOut*, int);
-template __global__ void k_pairs<PAIRS_CONTACT>(DS, int, PairOut*, int);
-template __global__ void k_pairs<PAIRS_BOND>(DS, int, PairOut*, int);
+template __global__ void k_pairs<PAIRS_CANDIDATE>(DS, int, int, PairOut*, int);
+template __global__ void k_pairs<PAIRS_CONTACT>(DS, int, int, PairOut*, int);
+template __global__ void k_pairs<PAIRS_BOND>(DS, int, int, PairOut*, int);
 template __global__ void k_sup<false>(DS);
 template __global__ void k_sup<true>(DS);
 template __global__ void k_sup_dense<false>(DS);

@@ -318,3 +318,40 @@ def test_lists_after_a_step_that_failed():
     _same(a, b, ma, mb)
     a.close()
     b.close()
+
+
+def test_pair_lists_after_the_last_storage_slots_are_freed():
+    """A member whose floes came first in the cell order but last in storage
+    leaves: the other's pair lists, totals and list capacities are what they
+    were, though its positions are past the floe slots in use now."""
+    f, p = _box()                                  # (first: 64 slots and cells enough for the guest)
+    mate, guest = kick(squeeze(packed_box(64, 11)), 4), kick(squeeze(packed_box(70, 12)), 5)
+    pm = config0_params(mate, sigmanc_crit=1e5)
+    pg = config0_params(guest, sigmanc_crit=1e5, rtree=9000.0)       # (a few large cells)
+    a, b = _ctx(f.n + mate.n + guest.n, 2), _ctx(mate.n)
+    ma, mm = a.add_field(p, f), a.add_field(pm, mate)
+    mb = b.add_field(pm, mate)
+    a.remove(ma)
+    mg = a.add_field(pg, guest)
+    a.step(12)
+    b.step(12)
+    kinds = ("candidate", "contact", "bond")
+    want = [[x.tolist() for x in b.pairs(mb, k)] for k in kinds]
+    assert len(want[0][0]) > 0 and len(want[1][0]) > 0
+    for gone in (False, True):
+        if gone:
+            a.remove(mg)
+            assert a.totals()["candidates"] == len(want[0][0])
+            assert a.totals()["contacts"] == len(want[1][0])
+            with pytest.raises(_lib.GodarError) as e:
+                a.reserve(outer=1)
+            assert e.value.code == _lib.GODAR_ERR_ARG
+        for k, w in zip(kinds, want):
+            assert [x.tolist() for x in a.pairs(mm, k)] == w, (gone, k)
+        s = a.stats(mm)
+        assert (s["candidates"], s["contacts"]) == (len(want[0][0]), len(want[1][0]))
+    a.step(5)
+    b.step(5)
+    _same(a, b, mm, mb)
+    a.close()
+    b.close()
