@@ -11,6 +11,7 @@
 #include <cstdio>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -35,7 +36,7 @@ __global__ void k_totals(DS, int, int64_t*);
 __global__ void k_status(DS, int, HostStatus*);
 __global__ void k_admit(DS, int, int, int, int, const FloeRec*, const int32_t*);
 template <int W> __global__ void k_read(DS, int, int, int, double*);
-template <int K> __global__ void k_pairs(DS, int, int, PairOut*, int);
+template <int K> __global__ void k_pairs(DS, int, int, int, int, typename PairKind<K>::Out*, int);
 __global__ void k_take_count(int32_t*, int32_t*);
 
 __global__ void k_fill_u8(uint8_t* p, int64_t n, uint8_t v) {
@@ -524,56 +525,61 @@ int read_rows(godar_ctx* c, int32_t m, int rows, double* const* dst) {
     return GODAR_OK;
 }
 
-// Member m's pairs of kind K (PAIRS_*): counted into *n, and where `want`
-// listed, in no order, in the staging area or, past its room, in `more`.
+// Member m's pairs of kind K (PAIRS_*) in order, for a caller with room for
+// `cap` of them; without room only counted.  They come through the staging
+// area, so a list of any length takes no device memory and one host copy: the
+// whole list at once where it fits (524,288 pairs, 43,690 bonds), else as many
+// floes at a time as fill about three quarters of the room, and the list of one
+// floe that is longer than it in parts.
 template <int K>
-int read_pairs(godar_ctx* c, int32_t m, bool want, const PairOut** list, std::vector<PairOut>& more, int* n) {
+int ordered_pairs(godar_ctx* c, int32_t m, int32_t cap, std::vector<typename PairKind<K>::Out>& out, int32_t* count) {
+    using Out = typename PairKind<K>::Out;
     int rc = settle(c);
     if (rc == GODAR_OK) rc = ensure_stage(c);
     if (rc != GODAR_OK) return rc;
-    sync_ds(c);
-    *list = nullptr;
-    *n = 0;
+    *count = 0;
     if (K != PAIRS_BOND && !c->lists) return GODAR_OK;
-    auto pass = [&](PairOut* out, int cap) -> hipError_t {
-        const int nt = std::max(c->N_pos, c->members[m].n);      // (a thread per position, or floe)
-        hipLaunchKernelGGL(k_pairs<K>, dim3((nt + 255) / 256), dim3(256), 0, c->stream, c->d, m, c->N_pos, out, cap);
-        hipLaunchKernelGGL(k_take_count, dim3(1), dim3(1), 0, c->stream, c->d.npairs, &c->status->npairs);
-        hipError_t e = hipGetLastError();
-        if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-        *n = c->status->npairs;
-        return e;
-    };
-    const int room = want ? (int)(STAGE_BYTES / sizeof(PairOut)) : 0;
-    *list = reinterpret_cast<const PairOut*>(c->stage);
-    HIPCHK(c, pass(reinterpret_cast<PairOut*>(c->stage), room));
-    if (!want || *n <= room) return GODAR_OK;
-    more.resize(*n);
-    const int cap = *n;
-    PairOut* dev = nullptr;
-    hipError_t e = hipMalloc(&dev, sizeof(PairOut) * cap);
-    if (e == hipSuccess) e = pass(dev, cap);
-    if (e == hipSuccess) e = hipMemcpy(more.data(), dev, sizeof(PairOut) * cap, hipMemcpyDeviceToHost);
-    (void)hipFree(dev);
-    HIPCHK(c, e);
-    *list = more.data();
-    return GODAR_OK;
-}
-
-// Member m's pairs of kind K in order, those wanted by a caller with room for
-// `cap` of them; without room only counted.
-template <int K>
-int ordered_pairs(godar_ctx* c, int32_t m, int32_t cap, std::vector<PairOut>& out, int32_t* count) {
-    const PairOut* list = nullptr;
-    std::vector<PairOut> more;
+    sync_ds(c);
+    const Out* stage = reinterpret_cast<const Out*>(c->stage);
+    const int room = cap > 0 ? (int)(STAGE_BYTES / sizeof(Out)) : 0;
+    // (positions, or the member's floes)
+    const int items = K == PAIRS_CANDIDATE ? c->N_pos : c->members[m].n;
     int n = 0;
-    int rc = read_pairs<K>(c, m, cap > 0, &list, more, &n);
-    if (rc != GODAR_OK) return rc;
-    *count = n;
-    if (cap > 0) out.assign(list, list + n);
-    std::sort(out.begin(), out.end(), [](const PairOut& a, const PairOut& b) {
-        return a.i != b.i ? a.i < b.i : a.j < b.j;
-    });
+    // the pairs of items [b, e): n of them, those from number `skip` on listed
+    auto pass = [&](int b, int e, int skip) -> hipError_t {
+        hipLaunchKernelGGL(k_pairs<K>, dim3((e - b + 255) / 256), dim3(256), 0, c->stream, c->d, m, b, e, skip,
+                           reinterpret_cast<Out*>(c->stage), room);
+        hipLaunchKernelGGL(k_take_count, dim3(1), dim3(1), 0, c->stream, c->d.npairs, &c->status->npairs);
+        hipError_t x = hipGetLastError();
+        if (x == hipSuccess) x = hipStreamSynchronize(c->stream);
+        n = c->status->npairs;
+        return x;
+    };
+    try {
+        HIPCHK(c, pass(0, items, 0));
+        *count = n;
+        if (cap == 0) return GODAR_OK;
+        out.reserve(n);
+        if (n <= room) {
+            out.assign(stage, stage + n);
+        } else {
+            int part = std::max(1, (int)((int64_t)items * room / n * 3 / 4));
+            for (int b = 0; b < items;) {
+                const int e = std::min(items, b + part);
+                HIPCHK(c, pass(b, e, 0));
+                if (n > room && e - b > 1) { part = (e - b) / 2; continue; }
+                out.insert(out.end(), stage, stage + std::min(n, room));
+                for (int at = room; at < n; at += room) {        // (one floe: listed in the same order again)
+                    HIPCHK(c, pass(b, e, at));
+                    out.insert(out.end(), stage, stage + std::min(n - at, room));
+                }
+                b = e;
+            }
+        }
+    } catch (const std::bad_alloc&) {
+        return fail(c, GODAR_ERR_NOMEM, "read-back: out of host memory for the pair list");
+    }
+    std::sort(out.begin(), out.end(), [](const Out& a, const Out& b) { return a.i != b.i ? a.i < b.i : a.j < b.j; });
     if ((int64_t)out.size() > cap) out.resize(cap);
     return GODAR_OK;
 }
@@ -2180,21 +2186,23 @@ int godar_get_pairs(godar_ctx* c, int32_t m, int32_t kind, int32_t cap, int32_t*
                     int32_t* count) {
     if (!valid_member(c, m) || !count || cap < 0 || (cap > 0 && (!pi || !pj)))
         return fail(c, GODAR_ERR_ARG, "get_pairs: bad argument");
-    std::vector<PairOut> out;
-    int rc;
-    if (kind == GODAR_PAIRS_CANDIDATE) rc = ordered_pairs<PAIRS_CANDIDATE>(c, m, cap, out, count);
-    else if (kind == GODAR_PAIRS_CONTACT) rc = ordered_pairs<PAIRS_CONTACT>(c, m, cap, out, count);
-    else if (kind == GODAR_PAIRS_BOND) rc = ordered_pairs<PAIRS_BOND>(c, m, cap, out, count);
-    else return fail(c, GODAR_ERR_ARG, "get_pairs: bad kind");
-    if (rc != GODAR_OK) return rc;
-    for (size_t k = 0; k < out.size(); ++k) { pi[k] = out[k].i; pj[k] = out[k].j; }
-    return GODAR_OK;
+    auto list = [&](auto&& out, int rc) -> int {
+        if (rc != GODAR_OK) return rc;
+        for (size_t k = 0; k < out.size(); ++k) { pi[k] = out[k].i; pj[k] = out[k].j; }
+        return GODAR_OK;
+    };
+    std::vector<PairOut> pairs;
+    std::vector<BondOut> bonds;
+    if (kind == GODAR_PAIRS_CANDIDATE) return list(pairs, ordered_pairs<PAIRS_CANDIDATE>(c, m, cap, pairs, count));
+    if (kind == GODAR_PAIRS_CONTACT) return list(pairs, ordered_pairs<PAIRS_CONTACT>(c, m, cap, pairs, count));
+    if (kind == GODAR_PAIRS_BOND) return list(bonds, ordered_pairs<PAIRS_BOND>(c, m, cap, bonds, count));
+    return fail(c, GODAR_ERR_ARG, "get_pairs: bad kind");
 }
 
 int godar_get_bond_state(godar_ctx* c, int32_t m, int32_t cap, double* st, int32_t* count) {
     if (!valid_member(c, m) || !count || cap < 0 || (cap > 0 && !st))
         return fail(c, GODAR_ERR_ARG, "get_bond_state: bad argument");
-    std::vector<PairOut> out;
+    std::vector<BondOut> out;
     int rc = ordered_pairs<PAIRS_BOND>(c, m, cap, out, count);
     if (rc != GODAR_OK) return rc;
     for (size_t k = 0; k < out.size(); ++k) std::memcpy(st + 11 * k, out[k].v, sizeof(out[k].v));

@@ -190,9 +190,12 @@ struct HostStatus {
 enum { READ_FLOES, READ_FORCES, READ_WALLS };
 enum { PAIRS_CANDIDATE, PAIRS_CONTACT, PAIRS_BOND };
 constexpr int NFORCE = 33;
-struct PairOut {
-    int32_t i, j;              // in the caller's indices
-    double v[11];              // PAIRS_BOND: the bond's state, as godar_set_bonds takes it
+struct PairOut { int32_t i, j; };   // in the caller's indices
+struct BondOut {
+    int32_t i, j;
+    double v[11];              // the bond's state, as godar_set_bonds takes it
 };
+template <int K> struct PairKind { using Out = PairOut; };
+template <> struct PairKind<PAIRS_BOND> { using Out = BondOut; };
 
 }  // namespace godar

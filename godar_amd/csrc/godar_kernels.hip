@@ -3073,45 +3073,46 @@ __global__ __launch_bounds__(64) void k_read(DS S, int m, int begin, int count, 
 }
 
 // Member m's pairs of the last step, in the caller's indices, in no order:
-// counted in *S.npairs, the first `cap` written to `out`.  Candidates come
-// from the supersets (thread k: position k of the step's np, which may be more
-// than the floe slots in use now), contacts from the step's lists and bonds
-// from the owners' records (thread k: the member's k-th floe).
+// counted in *S.npairs, those from number `skip` on, up to `cap`, written to
+// `out`.  Candidates come from the supersets (thread k: position b + k of the
+// step's [b, e), which may be more than the floe slots in use now), contacts
+// from the step's lists and bonds from the owners' records (thread k: floe
+// b + k of the member's [b, e)).
 template <int K>
-__global__ void k_pairs(DS S, int m, int np, PairOut* out, int cap) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void k_pairs(DS S, int m, int b, int e, int skip, typename PairKind<K>::Out* out, int cap) {
+    const int k = b + blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= e) return;
     const Member mb = S.members[m];
     if (K == PAIRS_CANDIDATE) {
-        if (k >= np) return;
         const GeoRec me = S.geo_new[k];
         if (me.member != m || !still_there(S, me, k)) return;
         each_candidate(S, k, me, [&](int j) {
-            const int at = atomicAdd(S.npairs, 1);
-            if (at < cap) { out[at].i = me.id - mb.first; out[at].j = j - mb.first; }
+            const int at = atomicAdd(S.npairs, 1) - skip;
+            if (at >= 0 && at < cap) { out[at].i = me.id - mb.first; out[at].j = j - mb.first; }
         });
         return;
     }
-    if (k >= mb.n) return;
     const int f = mb.first + k, i = S.gid_of[f] - mb.first;
     if (K == PAIRS_CONTACT) {
         const int q = S.pos_of[f];
-        if ((uint32_t)q >= (uint32_t)np) return;       // (-1: the member's first step is to come)
+        if (q < 0) return;                                  // (the member's first step is to come)
         const int no = min(S.ocnt[q], S.CO);
         for (int s = 0; s < no; ++s) {
             const int64_t at0 = (int64_t)s * S.S + q;
             const uint32_t fl = S.evf[at0];
             if ((fl & EV_REMOVED) || !(fl & EV_CONTACT)) continue;
-            const int at = atomicAdd(S.npairs, 1);
-            if (at < cap) { out[at].i = i; out[at].j = ent_id(S.oj[at0]) - mb.first; }
+            const int at = atomicAdd(S.npairs, 1) - skip;
+            if (at >= 0 && at < cap) { out[at].i = i; out[at].j = ent_id(S.oj[at0]) - mb.first; }
         }
-    } else {
+    }
+    if constexpr (K == PAIRS_BOND) {
         const int nb = min(S.bcnt_old[f], S.BC);
         for (int q = 0; q < nb; ++q) {
             const BondRec b = S.bond_old[(int64_t)q * S.S + f];
             if (b.j < 0 || b.bond != 1) continue;
-            const int at = atomicAdd(S.npairs, 1);
-            if (at >= cap) continue;
-            PairOut p;
+            const int at = atomicAdd(S.npairs, 1) - skip;
+            if (at < 0 || at >= cap) continue;
+            BondOut p;
             p.i = i; p.j = b.j - mb.first;
             const double v[11] = {(double)b.bond, b.damage, b.deltanb, b.deltatb, b.trb_ji, b.trb_ij, b.rb, b.hb,
                                   b.lb, b.sb, b.ib};
@@ -3169,9 +3170,9 @@ __global__ void k_status(DS S, int nmembers, HostStatus* out) {
 template __global__ void k_read<READ_FLOES>(DS, int, int, int, double*);
 template __global__ void k_read<READ_FORCES>(DS, int, int, int, double*);
 template __global__ void k_read<READ_WALLS>(DS, int, int, int, double*);
-template __global__ void k_pairs<PAIRS_CANDIDATE>(DS, int, int, PairOut*, int);
-template __global__ void k_pairs<PAIRS_CONTACT>(DS, int, int, PairOut*, int);
-template __global__ void k_pairs<PAIRS_BOND>(DS, int, int, PairOut*, int);
+template __global__ void k_pairs<PAIRS_CANDIDATE>(DS, int, int, int, int, PairOut*, int);
+template __global__ void k_pairs<PAIRS_CONTACT>(DS, int, int, int, int, PairOut*, int);
+template __global__ void k_pairs<PAIRS_BOND>(DS, int, int, int, int, BondOut*, int);
 template __global__ void k_sup<false>(DS);
 template __global__ void k_sup<true>(DS);
 template __global__ void k_sup_dense<false>(DS);

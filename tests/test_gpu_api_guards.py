@@ -10,6 +10,7 @@ import numpy as np
 import pytest
 
 from godar_amd import _lib
+from godar_amd import generators as g
 from godar_amd.params import GodarParams
 from workloads import config0_params, kick, packed_box, squeeze
 
@@ -355,3 +356,50 @@ def test_pair_lists_after_the_last_storage_slots_are_freed():
     _same(a, b, mm, mb)
     a.close()
     b.close()
+
+
+def _peak_rss():
+    with open("/proc/self/status") as f:
+        return int(re.search(r"VmHWM:\s+(\d+) kB", f.read()).group(1)) * 1024
+
+
+def test_long_pair_lists_in_parts():
+    """Lists longer than the staging area (524,288 pairs, 43,690 bonds) come in
+    parts: a lattice's candidates, and the bonds and contacts of its
+    neighbours, are those a tree search gives, and the candidate list takes
+    host memory for 8 bytes a pair, not for a bond's state."""
+    from scipy.spatial import cKDTree
+    n, side = 24000, 155
+    rng = np.random.default_rng(8)
+    f = g.config0_member(51, 100)
+    at = rng.permutation(side * side)[:n]
+    f.x, f.y = 2000.0 * (at % side) + 1000.0, 2000.0 * (at // side) + 1000.0
+    f.r, f.h = 1001.0 + rng.uniform(-2, 2, n), rng.uniform(0.8, 1.2, n)
+    f.theta, f.omega, f.u, f.v = np.zeros((4, n))
+    f.box = 2000.0 * side
+    p = config0_params(f, bond_lim=900.0, bond_frac=1.0, rtree=7500.0, ridging=0)
+    ctx = _ctx(n)
+    m = ctx.add_field(p, f)
+    ctx.step(1)
+    pq = cKDTree(np.stack([f.x, f.y], 1)).query_pairs(9000.0, output_type="ndarray")
+    pq = np.sort(pq, axis=1)
+    pq = pq[np.lexsort((pq[:, 1], pq[:, 0]))]
+    dx, dy = f.x[pq[:, 0]] - f.x[pq[:, 1]], f.y[pq[:, 0]] - f.y[pq[:, 1]]
+    d = np.sqrt(dx * dx + dy * dy)
+    gap = d - (f.r[pq[:, 0]] + f.r[pq[:, 1]])
+    want = {"candidate": pq[d <= f.r[pq[:, 0]] + p.rtree], "bond": pq[gap <= p.bond_lim], "contact": pq[gap < 0]}
+    assert len(want["candidate"]) > 524288 and len(want["bond"]) > 43690 and len(want["contact"]) > 10000
+    cnt = ctypes.c_int32()
+    got = np.empty((2, len(want["candidate"])), np.int32)
+    got[:] = 0
+    i32 = ctypes.POINTER(ctypes.c_int32)
+    before = _peak_rss()
+    _lib.check(ctx.h, _lib.load().godar_get_pairs(ctx.h, m, _lib.PAIRS_CANDIDATE, got.shape[1], got[0].ctypes.data_as(i32),
+                                                  got[1].ctypes.data_as(i32), ctypes.byref(cnt)))
+    assert _peak_rss() - before < 24 * got.shape[1]
+    assert cnt.value == got.shape[1]
+    for k, w in want.items():
+        assert np.array_equal(np.stack(ctx.pairs(m, k), 1), w), k
+    assert np.array_equal(got.T, want["candidate"])
+    assert ctx.bond_state(m)["bond"].size == len(want["bond"])
+    ctx.close()
