@@ -32,11 +32,11 @@ template <bool M> __global__ void k_walls(DS);
 template <bool M> __global__ void k_repair(DS, int);
 template <bool M> __global__ void k_fixup(DS);
 template <bool M, bool R> __global__ void k_final(DS);
-__global__ void k_totals(DS, int, int64_t*);
+__global__ void k_totals(DS, int, int, int64_t*);
 __global__ void k_status(DS, int, HostStatus*);
 __global__ void k_admit(DS, int, int, int, int, const FloeRec*, const int32_t*);
 template <int W> __global__ void k_read(DS, int, int, int, double*);
-template <int K> __global__ void k_pairs(DS, int, int, int, int, typename PairKind<K>::Out*, int);
+template <int K> __global__ void k_pairs(DS, int, int, int, int, int, typename PairKind<K>::Out*, int);
 __global__ void k_take_count(int32_t*, int32_t*);
 
 __global__ void k_fill_u8(uint8_t* p, int64_t n, uint8_t v) {
@@ -525,6 +525,14 @@ int read_rows(godar_ctx* c, int32_t m, int rows, double* const* dst) {
     return GODAR_OK;
 }
 
+// Floes per wavefront of the candidate lists (k_totals, k_pairs): with room on
+// the chip fewer, which end sooner.
+int list_floes(int n) {
+    int f = 64;
+    while (f > CAND_MIN_FLOES && n / f < CAND_WAVES) f /= 2;
+    return f;
+}
+
 // Member m's pairs of kind K (PAIRS_*) in order, for a caller with room for
 // `cap` of them; without room only counted.  They come through the staging
 // area, so a list of any length takes no device memory and one host copy: the
@@ -547,7 +555,8 @@ int ordered_pairs(godar_ctx* c, int32_t m, int32_t cap, std::vector<typename Pai
     int n = 0;
     // the pairs of items [b, e): n of them, those from number `skip` on listed
     auto pass = [&](int b, int e, int skip) -> hipError_t {
-        hipLaunchKernelGGL(k_pairs<K>, dim3((e - b + 255) / 256), dim3(256), 0, c->stream, c->d, m, b, e, skip,
+        const int floes = K == PAIRS_CANDIDATE ? list_floes(e - b) : 64;
+        hipLaunchKernelGGL(k_pairs<K>, dim3((e - b + floes - 1) / floes), dim3(64), 0, c->stream, c->d, m, b, e, floes, skip,
                            reinterpret_cast<Out*>(c->stage), room);
         hipLaunchKernelGGL(k_take_count, dim3(1), dim3(1), 0, c->stream, c->d.npairs, &c->status->npairs);
         hipError_t x = hipGetLastError();
@@ -2219,9 +2228,10 @@ int godar_get_totals(godar_ctx* c, int64_t* out) {
     sync_ds(c);
     // (on the context's stream, which the null stream's memset would not wait for)
     hipLaunchKernelGGL(k_zero_i64, dim3(1), dim3(64), 0, c->stream, dout, 5);
-    const int nt = std::max(c->N_pos, c->N_used);      // (a thread per position and storage slot)
+    const int nt = std::max(c->N_pos, c->N_used);      // (positions and storage slots)
+    const int floes = list_floes(nt);
     if (nt > 0)
-        hipLaunchKernelGGL(k_totals, dim3((nt + 255) / 256), dim3(256), 0, c->stream, c->d, c->lists ? c->N_pos : 0, dout);
+        hipLaunchKernelGGL(k_totals, dim3((nt + floes - 1) / floes), dim3(64), 0, c->stream, c->d, c->lists ? c->N_pos : 0, floes, dout);
     hipLaunchKernelGGL(k_member_totals, dim3(1), dim3(256), 0, c->stream, c->d, c->Mcap, dout + 3);
     hipError_t e = hipStreamSynchronize(c->stream);
     if (e == hipSuccess) e = hipMemcpy(out, dout, 3 * sizeof(int64_t), hipMemcpyDeviceToHost);
@@ -2256,9 +2266,10 @@ int godar_get_totals_noalloc(godar_ctx* c, int64_t* out) {
     HIPCHK(c, hipStreamSynchronize(c->stream));
     sync_ds(c);
     hipLaunchKernelGGL(k_zero_i64, dim3(1), dim3(64), 0, c->stream, w, GODAR_NTOTALS);
-    const int nt = std::max(c->N_pos, c->N_used);      // (a thread per position and storage slot)
+    const int nt = std::max(c->N_pos, c->N_used);      // (positions and storage slots)
+    const int floes = list_floes(nt);
     if (nt > 0)
-        hipLaunchKernelGGL(k_totals, dim3((nt + 255) / 256), dim3(256), 0, c->stream, c->d, c->lists ? c->N_pos : 0, w);
+        hipLaunchKernelGGL(k_totals, dim3((nt + floes - 1) / floes), dim3(64), 0, c->stream, c->d, c->lists ? c->N_pos : 0, floes, w);
     hipLaunchKernelGGL(k_queue_totals, dim3(1), dim3(64), 0, c->stream, c->d.qn_next, w + 3);
     hipLaunchKernelGGL(k_member_totals, dim3(1), dim3(256), 0, c->stream, c->d, c->Mcap, w + 6);
     HIPCHK(c, hipGetLastError());
