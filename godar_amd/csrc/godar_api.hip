@@ -1879,8 +1879,10 @@ int build_period(godar_ctx* c, double frac, double* period) {
 // cell span and the dense threshold, one after the other.  Each
 // candidate is priced as a build step plus `4 trial` steps after it: the
 // mean step cost over a build and the steps until the next one,
-// t_step + (t_build - t_step) / period.  The settings stay where they were
-// if no candidate is cheaper.
+// t_step + (t_build - t_step) / period.  (Contacts, bonds and walls are timed as
+// three kernels where other steps launch one; their work does not depend on the
+// search shape, so every candidate's price holds the same excess.)  The
+// settings stay where they were if no candidate is cheaper.
 int tune_search(godar_ctx* c, int trial) {
     const int n = std::max(4, 4 * trial);
     auto stage_sum = [&]() {
@@ -1955,7 +1957,9 @@ int godar_autotune(godar_ctx* c, int32_t trial) {
     for (int st = 0; st < GODAR_NSTAGES; ++st) {
         if (!tunable_stage(st)) continue;
         // (outside steps timed stage by stage, contacts, bonds and walls are
-        // one launch of single-wavefront blocks, whatever their sizes here)
+        // one launch of single-wavefront blocks, whatever their sizes here:
+        // nothing to time)
+        if (st == 4) continue;
         if (st == 5 || st == 7) {
             c->sblock[st] = 64;
             continue;

@@ -403,3 +403,21 @@ def test_long_pair_lists_in_parts():
     assert np.array_equal(got.T, want["candidate"])
     assert ctx.bond_state(m)["bond"].size == len(want["bond"])
     ctx.close()
+
+
+@pytest.mark.parametrize("trial", [1, 3])
+def test_autotune_times_no_stage_that_steps_do_not_launch(trial):
+    """The contact stage's block size is of the steps timed stage by stage
+    alone: no trial steps are spent on it and it stays as set (six stages of
+    three sizes each are timed, and six to eight search shapes: a skin or
+    threshold that was left for a better one is priced again)."""
+    f, p = _box()
+    a = _ctx(f.n)
+    m = a.add_field(p, f)
+    a.set_stage_block(4, 128)
+    a.profile(True)                      # (no launch mode to time)
+    blocks = a.autotune(trial)
+    assert blocks["contacts"] == 128
+    shapes, rest = divmod(a.tstep(m) - 1 - (1 + 3 * trial * 6), 1 + max(4, 4 * trial))
+    assert rest == 0 and 6 <= shapes <= 8
+    a.close()
