@@ -157,7 +157,6 @@ struct godar_ctx {
     double tuned_cost_ms = 0.0;         // the autotuner's price of the chosen search shape
     std::vector<double> rmax;           // largest radius of each member when it was added
     int64_t sup_cap = 0;                // superset pool entries
-    int32_t built_qseg = -1;            // queue share of the last step launched
     // captured graphs of the step with the build kernels, by parity
     hipGraphExec_t gexec[2] = {nullptr, nullptr};
     std::vector<unsigned char> gsig[2];
@@ -800,8 +799,8 @@ std::vector<unsigned char> launch_signature(godar_ctx* c) {
     std::memcpy(p, &c->d, sizeof(DS)); p += sizeof(DS);
     std::memcpy(p, &c->rs, sizeof(RadixScratch)); p += sizeof(RadixScratch);
     std::memcpy(p, c->sblock, sizeof(c->sblock)); p += sizeof(c->sblock);
-    // the dense kernels are launched, and their grid sized, by the members'
-    // dense floe count
+    // whether the dense members' build kernels are launched, and the floes per
+    // wavefront of the search (cand_floes)
     int dense_members = 0, dense_n = 0;
     for (int k = 0; k < c->Mcap; ++k)
         if (c->members[k].active && c->dparams[k].dense) { ++dense_members; dense_n += c->members[k].n; }
@@ -2024,13 +2023,6 @@ int godar_step_async(godar_ctx* c, int32_t nsteps) {
     // many more keep one that speeds up steadily from rest below 0.45
     const int run = (int)std::min<int64_t>(std::max<int64_t>(c->since_build / 5, LEAN_RUN), LEAN_RUN_MAX);
     for (int k = 0; k < nsteps; ++k) {
-        // the queues are laid out by the candidate search's XCD
-        // shares: a new block size or floe count needs a build
-        const int32_t q = qseg_of(c);
-        if (q != c->built_qseg) {
-            force_rebuild(c);
-            c->built_qseg = q;
-        }
         const bool lean = !c->need_full && !c->soon && c->full_hold == 0 && c->lean_run < run;
         int rc = graphs && !lean ? graph_step(c) : launch_step(c, lean);
         if (rc != GODAR_OK) return rc;

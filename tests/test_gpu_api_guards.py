@@ -421,3 +421,29 @@ def test_autotune_times_no_stage_that_steps_do_not_launch(trial):
     shapes, rest = divmod(a.tstep(m) - 1 - (1 + 3 * trial * 6), 1 + max(4, 4 * trial))
     assert rest == 0 and 6 <= shapes <= 8
     a.close()
+
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+def test_block_sizes_change_between_builds(prec):
+    """The work queues are laid out by the search's block size anew in every
+    step, so a size that changes in the middle of a run, on steps with the
+    supersets of an earlier build, changes nothing: the trajectory is that of
+    the sizes left alone, for a dense member beside one that is not."""
+    f, p = _box()
+    dense = kick(squeeze(packed_box(300, 9, box=4.3e4)), 6)
+    pd = config0_params(dense, sigmanc_crit=1e5, rtree=9000.0)
+    out = []
+    for sizes in ((), (128, 256, 64, 192)):
+        a = _ctx(f.n + dense.n, 2, prec)
+        ms = [a.add_field(p, f), a.add_field(pd, dense)]
+        a.step(6)
+        for k in range(4):
+            if sizes:
+                a.set_block(sizes[k])
+            a.step(5)
+        out.append([a.floes(m) for m in ms] + [a.totals()])
+        a.close()
+    for x, y in zip(*out):
+        for k in x:
+            assert np.array_equal(x[k], y[k]), k
+    assert out[0][2]["contacts"] > 0
