@@ -39,10 +39,6 @@ template <int W> __global__ void k_read(DS, int, int, int, double*);
 template <int K> __global__ void k_pairs(DS, int, int, int, int, int, typename PairKind<K>::Out*, int);
 __global__ void k_take_count(int32_t*, int32_t*);
 
-__global__ void k_fill_u8(uint8_t* p, int64_t n, uint8_t v) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
-}
 __global__ void k_fill_i32(int32_t* p, int64_t n, int32_t v) {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = v;
@@ -717,8 +713,7 @@ int launch_step(godar_ctx* c, bool lean) {
     if (!lean) {
         StageTimer t(c, 2);
         hipLaunchKernelGGL(k_ranges, grid_for(N, B[2], false), dim3(B[2]), 0, s, d);
-        // superset build: counts, offsets, entries (k_sup shares k_cand's
-        // grid)
+        // superset build: counts, offsets, entries
         const int ntiles = (N + SCAN_TILE - 1) / SCAN_TILE;
         hipLaunchKernelGGL(k_sup<false>, grid_for(N, B[3], true), dim3(B[3]), 0, s, d);
         if (any_dense) hipLaunchKernelGGL(k_sup_dense<false>, dim3(XCD_COUNT * 1024), dim3(64), 0, s, d);
