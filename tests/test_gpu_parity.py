@@ -19,7 +19,7 @@ import pytest
 
 from fixtures import load, load_long, pairs_at
 from godar_amd import generators as g
-from workloads import config0_params, kick, packed_box, squeeze
+from workloads import clusters, config0_params, kick, packed_box, squeeze
 
 pytestmark = pytest.mark.gpu
 
@@ -1017,3 +1017,35 @@ def test_long_run_error_budget():
           "reference 1-ulp envelope: max", env_max, "median", env_med)
     assert errs["fp64"]["max"] <= env_max
     assert errs["fp64"]["median"] <= env_med
+
+
+@pytest.mark.parametrize("prec,copies", [("fp64", 1), ("fp64", 5), ("mixed", 18), ("fp64", 66), ("mixed", 66)])
+def test_events_launch_matches_separate_kernels(prec, copies):
+    """Contacts, bonds and walls in one launch against the kernels of each that
+    steps timed stage by stage launch, bitwise: 64 packed boxes a member, bonded
+    and in contact at once, at 4,096 floes (more contact blocks than bond blocks)
+    and past the sizes where the wall (16,384 floes), contact (65,536) and bond
+    blocks (262,144) reach their caps and a wavefront takes 64 queued floes."""
+    f = clusters(8, 64, 5)
+    f.x, f.y = f.x - 60.0, f.y - 60.0            # (some floes cross the walls)
+    p = config0_params(f, sigmanc_crit=1e5, bond_lim=50.0, bond_frac=1.0)
+    out = []
+    for prof in (True, False):
+        ctx = _ctx(copies * f.n, copies, prec)
+        ms = [ctx.add_field(p, f) for _ in range(copies)]
+        ctx.profile(prof)
+        ctx.step(8)
+        some = sorted({0, copies // 2, copies - 1})
+        out.append([ctx.totals()] + [ctx.floes(ms[k]) for k in range(copies)] + [ctx.forces(ms[k]) for k in some])
+        out[-1].append({(k, kind, ij): v for k in some for kind in ("contact", "bond")
+                        for ij, v in enumerate(ctx.pairs(ms[k], kind))})
+        ctx.close()
+    for a, b in zip(*out):
+        assert a.keys() == b.keys()
+        for key in a:
+            assert np.array_equal(a[key], b[key]), key
+    one, floes = out[1][0], out[1][1]
+    assert one["contacts"] > 64 * copies and one["bonds"] > 1000 * copies and one["queued_wall"] >= 8 * copies
+    for other in out[1][2:copies + 1]:
+        for key in STATE:
+            assert np.array_equal(other[key], floes[key]), key
