@@ -99,6 +99,13 @@ struct godar_ctx {
     int precision = GODAR_FP64;
     int64_t S = 0;
     int Mcap = 0;
+    // Kept as members come and go, since every launch asks for them: the member
+    // slots up to the last one taken, which is what kernels and read-backs go
+    // over (one member of 1,000 floes in 65,536 slots: 382 -> 29 us a step), the
+    // dense members and their floes.
+    int Mtop = 0;
+    int dense_members = 0;
+    int64_t dense_n = 0;
     int CO = 32, CI = 32, HC = 16, BC = 16;
     int SEEDK = 2, HEAPK = 8;
     int block = 256;
@@ -333,10 +340,7 @@ void force_refresh(godar_ctx* c) {
 static int cand_floes(const godar_ctx* c) {
     const int N = std::max(c->N_used, 1);
     const int64_t slots = (int64_t)CAND_RESIDENT * c->ncu, waves = (N + 63) / 64;
-    int64_t dense = 0;
-    for (int k = 0; k < c->Mcap; ++k)
-        if (c->members[k].active && c->dparams[k].dense) dense += c->members[k].n;
-    if (2 * dense >= N && waves > slots && waves <= CAND_ROUNDS * slots) {
+    if (2 * c->dense_n >= N && waves > slots && waves <= CAND_ROUNDS * slots) {
         const int64_t rounds = (waves + slots - 1) / slots;
         return (int)std::min<int64_t>(64, ((N + rounds * slots - 1) / (rounds * slots) + 3) / 4 * 4);
     }
@@ -416,10 +420,12 @@ constexpr int FULL_HOLD = 64;      // full steps after a lean step found a build
 // word, the steps completed and the members (their step numbers).
 int read_status(godar_ctx* c) {
     sync_ds(c);
-    hipLaunchKernelGGL(k_status, dim3(1), dim3(256), 0, c->stream, c->d, c->Mcap, c->status);
+    const int words = c->Mtop * (int)(sizeof(Member) / sizeof(int32_t));
+    hipLaunchKernelGGL(k_status, dim3(std::min(std::max((words + 255) / 256, 1), 256)), dim3(256), 0, c->stream, c->d,
+                       words, c->status);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    std::memcpy(c->members.data(), c->status->members(), sizeof(Member) * c->Mcap);
+    std::memcpy(c->members.data(), c->status->members(), sizeof(Member) * c->Mtop);
     return GODAR_OK;
 }
 
@@ -695,7 +701,7 @@ int launch_step(godar_ctx* c, bool lean) {
     if (!lean) {
         StageTimer t(c, 0);
         const int nt = std::max({N, c->ncells_cap + 1, NQUEUE * XCD_COUNT});
-        hipLaunchKernelGGL(k_begin, grid_for(nt, B[0], false), dim3(B[0]), 0, s, d, (int)c->Mcap);
+        hipLaunchKernelGGL(k_begin, grid_for(nt, B[0], false), dim3(B[0]), 0, s, d, c->Mtop);
     }
     int bits = 1;
     while ((1u << bits) <= (uint32_t)c->ncells_cap && bits < 32) ++bits;
@@ -703,10 +709,9 @@ int launch_step(godar_ctx* c, bool lean) {
         StageTimer t(c, 1);
         HIPCHK(c, radix_sort_pairs(c->rs, d.ckey, d.cval, N, bits, d.err, d.rebuild, s));
     }
-    int nm = c->Mcap;
+    const int nm = c->Mtop;
     const bool mixed = c->precision == GODAR_MIXED;
-    bool any_dense = false;
-    for (int k = 0; k < c->Mcap; ++k) any_dense |= c->members[k].active && c->dparams[k].dense;
+    const bool any_dense = c->dense_members > 0;
     // (the superset builds of dense members keep 1,024 wavefronts per XCD:
     // they return at once on most steps, and dispatching many more would cost
     // more than they save)
@@ -796,10 +801,7 @@ std::vector<unsigned char> launch_signature(godar_ctx* c) {
     std::memcpy(p, c->sblock, sizeof(c->sblock)); p += sizeof(c->sblock);
     // whether the dense members' build kernels are launched, and the floes per
     // wavefront of the search (cand_floes)
-    int dense_members = 0, dense_n = 0;
-    for (int k = 0; k < c->Mcap; ++k)
-        if (c->members[k].active && c->dparams[k].dense) { ++dense_members; dense_n += c->members[k].n; }
-    int extra[5] = {c->precision, c->Mcap, c->N_used, dense_members, dense_n};
+    int extra[5] = {c->precision, c->Mtop, c->N_used, c->dense_members, (int)c->dense_n};
     std::memcpy(p, extra, sizeof(extra));
     return sig;
 }
@@ -1106,6 +1108,21 @@ void member_search(const godar_ctx* c, DevParams& dp, int n, double rmax, int64_
 // thread span, dense threshold), with cell ranges laid out one after the
 // other; the next step builds the supersets.  Nothing changes if the cell
 // table cannot grow.
+// The counts over the members anew from member m's being there (by 1) or not
+// (-1) and its search shape.
+static void count_member(godar_ctx* c, int m, int by) {
+    const int32_t n = c->members[m].n;
+    if (c->dparams[m].dense) {
+        c->dense_members += by;
+        c->dense_n += by * (int64_t)n;
+    }
+    if (by > 0) {
+        c->Mtop = std::max(c->Mtop, m + 1);
+    } else {
+        while (c->Mtop > 0 && !c->members[c->Mtop - 1].active) --c->Mtop;
+    }
+}
+
 int research_all(godar_ctx* c) {
     int rc = settle(c);
     if (rc != GODAR_OK) return rc;
@@ -1126,6 +1143,10 @@ int research_all(godar_ctx* c) {
     if (rc != GODAR_OK) return rc;
     c->dparams = dps;
     c->cell_n = cn;
+    c->dense_members = 0;
+    c->dense_n = 0;
+    for (int m = 0; m < c->Mcap; ++m)
+        if (c->members[m].active) count_member(c, m, 1);
     rc = upload_tables(c);
     if (rc != GODAR_OK) return rc;
     force_rebuild(c);
@@ -1262,6 +1283,7 @@ int godar_member_add(godar_ctx* c, const godar_params* p, int32_t n, const doubl
     c->members[m].tstep = tstep0;
     c->members[m].active = 1;
     c->members[m].tstop = 0;
+    count_member(c, m, 1);
     c->N_used = std::max<int32_t>(c->N_used, (int32_t)(first + n));
     rc = upload_tables(c);
     if (rc != GODAR_OK) return rc;
@@ -1552,6 +1574,7 @@ int godar_member_remove(godar_ctx* c, int32_t m) {
     hipLaunchKernelGGL(k_fill_i32, dim3((mm.n + 255) / 256), dim3(256), 0, c->stream,
                        c->d.member_of + mm.first, (int64_t)mm.n, -1);
     mm.active = 0;
+    count_member(c, m, -1);
     c->cell_n[m] = 0;
     int32_t hw = 0;
     for (const Member& q : c->members)
@@ -2223,7 +2246,7 @@ int godar_get_totals(godar_ctx* c, int64_t* out) {
     const int floes = list_floes(nt);
     if (nt > 0)
         hipLaunchKernelGGL(k_totals, dim3((nt + floes - 1) / floes), dim3(64), 0, c->stream, c->d, c->lists ? c->N_pos : 0, floes, dout);
-    hipLaunchKernelGGL(k_member_totals, dim3(1), dim3(256), 0, c->stream, c->d, c->Mcap, dout + 3);
+    hipLaunchKernelGGL(k_member_totals, dim3(1), dim3(256), 0, c->stream, c->d, c->Mtop, dout + 3);
     hipError_t e = hipStreamSynchronize(c->stream);
     if (e == hipSuccess) e = hipMemcpy(out, dout, 3 * sizeof(int64_t), hipMemcpyDeviceToHost);
     if (e == hipSuccess) e = hipMemcpy(out + 6, dout + 3, 2 * sizeof(int64_t), hipMemcpyDeviceToHost);
@@ -2262,7 +2285,7 @@ int godar_get_totals_noalloc(godar_ctx* c, int64_t* out) {
     if (nt > 0)
         hipLaunchKernelGGL(k_totals, dim3((nt + floes - 1) / floes), dim3(64), 0, c->stream, c->d, c->lists ? c->N_pos : 0, floes, w);
     hipLaunchKernelGGL(k_queue_totals, dim3(1), dim3(64), 0, c->stream, c->d.qn_next, w + 3);
-    hipLaunchKernelGGL(k_member_totals, dim3(1), dim3(256), 0, c->stream, c->d, c->Mcap, w + 6);
+    hipLaunchKernelGGL(k_member_totals, dim3(1), dim3(256), 0, c->stream, c->d, c->Mtop, w + 6);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipMemcpyAsync(out, w, GODAR_NTOTALS * sizeof(int64_t), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));

@@ -1049,3 +1049,34 @@ def test_events_launch_matches_separate_kernels(prec, copies):
     for other in out[1][2:copies + 1]:
         for key in STATE:
             assert np.array_equal(other[key], floes[key]), key
+
+
+@pytest.mark.parametrize("n,members", [(16, 700), (400, 300), (64, 257)])
+def test_many_members_step_as_alone(n, members):
+    """More members than compute units (every block of the search resets some of
+    them): each takes the steps it takes alone, and so does the last one left in
+    a high slot after the others have gone."""
+    f = kick(squeeze(packed_box(n, 3, box=2.0e4 * np.sqrt(n / 64))), 1)
+    p = config0_params(f, sigmanc_crit=1e5)
+    for prec in ("fp64", "mixed"):
+        a, b = _ctx(n * members, members, prec), _ctx(n, 1, prec)
+        ms, mb = [a.add_field(p, f) for _ in range(members)], b.add_field(p, f)
+        a.step(10)
+        b.step(10)
+        t, want = a.totals(), b.totals()
+        assert want["ridging_seeds"] > 0 and {k: v // members for k, v in t.items()} == want
+        assert all(v % members == 0 for v in t.values())
+        for m in ms[:-1]:
+            if m % 50 == 0:
+                got, alone = a.floes(m), b.floes(mb)
+                for k in STATE:
+                    assert np.array_equal(got[k], alone[k]), (prec, m, k)
+            a.remove(m)
+        a.step(5)
+        b.step(5)
+        got, alone = a.floes(ms[-1]), b.floes(mb)
+        for k in STATE:
+            assert np.array_equal(got[k], alone[k]), (prec, k)
+        assert a.totals() == b.totals() and a.tsteps()[ms[-1]] == b.tstep(mb)
+        a.close()
+        b.close()
