@@ -29,7 +29,7 @@ template <bool M> __global__ void k_contact(DS);
 template <bool M> __global__ void k_bond(DS);
 __global__ void k_stress(DS);
 template <bool M> __global__ void k_walls(DS);
-template <bool M> __global__ void k_repair(DS, int);
+template <bool M> __global__ void k_repair(DS, int, int);
 template <bool M> __global__ void k_fixup(DS);
 template <bool M, bool R> __global__ void k_final(DS);
 __global__ void k_totals(DS, int, int, int64_t*);
@@ -102,8 +102,10 @@ struct godar_ctx {
     // Kept as members come and go, since every launch asks for them: the member
     // slots up to the last one taken, which is what kernels and read-backs go
     // over (one member of 1,000 floes in 65,536 slots: 382 -> 29 us a step), the
-    // dense members and their floes.
+    // members, the largest's floes, the dense ones and their floes.
     int Mtop = 0;
+    int nmembers = 0;
+    int32_t nmax = 0;
     int dense_members = 0;
     int64_t dense_n = 0;
     int CO = 32, CI = 32, HC = 16, BC = 16;
@@ -688,6 +690,18 @@ static dim3 grid_queue(int N, int B) {
     return dim3(std::max(XCD_COUNT, std::min((int)g.x, cap)));
 }
 
+// Whether the repair takes one wavefront a member: with more than two members a
+// CU, other members' work fills the wavefronts that a wide block adds, and
+// blocks of 64 threads with short lists let more members run at once.  (Packed
+// boxes that ridge all at once, narrow against wide: 600 members of 2,000 floes
+// 1,267 and 2,056 us, 2,500 of 300 1,126 and 2,946, 16,384 of 16 304 and 382 and,
+// with lists of 1,024 entries, 327.  256 of 2,000 take 567 and 461; 512 fields of
+// 500 to 8,000 floes that ridge here and there 25.0 and 24.6.)  A member much
+// larger than the others keeps wide blocks: its chain would be the launch's.
+bool repair_narrow(const godar_ctx* c) {
+    return c->nmembers > 2 * c->ncu && (int64_t)c->nmax * c->nmembers <= 8 * (int64_t)c->N_used;
+}
+
 int launch_step(godar_ctx* c, bool lean) {
     DS& d = c->d;
     sync_ds(c);
@@ -764,8 +778,10 @@ int launch_step(godar_ctx* c, bool lean) {
     }
     {
         StageTimer t(c, 8);
-        hipLaunchKernelGGL(mixed ? k_repair<true> : k_repair<false>, dim3(nm), dim3(REPAIR_THREADS),
-                           0, s, d, nm);
+        const bool narrow = repair_narrow(c);
+        const int list = narrow ? REPAIR_LIST_NARROW : REPAIR_LIST;
+        hipLaunchKernelGGL(mixed ? k_repair<true> : k_repair<false>, dim3(nm), dim3(narrow ? 64 : REPAIR_THREADS),
+                           list * REPAIR_ENTRY, s, d, nm, list);
     }
     {
         StageTimer t(c, 9);
@@ -794,14 +810,14 @@ int launch_step(godar_ctx* c, bool lean) {
 std::vector<unsigned char> launch_signature(godar_ctx* c) {
     sync_ds(c);
     std::vector<unsigned char> sig(sizeof(DS) + sizeof(RadixScratch) + sizeof(c->sblock) +
-                                   5 * sizeof(int));
+                                   6 * sizeof(int));
     unsigned char* p = sig.data();
     std::memcpy(p, &c->d, sizeof(DS)); p += sizeof(DS);
     std::memcpy(p, &c->rs, sizeof(RadixScratch)); p += sizeof(RadixScratch);
     std::memcpy(p, c->sblock, sizeof(c->sblock)); p += sizeof(c->sblock);
     // whether the dense members' build kernels are launched, and the floes per
     // wavefront of the search (cand_floes)
-    int extra[5] = {c->precision, c->Mtop, c->N_used, c->dense_members, (int)c->dense_n};
+    int extra[6] = {c->precision, c->Mtop, c->N_used, c->dense_members, (int)c->dense_n, repair_narrow(c)};
     std::memcpy(p, extra, sizeof(extra));
     return sig;
 }
@@ -1112,14 +1128,21 @@ void member_search(const godar_ctx* c, DevParams& dp, int n, double rmax, int64_
 // (-1) and its search shape.
 static void count_member(godar_ctx* c, int m, int by) {
     const int32_t n = c->members[m].n;
+    c->nmembers += by;
     if (c->dparams[m].dense) {
         c->dense_members += by;
         c->dense_n += by * (int64_t)n;
     }
     if (by > 0) {
         c->Mtop = std::max(c->Mtop, m + 1);
+        c->nmax = std::max(c->nmax, n);
     } else {
         while (c->Mtop > 0 && !c->members[c->Mtop - 1].active) --c->Mtop;
+        if (n == c->nmax) {
+            c->nmax = 0;
+            for (int k = 0; k < c->Mtop; ++k)
+                if (c->members[k].active) c->nmax = std::max(c->nmax, c->members[k].n);
+        }
     }
 }
 
@@ -1143,7 +1166,7 @@ int research_all(godar_ctx* c) {
     if (rc != GODAR_OK) return rc;
     c->dparams = dps;
     c->cell_n = cn;
-    c->dense_members = 0;
+    c->nmembers = c->dense_members = 0;
     c->dense_n = 0;
     for (int m = 0; m < c->Mcap; ++m)
         if (c->members[m].active) count_member(c, m, 1);

@@ -29,6 +29,10 @@ constexpr int CAND_MIN_FLOES = 8;
 constexpr int CAND_RESIDENT = 16;          // wavefronts of the search a CU holds (registers, LDS)
 constexpr int CAND_ROUNDS = 4;             // rounds of them up to which the floes are spread evenly
 constexpr int WALL_GRID_WAVES = 256;     // wavefronts of the walls beside contacts and bonds at most
+constexpr int REPAIR_THREADS = 512;
+constexpr int REPAIR_LIST = 1024;          // entries of each list of the repair held in LDS
+constexpr int REPAIR_LIST_NARROW = 256;    // in blocks of one wavefront
+constexpr int REPAIR_ENTRY = 12;           // bytes of one entry of both
 constexpr int FIXUP_GRID_WAVES = 2048;   // wavefronts of the fix-up (about one resident round)
 
 // Per-floe record (96 bytes) by storage slot.  Between builds of the cell

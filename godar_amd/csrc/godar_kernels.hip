@@ -2007,8 +2007,6 @@ __global__ __launch_bounds__(FLOE_BLOCK) void k_walls(DS S) {
 // step; 24 such fields, 320,000 floes, mixed, 0.23-0.9 -> 0.023; 2,501 floes
 // with 50 seeds 0.26 -> 0.027; the 512-field ensemble 0.064 -> 0.026.)
 // ---------------------------------------------------------------------
-constexpr int REPAIR_THREADS = 512;
-constexpr int REPAIR_LIST = 1024;        // entries of each list held in LDS
 constexpr int REPAIR_ROUNDS = 1 << 20;   // (never reached: every round settles one more key)
 
 // slot of partner id g in the outer list of the floe at position kp
@@ -2055,23 +2053,26 @@ __device__ __forceinline__ LaterEvents later_events(const DS& S, int64_t key, in
 }
 
 template <bool MIXED>
-__global__ __launch_bounds__(REPAIR_THREADS) void k_repair(DS S, int nmembers) {
-    __shared__ uint64_t wl[REPAIR_LIST];   // events to evaluate: outer position << 16 | slot
-    __shared__ int cl[REPAIR_LIST];        // records that changed
+__global__ __launch_bounds__(REPAIR_THREADS) void k_repair(DS S, int nmembers, int list) {
+    // events to evaluate (outer position << 16 | slot) and records that
+    // changed, `list` entries of each
+    extern __shared__ __align__(16) unsigned char repair_lds[];
+    uint64_t* wl = reinterpret_cast<uint64_t*>(repair_lds);
+    int* cl = reinterpret_cast<int*>(repair_lds + 8 * (size_t)list);
     __shared__ int nw_, nc_, nn_, rep_, ns_, nt_, first_, nmem_, tstep_;
     __shared__ int64_t mean_;
     __shared__ uint32_t over_;
     // the member's parameters: the physics reads them at LDS latency
     __shared__ uint64_t pbuf[sizeof(DevParams) / 8];
-    static_assert(sizeof(DevParams) % 8 == 0 && sizeof(DevParams) / 8 <= 64, "DevParams copied by lane");
+    static_assert(sizeof(DevParams) % 8 == 0, "DevParams copied in 8-byte words");
     const int m = blockIdx.x;
     const int tid = (int)threadIdx.x, lane = tid & 63;
     if (m >= nmembers) return;
     // (the parameters and the mean superset length of the last build are
     // requested beside the seed count)
-    if (tid >= 64 && tid < 64 + (int)(sizeof(DevParams) / 8))
-        pbuf[tid - 64] = reinterpret_cast<const uint64_t*>(S.params + m)[tid - 64];
-    if (tid == 128) mean_ = 1 + S.sblk[(S.N + SCAN_TILE - 1) / SCAN_TILE] / S.N;
+    for (int i = tid; i < (int)(sizeof(DevParams) / 8); i += (int)blockDim.x)
+        pbuf[i] = reinterpret_cast<const uint64_t*>(S.params + m)[i];
+    if (tid == 63) mean_ = 1 + S.sblk[(S.N + SCAN_TILE - 1) / SCAN_TILE] / S.N;
     // (the error word is read once for the block: all its wavefronts take the
     // barriers below or none does)
     if (tid == 0) {
@@ -2087,13 +2088,13 @@ __global__ __launch_bounds__(REPAIR_THREADS) void k_repair(DS S, int nmembers) {
     __syncthreads();
     const int ns = ns_;
     if (ns == 0) return;
-    // as many wavefronts as the events after the seeds fill (by the mean
-    // superset length of the last build); where the caller allows fewer than
+    // as many of the block's wavefronts as the events after the seeds fill (by
+    // the mean superset length of the last build); where the caller allows fewer than
     // 64 lanes, the first wavefront with those
     const int lanes = min(max(S.repair_lanes, 1), 64);
     int waves = 1;
     if (lanes == 64) {
-        waves = (int)min((int64_t)(REPAIR_THREADS / 64), ((int64_t)ns * mean_ + 63) / 64);
+        waves = (int)min((int64_t)(blockDim.x / 64), ((int64_t)ns * mean_ + 63) / 64);
     }
     const int width = lanes < 64 ? lanes : waves * 64;
     if (tid >= waves * 64) return;
@@ -2105,7 +2106,7 @@ __global__ __launch_bounds__(REPAIR_THREADS) void k_repair(DS S, int nmembers) {
     Reshape* rec = S.shape + (int64_t)S.SEEDK * first;
     const int reccap = S.SEEDK * nmem;
     // lists beyond LDS: the member's share of `heap`, half for each
-    const int cap = min(max(S.repair_cap, 1), REPAIR_LIST);
+    const int cap = min(max(S.repair_cap, 1), list);
     uint64_t* whbm = S.heap + (int64_t)S.HEAPK * first;
     const int hcap = S.HEAPK / 2 * nmem;
     uint64_t* chbm = whbm + hcap;
@@ -2122,7 +2123,7 @@ __global__ __launch_bounds__(REPAIR_THREADS) void k_repair(DS S, int nmembers) {
     // one behind the other once instead of for every floe
     auto touch = [&](int k) {
         const int at = atomicAdd(&nt_, 1);
-        if (at < REPAIR_LIST) wl[at] = (uint64_t)(uint32_t)k;
+        if (at < list) wl[at] = (uint64_t)(uint32_t)k;
         else touch_floe(S, k);
     };
     auto put_change = [&](int p) {
@@ -2390,7 +2391,7 @@ __global__ __launch_bounds__(REPAIR_THREADS) void k_repair(DS S, int nmembers) {
     }
     atomicAdd(&rep_, counted);
     __syncthreads();
-    for (int t = tid; t < min(nt_, REPAIR_LIST); t += waves * 64) touch_floe(S, (int)wl[t]);
+    for (int t = tid; t < min(nt_, list); t += waves * 64) touch_floe(S, (int)wl[t]);
     if (tid == 0) {
         S.stats[4 * m + 2] = ns;
         S.stats[4 * m + 3] = rep_;
@@ -3227,8 +3228,8 @@ template __global__ void k_bond<false>(DS);
 template __global__ void k_bond<true>(DS);
 template __global__ void k_walls<false>(DS);
 template __global__ void k_walls<true>(DS);
-template __global__ void k_repair<false>(DS, int);
-template __global__ void k_repair<true>(DS, int);
+template __global__ void k_repair<false>(DS, int, int);
+template __global__ void k_repair<true>(DS, int, int);
 template __global__ void k_fixup<false>(DS);
 template __global__ void k_fixup<true>(DS);
 template __global__ void k_final<false, false>(DS);

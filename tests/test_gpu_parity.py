@@ -1051,11 +1051,12 @@ def test_events_launch_matches_separate_kernels(prec, copies):
             assert np.array_equal(other[key], floes[key]), key
 
 
-@pytest.mark.parametrize("n,members", [(16, 700), (400, 300), (64, 257)])
+@pytest.mark.parametrize("n,members", [(16, 700), (400, 520), (64, 512), (64, 513)])
 def test_many_members_step_as_alone(n, members):
-    """More members than compute units (every block of the search resets some of
-    them): each takes the steps it takes alone, and so does the last one left in
-    a high slot after the others have gone."""
+    """Two members a compute unit and more (then a wavefront each in the repair, its
+    lists past their room in LDS at 400 ridging floes; every block of the search
+    resets some members): each takes the steps it takes alone, and so does the
+    last one left in a high slot after the others have gone."""
     f = kick(squeeze(packed_box(n, 3, box=2.0e4 * np.sqrt(n / 64))), 1)
     p = config0_params(f, sigmanc_crit=1e5)
     for prec in ("fp64", "mixed"):
