@@ -430,9 +430,10 @@ def main():
     qc, qb = B["totals"]["queued_contact"], B["totals"]["queued_bond"]
     # algorithmic bytes per launch of each stage (partner records are re-reads
     # of other floes' rows and count once, in the floe's own term):
-    #  shelter: x, y, r, hfa, hfw + wind read, 2 minima written, history and
-    #    bond counts read, class written; per candidate pair one list entry
-    #    read on each side, flag and override words written
+    #  candidates: position, radius and identity (4 words) read, class and
+    #    counts written; 24 bytes of entry and flags on either side together for
+    #    each pair that acts (contacts and bonds: the search reads and lists only
+    #    the pairs near enough to matter; those that only shelter come on top)
     #  contacts: queued floe's 11 words read, 5 accumulators + count written;
     #    per contact two list entries read, history (16 B) read and written
     #  bonds: same per queued floe; per bond two list entries read, the
@@ -441,16 +442,15 @@ def main():
     #    written, 2 sheltering minima read; 5 force accumulators per contact
     #    floe; per bond its 10 terms read by each floe (the bond gather)
     per_stage_bytes = {
-        "shelter": nf * (7 * 8 + 2 * 8 + 2 * 4 + 1) + nc * (2 * 8 + 4 + 4),
         "contacts": qc * (11 * 8 + 5 * 8 + 4) + nk * (2 * 8 + 32),
         "bonds": qb * (11 * 8 + 5 * 8 + 4) + nb * (2 * 8 + 2 * 88),
-        "candidates": nf * (4 * 8 + 8) + 24.0 * nc,
+        "candidates": nf * (4 * 8 + 8) + 24.0 * (nk + nb),
         "integrate": nf * (12 * 8 + 6 * 8 + 2 * 8) + qc * 5 * 8 + nb * 2 * 10 * 8,
         "sort": nf * 8.0 * 2 * 3,
-        #  repair: per event re-evaluated, both floes' current properties and
-        #    rows (2 x (48 + 32 + 56) B) and the pair state (40 B history, 88 B
-        #    bond record) read, its 264-byte result written
-        "repair": B["totals"]["repaired_events"] * (2 * (48 + 32 + 56) + 40 + 88 + 264),
+        #  repair: per seed both floes' rows (2 x (32 + 32 + 56) B) read and its
+        #    80-byte record; per event after a reshape its superset entry and
+        #    the partner's position (8 + 32 B)
+        "repair": B["totals"]["ridging_seeds"] * (2 * (32 + 32 + 56) + 80) + B["totals"]["repaired_events"] * (8 + 32),
     }
     # the roofline is the dominant kernel's; a stage without a byte model
     # (fix-up, walls, build) passes the place to the next one

@@ -2064,15 +2064,17 @@ __global__ __launch_bounds__(REPAIR_THREADS) void k_repair(DS S, int nmembers, i
     __shared__ uint32_t over_;
     // the member's parameters: the physics reads them at LDS latency
     __shared__ uint64_t pbuf[sizeof(DevParams) / 8];
-    static_assert(sizeof(DevParams) % 8 == 0, "DevParams copied in 8-byte words");
+    static_assert(sizeof(DevParams) % 8 == 0 && sizeof(DevParams) / 8 <= 64, "DevParams copied by lane");
     const int m = blockIdx.x;
     const int tid = (int)threadIdx.x, lane = tid & 63;
     if (m >= nmembers) return;
     // (the parameters and the mean superset length of the last build are
-    // requested beside the seed count)
-    for (int i = tid; i < (int)(sizeof(DevParams) / 8); i += (int)blockDim.x)
-        pbuf[i] = reinterpret_cast<const uint64_t*>(S.params + m)[i];
-    if (tid == 63) mean_ = 1 + S.sblk[(S.N + SCAN_TILE - 1) / SCAN_TILE] / S.N;
+    // requested beside the seed count, by other wavefronts where the block has
+    // some: by the first one, a microsecond later)
+    const int lastw = (int)(blockDim.x >> 6) - 1;
+    if ((tid >> 6) == min(1, lastw) && lane < (int)(sizeof(DevParams) / 8))
+        pbuf[lane] = reinterpret_cast<const uint64_t*>(S.params + m)[lane];
+    if (tid == 64 * min(2, lastw)) mean_ = 1 + S.sblk[(S.N + SCAN_TILE - 1) / SCAN_TILE] / S.N;
     // (the error word is read once for the block: all its wavefronts take the
     // barriers below or none does)
     if (tid == 0) {

@@ -174,7 +174,8 @@ class Context:
         self._chk(self.L.godar_set_block(self.h, int(threads)))
 
     def set_dense_search(self, floes: int):
-        """Members added afterwards examining >= floes per search list only the pairs that can matter."""
+        """Members added afterwards examining >= floes per search are dense: builds
+        take a wavefront per floe of theirs.  Results do not depend on it."""
         self._chk(self.L.godar_set_dense_search(self.h, int(floes)))
 
     def set_skin(self, frac: float = 0.1):

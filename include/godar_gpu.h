@@ -224,9 +224,11 @@ int godar_set_block(godar_ctx *ctx, int32_t threads);
 int godar_set_stage_block(godar_ctx *ctx, int32_t stage, int32_t threads);
 /* Members added afterwards whose neighbour search examines at least `floes`
  * floes per floe (3x3 cells at their grid's mean density; default 96) are
- * dense: their supersets put the pairs that can come near enough to matter
- * first, and the step's lists hold only those (0: every member, a huge value:
- * none).  Results do not depend on it. */
+ * dense (0: every member, a huge value: none): a build collects the candidates
+ * of each of their floes with a wavefront over cells of half the size in place
+ * of a thread, and the step's search spreads their floes over full rounds of
+ * wavefronts.  The step's lists hold only the pairs near enough to matter,
+ * dense member or not.  Results do not depend on it. */
 int godar_set_dense_search(godar_ctx *ctx, int32_t floes);
 /* Ridging repair: the number of events one wavefront of a member evaluates
  * at once (1-64, default 64; fewer than 64: one wavefront per member) and the
