@@ -528,8 +528,9 @@ __global__ void k_begin(DS S, int nmembers) {
     if (!live) { S.bkey[f] = (uint32_t)S.ncells; return; }
     const DevParams& P = S.params[m];
     double x, y;
-    const GeoRec g = newer ? S.geo[S.pos_of[f]] : GeoRec{};
-    if (newer && g.member >= 0) { x = g.x; y = g.y; }
+    const int pos = newer ? S.pos_of[f] : -1;
+    const GeoRec g = pos >= 0 ? S.geo[pos] : GeoRec{};
+    if (pos >= 0 && g.member >= 0) { x = g.x; y = g.y; }
     else { x = S.rec[f].x; y = S.rec[f].y; }
     int cx = cell_coord(x, P.cell, P.gx), cy = cell_coord(y, P.cell, P.gy);
     S.bkey[f] = (uint32_t)(P.cell_base + cy * P.gx + cx);
@@ -3188,6 +3189,8 @@ __global__ __launch_bounds__(64) void k_admit(DS S, int m, int first, int b, int
     S.nbmin[f] = 0.0f;
     S.dirty[f] = 0;
     S.wnz[f] = 0;                  // (the wall history rows are all +0.0)
+    if (b + t == 0)                // (those of the slot's last member)
+        for (int k = 0; k < 4; ++k) S.stats[4 * m + k] = 0;
 }
 
 // The pair count to the host, and back to 0 for the next list.

@@ -163,8 +163,8 @@ def test_lists_of_a_member_that_left_are_not_walked(n):
     assert mc == ma
     t = a.totals()
     assert (t["candidates"], t["contacts"], t["bonds"]) == tuple(len(of_mate[k][0]) for k in kinds)
-    s = a.stats(mc)
-    assert (s["candidates"], s["contacts"]) == (0, 0)
+    assert set(a.stats(mc).values()) == {0}
+    assert t["ridging_seeds"] == a.stats(mb)["seeds"]
     for k in kinds:
         assert a.pairs(mc, k)[0].size == 0, k
         assert [x.tolist() for x in a.pairs(mb, k)] == of_mate[k], k
