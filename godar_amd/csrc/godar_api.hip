@@ -1806,9 +1806,11 @@ int godar_reserve(godar_ctx* c, int32_t outer, int32_t inner, int32_t histc, int
                 ok(rows(nl.ssb, ol.ssb, sizeof(double), c->CO, nCO)) &&
                 ok(rows(nl.ik, ol.ik, sizeof(int64_t), c->CI, nCI)) &&
                 ok(rows(nl.ibond, ol.ibond, sizeof(int32_t), c->CI, nCI)) &&
-                ok(rows(nl.bterm, ol.bterm, sizeof(BondTerms), c->BC, nBC)) &&
-                ok(rows(nl.hist[o], ol.hist[o], sizeof(HistRec), c->HC, nHC)) &&
-                ok(rows(nl.bond[o], ol.bond[o], sizeof(BondRec), c->BC, nBC));
+                ok(rows(nl.bterm, ol.bterm, sizeof(BondTerms), c->BC, nBC));
+    // (both buffers: stopped members' pair state stands in the two)
+    for (int k = 0; good && k < 2; ++k)
+        good = ok(rows(nl.hist[k], ol.hist[k], sizeof(HistRec), c->HC, nHC)) &&
+               ok(rows(nl.bond[k], ol.bond[k], sizeof(BondRec), c->BC, nBC));
     if (!good) {
         free_lists(nl);
         return fail(c, GODAR_ERR_HIP, std::string("reserve: ") + hipGetErrorString(e));

@@ -556,7 +556,17 @@ __global__ void k_ranges(DS S) {
     if (k >= S.N || *S.err || (!S.rebuild[0] && !S.rebuild[1])) return;
     int f = (int)S.cval[k];
     int m = S.member_of[f];
-    if (m >= 0 && !member_live(S.members[m])) m = -1;
+    if (m >= 0 && !member_live(S.members[m])) {
+        // The first step after a member stopped (and every build): its pair
+        // state into the other buffers too, which no step of its own writes
+        // any more while they go on changing place.
+        m = -1;
+        const int nh = S.hcnt_old[f], nb = S.bcnt_old[f];
+        for (int q = 0; q < nh; ++q) S.hist_new[(int64_t)q * S.S + f] = S.hist_old[(int64_t)q * S.S + f];
+        for (int q = 0; q < nb; ++q) S.bond_new[(int64_t)q * S.S + f] = S.bond_old[(int64_t)q * S.S + f];
+        S.hcnt_new[f] = nh;
+        S.bcnt_new[f] = nb;
+    }
     const FloeRec fr = S.rec[f];
     GeoRec g;
     g.x = fr.x; g.y = fr.y; g.r = fr.r; g.id = S.gid_of[f]; g.member = m;

@@ -447,3 +447,38 @@ def test_block_sizes_change_between_builds(prec):
         for k in x:
             assert np.array_equal(x[k], y[k]), k
     assert out[0][2]["contacts"] > 0
+
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+@pytest.mark.parametrize("extra", [1, 2, 3])
+def test_stopped_members_keep_their_pair_state(extra, prec):
+    """A member that stops keeps the contact histories and bonds of its last
+    step, however many steps the others take after it (the two buffers of the
+    pair state change place every step) and whatever the lists grow to: its
+    checkpoint and bonds stay what they are alone, and when it goes on it takes
+    the steps it takes alone."""
+    f, p = _box()
+    p = config0_params(f, sigmanc_crit=1e5, bond_lim=50.0, bond_frac=0.3)
+    mate = kick(squeeze(packed_box(64, 11)), 4)
+    a, b = _ctx(f.n + mate.n, 2, prec), _ctx(f.n, 1, prec)
+    ma, mb = a.add_field(p, f), b.add_field(p, f)
+    a.add_field(config0_params(mate, sigmanc_crit=1e5), mate)
+    a.run_until(ma, 10)
+    a.step(10)
+    b.step(10)
+    block, bonds = b.checkpoint(mb, p), b.bond_state(mb)
+    for step in range(3):
+        assert a.checkpoint(ma, p) == block, step
+        got = a.bond_state(ma)
+        assert all(np.array_equal(got[k], bonds[k]) for k in bonds)
+        if step == 1:
+            a.reserve(hist=40, bonds=40)
+        if step < 2:
+            a.step(extra)
+    a.run_until(ma, 0)
+    a.step(7)
+    b.step(7)
+    assert a.tstep(ma) == 18
+    _same(a, b, ma, mb)
+    a.close()
+    b.close()
