@@ -183,6 +183,8 @@ struct godar_ctx {
     int32_t builds = 0;
     int64_t since_build = 0;
     int64_t pend_launched = 0;          // steps launched since then
+    // whether each of those records forces: the flag from a step of theirs on
+    std::vector<std::pair<int64_t, int>> pend_record;
     int device = 0;                     // the GPU the context lives on
     int ncu = 256;                      // its compute units
     int64_t* totals_scratch = nullptr;  // device address of that GPU's `scratch`
@@ -463,13 +465,24 @@ int settle(godar_ctx* c) {
         // here, with the build kernels
         HIPCHK(c, hipMemsetAsync(c->d.dirty, 0, c->S, c->stream));
         HIPCHK(c, hipMemsetAsync(c->d.err, 0, sizeof(uint32_t), c->stream));
-        const int64_t left = c->pend_launched - (now - c->pend_done0);
+        const int64_t from = now - c->pend_done0, to = c->pend_launched;
+        std::vector<std::pair<int64_t, int>> flags;
+        flags.swap(c->pend_record);
+        const int record = c->record;
         c->pend_parity = c->parity;
         c->pend_done0 = now;
         c->pend_launched = 0;
         c->need_full = true;
         c->full_hold = FULL_HOLD;
-        rc = godar_step_async(c, (int32_t)std::max<int64_t>(left, 0));
+        for (size_t k = 0; rc == GODAR_OK && k < flags.size(); ++k) {
+            const int64_t a = std::max(flags[k].first, from), b = k + 1 < flags.size() ? flags[k + 1].first : to;
+            if (a >= b) continue;
+            c->record = flags[k].second;
+            c->pend_record.push_back({c->pend_launched, c->record});
+            rc = godar_step_async(c, (int32_t)(b - a));
+        }
+        c->record = record;
+        c->pend_record.push_back({c->pend_launched, record});
         if (rc != GODAR_OK) return rc;
     }
     return GODAR_OK;
@@ -2049,6 +2062,7 @@ int godar_autotune(godar_ctx* c, int32_t trial) {
 int godar_record_forces(godar_ctx* c, int32_t on) {
     if (!c) return GODAR_ERR_ARG;
     c->record = on ? 1 : 0;
+    if (c->pending) c->pend_record.push_back({c->pend_launched, c->record});
     return GODAR_OK;
 }
 
@@ -2059,6 +2073,7 @@ int godar_step_async(godar_ctx* c, int32_t nsteps) {
         c->pend_parity = c->parity;
         c->pending = true;
         c->pend_launched = 0;
+        c->pend_record.assign(1, {0, c->record});
     }
     const bool graphs = c->use_graphs && !c->prof;
     // a run of lean steps ends in a full one that builds early if it must: no

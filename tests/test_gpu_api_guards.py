@@ -482,3 +482,29 @@ def test_stopped_members_keep_their_pair_state(extra, prec):
     _same(a, b, ma, mb)
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("k", [1, 2, 5])
+def test_held_up_steps_record_forces_as_launched(k):
+    """Steps that a missed build held up run again with the force recording
+    they were launched with, whatever it was set to since."""
+    f, p = _box()
+    out = []
+    for sync in (True, False):
+        c = _ctx(f.n)
+        c.set_skin(0.0)
+        m = c.add_field(p, f)
+        c.step(1)
+        for on, n in ((0, k), (1, 1), (0, 3), (1, k), (0, 2)):
+            c.record_forces(bool(on))
+            c.step_async(n)
+            if sync:
+                c.sync()
+        out.append([c.forces(m), c.floes(m)])
+        c.record_forces(True)
+        c.step(1)
+        out[-1] += [c.forces(m), {"t": c.tstep(m)}]
+        c.close()
+    for a, b in zip(*out):
+        for key in a:
+            assert np.array_equal(a[key], b[key]), key
